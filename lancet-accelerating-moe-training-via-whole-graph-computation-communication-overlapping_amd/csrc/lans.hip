@@ -391,17 +391,6 @@ __device__ __forceinline__ void chunk_update(const LansTables& t, const ChunkVie
   }
 }
 
-// sqrt of the sum of a tensor's chunk partials: one wave, lane-strided double sums, xor tree
-// (fixed order, so every caller gets the same bits).  get(c) returns the partial of chunk c.
-template <typename Get>
-__device__ __forceinline__ float wave_norm(int lo, int hi, Get get) {
-  double acc = 0.0;
-  for (int c = lo + lane_id(); c < hi; c += kWave) acc += static_cast<double>(get(c));
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kWave);
-  return static_cast<float>(sqrt(acc));
-}
-
 // =======================================================================================
 // schedule "sweeps": three launches + two per-tensor reductions
 // =======================================================================================
@@ -455,18 +444,36 @@ __global__ __launch_bounds__(kLansThreads) void lans_norm_g_kernel(LansTables t,
   if (threadIdx.x == 0) t.partial[chunk] = sg;
 }
 
-// per-tensor sqrt(sum of chunk partials) (cleanup, multi_tensor_lans.cu:169-185)
-// split: partial sums per chunk (1 after the sweep over g, kSweepSplit after the moments sweep)
-__global__ __launch_bounds__(kLansThreads) void lans_reduce_kernel(LansTables t, int first_norm, int tensor_base,
-                                                                   int tensor_end, int count, int split) {
+// per-tensor sqrt(sum of chunk partials) (cleanup, multi_tensor_lans.cu:169-185): one workgroup per tensor and norm.
+// split: partial sums per chunk (1 after the sweep over g, kSweepSplit after the moments sweep).
+// Bound by load latency alone: a tensor of 20M parameters has 19544 partials per norm after the moments sweep.  A
+// workgroup of 1024 threads keeps kReduceBatch loads in flight per thread: 10 us for the three norms of that tensor
+// (4 us for the 2443 partials of its g), where one wave per tensor, one load at a time, took 220 us (12 us).
+constexpr int kReduceThreads = 1024;
+constexpr int kReduceBatch = 8;
+__global__ __launch_bounds__(kReduceThreads) void lans_reduce_kernel(LansTables t, int first_norm, int tensor_base, int split) {
   if (step_is_skipped(t)) return;  // the norms of the last step that ran stay
-  const int tensor = tensor_base + blockIdx.x * (kLansThreads / kWave) + threadIdx.x / kWave;
-  if (tensor >= tensor_end) return;
-  const int lo = t.tensor_first[tensor], hi = lo + t.tensor_chunks[tensor];
-  for (int k = 0; k < count; ++k) {
-    const float* part = t.partial + static_cast<size_t>(k) * t.nchunks * split;
-    const float n = wave_norm(lo * split, hi * split, [&](int c) { return part[c]; });
-    if (lane_id() == 0) t.norms[(first_norm + k) * t.T + tensor] = n;
+  __shared__ double s_sum[kReduceThreads / kWave];
+  const int tensor = tensor_base + static_cast<int>(blockIdx.x), k = blockIdx.y;
+  const float* part = t.partial + static_cast<size_t>(k) * t.nchunks * split + static_cast<size_t>(t.tensor_first[tensor]) * split;
+  const int n = t.tensor_chunks[tensor] * split;
+  double acc = 0.0;  // fixed order: every run gets the same bits
+  for (int c = threadIdx.x; c < n; c += kReduceBatch * kReduceThreads) {
+    float x[kReduceBatch];
+#pragma unroll
+    for (int j = 0; j < kReduceBatch; ++j) x[j] = c + j * kReduceThreads < n ? part[c + j * kReduceThreads] : 0.f;
+#pragma unroll
+    for (int j = 0; j < kReduceBatch; ++j) acc += static_cast<double>(x[j]);
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kWave);
+  if (lane_id() == 0) s_sum[threadIdx.x / kWave] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < kReduceThreads / kWave; ++w) sum += s_sum[w];
+    t.norms[(first_norm + k) * t.T + tensor] = static_cast<float>(sqrt(sum));
   }
 }
 
@@ -769,8 +776,8 @@ __device__ __noinline__ void regather(const uint64_t* part_word, int nchunks, ui
   }
 }
 
-// wave_norm over nc <= kMaxResidentChunks sums in LDS: the same additions in the same order (a sum that is not
-// there counts as +0, which changes no bit of a sum of squares), with all of a lane's reads issued at once.
+// sqrt of the sum of nc <= kMaxResidentChunks chunk sums in LDS: one wave, lane-strided double sums, xor tree (a fixed
+// order, so every workgroup gets the same bits), with all of a lane's reads issued at once.
 __device__ __forceinline__ float wave_norm_lds(const float* part, int nc) {
   float x[kMaxResidentChunks / kWave];
 #pragma unroll
@@ -800,7 +807,7 @@ __device__ __forceinline__ void forget(f32x4 (&a)[kVecPerThread], f32x4 (&b)[kVe
 //
 // Norms.  Every workgroup publishes the sums of its chunks (one word for stage N, three for stage M) and
 // every workgroup forms the norms it needs itself, from the published sums of all the tensor's chunks, in
-// the fixed order of wave_norm: they all get the same bits, nobody waits for a workgroup in charge, and the
+// the fixed order of wave_norm_lds: they all get the same bits, nobody waits for a workgroup in charge, and the
 // workgroup that is behind the others has no more to do than they.  A tensor has at most
 // kMaxResidentChunks chunks: kGatherPerThread words per thread and norm.
 //
@@ -1399,14 +1406,13 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   }
   const int nsweep = t.nchunks - chunk_base;
   if (nsweep > 0) {
-    const int per_block = kLansThreads / kWave;
-    const int rblocks = (T - tensor_base + per_block - 1) / per_block;
+    const int rest = T - tensor_base;
     if (!grad_norms) {
       LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_norm_g_kernel<GT><<<nsweep, kLansThreads, 0, st>>>(t, chunk_base)))
-      lans_reduce_kernel<<<rblocks, kLansThreads, 0, st>>>(t, 0, tensor_base, T, 1, 1);
+      lans_reduce_kernel<<<dim3(rest, 1), kReduceThreads, 0, st>>>(t, 0, tensor_base, 1);
     }
     LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_moments_kernel<GT><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, chunk_base)))
-    lans_reduce_kernel<<<rblocks, kLansThreads, 0, st>>>(t, 1, tensor_base, T, 3, kSweepSplit);
+    lans_reduce_kernel<<<dim3(rest, 3), kReduceThreads, 0, st>>>(t, 1, tensor_base, kSweepSplit);
     LANS_TYPE_SWITCH(g_dtype, plt, (lans_update_kernel<GT, PL><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, chunk_base)))
   }
   return static_cast<int>(hipGetLastError());

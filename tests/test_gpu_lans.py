@@ -523,3 +523,21 @@ def test_stepper_keeps_master_weights_for_a_16_bit_model(pkg):
         for a, master in zip(ref_p, opt.master):
             assert_close_scaled(to_np(master), a, 2e-6, "master parameter")
             a[...] = to_np(master)
+
+
+def test_lans_norms_of_tensors_with_many_partial_sums(pkg):
+    """Norms of tensors whose per-chunk sums are one less than, as many as and one more than a workgroup of the reduction
+    reads at a time (8 x 1024 of the moments sweep, 1024 chunks), and more than it reads in one go.  A chunk's sum is
+    formed in fp32 from at most 40 roundings per term, half of which a square root keeps: 1.2e-6."""
+    capi = pkg.capi
+    numels = [1023 * 8192, 1024 * 8192, 1024 * 8192 + 1, 2100 * 8192 + 77]
+    state = _fresh_state(numels, 17)
+    before = [t.double() for t in state[1]]
+    plan = pkg.ops.LansPlan(numels, schedule=capi.LANS_SWEEPS)
+    plan.step(*state, 1, capi.LansHyper(1e-3, 0.9, 0.999, 1e-6, 1, 0.01, 1, 1, 1))
+    norms = plan.norms().double()
+    for i in range(len(numels)):
+        for k, t in ((0, state[0][i].double()), (1, before[i])):
+            want = float(t.norm())
+            assert abs(float(norms[k, i]) - want) <= 1.2e-6 * want
+    plan.close()
