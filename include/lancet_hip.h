@@ -402,14 +402,17 @@ int lancet_lans_step_mixed(lancet_lans_plan_t plan, const void* const* g, int g_
  * replay is a new step.  The pointer tables are uploaded (one host-to-device copy) by the first call that
  * sees a new set of pointers: make that call once before recording. */
 /* Schedules of the step.
- * LANCET_LANS_RESIDENT (what a new plan has when at least one tensor fits it): one persistent kernel that
+ * LANCET_LANS_RESIDENT (what a new plan has when at least one tensor fits it: at most the capacity in chunks, and either whole chunks
+ * or more than two): one persistent kernel that
  * reads and writes every array once (28 B/param).  Each workgroup runs a three-stage pipeline over chunks of
  * 8192 parameters (sum of g^2 / moments and the two updates / parameter write) and keeps a chunk on chip
  * between the stages; it publishes the sums of its chunks and forms the norms it needs from the published
- * sums of all the tensor's chunks.  The kernel takes the tensors that are whole multiples of 8192
- * parameters and have at most lancet_lans_plan_resident_capacity() chunks; the other tensors of the plan
- * take the three sweeps in the same step, and so does every tensor of a step in which an array of a tensor
- * the kernel would take is not 16-byte aligned.
+ * sums of all the tensor's chunks.  The kernel takes the tensors of at most
+ * lancet_lans_plan_resident_capacity() chunks (the last chunk of a tensor may be a partial one); larger tensors of the
+ * plan take the three sweeps in the same step, and so does every tensor of a step in which an array of a tensor
+ * the kernel would take is not 16-byte aligned (and every tensor that is not a multiple of 8192 parameters of a step
+ * with eps < 1e-30).  Tensors of at most two chunks that are not whole chunks are updated by one workgroup each, under
+ * either schedule.
  * Contract of this schedule: its workgroups wait for one another (for chunks of the same tensor only), so
  * at least half of them must be running on the device at the same time.  The grid is sized to what an
  * otherwise idle device runs at once; other kernels on the device delay the step until enough of its

@@ -5,7 +5,7 @@
 //   phase M  reads g, p, m, v      -> writes m, v; per-chunk sums of p^2, u_m^2 and u_g^2
 //   phase U  reads g, p, m, v      -> recomputes u_m, u_g (never stored) and writes p
 // and two schedules:
-//   * sweeps: three plain launches + two tiny per-tensor reductions.  Real HBM traffic
+//   * sweeps: three plain launches + two short per-tensor reductions.  Real HBM traffic
 //     is 48 B/param (g read three times, p, m, v twice).  No workgroup waits for another.
 //   * resident (what a new plan runs): ONE persistent kernel in which every array is read once and written
 //     once (28 B/param).  A workgroup runs a three-stage software pipeline over the chunks it draws from a
@@ -22,7 +22,10 @@
 //     chunks of a tensor are drawn in the same pipeline iteration.  A workgroup waits only for chunks of
 //     tensors it holds, chunks are drawn in order, and a workgroup holds at most two chunks that have not
 //     passed stage M: the kernel drains as long as half as many workgroups as the largest tensor has
-//     chunks are running.  Larger tensors go through the sweeps in the same step.  Waits are bounded; a
+//     chunks are running.  Larger tensors go through the sweeps in the same step, and those of at most two chunks
+//     through one workgroup each of the step's first kernel.  A tensor need not be whole chunks: the last one is
+//     accessed through a bounds-checked buffer descriptor (40M parameters in 34 tensors that are multiples of
+//     nothing: 224 us, 325 us in the sweeps; 2M in 30: 42 and 43 us; nowhere slower).  Waits are bounded; a
 //     wait that gives up poisons what it would have fed, so that no parameter is written from an unknown
 //     norm, and raises a sticky error the next step reports.
 // Work is cut into fixed-size chunks described by device-resident tables built once per
@@ -61,10 +64,11 @@ struct LansTables {
   const int64_t* numel;        // [T]
   const int32_t* chunk_tensor; // [nchunks] tensor of a chunk slot, -1 = padding slot of a round
   const int32_t* tensor_first; // [T] first chunk slot of each tensor (its chunks are consecutive)
+  const int32_t* res_tensor;   // [nres] tensor of a slot the resident kernel hands out, -1 = padding slot of a round
+  const int32_t* res_first;    // [T] first of those slots of each tensor the resident kernel takes
   const int32_t* tensor_chunks;// [T] chunks of each tensor
   float* partial;              // [3][nchunks * kSweepSplit]  (sweeps: one sum per slice)
-  uint64_t* part_word;         // [4][nchunks]      (resident schedule: tag | fp32 sum of squares)
-  uint64_t* norm_word;         // [4][T]            (resident schedule: tag | fp32 norm)
+  uint64_t* part_word;         // [4][res_stride]   (resident schedule: tag | fp32 sum of squares)
   uint32_t* ctl;               // control words, see kCtl*
   uint32_t* host_status;       // device view of a pinned host word: set with the error word, read by the next step
   float* norms;                // [4][T]: g, p, u_m, u_g
@@ -73,7 +77,8 @@ struct LansTables {
   const float* grad_norms;     // [T] ||g|| per tensor in the caller's order, or null: computed by the step
   int T;
   int nchunks;                 // chunk slots, padding included
-  int nres;                    // slots [0, nres) are handed out by the resident kernel
+  int nres;                    // slots the resident kernel hands out in this step
+  int res_stride;              // slots it can hand out
   uint32_t debug_flags;        // bit 0: nothing is published (exercises the bounded waits); bit 1 is the host's
 };
 
@@ -186,14 +191,22 @@ __device__ __forceinline__ LansElem make_elem(const LansScalars& sc, float gn, f
 
 // bias corrections 1 - beta^step (src/op/dialect/cuda/lans.cc:108-113), from a host step or
 // from the fp32 step scalar in device memory (no host synchronisation, unlike lans.cc:102-107)
+// (The powers by repeated squaring in double: at most 62 products, 1e-14 relative, where the float result has 6e-8;
+// the general pow takes several microseconds on its one lane, which every step waits for.)
 __device__ __forceinline__ void bias_corrections(const LansScalars& sc, float& bc1, float& bc2) {
   int step = sc.step_host;
   if (sc.step_dev) step = static_cast<int>(*sc.step_dev);
   bc1 = 1.f;
   bc2 = 1.f;
   if (sc.bias_correction) {
-    bc1 = static_cast<float>(1.0 - pow(static_cast<double>(sc.beta1), step));
-    bc2 = static_cast<float>(1.0 - pow(static_cast<double>(sc.beta2), step));
+    double b1 = sc.beta1, b2 = sc.beta2, p1 = 1.0, p2 = 1.0;
+    if (step < 0) b1 = 1.0 / b1, b2 = 1.0 / b2;
+    for (uint32_t n = static_cast<uint32_t>(step < 0 ? -static_cast<int64_t>(step) : step); n != 0u; n >>= 1) {
+      if (n & 1u) p1 *= b1, p2 *= b2;
+      b1 *= b1, b2 *= b2;
+    }
+    bc1 = static_cast<float>(1.0 - p1);
+    bc2 = static_cast<float>(1.0 - p2);
   }
 }
 
@@ -402,13 +415,6 @@ __device__ __forceinline__ bool step_is_skipped(const LansTables& t) {
   return __builtin_amdgcn_readfirstlane(static_cast<int>(ld_agent(t.ctl + kCtlSkip))) != 0;
 }
 
-__global__ void lans_prepare_kernel(LansTables t, LansScalars sc) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    t.ctl[kCtlSkip] = ld_agent(t.ctl + kCtlError) != 0u ? 1u : 0u;
-    bias_corrections(sc, t.consts[0], t.consts[1]);
-  }
-}
-
 // The sweeps hand every chunk to kSweepSplit workgroups (a slice of kLansChunk / kSweepSplit elements each:
 // one float4 per thread and array).  Short workgroups in address order stream a few percent faster than
 // workgroups that loop over a whole chunk; the chunk stays the unit of the tables and of the resident kernel.
@@ -505,13 +511,6 @@ __global__ __launch_bounds__(kLansThreads) void lans_update_kernel(LansTables t,
   chunk_update<GT, PL>(t, c, el, sc, t.norms[1 * t.T + c.tensor], t.norms[2 * t.T + c.tensor], t.norms[3 * t.T + c.tensor]);
 }
 
-// ||g|| per tensor supplied by the caller (in the order of its lists) instead of the sweep over g
-__global__ void lans_take_grad_norms_kernel(LansTables t) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (step_is_skipped(t)) return;
-  if (i < t.T) t.norms[i] = t.grad_norms[t.order[i]];
-}
-
 // norms live in the plan's tensor order; callers get them in the order of their lists
 __global__ void lans_gather_norms_kernel(LansTables t, float* dst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -592,13 +591,13 @@ struct Slot {
   int tensor;  // -1: padding slot, nothing to do
   int dead;    // stage M was skipped (||g|| unknown): the parameters stay as they are
   int lo, nc;  // first chunk slot and number of chunks of the tensor
+  int n;       // elements in the chunk
   int64_t begin;
   __device__ __forceinline__ bool real() const { return chunk >= 0 && tensor >= 0; }
 };
 
-// The resident kernel only takes whole chunks of 16-byte aligned arrays (the plan leaves tensors that are not a
-// multiple of the chunk to the sweeps; a step whose pointers are not aligned runs as sweeps altogether): every
-// access is an unconditional, non-temporal float4.
+// The resident kernel only takes 16-byte aligned arrays (a step whose pointers are not aligned runs as sweeps
+// altogether): every access is an unconditional, non-temporal float4.
 // A table entry (tensor pointers, chunk tables) read as constant memory: nothing writes the tables while a
 // kernel runs, and said this way the read goes through the scalar unit and its result stays in scalar
 // registers.  A plain read behind the kernel's own stores has to assume they changed the table, takes the
@@ -608,27 +607,68 @@ __device__ __forceinline__ T ld_table(const T* p) {
   return *(const __attribute__((address_space(4))) T*)(p);
 }
 
+// A chunk of one array as a buffer: accesses carry a byte offset per lane and the hardware compares it with the size,
+// so that what lies past the tensor's end reads as zero and is not written, dword by dword.  The last chunk of a tensor
+// thereby takes the same straight-line code as a whole one: zeros for g, p, m and v make zero moments and updates (the
+// host sees to it that eps is not so small that 0 / eps is no number) and add nothing to any sum.
+typedef __amdgpu_buffer_rsrc_t ChunkBuf;
+constexpr int kBufNonTemporal = 2;  // cache policy bits of a buffer access
+template <typename T>
+__device__ __forceinline__ ChunkBuf chunk_buf(const T* a, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(static_cast<const void*>(a)), 0, bytes, 0x00027000);
+}
 // float4 k of a thread: the wave's quarter of the chunk starts lane_offset() elements into it, float4 k lies
-// k * 256 elements further on (one load instruction of a wave covers 1 KB of consecutive memory).  The
-// address is a uniform 64-bit base plus an unsigned 32-bit offset per lane, the form that takes its base
-// from scalar registers and one vector register for the offset.
+// k * 256 elements further on (one load instruction of a wave covers 1 KB of consecutive memory).
 __device__ __forceinline__ uint32_t lane_offset(int wave) {
   return static_cast<uint32_t>(wave * (kLansChunk / kWavesPerTile) + 4 * fresh_lane());
 }
-__device__ __forceinline__ f32x4 ld_chunk4(const LANCET_GLOBAL float* a, int k, int wave) {
-  return __builtin_nontemporal_load((const LANCET_GLOBAL f32x4*)(a + k * (4 * kWave) + lane_offset(wave)));
+__device__ __forceinline__ f32x4 ld_chunk4(ChunkBuf a, int k, int wave) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a, 4u * lane_offset(wave) + k * (16 * kWave), 0, kBufNonTemporal));
 }
-__device__ __forceinline__ void st_chunk4(LANCET_GLOBAL float* a, int k, f32x4 x, int wave) {
-  __builtin_nontemporal_store(x, (LANCET_GLOBAL f32x4*)(a + k * (4 * kWave) + lane_offset(wave)));
+__device__ __forceinline__ void st_chunk4(ChunkBuf a, int k, f32x4 x, int wave) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), a, 4u * lane_offset(wave) + k * (16 * kWave), 0, kBufNonTemporal);
 }
-// the same four elements of a gradient chunk in its own type, as fp32, and of the 16-bit parameter copy
+// the same four elements of a gradient chunk in its own type (two 16-bit elements are one dword: the one that holds the
+// last element of an odd-sized tensor is read whole, see mask_odd_grad)
 template <int GT>
-__device__ __forceinline__ typename Grad<GT>::R ld_grad4(const LANCET_GLOBAL typename Grad<GT>::S* a, int k, int wave) {
-  return Grad<GT>::ldr4(a + k * (4 * kWave) + lane_offset(wave));
+__device__ __forceinline__ ChunkBuf grad_buf(const void* g, int64_t begin, int n) {
+  typedef typename Grad<GT>::S S;
+  return chunk_buf(static_cast<const S*>(g) + begin, (static_cast<uint32_t>(n) * static_cast<uint32_t>(sizeof(S)) + 3u) & ~3u);
 }
+template <int GT>
+__device__ __forceinline__ typename Grad<GT>::R ld_grad4(ChunkBuf a, int k, int wave) {
+  typedef typename Grad<GT>::R R;
+  if constexpr (GT == LANCET_F32) return __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b128(a, 4u * lane_offset(wave) + k * (16 * kWave), 0, kBufNonTemporal));
+  else return __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b64(a, 2u * lane_offset(wave) + k * (8 * kWave), 0, kBufNonTemporal));
+}
+// 16-bit gradients of a chunk with an odd number n of elements: the dword of the last one also holds two bytes that
+// are not the tensor's; they count as zero
+template <int GT>
+__device__ __forceinline__ void mask_odd_grad(typename Grad<GT>::R (&g)[kVecPerThread], int n, int wave) {
+  if constexpr (GT != LANCET_F32) {
+#pragma unroll
+    for (int k = 0; k < kVecPerThread; ++k) {
+      const uint32_t e = lane_offset(wave) + k * (4 * kWave);
+      if (e == static_cast<uint32_t>(n - 1)) g[k].x &= 0xffffu;
+      if (e + 2 == static_cast<uint32_t>(n - 1)) g[k].y &= 0xffffu;
+    }
+  }
+}
+// the 16-bit copy of four new parameters: whole dwords through the buffer, the last element of an odd-sized chunk (its
+// dword's other half belongs to somebody else) on its own
 template <int PL>
-__device__ __forceinline__ void st_lowp_chunk4(LANCET_GLOBAL uint16_t* a, int k, f32x4 x, int wave) {
-  st_lowp4<PL>(a + k * (4 * kWave) + lane_offset(wave), x);
+__device__ __forceinline__ void st_lowp_chunk4(ChunkBuf a, LANCET_GLOBAL uint16_t* pl, int n, int k, f32x4 x, int wave) {
+  if constexpr (PL != kNoLowp) {
+    u32x2 y;
+    y.x = (f32_to_half<PL>(x.x) & 0xffffu) | (f32_to_half<PL>(x.y) << 16);
+    y.y = (f32_to_half<PL>(x.z) & 0xffffu) | (f32_to_half<PL>(x.w) << 16);
+    __builtin_amdgcn_raw_buffer_store_b64(y, a, 2u * lane_offset(wave) + k * (8 * kWave), 0, kBufNonTemporal);
+    if (UNLIKELY((n & 1) != 0)) {
+      const uint32_t e = lane_offset(wave) + k * (4 * kWave);
+      if (e == static_cast<uint32_t>(n - 1)) pl[n - 1] = static_cast<uint16_t>(y.x);
+      if (e + 2 == static_cast<uint32_t>(n - 1)) pl[n - 1] = static_cast<uint16_t>(y.y);
+    }
+  }
 }
 
 // Thread 0: publishes the N chunk sums a[] of slot s as words first .. first+N-1 (fire and forget).
@@ -638,12 +678,12 @@ __device__ __forceinline__ void publish(const LansTables& t, const LansScalars& 
   if (t.debug_flags & 1u) return;  // test hook: nothing is ever published, every wait runs into its bound
   const uint32_t tag = sc.epoch | (poison ? kPoison : 0u);
 #pragma unroll
-  for (int k = 0; k < N; ++k) st_word(t.part_word + static_cast<size_t>(first + k) * t.nchunks + s.chunk, tag, a[k]);
+  for (int k = 0; k < N; ++k) st_word(t.part_word + static_cast<size_t>(first + k) * t.res_stride + s.chunk, tag, a[k]);
 }
 
 // the partials of one norm of slot s's tensor as this thread reads them (issued, not yet looked at)
 __device__ __forceinline__ void gather_issue(const LansTables& t, int kind, const Slot& s, uint64_t (&word)[kGatherPerThread], int wave) {
-  const uint64_t* src = t.part_word + static_cast<size_t>(kind) * t.nchunks + s.lo;
+  const uint64_t* src = t.part_word + static_cast<size_t>(kind) * t.res_stride + s.lo;
 #pragma unroll
   for (int i = 0; i < kGatherPerThread; ++i) {
     const int c = fresh_tid(wave) + i * kLansThreads;
@@ -674,9 +714,10 @@ template <int PAR, int GT>
 __device__ __forceinline__ void moments_chunk(const LansTables& t, const Slot& s, const LansElem& el,
                                               const typename Grad<GT>::R (&g)[kVecPerThread], f32x4 (&um)[kVecPerThread],
                                               f32x4 (&ug)[kVecPerThread], PipeShared& sh, float (&a)[3], uint32_t ticket, int wave) {
-  const LANCET_GLOBAL float* p = as_global(ld_table(t.p + s.tensor) + s.begin);
-  LANCET_GLOBAL float* m = as_global(ld_table(t.m + s.tensor) + s.begin);
-  LANCET_GLOBAL float* v = as_global(ld_table(t.v + s.tensor) + s.begin);
+  const uint32_t bytes = 4u * static_cast<uint32_t>(s.n);
+  const ChunkBuf p = chunk_buf(ld_table(t.p + s.tensor) + s.begin, bytes);
+  const ChunkBuf m = chunk_buf(ld_table(t.m + s.tensor) + s.begin, bytes);
+  const ChunkBuf v = chunk_buf(ld_table(t.v + s.tensor) + s.begin, bytes);
   float a0 = 0.f, a1 = 0.f, a2 = 0.f;
   // kPrefetch float4 of each array are in flight ahead of the one being worked on
   f32x4 np[kPrefetch], nm[kPrefetch], nv[kPrefetch];
@@ -733,7 +774,7 @@ __device__ __forceinline__ void moments_chunk(const LansTables& t, const Slot& s
 // that kind; lo_g / lo_u: first chunk slot of the tensor whose g sums / whose other sums are gathered) until
 // they are all there, or until the bound.  A function of its own on purpose: it runs rarely, is full of
 // loops, and inlined it misleads the register allocation of the straight-line code around it.
-__device__ __noinline__ void regather(const uint64_t* part_word, int nchunks, uint32_t* ctl, uint32_t* host_status,
+__device__ __noinline__ void regather(const uint64_t* part_word, int stride, uint32_t* ctl, uint32_t* host_status,
                                       uint32_t epoch, uint32_t spin_limit, int lo_g, int lo_u, uint32_t missing,
                                       PipeShared* shp, int wave) {
   PipeShared& sh = *shp;
@@ -761,7 +802,7 @@ __device__ __noinline__ void regather(const uint64_t* part_word, int nchunks, ui
       const int bit = __builtin_ctz(left);
       const int kind = bit / kGatherPerThread;
       const int c = fresh_tid(wave) + (bit % kGatherPerThread) * kLansThreads;
-      const uint64_t x = ld_word(part_word + static_cast<size_t>(kind) * nchunks + (kind == 0 ? lo_g : lo_u) + c);
+      const uint64_t x = ld_word(part_word + static_cast<size_t>(kind) * stride + (kind == 0 ? lo_g : lo_u) + c);
       if (word_is_current(x, epoch)) {
         missing &= ~(1u << bit);
         sh.part[kind][c] = __uint_as_float(static_cast<uint32_t>(x));
@@ -892,11 +933,13 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
     s3.tensor = -1;
     s3.dead = 0;
     if (s3.chunk >= 0) {
-      s3.tensor = ld_table(t.chunk_tensor + s3.chunk);
+      s3.tensor = ld_table(t.res_tensor + s3.chunk);
       if (s3.tensor >= 0) {
-        s3.lo = ld_table(t.tensor_first + s3.tensor);
+        s3.lo = ld_table(t.res_first + s3.tensor);
         s3.nc = ld_table(t.tensor_chunks + s3.tensor);
         s3.begin = static_cast<int64_t>(s3.chunk - s3.lo) * kLansChunk;
+        const int64_t left = ld_table(t.numel + s3.tensor) - s3.begin;
+        s3.n = static_cast<int>(left < kLansChunk ? left : kLansChunk);
       }
     }
   }
@@ -904,8 +947,7 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
   // the sums other workgroups have published: read as late as possible, and still back before anything waits
   // for them alone
   if (LIKELY(s3.real())) {
-    typedef typename Grad<GT>::S GS;
-    const LANCET_GLOBAL GS* src = as_global(static_cast<const GS*>(ld_table(t.g + s3.tensor)) + s3.begin);
+    const ChunkBuf src = grad_buf<GT>(ld_table(t.g + s3.tensor), s3.begin, s3.n);
 #pragma unroll
     for (int k = 0; k < kVecPerThread; ++k) g[k] = ld_grad4<GT>(src, k, wave);
   }
@@ -916,6 +958,7 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
   if (LIKELY(need_g)) gather_issue(t, 0, s2, words_g, wave);
   if (LIKELY(s3.real())) {
     float a = 0.f;
+    if (GT != LANCET_F32 && UNLIKELY((s3.n & 1) != 0)) mask_odd_grad<GT>(g, s3.n, wave);
 #pragma unroll
     for (int k = 0; k < kVecPerThread; ++k) {
       const f32x4 x = Grad<GT>::wide(g[k]);
@@ -952,7 +995,7 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
   // once any wait of the plan has given up the others stop at their next look, so that a stalled step ends
   // after about one bound, not one per chunk.
   if (UNLIKELY(__builtin_amdgcn_readfirstlane(sh.retry) != 0)) {
-    regather(t.part_word, t.nchunks, t.ctl, t.host_status, sc.epoch, sc.spin_limit, s2.lo, s0.lo, missing, &sh, wave);
+    regather(t.part_word, t.res_stride, t.ctl, t.host_status, sc.epoch, sc.spin_limit, s2.lo, s0.lo, missing, &sh, wave);
   }
   {
     const int w = wave;  // wave w sums norm w: the same fixed order in every workgroup
@@ -982,9 +1025,14 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
     float ratio_g = (ugn != 0.f && pn != 0.f) ? sc.lr * (pn / ugn) : sc.lr;
     ratio_m = uniform(ratio_m * sc.beta1);
     ratio_g = uniform(ratio_g * sc.beta3);
-    LANCET_GLOBAL float* p = as_global(ld_table(t.p + s0.tensor) + s0.begin);
+    const ChunkBuf p = chunk_buf(ld_table(t.p + s0.tensor) + s0.begin, 4u * static_cast<uint32_t>(s0.n));
     LANCET_GLOBAL uint16_t* pl = nullptr;
-    if (PL != kNoLowp) pl = as_global(static_cast<uint16_t*>(ld_table(t.plow + s0.tensor)) + s0.begin);
+    ChunkBuf pl_buf = p;
+    if (PL != kNoLowp) {
+      uint16_t* q = static_cast<uint16_t*>(ld_table(t.plow + s0.tensor)) + s0.begin;
+      pl = as_global(q);
+      pl_buf = chunk_buf(q, 4u * (static_cast<uint32_t>(s0.n) / 2u));
+    }
 #pragma unroll
     for (int k = 0; k < kVecPerThread; ++k) {
       f32x4 xp = sh.p[PAR ^ 1][k][fresh_tid(wave)];
@@ -994,7 +1042,7 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
         xp[j] = xp[j] - (ratio_m * um_old[k][j]) - (ratio_g * ug_old[k][j]);
       }
       st_chunk4(p, k, xp, wave);
-      st_lowp_chunk4<PL>(pl, k, xp, wave);
+      st_lowp_chunk4<PL>(pl_buf, pl, s0.n, k, xp, wave);
     }
   }
   // ---- the slots move up ------------------------------------------------------------------------------------
@@ -1009,22 +1057,199 @@ __device__ __forceinline__ bool pipeline_pass(const LansTables& t, const LansSca
 // LDS for parameters.
 constexpr int kResidentWavesPerSimd = 2;
 
-// Start of a resident step: clears the ticket, moves the step epoch on and forms the two bias corrections
-// (pow in double: kept out of the resident kernel, whose registers are all spoken for).  The epoch lives on the device so
-// that a step recorded in a graph tags every replay differently; when it wraps (2^31 steps) every word of
-// earlier steps is forgotten.  The error word is left alone.
-__global__ __launch_bounds__(kLansThreads) void lans_begin_kernel(LansTables t, LansScalars sc, size_t nwords) {
-  uint32_t* ep = t.ctl + kCtlEpoch;
-  const uint32_t e = (*ep + 1u) & ~kPoison;
-  if (e == 0u)
-    for (size_t k = threadIdx.x; k < nwords; k += kLansThreads) t.part_word[k] = 0;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    *ep = e == 0u ? 1u : e;
-    t.ctl[kCtlTicket] = 0u;
-    t.ctl[kCtlSkip] = ld_agent(t.ctl + kCtlError) != 0u ? 1u : 0u;  // step_is_skipped
-    bias_corrections(sc, t.consts[0], t.consts[1]);
+// =======================================================================================
+// first kernel of a step (either schedule), and the whole step of the small tensors
+// =======================================================================================
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallChunks = 2;
+constexpr int kSmallQuads = kSmallChunks * kLansChunk / 4 / kSmallThreads;  // groups of four elements per thread and array
+
+// sums over the workgroup, on every thread, in a fixed order
+template <int N>
+__device__ __forceinline__ void small_sums(double (&v)[N], double* s_red) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) v[i] += __shfl_xor(v[i], o, kWave);
+  __syncthreads();  // s_red may still be read from the sums before
+  if (lane_id() == 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) s_red[i * (kSmallThreads / kWave) + threadIdx.x / kWave] = v[i];
   }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    v[i] = 0.0;
+#pragma unroll
+    for (int w = 0; w < kSmallThreads / kWave; ++w) v[i] += s_red[i * (kSmallThreads / kWave) + w];
+  }
+}
+
+// elements e .. e + 3 of an array of n, zeros past its end; VEC: the array is aligned to such a group
+template <bool VEC>
+__device__ __forceinline__ f32x4 small_ld(const LANCET_GLOBAL float* a, int e, int n) {
+  if (VEC && e + 4 <= n) return ldn((const LANCET_GLOBAL f32x4*)(a + e));
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (e + j < n) x[j] = a[e + j];
+  return x;
+}
+template <bool VEC>
+__device__ __forceinline__ void small_st(LANCET_GLOBAL float* a, int e, int n, f32x4 x) {
+  if (VEC && e + 4 <= n) {
+    stn((LANCET_GLOBAL f32x4*)(a + e), x);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (e + j < n) a[e + j] = x[j];
+}
+
+// One workgroup takes a tensor of at most kSmallChunks chunks through all three phases: its sums never leave the
+// workgroup, so every array is read once and written once and nothing is launched per phase.  Such tensors (biases,
+// norms) have no bytes to speak of; what they cost is launches: 194 of them beside 480 large ones took five, 37 us.
+// Arithmetic is free here: sums in double, and the gradient divided by its norm instead of multiplied by a reciprocal.
+template <int GT, int PL, bool VEC>
+__device__ __forceinline__ void small_step(const LansTables& t, const LansScalars& sc, int tensor, float bc1, float bc2, double* s_red) {
+  typedef Grad<GT> G;
+  const int n = static_cast<int>(t.numel[tensor]);
+  const LANCET_GLOBAL typename G::S* g = as_global(static_cast<const typename G::S*>(t.g[tensor]));
+  LANCET_GLOBAL float* p = as_global(t.p[tensor]);
+  LANCET_GLOBAL float* m = as_global(t.m[tensor]);
+  LANCET_GLOBAL float* v = as_global(t.v[tensor]);
+  f32x4 xg[kSmallQuads], xp[kSmallQuads], xm[kSmallQuads], xv[kSmallQuads];
+#pragma unroll
+  for (int k = 0; k < kSmallQuads; ++k) {
+    const int e = 4 * (static_cast<int>(threadIdx.x) + k * kSmallThreads);
+    if (4 * k * kSmallThreads >= n) {  // most tensors end in the first round: the others cost nothing
+      xg[k] = xp[k] = xm[k] = xv[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      continue;
+    }
+    if (VEC && e + 4 <= n) {
+      xg[k] = G::ld4(g + e);
+    } else {
+      xg[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (e + j < n) xg[k][j] = G::ld1(g + e + j);
+    }
+    xp[k] = small_ld<VEC>(p, e, n);
+    xm[k] = small_ld<VEC>(m, e, n);
+    xv[k] = small_ld<VEC>(v, e, n);
+  }
+  double sum = 0.0;
+#pragma unroll
+  for (int k = 0; k < kSmallQuads; ++k) {
+    if (4 * k * kSmallThreads >= n) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sum += static_cast<double>(xg[k][j]) * xg[k][j];
+  }
+  double sum_g[1] = {sum};
+  if (!t.grad_norms) small_sums<1>(sum_g, s_red);
+  const float gn = t.grad_norms ? t.grad_norms[t.order[tensor]] : static_cast<float>(sqrt(sum_g[0]));
+  LansElem el = make_elem(sc, gn, bc1, bc2);
+  const float divisor = el.normalize ? gn + sc.eps : 1.f;
+  el.normalize = false;
+  f32x4 um[kSmallQuads], ug[kSmallQuads];
+  double ap = 0.0, am = 0.0, ag = 0.0;
+#pragma unroll
+  for (int k = 0; k < kSmallQuads; ++k) {
+    const int e = 4 * (static_cast<int>(threadIdx.x) + k * kSmallThreads);
+    if (4 * k * kSmallThreads >= n) {
+      um[k] = ug[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      continue;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float sg = el.scaled_grad(xg[k][j] / divisor, xp[k][j]);
+      float mm = xm[k][j], vv = xv[k][j], u0, u1;
+      el.moments(sg, mm, vv);
+      el.updates(sg, xp[k][j], mm, vv, u0, u1);
+      if (e + j >= n) u0 = u1 = 0.f;  // 0 / eps may be no number
+      xm[k][j] = mm;
+      xv[k][j] = vv;
+      um[k][j] = u0;
+      ug[k][j] = u1;
+      ap += static_cast<double>(xp[k][j]) * xp[k][j];
+      am += static_cast<double>(u0) * u0;
+      ag += static_cast<double>(u1) * u1;
+    }
+    small_st<VEC>(m, e, n, xm[k]);
+    small_st<VEC>(v, e, n, xv[k]);
+  }
+  double sums[3] = {ap, am, ag};
+  small_sums<3>(sums, s_red);
+  const float pn = static_cast<float>(sqrt(sums[0])), umn = static_cast<float>(sqrt(sums[1])), ugn = static_cast<float>(sqrt(sums[2]));
+  if (threadIdx.x == 0) {
+    t.norms[tensor] = gn;
+    t.norms[1 * t.T + tensor] = pn;
+    t.norms[2 * t.T + tensor] = umn;
+    t.norms[3 * t.T + tensor] = ugn;
+  }
+  const float ratio_m = ((umn != 0.f && pn != 0.f) ? sc.lr * (pn / umn) : sc.lr) * sc.beta1;
+  const float ratio_g = ((ugn != 0.f && pn != 0.f) ? sc.lr * (pn / ugn) : sc.lr) * sc.beta3;
+  LANCET_GLOBAL uint16_t* pl = PL == kNoLowp ? nullptr : as_global(static_cast<uint16_t*>(t.plow[tensor]));
+#pragma unroll
+  for (int k = 0; k < kSmallQuads; ++k) {
+    const int e = 4 * (static_cast<int>(threadIdx.x) + k * kSmallThreads);
+    if (4 * k * kSmallThreads >= n) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma clang fp contract(off)
+      xp[k][j] = xp[k][j] - (ratio_m * um[k][j]) - (ratio_g * ug[k][j]);
+    }
+    small_st<VEC>(p, e, n, xp[k]);
+    if (PL != kNoLowp) {
+      if (VEC && e + 4 <= n) {
+        st_lowp4<PL>(pl + e, xp[k]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (e + j < n) st_lowp1<PL>(pl + e + j, xp[k][j]);
+      }
+    }
+  }
+}
+
+// Workgroup 0 begins the step: clears the resident kernel's ticket, moves the step epoch on, decides whether the step
+// runs at all (step_is_skipped), forms the two bias corrections (pow in double: kept out of the resident kernel, whose
+// registers are all spoken for) and brings the caller's gradient norms into the plan's order.  The epoch lives on the
+// device so that a step recorded in a graph tags every replay differently; when it wraps (2^31 steps) every word of
+// earlier steps is forgotten.  The error word is left alone.
+// The other workgroups update one small tensor each; they look at the error word itself, which no workgroup of this
+// launch writes.
+template <int GT, int PL>
+__global__ __launch_bounds__(kSmallThreads) void lans_begin_kernel(LansTables t, LansScalars sc, size_t nwords, int small_base) {
+  __shared__ double s_red[3 * kSmallThreads / kWave];
+  __shared__ float s_bc[2];
+  const bool skip = ld_agent(t.ctl + kCtlError) != 0u;
+  if (blockIdx.x == 0) {
+    uint32_t* ep = t.ctl + kCtlEpoch;
+    const uint32_t e = (*ep + 1u) & ~kPoison;
+    if (e == 0u)
+      for (size_t k = threadIdx.x; k < nwords; k += kSmallThreads) t.part_word[k] = 0;
+    if (t.grad_norms && !skip)
+      for (int i = threadIdx.x; i < small_base; i += kSmallThreads) t.norms[i] = t.grad_norms[t.order[i]];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      *ep = e == 0u ? 1u : e;
+      t.ctl[kCtlTicket] = 0u;
+      t.ctl[kCtlSkip] = skip ? 1u : 0u;
+      bias_corrections(sc, t.consts[0], t.consts[1]);
+    }
+    return;
+  }
+  if (skip) return;
+  const int tensor = small_base + static_cast<int>(blockIdx.x) - 1;
+  if (threadIdx.x == 0) bias_corrections(sc, s_bc[0], s_bc[1]);
+  __syncthreads();
+  const float bc1 = s_bc[0], bc2 = s_bc[1];
+  const uintptr_t g = reinterpret_cast<uintptr_t>(t.g[tensor]), lo = PL == kNoLowp ? 0u : reinterpret_cast<uintptr_t>(t.plow[tensor]);
+  if (vec_ok(t.p[tensor], t.p[tensor], t.m[tensor], t.v[tensor]) && (g & Grad<GT>::kAlign4) == 0 && (lo & 7u) == 0)
+    small_step<GT, PL, true>(t, sc, tensor, bc1, bc2, s_red);
+  else
+    small_step<GT, PL, false>(t, sc, tensor, bc1, bc2, s_red);
 }
 
 template <int GT, int PL>
@@ -1042,6 +1267,7 @@ __global__ __launch_bounds__(kLansThreads, kResidentWavesPerSimd) void lans_resi
   s0.chunk = s1.chunk = s2.chunk = -1;
   s0.tensor = s1.tensor = s2.tensor = -1;
   s0.dead = s1.dead = s2.dead = 0;
+  s0.n = s1.n = s2.n = 0;
   if (threadIdx.x == 0) {
     sh.g_next = 0.f;
     sh.g_next_bad = 0;
@@ -1079,8 +1305,12 @@ struct lancet_lans_plan {
   int resident_grid;      // workgroups of the resident schedule the device runs at once
   int max_tensor_chunks;  // chunks of the largest tensor
   int resident_limit;     // chunks of the largest tensor the resident schedule takes on this device
-  int n_res_tensors;      // tensors within that limit: the first ones in the plan's own order
-  int n_res_chunks;       // chunk slots the resident kernel hands out (padding included)
+  // the plan's own order: tensors of whole chunks within that limit, larger ones, ragged ones within the limit, and
+  // small ones; the last three start at:
+  int big_first, ragged_first, small_first;
+  int n_whole_slots;      // chunk slots of the whole tensors (padding included): the first ones the resident kernel hands out
+  int n_res_slots;        // ... and of the ragged ones behind them
+  int big_slot, ragged_slot, small_slot;  // first chunk slot of each group in the table of all tensors
   std::vector<int32_t> order;  // plan position -> position in the caller's lists
   std::vector<char> is_resident;  // by position in the caller's lists: the resident kernel takes this tensor
   size_t words_bytes;
@@ -1111,47 +1341,80 @@ static inline int chunks_of(int64_t numel) { return static_cast<int>((numel + kL
 
 // The plan's own tensor order and chunk slots.  Tensors of at most `limit` whole chunks come first, largest first
 // (list order among equals), packed into rounds of `round` slots: a tensor that does not fit into what is
-// left of a round starts the next one and the rest of the round is padding (chunk_tensor -1), so that all
-// chunks of a tensor are drawn in the same pass of the resident kernel's workgroups.  The other tensors (larger,
-// or not a multiple of the chunk) follow in list order, without padding: they go through the sweeps.  first[i] / ctensor are in plan order.
+// left of a round starts the next one and the rest of the round is padding (-1), so that all chunks of a tensor are
+// drawn in the same pass of the resident kernel's workgroups.  The other tensors follow without padding, in list order
+// inside each group: those of more than `limit` chunks (they go through the sweeps), those within the limit that are
+// not whole chunks (ragged), and those of at most kSmallChunks chunks (small: one workgroup each).  first / ctensor are in
+// plan order.  The resident kernel hands out the whole tensors' slots and behind them, in res_tensor / res_first, slots
+// of the ragged ones, packed the same way.
 struct ChunkLayout {
   std::vector<int32_t> order, ctensor, first, count;
-  int n_fit = 0;       // tensors the resident kernel takes
-  int n_res_slots = 0; // slots it hands out
+  std::vector<int32_t> res_tensor, res_first;
+  int big_first = 0, ragged_first = 0, small_first = 0;  // plan positions
+  int big_slot = 0, ragged_slot = 0, small_slot = 0;     // slots in ctensor
+  int n_whole_slots = 0;                                 // slots of the whole tensors, padding included
 };
 
 static ChunkLayout chunk_layout(const int64_t* numels, int T, int limit, int round) {
   ChunkLayout L;
-  std::vector<int32_t> fit, big;
-  // the resident kernel takes whole chunks only
-  for (int i = 0; i < T; ++i)
-    ((chunks_of(numels[i]) <= limit && numels[i] % kLansChunk == 0) ? fit : big).push_back(i);
-  std::stable_sort(fit.begin(), fit.end(), [&](int a, int b) { return chunks_of(numels[a]) > chunks_of(numels[b]); });
-  L.n_fit = static_cast<int>(fit.size());
-  L.order = fit;
-  L.order.insert(L.order.end(), big.begin(), big.end());
+  std::vector<int32_t> whole, big, ragged, small;
+  for (int i = 0; i < T; ++i) {
+    const int k = chunks_of(numels[i]);
+    if (k <= limit && numels[i] % kLansChunk == 0) whole.push_back(i);
+    else if (k <= kSmallChunks) small.push_back(i);
+    else if (k <= limit) ragged.push_back(i);
+    else big.push_back(i);
+  }
+  const auto larger = [&](int a, int b) { return chunks_of(numels[a]) > chunks_of(numels[b]); };
+  std::stable_sort(whole.begin(), whole.end(), larger);
+  if (round < 1) round = 1;
+  const auto pack = [&](std::vector<int32_t>& slots, int k, int i) {
+    const int used = static_cast<int>(slots.size()) % round;
+    if (k <= round && used + k > round) slots.insert(slots.end(), round - used, -1);
+    const int32_t at = static_cast<int32_t>(slots.size());
+    slots.insert(slots.end(), k, i);
+    return at;
+  };
   L.first.assign(T, 0);
   L.count.assign(T, 0);
-  if (round < 1) round = 1;
-  for (int i = 0; i < T; ++i) {
-    const int k = chunks_of(numels[L.order[i]]);
-    if (i < L.n_fit && k <= round) {
-      const int used = static_cast<int>(L.ctensor.size()) % round;
-      if (used + k > round) L.ctensor.insert(L.ctensor.end(), round - used, -1);
+  L.res_first.assign(T, 0);
+  const auto place = [&](const std::vector<int32_t>& group, bool rounds) {
+    for (int u : group) {
+      const int i = static_cast<int>(L.order.size()), k = chunks_of(numels[u]);
+      L.order.push_back(u);
+      L.count[i] = k;
+      if (rounds) {
+        L.first[i] = pack(L.ctensor, k, i);
+      } else {
+        L.first[i] = static_cast<int32_t>(L.ctensor.size());
+        L.ctensor.insert(L.ctensor.end(), k, i);
+      }
     }
-    if (i == L.n_fit) L.n_res_slots = static_cast<int>(L.ctensor.size());
-    L.first[i] = static_cast<int32_t>(L.ctensor.size());
-    L.count[i] = k;
-    L.ctensor.insert(L.ctensor.end(), k, i);
-  }
-  if (L.n_fit == T) L.n_res_slots = static_cast<int>(L.ctensor.size());
+  };
+  place(whole, true);
+  L.res_tensor = L.ctensor;
+  L.res_first = L.first;
+  L.n_whole_slots = static_cast<int>(L.ctensor.size());
+  L.big_first = static_cast<int>(L.order.size());
+  L.big_slot = static_cast<int>(L.ctensor.size());
+  place(big, false);
+  L.ragged_first = static_cast<int>(L.order.size());
+  L.ragged_slot = static_cast<int>(L.ctensor.size());
+  place(ragged, false);
+  L.small_first = static_cast<int>(L.order.size());
+  L.small_slot = static_cast<int>(L.ctensor.size());
+  place(small, false);
+  std::vector<int32_t> by_size(L.small_first - L.ragged_first);
+  for (size_t k = 0; k < by_size.size(); ++k) by_size[k] = L.ragged_first + static_cast<int32_t>(k);
+  std::stable_sort(by_size.begin(), by_size.end(), [&](int a, int b) { return L.count[a] > L.count[b]; });
+  for (int i : by_size) L.res_first[i] = pack(L.res_tensor, L.count[i], i);
   return L;
 }
 
 // Host-only view of what a plan builds for `numels` when the resident kernel takes tensors of up to
 // `resident_limit` chunks and runs `round` workgroups (no device needed): for every chunk slot, in ticket
-// order, the position of its tensor in the caller's list (-1: padding); *n_resident_chunks = slots the
-// resident kernel hands out.
+// order, the position of its tensor in the caller's list (-1: padding); *n_resident_chunks = slots of the tensors of
+// whole chunks, the first ones the resident kernel hands out.
 extern "C" int64_t lancet_lans_debug_chunk_table(const int64_t* numels, int T, int resident_limit, int round,
                                                  int32_t* chunk_tensor_out, int64_t capacity,
                                                  int64_t* n_resident_chunks) {
@@ -1161,7 +1424,7 @@ extern "C" int64_t lancet_lans_debug_chunk_table(const int64_t* numels, int T, i
   const ChunkLayout L = chunk_layout(numels, T, resident_limit, round);
   for (int64_t i = 0; i < capacity && i < static_cast<int64_t>(L.ctensor.size()); ++i)
     if (chunk_tensor_out) chunk_tensor_out[i] = L.ctensor[i] < 0 ? -1 : L.order[L.ctensor[i]];
-  if (n_resident_chunks) *n_resident_chunks = L.n_res_slots;
+  if (n_resident_chunks) *n_resident_chunks = L.n_whole_slots;
   return static_cast<int64_t>(L.ctensor.size());
 }
 
@@ -1215,15 +1478,23 @@ extern "C" int lancet_lans_plan_create(const int64_t* numels, int T, lancet_lans
   pl->resident_limit = std::min(pl->resident_grid, kMaxResidentChunks);
   const ChunkLayout L = chunk_layout(numels, T, pl->resident_limit, pl->resident_grid);
   pl->order = L.order;
-  pl->n_res_tensors = L.n_fit;
-  pl->n_res_chunks = L.n_res_slots;
+  pl->big_first = L.big_first;
+  pl->ragged_first = L.ragged_first;
+  pl->small_first = L.small_first;
+  pl->big_slot = L.big_slot;
+  pl->ragged_slot = L.ragged_slot;
+  pl->small_slot = L.small_slot;
+  pl->n_whole_slots = L.n_whole_slots;
+  pl->n_res_slots = static_cast<int>(L.res_tensor.size());
   pl->nchunks = static_cast<int>(L.ctensor.size());
-  if (pl->n_res_chunks > 0) pl->schedule = LANCET_LANS_RESIDENT;
+  if (pl->n_res_slots > 0) pl->schedule = LANCET_LANS_RESIDENT;
   pl->is_resident.assign(T, 0);
-  for (int k = 0; k < pl->n_res_tensors; ++k) pl->is_resident[pl->order[k]] = 1;
+  for (int k = 0; k < pl->small_first; ++k)
+    if (k < pl->big_first || k >= pl->ragged_first) pl->is_resident[pl->order[k]] = 1;
   // device block layout
   const size_t n = static_cast<size_t>(pl->nchunks);
   const size_t n1 = n ? n : 1;
+  const size_t nr = L.res_tensor.size(), nr1 = nr ? nr : 1;
   size_t off = 0;
   const size_t o_ptrs = off;      off = align_up(off + 5 * T * sizeof(void*), 256);
   const size_t o_numel = off;     off = align_up(off + T * sizeof(int64_t), 256);
@@ -1233,11 +1504,13 @@ extern "C" int lancet_lans_plan_create(const int64_t* numels, int T, lancet_lans
   const size_t o_partial = off;   off = align_up(off + 3 * n1 * kSweepSplit * sizeof(float), 256);
   const size_t o_norms = off;     off = align_up(off + 4 * T * sizeof(float), 256);
   const size_t o_consts = off;    off = align_up(off + 2 * sizeof(float), 256);
-  const size_t o_words = off;     off = align_up(off + 4 * (n1 + T) * sizeof(uint64_t), 256);
+  const size_t o_rtensor = off;   off = align_up(off + nr1 * sizeof(int32_t), 256);
+  const size_t o_rfirst = off;    off = align_up(off + T * sizeof(int32_t), 256);
+  const size_t o_words = off;     off = align_up(off + 4 * nr1 * sizeof(uint64_t), 256);
   const size_t n_ctl = kCtlWords;
   const size_t o_ctl = off;       off = align_up(off + n_ctl * sizeof(uint32_t), 256);
   const size_t o_order = off;     off = align_up(off + T * sizeof(int32_t), 256);
-  pl->words_bytes = 4 * (n1 + T) * sizeof(uint64_t);
+  pl->words_bytes = 4 * nr1 * sizeof(uint64_t);
   if (err == hipSuccess) err = hipMalloc(&pl->dev_block, off);
   if (err == hipSuccess) err = hipHostMalloc(reinterpret_cast<void**>(&pl->h_ptrs), 5 * T * sizeof(void*), hipHostMallocDefault);
   if (err == hipSuccess) err = hipHostMalloc(reinterpret_cast<void**>(&pl->h_status), 64, hipHostMallocDefault);
@@ -1251,13 +1524,14 @@ extern "C" int lancet_lans_plan_create(const int64_t* numels, int T, lancet_lans
     if (err == hipSuccess) err = hipMemcpy(base + o_order, pl->order.data(), T * sizeof(int32_t), hipMemcpyHostToDevice);
     if (err == hipSuccess && n) err = hipMemcpy(base + o_ctensor, L.ctensor.data(), n * sizeof(int32_t), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(base + o_first, L.first.data(), T * sizeof(int32_t), hipMemcpyHostToDevice);
+    if (err == hipSuccess && nr) err = hipMemcpy(base + o_rtensor, L.res_tensor.data(), nr * sizeof(int32_t), hipMemcpyHostToDevice);
+    if (err == hipSuccess) err = hipMemcpy(base + o_rfirst, L.res_first.data(), T * sizeof(int32_t), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(base + o_count, L.count.data(), T * sizeof(int32_t), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemset(base + o_norms, 0, 4 * T * sizeof(float));
     if (err == hipSuccess) err = hipMemset(base + o_words, 0, pl->words_bytes);
     if (err == hipSuccess) err = hipMemset(base + o_ctl, 0, n_ctl * sizeof(uint32_t));
     LansTables& t = pl->tables;
     t.part_word = reinterpret_cast<uint64_t*>(base + o_words);
-    t.norm_word = t.part_word + 4 * n1;
     t.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
     t.host_status = nullptr;
     if (err == hipSuccess) err = hipHostGetDevicePointer(reinterpret_cast<void**>(&t.host_status), pl->h_status, 0);
@@ -1271,6 +1545,8 @@ extern "C" int lancet_lans_plan_create(const int64_t* numels, int T, lancet_lans
     t.chunk_tensor = reinterpret_cast<const int32_t*>(base + o_ctensor);
     t.tensor_first = reinterpret_cast<const int32_t*>(base + o_first);
     t.tensor_chunks = reinterpret_cast<const int32_t*>(base + o_count);
+    t.res_tensor = reinterpret_cast<const int32_t*>(base + o_rtensor);
+    t.res_first = reinterpret_cast<const int32_t*>(base + o_rfirst);
     t.partial = reinterpret_cast<float*>(base + o_partial);
     t.norms = reinterpret_cast<float*>(base + o_norms);
     t.consts = reinterpret_cast<float*>(base + o_consts);
@@ -1278,7 +1554,8 @@ extern "C" int lancet_lans_plan_create(const int64_t* numels, int T, lancet_lans
     t.grad_norms = nullptr;
     t.T = T;
     t.nchunks = pl->nchunks;
-    t.nres = pl->n_res_chunks;
+    t.nres = pl->n_res_slots;
+    t.res_stride = static_cast<int>(nr1);
     t.debug_flags = 0u;
   }
   if (err != hipSuccess) {
@@ -1388,32 +1665,30 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   t.grad_norms = grad_norms;
   sc.spin_limit = pl->spin_limit;
   sc.epoch = 0;
-  // slots [0, chunk_base) and tensors [0, tensor_base) go through the resident kernel, the rest
-  // (everything, under the sweeps schedule) through the three sweeps
-  int chunk_base = 0, tensor_base = 0;
-  pl->last_resident_slots = 0;
-  const bool resident = pl->schedule == LANCET_LANS_RESIDENT && pl->n_res_chunks > 0 && aligned16;
-  // the first kernel of a step forms the bias corrections and decides whether the step runs at all
-  if (resident) lans_begin_kernel<<<1, kLansThreads, 0, st>>>(t, sc, pl->words_bytes / sizeof(uint64_t));
-  else lans_prepare_kernel<<<1, 64, 0, st>>>(t, sc);
-  if (grad_norms) lans_take_grad_norms_kernel<<<(T + 255) / 256, 256, 0, st>>>(t);
-  if (resident) {
-    const int grid = std::min(pl->resident_grid, pl->n_res_chunks);
+  // The resident kernel takes the whole and the ragged tensors, the sweeps the large ones; under the sweeps schedule,
+  // and in a step whose arrays are not aligned, the sweeps take all three groups.  Its ragged chunks are padded with
+  // zeros, whose updates are 0 / eps: a step with an eps whose reciprocal is not safely finite leaves them to the sweeps.
+  const bool resident = pl->schedule == LANCET_LANS_RESIDENT && pl->n_res_slots > 0 && aligned16;
+  const bool ragged = resident && h->eps >= 1e-30f;
+  t.nres = !resident ? 0 : ragged ? pl->n_res_slots : pl->n_whole_slots;
+  pl->last_resident_slots = t.nres;
+  const int sweep_tensor = resident ? pl->big_first : 0, sweep_slot = resident ? pl->big_slot : 0;
+  const int sweep_tensor_end = ragged ? pl->ragged_first : pl->small_first, sweep_slot_end = ragged ? pl->ragged_slot : pl->small_slot;
+  LANS_TYPE_SWITCH(g_dtype, plt, (lans_begin_kernel<GT, PL><<<1 + (T - pl->small_first), kSmallThreads, 0, st>>>(
+                                     t, sc, pl->words_bytes / sizeof(uint64_t), pl->small_first)))
+  if (t.nres > 0) {
+    const int grid = std::min(pl->resident_grid, t.nres);
     LANS_TYPE_SWITCH(g_dtype, plt, (lans_resident_kernel<GT, PL><<<grid, kLansThreads, 0, st>>>(t, sc)))
-    chunk_base = pl->n_res_chunks;
-    tensor_base = pl->n_res_tensors;
-    pl->last_resident_slots = chunk_base;
   }
-  const int nsweep = t.nchunks - chunk_base;
+  const int nsweep = sweep_slot_end - sweep_slot, rest = sweep_tensor_end - sweep_tensor;
   if (nsweep > 0) {
-    const int rest = T - tensor_base;
     if (!grad_norms) {
-      LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_norm_g_kernel<GT><<<nsweep, kLansThreads, 0, st>>>(t, chunk_base)))
-      lans_reduce_kernel<<<dim3(rest, 1), kReduceThreads, 0, st>>>(t, 0, tensor_base, 1);
+      LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_norm_g_kernel<GT><<<nsweep, kLansThreads, 0, st>>>(t, sweep_slot)))
+      lans_reduce_kernel<<<dim3(rest, 1), kReduceThreads, 0, st>>>(t, 0, sweep_tensor, 1);
     }
-    LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_moments_kernel<GT><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, chunk_base)))
-    lans_reduce_kernel<<<dim3(rest, 3), kReduceThreads, 0, st>>>(t, 1, tensor_base, kSweepSplit);
-    LANS_TYPE_SWITCH(g_dtype, plt, (lans_update_kernel<GT, PL><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, chunk_base)))
+    LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_moments_kernel<GT><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, sweep_slot)))
+    lans_reduce_kernel<<<dim3(rest, 3), kReduceThreads, 0, st>>>(t, 1, sweep_tensor, kSweepSplit);
+    LANS_TYPE_SWITCH(g_dtype, plt, (lans_update_kernel<GT, PL><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, sweep_slot)))
   }
   return static_cast<int>(hipGetLastError());
 }
@@ -1440,7 +1715,7 @@ extern "C" int lancet_lans_plan_set_schedule(lancet_lans_plan_t pl, int schedule
   if (schedule != LANCET_LANS_SWEEPS && schedule != LANCET_LANS_RESIDENT) return LANCET_ERR_SHAPE;
   // tensors too large for the resident kernel go through the sweeps inside the same step; a plan made only
   // of such tensors has no use for the kernel
-  if (schedule == LANCET_LANS_RESIDENT && pl->n_res_chunks == 0 && pl->nchunks > 0) return LANCET_ERR_SHAPE;
+  if (schedule == LANCET_LANS_RESIDENT && pl->n_res_slots == 0 && pl->nchunks > 0) return LANCET_ERR_SHAPE;
   pl->schedule = schedule;
   return LANCET_OK;
 }

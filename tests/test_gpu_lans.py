@@ -525,6 +525,54 @@ def test_stepper_keeps_master_weights_for_a_16_bit_model(pkg):
             a[...] = to_np(master)
 
 
+@pytest.mark.parametrize("gdt,pdt", [("f32", None), ("bf16", "bf16"), ("f16", None)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_lans_tensors_that_end_anywhere(pkg, gdt, pdt, offset):
+    """Tensors that are not whole chunks of 8192 parameters: the last chunk of 1 .. 8191 elements in the resident kernel
+    (every remainder of the four-element accesses, odd sizes with 16-bit arrays) and tensors of at most two chunks in one
+    workgroup (around its 4096 elements per load), against the oracle; with offset 1 the arrays are unaligned and the
+    element paths run.  Nothing past a tensor's end changes, also for an eps so small that the ragged tensors are left to the sweeps."""
+    capi = pkg.capi
+    numels = [16385, 16386, 16387, 16388, 3 * 8192 - 1, 3 * 8192 + 4097, 5 * 8192,
+              1, 2, 3, 1000, 1003, 4095, 4096, 4097, 8191, 8193, 16383]
+    rng, p, m, v = make_state(31, [(n,) for n in numels])
+    g = [_rounder(gdt)(rng.normal(0, 1e-3, n).astype(np.float32)).astype(np.float32) for n in numels]
+
+    def inside(a, dtype=torch.float32):        # the tensor inside a buffer of sevens
+        buf = torch.full((offset + a.size + 8,), 7.0, dtype=dtype, device="cuda")
+        buf[offset:offset + a.size] = torch.from_numpy(a).cuda().to(dtype)
+        return buf
+
+    def cut(bufs):
+        return [b[offset:offset + n] for b, n in zip(bufs, numels)]
+
+    bufs = {k: [inside(a) for a in lst] for k, lst in (("p", p), ("m", m), ("v", v))}
+    bufs["g"] = [inside(a, _TORCH[gdt]) for a in g]
+    bufs["low"] = [inside(a, _TORCH[pdt]) for a in p] if pdt else None
+    dp, dm, dv, dg = (cut(bufs[k]) for k in "pmvg")
+    dlow = cut(bufs["low"]) if pdt else None
+    plan = pkg.ops.LansPlan(numels)
+    for step in range(1, 4):
+        lo.lans_step(g, p, m, v, step)
+        plan.step(dg, dp, dm, dv, step, capi.LansHyper(1e-3, 0.9, 0.999, 1e-6, 1, 0.01, 1, 1, 1), p_lowp=dlow)
+    assert plan.error() == 0
+    assert (plan.last_resident_slots() >= sum((n + 8191) // 8192 for n in numels if n > 16384)) == (offset == 0)
+    for i in range(len(numels)):
+        assert_close_scaled(to_np(dp[i]), p[i], P_RTOL, "p[%d]" % i)
+        assert_close_scaled(to_np(dm[i]), m[i], 1e-5, "m[%d]" % i)
+        assert_close_scaled(to_np(dv[i]), v[i], 1e-5, "v[%d]" % i)
+        if pdt:
+            assert torch.equal(dlow[i], dp[i].to(_TORCH[pdt]))
+    for lst in bufs.values():
+        for b, n in zip(lst or [], numels):
+            assert bool((b[:offset] == 7).all()) and bool((b[offset + n:] == 7).all())
+    plan.step(dg, dp, dm, dv, 4, capi.LansHyper(1e-3, 0.9, 0.999, 1e-36, 1, 0.01, 1, 1, 1), p_lowp=dlow)
+    assert plan.error() == 0
+    for i in range(len(numels)):
+        assert bool(torch.isfinite(dp[i]).all())
+    plan.close()
+
+
 def test_lans_norms_of_tensors_with_many_partial_sums(pkg):
     """Norms of tensors whose per-chunk sums are one less than, as many as and one more than a workgroup of the reduction
     reads at a time (8 x 1024 of the moments sweep, 1024 chunks), and more than it reads in one go.  A chunk's sum is
