@@ -11,27 +11,53 @@ namespace lancet {
 constexpr int kRowsPerBlock = kTile / kWave;  // waves per workgroup; a wave moves a row or a share of one
 constexpr int kTailRows = 16;                 // rows zero-filled by one tail workgroup
 
-// Access granule: 16 bytes when the row size and the pointers allow, else one element.
-template <typename V>
-__device__ __forceinline__ V ldv(const V* p) { return __builtin_nontemporal_load(p); }
-template <typename V>
-__device__ __forceinline__ void stv(V* p, V v) { __builtin_nontemporal_store(v, p); }
-template <typename V>
-__device__ __forceinline__ void stv(LANCET_GLOBAL V* p, V v) { __builtin_nontemporal_store(v, p); }
-template <typename V>
-__device__ __forceinline__ V zero_v() { return V(0); }
+// How a row is cut into the pieces its lanes move:
+//   kWhole16  16-byte granules, rows and pointers aligned to them;
+//   kAny16    rows of at least 16 bytes that end anywhere and start wherever their elements are aligned: 16-byte
+//             granules at unaligned addresses (the hardware takes them), the last one drawn back so that it ends with
+//             the row.  Its first bytes are then moved twice, with the same values.  At 10007 rows of 1003 bf16 values
+//             (60 experts, top-2) the scatter takes 17 us this way and 44 an element per lane, the decode 12 and 33;
+//   kElem2 / kElem4  one element per lane: rows of less than 16 bytes.
+enum RowMode { kWhole16, kAny16, kElem2, kElem4 };
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+
+template <int MODE>
+struct Granule {
+  typedef u32x4 V;
+  static __device__ __forceinline__ uint32_t at(int v, uint32_t) { return 16u * static_cast<uint32_t>(v); }
+  static __device__ __forceinline__ V ld(const char* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
+  static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { __builtin_nontemporal_store(x, (LANCET_GLOBAL u32x4*)p); }
+  static __device__ __forceinline__ V zero() { return u32x4{0u, 0u, 0u, 0u}; }
+};
 template <>
-__device__ __forceinline__ u32x4 zero_v<u32x4>() { return u32x4{0u, 0u, 0u, 0u}; }
+struct Granule<kAny16> {
+  typedef u32x4 V;
+  static __device__ __forceinline__ uint32_t at(int v, uint32_t row_bytes) { return min(16u * static_cast<uint32_t>(v), row_bytes - 16u); }
+  static __device__ __forceinline__ V ld(const char* p) { return *reinterpret_cast<const u32x4_any*>(p); }
+  static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { *(LANCET_GLOBAL u32x4_any*)p = x; }
+  static __device__ __forceinline__ V zero() { return u32x4{0u, 0u, 0u, 0u}; }
+};
+template <typename E>
+struct GranuleElem {
+  typedef E V;
+  static __device__ __forceinline__ uint32_t at(int v, uint32_t) { return static_cast<uint32_t>(sizeof(E)) * static_cast<uint32_t>(v); }
+  static __device__ __forceinline__ V ld(const char* p) { return __builtin_nontemporal_load(reinterpret_cast<const E*>(p)); }
+  static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { __builtin_nontemporal_store(x, (LANCET_GLOBAL E*)p); }
+  static __device__ __forceinline__ V zero() { return E(0); }
+};
+template <>
+struct Granule<kElem2> : GranuleElem<uint16_t> {};
+template <>
+struct Granule<kElem4> : GranuleElem<uint32_t> {};
 
 // ---------------------------------------------------------------------------------------
 // encode_forward: out[idx, loc, :] = data[s, :]; rows no token lands on are zero.
 // Replaces cudaMemsetAsync + atomicAdd per element of
 // src/op/dialect/cuda/kernels/tutel_moe_dispatch.cu:61-81,461-484.
 // ---------------------------------------------------------------------------------------
-template <typename V>
 struct ScatterArgs {
-  const V* data;
-  V* out;
+  const char* data;
+  char* out;
   const int32_t* idx;         // [K*S]
   const int32_t* loc;         // [K*S]
   const int32_t* dest;        // [K*S] or null: destination row e * C + location (-1: none) in ONE word per slot,
@@ -43,14 +69,17 @@ struct ScatterArgs {
   int S, E, C, K;
   int slot_stride;            // distance between the slots of one token in idx / loc (S, or the whole batch's
                               // token count when this call moves a token range of a larger mask)
+  uint32_t row_bytes;
   int row_vecs;               // granules per row
   int wpr_shift;              // 2^wpr_shift waves share one token row
   int token_blocks;
   int tail_chunks;            // tail workgroups per expert
 };
 
-template <typename V, int K, bool DEST = false>
-__global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs<V> a) {
+template <int MODE, int K, bool DEST = false>
+__global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
+  typedef Granule<MODE> G;
+  typedef typename G::V V;
   const int w = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   if (static_cast<int>(blockIdx.x) < a.token_blocks) {
@@ -64,24 +93,25 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs<V> a) {
     // The row's granules do not depend on the routing, only their destinations do: the first loads of the row
     // go out before idx / loc are known, so that a wave waits for the longer of the two latencies and not for
     // their sum (a dropped token's row is then read for nothing).  338 -> 333 us at the headline shape.
-    const V* src = a.data + static_cast<size_t>(s) * a.row_vecs;
+    const char* src = a.data + static_cast<size_t>(s) * a.row_bytes;
     const int step = kWave << a.wpr_shift;
     int v = part * kWave + lane;
     const bool has0 = v < a.row_vecs, has1 = v + step < a.row_vecs;
-    V x0 = zero_v<V>(), x1 = zero_v<V>();
-    if (has0) x0 = ldv(src + v);
-    if (has1) x1 = ldv(src + v + step);
+    const uint32_t o0 = G::at(v, a.row_bytes), o1 = G::at(v + step, a.row_bytes);
+    V x0 = G::zero(), x1 = G::zero();
+    if (has0) x0 = G::ld(src + o0);
+    if (has1) x1 = G::ld(src + o1);
     // destinations picked at run time: typed as global memory so the stores are not flat.  (The routing words of a
     // row are the same for every lane; loading them through the scalar cache, or forming the row addresses on the
     // scalar unit from vector-loaded words, was measured slower: 346 and 340 us against 333 at the headline shape.)
-    LANCET_GLOBAL V* dst[K];
+    LANCET_GLOBAL char* dst[K];
     int nd = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       if (DEST) {
         const int d = a.dest[static_cast<size_t>(j) * a.slot_stride + s];
         dst[j] = as_global(a.out);
-        if (d >= 0 && d < a.E * a.C) dst[nd++] = as_global(a.out + static_cast<size_t>(d) * a.row_vecs);
+        if (d >= 0 && d < a.E * a.C) dst[nd++] = as_global(a.out + static_cast<size_t>(d) * a.row_bytes);
         continue;
       }
       const int e = a.idx[static_cast<size_t>(j) * a.slot_stride + s];
@@ -93,32 +123,22 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs<V> a) {
         l += a.row_base[e];
         ok = l < a.C;
       }
-      if (ok) dst[nd++] = as_global(a.out + (static_cast<size_t>(e) * a.C + l) * a.row_vecs);
+      if (ok) dst[nd++] = as_global(a.out + (static_cast<size_t>(e) * a.C + l) * a.row_bytes);
     }
     if (nd == 0) return;
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       if (j < nd) {
-        if (has0) stv(dst[j] + v, x0);
-        if (has1) stv(dst[j] + v + step, x1);
+        if (has0) G::st(dst[j] + o0, x0);
+        if (has1) G::st(dst[j] + o1, x1);
       }
     }
-    v += 2 * step;
-    for (; v + step < a.row_vecs; v += 2 * step) {
-      const V x0 = ldv(src + v), x1 = ldv(src + v + step);
-#pragma unroll
-      for (int j = 0; j < K; ++j) {
-        if (j < nd) {
-          stv(dst[j] + v, x0);
-          stv(dst[j] + v + step, x1);
-        }
-      }
-    }
-    if (v < a.row_vecs) {
-      const V x = ldv(src + v);
+    for (v += 2 * step; v < a.row_vecs; v += step) {
+      const uint32_t o = G::at(v, a.row_bytes);
+      const V x = G::ld(src + o);
 #pragma unroll
       for (int j = 0; j < K; ++j)
-        if (j < nd) stv(dst[j] + v, x);
+        if (j < nd) G::st(dst[j] + o, x);
     }
   } else {
     // tail: zero rows [used, C) of expert e, kTailRows rows per workgroup
@@ -128,10 +148,9 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs<V> a) {
     const int used = a.rows_hi[e] - (a.rows_lo ? a.rows_lo[e] : 0);
     const int first = max(used, 0) + ch * kTailRows;
     const int last = min(first + kTailRows, a.C);
-    const V z = zero_v<V>();
     for (int r = first + w; r < last; r += kRowsPerBlock) {
-      V* row = a.out + (static_cast<size_t>(e) * a.C + r) * a.row_vecs;
-      for (int v = lane; v < a.row_vecs; v += kWave) stv(row + v, z);
+      LANCET_GLOBAL char* row = as_global(a.out + (static_cast<size_t>(e) * a.C + r) * a.row_bytes);
+      for (int v = lane; v < a.row_vecs; v += kWave) G::st(row + G::at(v, a.row_bytes), G::zero());
     }
   }
 }
@@ -221,7 +240,7 @@ struct DecodeArgs {
   int wpr_shift;         // 2^wpr_shift waves share one token row (each takes every 2^wpr_shift-th run of 64 granules)
 };
 
-template <int DT, int K, bool VEC, bool DEST = false>
+template <int DT, int K, int MODE, bool DEST = false>
 __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
   typedef Codec<DT> Cd;
   const int w = threadIdx.x / kWave;
@@ -250,31 +269,37 @@ __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
     g[j] = ok[j] ? (a.gates ? ld_gate(a.gates, static_cast<size_t>(j) * a.slot_stride + s, a.gate_dtype) : 1.f) : 0.f;
     any = any || ok[j];
   }
-  if (VEC) {
-    const int row_vecs = a.M / Cd::kPerVec;
-    u32x4* dst = static_cast<u32x4*>(a.out) + static_cast<size_t>(s) * row_vecs;
-    const u32x4* base = static_cast<const u32x4*>(a.expert_out);
+  if constexpr (MODE == kWhole16 || MODE == kAny16) {
+    typedef Granule<MODE> G;
+    const uint32_t row_bytes = static_cast<uint32_t>(a.M) * static_cast<uint32_t>(sizeof(typename Cd::S));
+    const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
+    LANCET_GLOBAL char* dst = as_global(static_cast<char*>(a.out) + static_cast<size_t>(s) * row_bytes);
+    const char* src[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) src[j] = static_cast<const char*>(a.expert_out) + row[j] * row_bytes;
     const u32x4 z = {0u, 0u, 0u, 0u};
     int v = part * kWave + lane;
     if (!any) {
-      for (; v < row_vecs; v += step) st_stream(dst + v, z);
+      for (; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), z);
       return;
     }
     for (; v + step < row_vecs; v += 2 * step) {  // two granules in flight per slot
+      const uint32_t oa = G::at(v, row_bytes), ob = G::at(v + step, row_bytes);
       u32x4 xa[K], xb[K];
 #pragma unroll
       for (int j = 0; j < K; ++j) {
-        xa[j] = ok[j] ? ld_stream(base + row[j] * row_vecs + v) : z;
-        xb[j] = ok[j] ? ld_stream(base + row[j] * row_vecs + v + step) : z;
+        xa[j] = ok[j] ? G::ld(src[j] + oa) : z;
+        xb[j] = ok[j] ? G::ld(src[j] + ob) : z;
       }
-      st_stream(dst + v, combine_vec<DT, K>(xa, g));
-      st_stream(dst + v + step, combine_vec<DT, K>(xb, g));
+      G::st(dst + oa, combine_vec<DT, K>(xa, g));
+      G::st(dst + ob, combine_vec<DT, K>(xb, g));
     }
     if (v < row_vecs) {
+      const uint32_t oa = G::at(v, row_bytes);
       u32x4 xa[K];
 #pragma unroll
-      for (int j = 0; j < K; ++j) xa[j] = ok[j] ? ld_stream(base + row[j] * row_vecs + v) : z;
-      st_stream(dst + v, combine_vec<DT, K>(xa, g));
+      for (int j = 0; j < K; ++j) xa[j] = ok[j] ? G::ld(src[j] + oa) : z;
+      G::st(dst + oa, combine_vec<DT, K>(xa, g));
     }
   } else {
     typedef typename Cd::S St;
@@ -341,10 +366,12 @@ __global__ __launch_bounds__(kTile) void merge_masks_kernel(PtrTable t, int P, i
 
 // out[e, off_p[e] + r, :] = buf_p[e, r, :] for r < kept[p][e]; other rows zero
 // (tutel_moe_dispatch.cu:365-408, which leaves them uninitialised).
-template <typename V>
-__global__ __launch_bounds__(kTile) void redispatch_rows_kernel(PtrTable bufs, int P, int E, int C,
+template <int MODE>
+__global__ __launch_bounds__(kTile) void redispatch_rows_kernel(PtrTable bufs, int P, int E, int C, uint32_t row_bytes,
                                                                 int row_vecs, int wpr_shift,
-                                                                const uint32_t* counts, V* out) {
+                                                                const uint32_t* counts, char* out) {
+  typedef Granule<MODE> G;
+  typedef typename G::V V;
   const int w = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const uint32_t gw = blockIdx.x * static_cast<uint32_t>(kRowsPerBlock) + w;
@@ -365,21 +392,24 @@ __global__ __launch_bounds__(kTile) void redispatch_rows_kernel(PtrTable bufs, i
   }
   const uint32_t excl = incl - k;
   const uint64_t owner = __ballot(lane < P && static_cast<uint32_t>(c) >= excl && static_cast<uint32_t>(c) < incl);
-  V* dst = out + static_cast<size_t>(r) * row_vecs;
+  LANCET_GLOBAL char* dst = as_global(out + static_cast<size_t>(r) * row_bytes);
   if (owner) {
     const int q = __ffsll(static_cast<unsigned long long>(owner)) - 1;
     const int off = static_cast<int>(__shfl(excl, q, kWave));
-    const V* src = static_cast<const V*>(bufs.p[q]) + (static_cast<size_t>(e) * C + (c - off)) * row_vecs;
+    const char* src = static_cast<const char*>(bufs.p[q]) + (static_cast<size_t>(e) * C + (c - off)) * row_bytes;
     int v = part * kWave + lane;
     for (; v + step < row_vecs; v += 2 * step) {
-      const V x0 = ldv(src + v), x1 = ldv(src + v + step);
-      stv(dst + v, x0);
-      stv(dst + v + step, x1);
+      const uint32_t o0 = G::at(v, row_bytes), o1 = G::at(v + step, row_bytes);
+      const V x0 = G::ld(src + o0), x1 = G::ld(src + o1);
+      G::st(dst + o0, x0);
+      G::st(dst + o1, x1);
     }
-    if (v < row_vecs) stv(dst + v, ldv(src + v));
+    if (v < row_vecs) {
+      const uint32_t o0 = G::at(v, row_bytes);
+      G::st(dst + o0, G::ld(src + o0));
+    }
   } else {
-    const V z = zero_v<V>();
-    for (int v = part * kWave + lane; v < row_vecs; v += step) stv(dst + v, z);
+    for (int v = part * kWave + lane; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), G::zero());
   }
 }
 
@@ -501,7 +531,7 @@ __global__ __launch_bounds__(kTile) void inverse_map_kernel(const int32_t* idx, 
 // grad_expert_out[e, l, :] = gates[i] * dy[s, :] for the slot-token i = src[e*C+l] (s = i mod S), zero
 // for rows nobody owns: decode_backward_data_kernel (tutel_moe_dispatch.cu:118-124, 523-533) without
 // the memset + atomicAdd; every output byte is written once.
-template <int DT, bool VEC>
+template <int DT, int MODE>
 __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, const void* gates, int gd,
                                                                const int32_t* src, void* out, int S, int M,
                                                                long rows, int wpr_shift) {
@@ -516,25 +546,29 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
   const int i = src[r];
   const float g1[1] = {i >= 0 ? ld_gate(gates, i, gd) : 0.f};
   const size_t s = i >= 0 ? static_cast<size_t>(i % S) : 0;
-  if (VEC) {
-    const int row_vecs = M / Cd::kPerVec;
-    u32x4* dst = static_cast<u32x4*>(out) + static_cast<size_t>(r) * row_vecs;
+  if constexpr (MODE == kWhole16 || MODE == kAny16) {
+    typedef Granule<MODE> G;
+    const uint32_t row_bytes = static_cast<uint32_t>(M) * static_cast<uint32_t>(sizeof(typename Cd::S));
+    const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
+    LANCET_GLOBAL char* dst = as_global(static_cast<char*>(out) + static_cast<size_t>(r) * row_bytes);
     const u32x4 z = {0u, 0u, 0u, 0u};
     int v = part * kWave + lane;
     if (i < 0) {
-      for (; v < row_vecs; v += step) st_stream(dst + v, z);
+      for (; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), z);
       return;
     }
-    const u32x4* sp = static_cast<const u32x4*>(dy) + s * row_vecs;
+    const char* sp = static_cast<const char*>(dy) + s * row_bytes;
     for (; v + step < row_vecs; v += 2 * step) {
-      const u32x4 xa[1] = {ld_stream(sp + v)};
-      const u32x4 xb[1] = {ld_stream(sp + v + step)};
-      st_stream(dst + v, combine_vec<DT, 1>(xa, g1));
-      st_stream(dst + v + step, combine_vec<DT, 1>(xb, g1));
+      const uint32_t oa = G::at(v, row_bytes), ob = G::at(v + step, row_bytes);
+      const u32x4 xa[1] = {G::ld(sp + oa)};
+      const u32x4 xb[1] = {G::ld(sp + ob)};
+      G::st(dst + oa, combine_vec<DT, 1>(xa, g1));
+      G::st(dst + ob, combine_vec<DT, 1>(xb, g1));
     }
     if (v < row_vecs) {
-      const u32x4 xa[1] = {ld_stream(sp + v)};
-      st_stream(dst + v, combine_vec<DT, 1>(xa, g1));
+      const uint32_t oa = G::at(v, row_bytes);
+      const u32x4 xa[1] = {G::ld(sp + oa)};
+      G::st(dst + oa, combine_vec<DT, 1>(xa, g1));
     }
   } else {
     typedef typename Cd::S St;
@@ -545,10 +579,37 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
   }
 }
 
+// acc + the products of the elements of two granules, in order
+template <int DT>
+__device__ __forceinline__ float dot_vec(const u32x4& x, const u32x4& y, float acc) {
+  typedef Codec<DT> Cd;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (Cd::kPerVec == 4) {
+      acc += Cd::get(x[k]) * Cd::get(y[k]);
+    } else {
+      acc += Cd::get(static_cast<typename Cd::S>(x[k] & 0xffffu)) * Cd::get(static_cast<typename Cd::S>(y[k] & 0xffffu));
+      acc += Cd::get(static_cast<typename Cd::S>(x[k] >> 16)) * Cd::get(static_cast<typename Cd::S>(y[k] >> 16));
+    }
+  }
+  return acc;
+}
+// a granule with its first n bytes (whole elements) as zeros: the last granule of a row that was drawn back over bytes
+// another lane has already counted
+template <int DT>
+__device__ __forceinline__ u32x4 drop_bytes(u32x4 x, uint32_t n) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (4u * k + 4u <= n) x[k] = 0u;
+    else if (Codec<DT>::kPerVec == 8 && 4u * k + 2u == n) x[k] &= 0xffff0000u;
+  }
+  return x;
+}
+
 // grad_gates_s[i] = <expert_out[idx, loc, :], dy[s, :]> for slot-token i, 0 when the slot is dropped
 // (decode_backward_gate_kernel, tutel_moe_dispatch.cu:126-157): one wave per slot-token, fp32 partial
 // sums per lane, xor-tree over the wave.
-template <int DT, bool VEC>
+template <int DT, int MODE>
 __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const void* expert_out,
                                                           const int32_t* idx, const int32_t* loc, void* out, int gd,
                                                           int S, int M, int E, int C, int n) {
@@ -565,21 +626,17 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
   const size_t s = static_cast<size_t>(i % S);
   const size_t row = static_cast<size_t>(e) * C + l;
   float acc = 0.f;
-  if (VEC) {
-    const int row_vecs = M / Cd::kPerVec;
-    const u32x4* a = static_cast<const u32x4*>(expert_out) + row * row_vecs;
-    const u32x4* b = static_cast<const u32x4*>(dy) + s * row_vecs;
+  if constexpr (MODE == kWhole16 || MODE == kAny16) {
+    typedef Granule<MODE> G;
+    const uint32_t row_bytes = static_cast<uint32_t>(M) * static_cast<uint32_t>(sizeof(typename Cd::S));
+    const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
+    const char* a = static_cast<const char*>(expert_out) + row * row_bytes;
+    const char* b = static_cast<const char*>(dy) + s * row_bytes;
     for (int v = lane; v < row_vecs; v += kWave) {
-      const u32x4 x = ld_stream(a + v), y = ld_stream(b + v);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (Cd::kPerVec == 4) {
-          acc += Cd::get(x[k]) * Cd::get(y[k]);
-        } else {
-          acc += Cd::get(static_cast<typename Cd::S>(x[k] & 0xffffu)) * Cd::get(static_cast<typename Cd::S>(y[k] & 0xffffu));
-          acc += Cd::get(static_cast<typename Cd::S>(x[k] >> 16)) * Cd::get(static_cast<typename Cd::S>(y[k] >> 16));
-        }
-      }
+      const uint32_t o = G::at(v, row_bytes);
+      u32x4 x = G::ld(a + o), y = G::ld(b + o);
+      if (MODE == kAny16 && o != 16u * static_cast<uint32_t>(v)) x = drop_bytes<DT>(x, 16u * static_cast<uint32_t>(v) - o);
+      acc = dot_vec<DT>(x, y, acc);
     }
   } else {
     typedef typename Cd::S St;
@@ -609,15 +666,43 @@ static inline int split_waves(long units, long rows, int per_lane = 1) {
   return shift;
 }
 
-template <typename V>
-static hipError_t scatter_launch(const void* data, void* out, const int32_t* idx, const int32_t* loc,
-                                 const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
-                                 const int32_t* rows_hi, int S, int E, int C, int K, int row_vecs,
-                                 int slot_stride, hipStream_t st, const int32_t* dest = nullptr) {
-  ScatterArgs<V> a;
+// the way rows of row_bytes bytes in arrays at the given addresses are cut
+static inline RowMode row_mode(size_t row_bytes, int elem_bytes, bool aligned) {
+  if (row_bytes < 16) return elem_bytes == 4 ? kElem4 : kElem2;
+  return row_bytes % 16 == 0 && aligned ? kWhole16 : kAny16;
+}
+// granules of such a row
+static inline int row_granules(RowMode mode, size_t row_bytes, int elem_bytes) {
+  return static_cast<int>(mode == kWhole16 || mode == kAny16 ? (row_bytes + 15) / 16 : row_bytes / elem_bytes);
+}
+// MODE as a compile-time constant inside `...` (the second form: for rows of a known type, whose elements have one size)
+#define LANCET_CODED_ROW_SWITCH(DT, mode, ...)                         \
+  switch (mode) {                                                      \
+    case kWhole16: { constexpr int MODE = kWhole16; __VA_ARGS__; } break; \
+    case kAny16: { constexpr int MODE = kAny16; __VA_ARGS__; } break;     \
+    default: { constexpr int MODE = DT == LANCET_F32 ? kElem4 : kElem2; __VA_ARGS__; } break; \
+  }
+#define LANCET_ROW_SWITCH(mode, ...)                                   \
+  switch (mode) {                                                      \
+    case kWhole16: { constexpr int MODE = kWhole16; __VA_ARGS__; } break; \
+    case kAny16: { constexpr int MODE = kAny16; __VA_ARGS__; } break;     \
+    case kElem2: { constexpr int MODE = kElem2; __VA_ARGS__; } break;     \
+    default: { constexpr int MODE = kElem4; __VA_ARGS__; } break;         \
+  }
+
+hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, const int32_t* loc,
+                            const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
+                            const int32_t* rows_hi,
+                            int S, int M, int E, int C, int K, int elem_bytes, hipStream_t st, int slot_stride,
+                            const int32_t* dest) {
+  const size_t row_bytes = static_cast<size_t>(M) * elem_bytes;
+  if (row_bytes == 0) return hipSuccess;
+  const RowMode mode = row_mode(row_bytes, elem_bytes, aligned16(data) && aligned16(out));
+  if (dest && mode != kWhole16) return hipErrorInvalidValue;  // the one-word form is for rows of 16-byte granules
+  ScatterArgs a;
   a.dest = dest;
-  a.data = static_cast<const V*>(data);
-  a.out = static_cast<V*>(out);
+  a.data = static_cast<const char*>(data);
+  a.out = static_cast<char*>(out);
   a.idx = idx;
   a.loc = loc;
   a.avail_used = avail_used;
@@ -628,36 +713,23 @@ static hipError_t scatter_launch(const void* data, void* out, const int32_t* idx
   a.E = E;
   a.C = C;
   a.K = K;
-  a.slot_stride = slot_stride;
-  a.row_vecs = row_vecs;
-  a.wpr_shift = split_waves(row_vecs, S);
+  a.slot_stride = slot_stride < 0 ? S : slot_stride;
+  a.row_bytes = static_cast<uint32_t>(row_bytes);  // M < 2^30
+  a.row_vecs = row_granules(mode, row_bytes, elem_bytes);
+  a.wpr_shift = split_waves(a.row_vecs, S);
   a.token_blocks = static_cast<int>(((static_cast<long>(S) << a.wpr_shift) + kRowsPerBlock - 1) / kRowsPerBlock);
   a.tail_chunks = rows_hi ? (C + kTailRows - 1) / kTailRows : 0;
   const long blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_chunks) * E;
   if (blocks == 0) return hipSuccess;
   if (dest) {
-    if (K == 1) scatter_rows_kernel<V, 1, true><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
-    else scatter_rows_kernel<V, 2, true><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
-  } else if (K == 1) scatter_rows_kernel<V, 1><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
-  else scatter_rows_kernel<V, 2><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
+    if (K == 1) scatter_rows_kernel<kWhole16, 1, true><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
+    else scatter_rows_kernel<kWhole16, 2, true><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
+    return hipGetLastError();
+  }
+  LANCET_ROW_SWITCH(mode,
+    if (K == 1) scatter_rows_kernel<MODE, 1><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
+    else scatter_rows_kernel<MODE, 2><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a))
   return hipGetLastError();
-}
-
-hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, const int32_t* loc,
-                            const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
-                            const int32_t* rows_hi,
-                            int S, int M, int E, int C, int K, int elem_bytes, hipStream_t st, int slot_stride,
-                            const int32_t* dest) {
-  const size_t row_bytes = static_cast<size_t>(M) * elem_bytes;
-  if (row_bytes == 0) return hipSuccess;
-  const int ss = slot_stride < 0 ? S : slot_stride;
-  if (row_bytes % 16 == 0 && aligned16(data) && aligned16(out))
-    return scatter_launch<u32x4>(data, out, idx, loc, avail_used, row_base, rows_lo, rows_hi, S, E, C, K,
-                                 static_cast<int>(row_bytes / 16), ss, st, dest);
-  if (dest) return hipErrorInvalidValue;  // the one-word form is for rows of 16-byte granules
-  if (elem_bytes == 4)
-    return scatter_launch<uint32_t>(data, out, idx, loc, avail_used, row_base, rows_lo, rows_hi, S, E, C, K, M, ss, st);
-  return scatter_launch<uint16_t>(data, out, idx, loc, avail_used, row_base, rows_lo, rows_hi, S, E, C, K, M, ss, st);
 }
 
 hipError_t run_zero_bytes(void* p, size_t nbytes, hipStream_t st) {
@@ -682,21 +754,19 @@ hipError_t run_zero_bytes(void* p, size_t nbytes, hipStream_t st) {
 }
 
 template <int DT>
-static hipError_t decode_launch(DecodeArgs a, int K, bool vec, hipStream_t st) {
+static hipError_t decode_launch(DecodeArgs a, int K, RowMode mode, hipStream_t st) {
   if (a.S == 0 || a.M == 0) return hipSuccess;
-  a.wpr_shift = split_waves(vec ? a.M / Codec<DT>::kPerVec : a.M, a.S, 2);
+  a.wpr_shift = split_waves(row_granules(mode, static_cast<size_t>(a.M) * sizeof(typename Codec<DT>::S), sizeof(typename Codec<DT>::S)), a.S, 2);
   const unsigned blocks = static_cast<unsigned>(((static_cast<long>(a.S) << a.wpr_shift) + kRowsPerBlock - 1) / kRowsPerBlock);
   if (a.dest) {
-    if (!vec) return hipErrorInvalidValue;
-    if (K == 1) decode_rows_kernel<DT, 1, true, true><<<blocks, kTile, 0, st>>>(a);
-    else decode_rows_kernel<DT, 2, true, true><<<blocks, kTile, 0, st>>>(a);
-  } else if (K == 1) {
-    if (vec) decode_rows_kernel<DT, 1, true><<<blocks, kTile, 0, st>>>(a);
-    else decode_rows_kernel<DT, 1, false><<<blocks, kTile, 0, st>>>(a);
-  } else {
-    if (vec) decode_rows_kernel<DT, 2, true><<<blocks, kTile, 0, st>>>(a);
-    else decode_rows_kernel<DT, 2, false><<<blocks, kTile, 0, st>>>(a);
+    if (mode != kWhole16) return hipErrorInvalidValue;
+    if (K == 1) decode_rows_kernel<DT, 1, kWhole16, true><<<blocks, kTile, 0, st>>>(a);
+    else decode_rows_kernel<DT, 2, kWhole16, true><<<blocks, kTile, 0, st>>>(a);
+    return hipGetLastError();
   }
+  LANCET_CODED_ROW_SWITCH(DT, mode,
+    if (K == 1) decode_rows_kernel<DT, 1, MODE><<<blocks, kTile, 0, st>>>(a);
+    else decode_rows_kernel<DT, 2, MODE><<<blocks, kTile, 0, st>>>(a))
   return hipGetLastError();
 }
 
@@ -716,12 +786,12 @@ hipError_t run_decode_rows(const void* expert_out, const void* gates, int gate_d
   a.E = E;
   a.C = C;
   a.slot_stride = slot_stride < 0 ? S : slot_stride;
-  const int per_vec = (dtype == LANCET_F32) ? 4 : 8;
-  const bool vec = (M % per_vec == 0) && aligned16(expert_out) && aligned16(out);
+  const int eb = dtype == LANCET_F32 ? 4 : 2;
+  const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(expert_out) && aligned16(out));
   switch (dtype) {
-    case LANCET_F32: return decode_launch<LANCET_F32>(a, K, vec, st);
-    case LANCET_BF16: return decode_launch<LANCET_BF16>(a, K, vec, st);
-    default: return decode_launch<LANCET_F16>(a, K, vec, st);
+    case LANCET_F32: return decode_launch<LANCET_F32>(a, K, mode, st);
+    case LANCET_BF16: return decode_launch<LANCET_BF16>(a, K, mode, st);
+    default: return decode_launch<LANCET_F16>(a, K, mode, st);
   }
 }
 
@@ -746,19 +816,14 @@ hipError_t run_redispatch_rows(const PtrTable& bufs, int P, int M, int C, int E,
   const size_t row_bytes = static_cast<size_t>(M) * elem_bytes;
   const long rows = static_cast<long>(E) * C;
   if (rows == 0 || row_bytes == 0) return hipSuccess;
-  bool vec = row_bytes % 16 == 0 && aligned16(out);
-  for (int p = 0; p < P; ++p) vec = vec && aligned16(bufs.p[p]);
-  const int units = vec ? static_cast<int>(row_bytes / 16) : M;
+  bool aligned = aligned16(out);
+  for (int p = 0; p < P; ++p) aligned = aligned && aligned16(bufs.p[p]);
+  const RowMode mode = row_mode(row_bytes, elem_bytes, aligned);
+  const int units = row_granules(mode, row_bytes, elem_bytes);
   const int shift = split_waves(units, rows, 2);  // two granules per lane: 426 -> 408 us
   const unsigned blocks = static_cast<unsigned>(((rows << shift) + kRowsPerBlock - 1) / kRowsPerBlock);
-  if (vec)
-    redispatch_rows_kernel<u32x4><<<blocks, kTile, 0, st>>>(bufs, P, E, C, units, shift, counts, static_cast<u32x4*>(out));
-  else if (elem_bytes == 4)
-    redispatch_rows_kernel<uint32_t><<<blocks, kTile, 0, st>>>(bufs, P, E, C, units, shift, counts,
-                                                               static_cast<uint32_t*>(out));
-  else
-    redispatch_rows_kernel<uint16_t><<<blocks, kTile, 0, st>>>(bufs, P, E, C, units, shift, counts,
-                                                               static_cast<uint16_t*>(out));
+  LANCET_ROW_SWITCH(mode, (redispatch_rows_kernel<MODE><<<blocks, kTile, 0, st>>>(
+                              bufs, P, E, C, static_cast<uint32_t>(row_bytes), units, shift, counts, static_cast<char*>(out))))
   return hipGetLastError();
 }
 
@@ -773,11 +838,11 @@ hipError_t run_encode_dg(const void* dy, const int32_t* idx, int S, int E, int K
 
 template <int DT>
 static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, void* out, int S, int M,
-                                   long rows, bool vec, hipStream_t st) {
-  const int shift = split_waves(vec ? M / Codec<DT>::kPerVec : M, rows, 2);  // two granules per lane: 442 -> 408 us
+                                   long rows, RowMode mode, hipStream_t st) {
+  constexpr int eb = sizeof(typename Codec<DT>::S);
+  const int shift = split_waves(row_granules(mode, static_cast<size_t>(M) * eb, eb), rows, 2);  // two granules per lane: 442 -> 408 us
   const unsigned blocks = static_cast<unsigned>(((rows << shift) + kRowsPerBlock - 1) / kRowsPerBlock);
-  if (vec) decode_dx_rows_kernel<DT, true><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift);
-  else decode_dx_rows_kernel<DT, false><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift);
+  LANCET_CODED_ROW_SWITCH(DT, mode, (decode_dx_rows_kernel<DT, MODE><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift)))
   return hipGetLastError();
 }
 
@@ -793,21 +858,20 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
     err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
-  const int per_vec = (dtype == LANCET_F32) ? 4 : 8;
-  const bool vec = (M % per_vec == 0) && aligned16(dy) && aligned16(out);
+  const int eb = dtype == LANCET_F32 ? 4 : 2;
+  const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(dy) && aligned16(out));
   switch (dtype) {
-    case LANCET_F32: return decode_dx_launch<LANCET_F32>(dy, gates, gate_dtype, src_map, out, S, M, rows, vec, st);
-    case LANCET_BF16: return decode_dx_launch<LANCET_BF16>(dy, gates, gate_dtype, src_map, out, S, M, rows, vec, st);
-    default: return decode_dx_launch<LANCET_F16>(dy, gates, gate_dtype, src_map, out, S, M, rows, vec, st);
+    case LANCET_F32: return decode_dx_launch<LANCET_F32>(dy, gates, gate_dtype, src_map, out, S, M, rows, mode, st);
+    case LANCET_BF16: return decode_dx_launch<LANCET_BF16>(dy, gates, gate_dtype, src_map, out, S, M, rows, mode, st);
+    default: return decode_dx_launch<LANCET_F16>(dy, gates, gate_dtype, src_map, out, S, M, rows, mode, st);
   }
 }
 
 template <int DT>
 static hipError_t decode_dg_launch(const void* dy, const void* expert_out, const int32_t* idx, const int32_t* loc,
-                                   void* out, int gd, int S, int M, int E, int C, int n, bool vec, hipStream_t st) {
+                                   void* out, int gd, int S, int M, int E, int C, int n, RowMode mode, hipStream_t st) {
   const int blocks = (n + kRowsPerBlock - 1) / kRowsPerBlock;
-  if (vec) decode_dg_kernel<DT, true><<<blocks, kTile, 0, st>>>(dy, expert_out, idx, loc, out, gd, S, M, E, C, n);
-  else decode_dg_kernel<DT, false><<<blocks, kTile, 0, st>>>(dy, expert_out, idx, loc, out, gd, S, M, E, C, n);
+  LANCET_CODED_ROW_SWITCH(DT, mode, (decode_dg_kernel<DT, MODE><<<blocks, kTile, 0, st>>>(dy, expert_out, idx, loc, out, gd, S, M, E, C, n)))
   return hipGetLastError();
 }
 
@@ -815,12 +879,12 @@ hipError_t run_decode_dg(const void* dy, const void* expert_out, const int32_t* 
                          int gate_dtype, int S, int M, int E, int C, int K, int dtype, hipStream_t st) {
   const int n = K * S;
   if (n == 0) return hipSuccess;
-  const int per_vec = (dtype == LANCET_F32) ? 4 : 8;
-  const bool vec = (M % per_vec == 0) && aligned16(dy) && aligned16(expert_out);
+  const int eb = dtype == LANCET_F32 ? 4 : 2;
+  const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(dy) && aligned16(expert_out));
   switch (dtype) {
-    case LANCET_F32: return decode_dg_launch<LANCET_F32>(dy, expert_out, idx, loc, out, gate_dtype, S, M, E, C, n, vec, st);
-    case LANCET_BF16: return decode_dg_launch<LANCET_BF16>(dy, expert_out, idx, loc, out, gate_dtype, S, M, E, C, n, vec, st);
-    default: return decode_dg_launch<LANCET_F16>(dy, expert_out, idx, loc, out, gate_dtype, S, M, E, C, n, vec, st);
+    case LANCET_F32: return decode_dg_launch<LANCET_F32>(dy, expert_out, idx, loc, out, gate_dtype, S, M, E, C, n, mode, st);
+    case LANCET_BF16: return decode_dg_launch<LANCET_BF16>(dy, expert_out, idx, loc, out, gate_dtype, S, M, E, C, n, mode, st);
+    default: return decode_dg_launch<LANCET_F16>(dy, expert_out, idx, loc, out, gate_dtype, S, M, E, C, n, mode, st);
   }
 }
 

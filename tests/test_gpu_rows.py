@@ -1,0 +1,65 @@
+"""Row movers at the row lengths where their pieces can go wrong: rows of less than 16 bytes (moved by elements), rows
+that end inside a 16-byte granule (the last one drawn back over the one before), rows of whole granules at addresses that
+are not aligned to them.  Against the oracle: rows bit-exact, 16-bit products within one unit in the last place, dot
+products within 1e-5 of sum|a_i * b_i| (fp32 sums of up to 1003 terms in another order)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as mo
+from tests.gpu_util import dev, make_inputs, rows_as_oracle, rows_to_torch, to_np, ulp_distance
+
+pytestmark = pytest.mark.gpu
+
+_TORCH = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+
+
+def _at(t, offset):
+    """t's values in memory that starts `offset` elements into an allocation."""
+    buf = torch.empty(t.numel() + offset, dtype=t.dtype, device=t.device)
+    view = buf[offset:].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("dt,M,offset", [("f32", 3, 0), ("f32", 4, 1), ("f32", 5, 0), ("f32", 255, 0), ("f32", 258, 3), ("bf16", 7, 0),
+                                         ("bf16", 8, 1), ("bf16", 9, 0), ("f16", 15, 1), ("bf16", 513, 0), ("f16", 1003, 0), ("bf16", 512, 3)])
+@pytest.mark.parametrize("k", [1, 2])
+def test_rows_of_any_length_and_alignment(pkg, dt, M, offset, k):
+    ops = pkg.ops
+    S, E, cf = 300, 6, 0.7
+    data, logits = make_inputs(M + k, S, M, E, zipf_bias=True)
+    x = rows_as_oracle(data, dt)
+    enc = mo.moe_encode_top2 if k == 2 else mo.moe_encode
+    g, il, used, _, disp = enc(x, logits, np.zeros(E, np.int32), cf, gate_is_logits=True, fast_scatter=True)
+    C = disp.shape[1]
+    assert (il[0] < 0).any() and (used < C).any()
+    rng = np.random.default_rng(M)
+    outs = [torch.empty(k * S, device="cuda"), torch.empty((2, k * S), dtype=torch.int32, device="cuda"),
+            torch.empty(E, dtype=torch.int32, device="cuda"), torch.empty(E, dtype=torch.int64, device="cuda"),
+            _at(torch.full((E, C, M), 7.0, dtype=_TORCH[dt], device="cuda"), offset)]
+    d_g, d_il, _, _, d_disp = ops.moe_encode(_at(rows_to_torch(data, dt), offset), dev(logits), None, cf, top_k=k, gate_is_logits=True, out=outs)
+    np.testing.assert_array_equal(to_np(d_il), il)
+    np.testing.assert_array_equal(to_np(d_disp), disp)
+
+    def near(got, want):                       # products and sums of two, rounded once
+        if dt == "f32":
+            np.testing.assert_array_equal(to_np(got), want)
+        else:
+            assert ulp_distance(got, torch.from_numpy(want).to(_TORCH[dt]).cuda()) <= 1
+
+    buf = rows_as_oracle(rng.standard_normal((E, C, M), dtype=np.float32), dt)
+    tok = rows_as_oracle(rng.standard_normal((S, M), dtype=np.float32), dt)
+    d_buf, d_tok = _at(rows_to_torch(buf, dt), offset), _at(rows_to_torch(tok, dt), offset)
+    w = to_np(d_g)                              # the GPU's own combine weights, so that products compare exactly
+    out = _at(torch.full((S, M), 7.0, dtype=_TORCH[dt], device="cuda"), offset)
+    rows = _at(torch.full((E, C, M), 7.0, dtype=_TORCH[dt], device="cuda"), offset)
+    near(ops.moe_decode(d_buf, d_g, d_il, top_k=k, out=out), mo.moe_decode(buf, w, il, k=k))
+    near(ops.moe_encode_dx(d_buf, d_il, top_k=k, out=out), mo.moe_encode_dx(buf, il, k))
+    near(ops.moe_decode_dx(d_tok, d_g, d_il, E, C, top_k=k, out=rows), mo.moe_decode_dx(tok, w, il, E, C, k))
+    dg = to_np(ops.moe_decode_dg(d_tok, d_buf, d_il, top_k=k))
+    bound = mo.moe_decode_dg(np.abs(tok), np.abs(buf), il, k)
+    assert (np.abs(dg - mo.moe_decode_dg(tok, buf, il, k)) <= 1e-5 * bound).all()
+    if k == 1:                                  # partition buffers: the same rows, the tail zero-filled again
+        merged = ops.moe_redispatch([d_disp], [d_il], out=rows)
+        np.testing.assert_array_equal(to_np(merged), disp)
