@@ -11,13 +11,26 @@ namespace lancet {
 constexpr int kRowsPerBlock = kTile / kWave;  // waves per workgroup; a wave moves a row or a share of one
 constexpr int kTailRows = 16;                 // rows zero-filled by one tail workgroup
 
+// A load that is issued where it stands: the compiler moves an ordinary one down to its use, behind other waits and
+// branches.  (A relaxed atomic of the narrowest scope is the same instruction.)
+template <typename T>
+__device__ __forceinline__ T ld_now(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // How a row is cut into the pieces its lanes move:
 //   kWhole16  16-byte granules, rows and pointers aligned to them;
 //   kAny16    rows of at least 16 bytes that end anywhere and start wherever their elements are aligned: 16-byte
 //             granules at unaligned addresses (the hardware takes them), the last one drawn back so that it ends with
 //             the row.  Its first bytes are then moved twice, with the same values.  At 10007 rows of 1003 bf16 values
-//             (60 experts, top-2) the scatter takes 17 us this way and 44 an element per lane, the decode 12 and 33;
+//             (60 experts, top-2) the scatter takes 13 us this way and 44 an element per lane, the decode 10 and 26;
 //   kElem2 / kElem4  one element per lane: rows of less than 16 bytes.
+// Loads: non-temporal (ld), except where rows come twice (ld_keep: the top-2 decode_dx reads every token row for both
+// slots, 402 -> 380 us at 65536 x 4096 bf16 and 39 -> 33 at 16384 x 1024 fp32; top-1 reads it once, 199 against 206) and
+// in the scatter (65536 x 4096 top-2 312 -> 307, 16384 x 2048 top-2 40 -> 36, nowhere slower).  The decode and the dot
+// products read every row once: 259 against 280 and 321 against 346 us with plain loads.  Stores are non-temporal
+// (plain: scatter 304 there, but 38 against 33 at 16384 x 1024 fp32 and 211 against 203 top-1).  Unaligned granules
+// share lines with their neighbours and are accessed plainly (10007 x 1003 bf16 scatter 13 against 16 us).
 enum RowMode { kWhole16, kAny16, kElem2, kElem4 };
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 
@@ -26,6 +39,7 @@ struct Granule {
   typedef u32x4 V;
   static __device__ __forceinline__ uint32_t at(int v, uint32_t) { return 16u * static_cast<uint32_t>(v); }
   static __device__ __forceinline__ V ld(const char* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
+  static __device__ __forceinline__ V ld_keep(const char* p) { return *reinterpret_cast<const u32x4*>(p); }
   static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { __builtin_nontemporal_store(x, (LANCET_GLOBAL u32x4*)p); }
   static __device__ __forceinline__ V zero() { return u32x4{0u, 0u, 0u, 0u}; }
 };
@@ -34,6 +48,7 @@ struct Granule<kAny16> {
   typedef u32x4 V;
   static __device__ __forceinline__ uint32_t at(int v, uint32_t row_bytes) { return min(16u * static_cast<uint32_t>(v), row_bytes - 16u); }
   static __device__ __forceinline__ V ld(const char* p) { return *reinterpret_cast<const u32x4_any*>(p); }
+  static __device__ __forceinline__ V ld_keep(const char* p) { return ld(p); }
   static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { *(LANCET_GLOBAL u32x4_any*)p = x; }
   static __device__ __forceinline__ V zero() { return u32x4{0u, 0u, 0u, 0u}; }
 };
@@ -42,6 +57,7 @@ struct GranuleElem {
   typedef E V;
   static __device__ __forceinline__ uint32_t at(int v, uint32_t) { return static_cast<uint32_t>(sizeof(E)) * static_cast<uint32_t>(v); }
   static __device__ __forceinline__ V ld(const char* p) { return __builtin_nontemporal_load(reinterpret_cast<const E*>(p)); }
+  static __device__ __forceinline__ V ld_keep(const char* p) { return ld(p); }
   static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { __builtin_nontemporal_store(x, (LANCET_GLOBAL E*)p); }
   static __device__ __forceinline__ V zero() { return E(0); }
 };
@@ -99,12 +115,20 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
     const bool has0 = v < a.row_vecs, has1 = v + step < a.row_vecs;
     const uint32_t o0 = G::at(v, a.row_bytes), o1 = G::at(v + step, a.row_bytes);
     V x0 = G::zero(), x1 = G::zero();
-    if (has0) x0 = G::ld(src + o0);
-    if (has1) x1 = G::ld(src + o1);
+    if (has0) x0 = G::ld_keep(src + o0);
+    if (has1) x1 = G::ld_keep(src + o1);
     // destinations picked at run time: typed as global memory so the stores are not flat.  (The routing words of a
     // row are the same for every lane; loading them through the scalar cache, or forming the row addresses on the
     // scalar unit from vector-loaded words, was measured slower: 346 and 340 us against 333 at the headline shape.)
     LANCET_GLOBAL char* dst[K];
+    int es[K], ls[K];
+    if (!DEST) {
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+        es[j] = ld_now(a.idx + static_cast<size_t>(j) * a.slot_stride + s);
+        ls[j] = ld_now(a.loc + static_cast<size_t>(j) * a.slot_stride + s);
+      }
+    }
     int nd = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j) {
@@ -114,9 +138,9 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
         if (d >= 0 && d < a.E * a.C) dst[nd++] = as_global(a.out + static_cast<size_t>(d) * a.row_bytes);
         continue;
       }
-      const int e = a.idx[static_cast<size_t>(j) * a.slot_stride + s];
-      int l = a.loc[static_cast<size_t>(j) * a.slot_stride + s];
-      bool ok = e >= 0 && e < a.E && l >= 0 && l < a.C;
+      const int e = es[j];
+      int l = ls[j];
+      bool ok = (e >= 0) & (e < a.E) & (l >= 0) & (l < a.C);
       if (ok && a.avail_used) ok = l < a.C - a.avail_used[e];
       dst[j] = as_global(a.out);
       if (ok && a.row_base) {
@@ -135,7 +159,7 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
     }
     for (v += 2 * step; v < a.row_vecs; v += step) {
       const uint32_t o = G::at(v, a.row_bytes);
-      const V x = G::ld(src + o);
+      const V x = G::ld_keep(src + o);
 #pragma unroll
       for (int j = 0; j < K; ++j)
         if (j < nd) G::st(dst[j] + o, x);
@@ -227,6 +251,50 @@ __device__ __forceinline__ u32x4 combine_vec(const u32x4 (&x)[K], const float (&
   return r;
 }
 
+// A gate value as it lies in memory: the aligned word that holds it.  (A 16-bit value's word may reach two bytes past
+// either end of the array, never past an aligned word of it.)
+struct GateWord {
+  uint32_t w, shift;
+  __device__ __forceinline__ void load(const void* p, size_t i, int gd) {
+    const char* at = static_cast<const char*>(p) + (i << (gd == 0 ? 2 : 1));
+    const uint32_t odd = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(at)) & 2u;
+    w = ld_now(reinterpret_cast<const uint32_t*>(at - odd));
+    shift = odd * 8u;
+  }
+  __device__ __forceinline__ float value(int gd) const {
+    const uint32_t h = w >> shift;
+    return gd == 0 ? __uint_as_float(w) : gd == 1 ? bf16_to_f32(h) : f16_to_f32(h & 0xffffu);
+  }
+};
+
+// routing words and combine weights of a token's K slots
+template <int K>
+struct RowWords {
+  int e[K], l[K];
+  GateWord g[K];
+  bool unit;  // no gates: every weight is one
+  int gd;
+  __device__ __forceinline__ void load(const int32_t* idx, const int32_t* loc, const void* gates, int gate_dtype, int stride, int s) {
+    load_dest(idx, gates, gate_dtype, stride, s);
+#pragma unroll
+    for (int j = 0; j < K; ++j) l[j] = ld_now(loc + static_cast<size_t>(j) * stride + s);
+  }
+  __device__ __forceinline__ void load_dest(const int32_t* dest, const void* gates, int gate_dtype, int stride, int s) {
+    unit = gates == nullptr;
+    gd = unit ? 0 : gate_dtype;
+    const void* gp = unit ? static_cast<const void*>(dest) : gates;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      e[j] = ld_now(dest + static_cast<size_t>(j) * stride + s);
+      l[j] = 0;
+      g[j].load(gp, static_cast<size_t>(j) * stride + s, gd);
+    }
+  }
+  __device__ __forceinline__ float weight(int j, bool ok) const { return ok ? (unit ? 1.f : g[j].value(gd)) : 0.f; }
+};
+
+// (Granules per lane: one for top-2, two for top-1, so that a wave has two row loads in flight either way.  65536 x 4096
+// bf16: top-2 264 us with one, 270 with two, 273 with four; top-1 193 / 177 / 188.)
 struct DecodeArgs {
   const void* expert_out;
   const void* gates;     // [K*S] of gate_dtype; null = all ones (moe_encode_dx)
@@ -250,23 +318,24 @@ __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
   const int part = static_cast<int>(gw & ((1u << a.wpr_shift) - 1u));
   if (s >= a.S) return;
   const int step = kWave << a.wpr_shift;
-  float g[K];
+  // Everything a row's addresses and weights come from is asked for at once and without a branch in between: asked
+  // for one after the other, each behind the test of the one before, the three words of a slot are three round trips
+  // to memory in front of the row's own.
+  RowWords<K> words;
+  if (DEST) words.load_dest(a.dest, a.gates, a.gate_dtype, a.slot_stride, s);
+  else words.load(a.idx, a.loc, a.gates, a.gate_dtype, a.slot_stride, s);
   size_t row[K];
   bool ok[K];
   bool any = false;
 #pragma unroll
   for (int j = 0; j < K; ++j) {
     if (DEST) {
-      const int d = a.dest[static_cast<size_t>(j) * a.slot_stride + s];
-      ok[j] = d >= 0 && d < a.E * a.C;
-      row[j] = ok[j] ? static_cast<size_t>(d) : 0;
+      ok[j] = (words.e[j] >= 0) & (words.e[j] < a.E * a.C);
+      row[j] = ok[j] ? static_cast<size_t>(words.e[j]) : 0;
     } else {
-      const int e = a.idx[static_cast<size_t>(j) * a.slot_stride + s];
-      const int l = a.loc[static_cast<size_t>(j) * a.slot_stride + s];
-      ok[j] = e >= 0 && e < a.E && l >= 0 && l < a.C;
-      row[j] = ok[j] ? (static_cast<size_t>(e) * a.C + l) : 0;
+      ok[j] = (words.e[j] >= 0) & (words.e[j] < a.E) & (words.l[j] >= 0) & (words.l[j] < a.C);
+      row[j] = ok[j] ? (static_cast<size_t>(words.e[j]) * a.C + words.l[j]) : 0;
     }
-    g[j] = ok[j] ? (a.gates ? ld_gate(a.gates, static_cast<size_t>(j) * a.slot_stride + s, a.gate_dtype) : 1.f) : 0.f;
     any = any || ok[j];
   }
   if constexpr (MODE == kWhole16 || MODE == kAny16) {
@@ -283,28 +352,34 @@ __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
       for (; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), z);
       return;
     }
-    for (; v + step < row_vecs; v += 2 * step) {  // two granules in flight per slot
-      const uint32_t oa = G::at(v, row_bytes), ob = G::at(v + step, row_bytes);
-      u32x4 xa[K], xb[K];
+    // two granules in flight per slot; the weights are looked at behind the first loads
+    u32x4 xa[K], xb[K];
+    const auto load = [&](int u) {
 #pragma unroll
       for (int j = 0; j < K; ++j) {
-        xa[j] = ok[j] ? G::ld(src[j] + oa) : z;
-        xb[j] = ok[j] ? G::ld(src[j] + ob) : z;
+        xa[j] = xb[j] = z;
+        if (ok[j] && u < row_vecs) xa[j] = G::ld(src[j] + G::at(u, row_bytes));
+        if (ok[j] && u + step < row_vecs) xb[j] = G::ld(src[j] + G::at(u + step, row_bytes));
       }
-      G::st(dst + oa, combine_vec<DT, K>(xa, g));
-      G::st(dst + ob, combine_vec<DT, K>(xb, g));
-    }
-    if (v < row_vecs) {
-      const uint32_t oa = G::at(v, row_bytes);
-      u32x4 xa[K];
+    };
+    load(v);
+    float g[K];
 #pragma unroll
-      for (int j = 0; j < K; ++j) xa[j] = ok[j] ? G::ld(src[j] + oa) : z;
-      G::st(dst + oa, combine_vec<DT, K>(xa, g));
+    for (int j = 0; j < K; ++j) g[j] = words.weight(j, ok[j]);
+    for (;;) {
+      if (v < row_vecs) G::st(dst + G::at(v, row_bytes), combine_vec<DT, K>(xa, g));
+      if (v + step < row_vecs) G::st(dst + G::at(v + step, row_bytes), combine_vec<DT, K>(xb, g));
+      v += 2 * step;
+      if (v >= row_vecs) break;
+      load(v);
     }
   } else {
     typedef typename Cd::S St;
     St* dst = static_cast<St*>(a.out) + static_cast<size_t>(s) * a.M;
     const St* base = static_cast<const St*>(a.expert_out);
+    float g[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) g[j] = words.weight(j, ok[j]);
     for (int i = part * kWave + lane; i < a.M; i += step) {
 #pragma clang fp contract(off)
       float acc = ok[0] ? mul_rn(g[0], Cd::get(base[row[0] * a.M + i])) : 0.f;
@@ -531,7 +606,7 @@ __global__ __launch_bounds__(kTile) void inverse_map_kernel(const int32_t* idx, 
 // grad_expert_out[e, l, :] = gates[i] * dy[s, :] for the slot-token i = src[e*C+l] (s = i mod S), zero
 // for rows nobody owns: decode_backward_data_kernel (tutel_moe_dispatch.cu:118-124, 523-533) without
 // the memset + atomicAdd; every output byte is written once.
-template <int DT, int MODE>
+template <int DT, int MODE, int K>
 __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, const void* gates, int gd,
                                                                const int32_t* src, void* out, int S, int M,
                                                                long rows, int wpr_shift) {
@@ -544,6 +619,8 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
   const int step = kWave << wpr_shift;
   if (r >= rows) return;
   const int i = src[r];
+  // the weight first, then the row: with both asked for at once the reads crowd out the writes here (262144 x 512 bf16
+  // top-1: 83 against 90 us)
   const float g1[1] = {i >= 0 ? ld_gate(gates, i, gd) : 0.f};
   const size_t s = i >= 0 ? static_cast<size_t>(i % S) : 0;
   if constexpr (MODE == kWhole16 || MODE == kAny16) {
@@ -557,17 +634,18 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
       for (; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), z);
       return;
     }
+    const auto ld = [](const char* q) { return K == 2 ? G::ld_keep(q) : G::ld(q); };
     const char* sp = static_cast<const char*>(dy) + s * row_bytes;
     for (; v + step < row_vecs; v += 2 * step) {
       const uint32_t oa = G::at(v, row_bytes), ob = G::at(v + step, row_bytes);
-      const u32x4 xa[1] = {G::ld(sp + oa)};
-      const u32x4 xb[1] = {G::ld(sp + ob)};
+      const u32x4 xa[1] = {ld(sp + oa)};
+      const u32x4 xb[1] = {ld(sp + ob)};
       G::st(dst + oa, combine_vec<DT, 1>(xa, g1));
       G::st(dst + ob, combine_vec<DT, 1>(xb, g1));
     }
     if (v < row_vecs) {
       const uint32_t oa = G::at(v, row_bytes);
-      const u32x4 xa[1] = {G::ld(sp + oa)};
+      const u32x4 xa[1] = {ld(sp + oa)};
       G::st(dst + oa, combine_vec<DT, 1>(xa, g1));
     }
   } else {
@@ -619,7 +697,7 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
   const int i = blockIdx.x * kRowsPerBlock + w;
   if (i >= n) return;
   const int e = idx[i], l = loc[i];
-  if (!(e >= 0 && e < E && l >= 0 && l < C)) {
+  if (!((e >= 0) & (e < E) & (l >= 0) & (l < C))) {
     if (lane == 0) st_gate(out, i, 0.f, gd);
     return;
   }
@@ -690,6 +768,12 @@ static inline int row_granules(RowMode mode, size_t row_bytes, int elem_bytes) {
     default: { constexpr int MODE = kElem4; __VA_ARGS__; } break;         \
   }
 
+// The scatter of rows that several waves share (more than 1 KB) asks for LDS it does not use, which keeps 5 of its
+// workgroups on a CU instead of 8: with all wave slots taken its reads crowd out its writes.  8 / 6 / 5 / 4 / 3 workgroups:
+// 344 / 337 / 324 / 350 / 420 us at 65536 x 4096 bf16 top-2, 206 / 208 / 200 / 221 / 243 top-1, 165 against 160 at rows of
+// 2048.  Rows of one wave want every slot: 90 / 92 / 99 / 108 us at 262144 x 512.  The gather kernels do not gain.
+constexpr size_t kScatterLds = 27000;
+
 hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, const int32_t* loc,
                             const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
                             const int32_t* rows_hi,
@@ -721,14 +805,15 @@ hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, con
   a.tail_chunks = rows_hi ? (C + kTailRows - 1) / kTailRows : 0;
   const long blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_chunks) * E;
   if (blocks == 0) return hipSuccess;
+  const size_t lds = a.row_vecs > kWave ? kScatterLds : 0;
   if (dest) {
-    if (K == 1) scatter_rows_kernel<kWhole16, 1, true><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
-    else scatter_rows_kernel<kWhole16, 2, true><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
+    if (K == 1) scatter_rows_kernel<kWhole16, 1, true><<<static_cast<unsigned>(blocks), kTile, lds, st>>>(a);
+    else scatter_rows_kernel<kWhole16, 2, true><<<static_cast<unsigned>(blocks), kTile, lds, st>>>(a);
     return hipGetLastError();
   }
   LANCET_ROW_SWITCH(mode,
-    if (K == 1) scatter_rows_kernel<MODE, 1><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a);
-    else scatter_rows_kernel<MODE, 2><<<static_cast<unsigned>(blocks), kTile, 0, st>>>(a))
+    if (K == 1) scatter_rows_kernel<MODE, 1><<<static_cast<unsigned>(blocks), kTile, lds, st>>>(a);
+    else scatter_rows_kernel<MODE, 2><<<static_cast<unsigned>(blocks), kTile, lds, st>>>(a))
   return hipGetLastError();
 }
 
@@ -756,7 +841,7 @@ hipError_t run_zero_bytes(void* p, size_t nbytes, hipStream_t st) {
 template <int DT>
 static hipError_t decode_launch(DecodeArgs a, int K, RowMode mode, hipStream_t st) {
   if (a.S == 0 || a.M == 0) return hipSuccess;
-  a.wpr_shift = split_waves(row_granules(mode, static_cast<size_t>(a.M) * sizeof(typename Codec<DT>::S), sizeof(typename Codec<DT>::S)), a.S, 2);
+  a.wpr_shift = split_waves(row_granules(mode, static_cast<size_t>(a.M) * sizeof(typename Codec<DT>::S), sizeof(typename Codec<DT>::S)), a.S, K == 1 ? 2 : 1);
   const unsigned blocks = static_cast<unsigned>(((static_cast<long>(a.S) << a.wpr_shift) + kRowsPerBlock - 1) / kRowsPerBlock);
   if (a.dest) {
     if (mode != kWhole16) return hipErrorInvalidValue;
@@ -838,11 +923,13 @@ hipError_t run_encode_dg(const void* dy, const int32_t* idx, int S, int E, int K
 
 template <int DT>
 static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, void* out, int S, int M,
-                                   long rows, RowMode mode, hipStream_t st) {
+                                   long rows, int K, RowMode mode, hipStream_t st) {
   constexpr int eb = sizeof(typename Codec<DT>::S);
   const int shift = split_waves(row_granules(mode, static_cast<size_t>(M) * eb, eb), rows, 2);  // two granules per lane: 442 -> 408 us
   const unsigned blocks = static_cast<unsigned>(((rows << shift) + kRowsPerBlock - 1) / kRowsPerBlock);
-  LANCET_CODED_ROW_SWITCH(DT, mode, (decode_dx_rows_kernel<DT, MODE><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift)))
+  LANCET_CODED_ROW_SWITCH(DT, mode,
+    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift);
+    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift))
   return hipGetLastError();
 }
 
@@ -861,9 +948,9 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
   const int eb = dtype == LANCET_F32 ? 4 : 2;
   const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(dy) && aligned16(out));
   switch (dtype) {
-    case LANCET_F32: return decode_dx_launch<LANCET_F32>(dy, gates, gate_dtype, src_map, out, S, M, rows, mode, st);
-    case LANCET_BF16: return decode_dx_launch<LANCET_BF16>(dy, gates, gate_dtype, src_map, out, S, M, rows, mode, st);
-    default: return decode_dx_launch<LANCET_F16>(dy, gates, gate_dtype, src_map, out, S, M, rows, mode, st);
+    case LANCET_F32: return decode_dx_launch<LANCET_F32>(dy, gates, gate_dtype, src_map, out, S, M, rows, K, mode, st);
+    case LANCET_BF16: return decode_dx_launch<LANCET_BF16>(dy, gates, gate_dtype, src_map, out, S, M, rows, K, mode, st);
+    default: return decode_dx_launch<LANCET_F16>(dy, gates, gate_dtype, src_map, out, S, M, rows, K, mode, st);
   }
 }
 
