@@ -318,6 +318,13 @@ int lancet_moe_decode_dx(const void* dy, const void* gates_s, const int32_t* ind
                          int64_t S, int64_t M, int64_t E, int64_t C, int top_k, int dtype, int gate_dtype,
                          void* grad_expert_out, void* workspace, size_t workspace_bytes,
                          lancet_stream_t stream);
+/* Both gradients of one moe_decode (MoeDecodeGrad, src/op/grad/moe.cc:60-90, which asks for the two ops) in one pass over
+ * the rows: grad_expert_out as moe_decode_dx, grad_gates_s as moe_decode_dg (the dot products summed in another order).
+ * The workspace is moe_decode_dx's. */
+int lancet_moe_decode_grad(const void* dy, const void* expert_out, const void* gates_s, const int32_t* indices_locations,
+                           int64_t S, int64_t M, int64_t E, int64_t C, int top_k, int dtype, int gate_dtype,
+                           void* grad_expert_out, void* grad_gates_s, void* workspace, size_t workspace_bytes,
+                           lancet_stream_t stream);
 /* moe_decode_dg: grad_gates_s[slot-token] = <expert_out[idx, loc, :], dy[s, :]>, 0 for dropped slots.
  * Replaces MoeDecodeDg / launch_decode_backward_gate (moe.cc:1397-1481; kernel_util.cuh:49;
  * tutel_moe_dispatch.cu:126-157,535-546). */

@@ -81,6 +81,7 @@ SIGNATURES = {
     "lancet_moe_encode_dgate": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _int, _u32, _vp, _vp]),
     "lancet_moe_decode_dx_workspace_bytes": (_sz, [_i64, _i64]),
     "lancet_moe_decode_dx": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp, _vp, _sz, _vp]),
+    "lancet_moe_decode_grad": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp, _vp, _vp, _sz, _vp]),
     "lancet_moe_decode_dg": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp, _vp]),
     "lancet_moe_top2_normalize_gates": (_int, [_vp, _vp, _i64, _int, _vp, _vp]),
     "lancet_moe_merge_masks_workspace_bytes": (_sz, [_int, _i64]),

@@ -637,6 +637,27 @@ extern "C" int lancet_moe_decode_dx(const void* dy, const void* gates_s, const i
                           static_cast<int>(E), static_cast<int>(C), top_k, dtype, S_(stream)));
 }
 
+extern "C" int lancet_moe_decode_grad(const void* dy, const void* expert_out, const void* gates_s, const int32_t* indices_locations,
+                                      int64_t S, int64_t M, int64_t E, int64_t C, int top_k, int dtype, int gate_dtype,
+                                      void* grad_expert_out, void* grad_gates_s, void* workspace, size_t workspace_bytes,
+                                      lancet_stream_t stream) {
+  if (((!dy && M > 0) || !gates_s || !indices_locations || !grad_gates_s) && S > 0) return LANCET_ERR_NULL;
+  if ((!grad_expert_out || (!expert_out && S > 0)) && C > 0 && M > 0) return LANCET_ERR_NULL;
+  const int eb = elem_bytes(dtype), gb = elem_bytes(gate_dtype);
+  if (!eb || !gb) return LANCET_ERR_DTYPE;
+  if (int r = check_dims(S, M, E, C)) return r;
+  if (top_k != 1 && top_k != 2) return LANCET_ERR_TOPK;
+  if (C > 0 && (!workspace || workspace_bytes < lancet_moe_decode_dx_workspace_bytes(E, C))) return LANCET_ERR_WORKSPACE;
+  if (misaligned(dy, eb) || misaligned(expert_out, eb) || misaligned(grad_expert_out, eb) || misaligned(gates_s, gb) ||
+      misaligned(grad_gates_s, gb) || misaligned(indices_locations, 4) || misaligned(workspace, 4))
+    return LANCET_ERR_ALIGN;
+  const int s = static_cast<int>(S);
+  return rc(run_decode_grad(dy, expert_out, gates_s, gate_dtype, indices_locations,
+                            indices_locations + static_cast<size_t>(top_k) * s, grad_expert_out, grad_gates_s,
+                            static_cast<int32_t*>(workspace), s, static_cast<int>(M), static_cast<int>(E), static_cast<int>(C),
+                            top_k, dtype, S_(stream)));
+}
+
 extern "C" int lancet_moe_decode_dg(const void* dy, const void* expert_out, const int32_t* indices_locations, int64_t S,
                                     int64_t M, int64_t E, int64_t C, int top_k, int dtype, int gate_dtype, void* grad_gates_s,
                                     lancet_stream_t stream) {

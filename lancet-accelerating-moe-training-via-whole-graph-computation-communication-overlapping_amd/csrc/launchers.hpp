@@ -67,6 +67,9 @@ hipError_t run_encode_dgate(const void* dy, const void* gate, const int32_t* idx
                             int gate_dtype, void* out, hipStream_t st);
 hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, const int32_t* idx, const int32_t* loc, void* out,
                          int32_t* src_map, int S, int M, int E, int C, int K, int dtype, hipStream_t st);
+hipError_t run_decode_grad(const void* dy, const void* expert_out, const void* gates, int gate_dtype, const int32_t* idx,
+                           const int32_t* loc, void* d_expert_out, void* d_gates, int32_t* src_map, int S, int M, int E,
+                           int C, int K, int dtype, hipStream_t st);
 hipError_t run_decode_dg(const void* dy, const void* expert_out, const int32_t* idx, const int32_t* loc, void* out,
                          int gate_dtype, int S, int M, int E, int C, int K, int dtype, hipStream_t st);
 

@@ -5,6 +5,7 @@ that differentiate with torch.autograd.
       d data = moe_encode_dx(dy[4], y[1]);  d gate = moe_encode_dg(dy[0], y[1], E);  used_capacity: none
   moe_decode (MoeDecodeGrad, :60-90):
       d data = moe_decode_dx(dy, gate, indices_locations, E, C);  d gate = moe_decode_dg(dy, data, indices_locations)
+      (moe_decode_grad: both in one pass over the rows)
 
 The reference differentiates the one form of the op it has: top-1 on a gate that holds probabilities.  The forms
 this library adds (top_k = 2 with GShard's normalised combine weights, docker/resources/sharded_moe.py:253-324, and
@@ -73,10 +74,14 @@ class _MoeDecode(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         data, gate, indloc = ctx.saved_tensors
-        E, C, _ = data.shape
         dy = dy.contiguous()
-        return (ops.moe_decode_dx(dy, gate, indloc, E, C, top_k=ctx.top_k),
-                ops.moe_decode_dg(dy, data, indloc, top_k=ctx.top_k, gate_dtype=gate.dtype), None, None)
+        # both gradients in one pass over the rows, or the one that is asked for
+        if all(ctx.needs_input_grad[:2]):
+            return ops.moe_decode_grad(dy, data, gate, indloc, top_k=ctx.top_k) + (None, None)
+        E, C, _ = data.shape
+        return (ops.moe_decode_dx(dy, gate, indloc, E, C, top_k=ctx.top_k) if ctx.needs_input_grad[0] else None,
+                ops.moe_decode_dg(dy, data, indloc, top_k=ctx.top_k, gate_dtype=gate.dtype) if ctx.needs_input_grad[1] else None,
+                None, None)
 
 
 def moe_encode(data, gate, used_capacity=None, capacity_factor=1.0, top_k=1, gate_is_logits=False, gate2_noise=None,

@@ -445,6 +445,27 @@ def moe_decode_dg(dy, data, indices_locations, top_k=1, gate_dtype=torch.float32
     return out
 
 
+def moe_decode_grad(dy, data, gate, indices_locations, top_k=1, workspace=None, out=None):
+    """Both gradients of moe_decode(data [E,C,M], gate [k*S], indices_locations) given dy [S,M], in one pass over the rows:
+    what moe_decode_dx and moe_decode_dg return (MoeDecodeGrad, src/op/grad/moe.cc:60-90)."""
+    lib = capi.load()
+    _dev(dy, "dy"), _dev(data, "data"), _dev(gate, "gate")
+    _need(dy.dim() == 2 and data.dim() == 3 and dy.dtype == data.dtype and dy.shape[1] == data.shape[2],
+          "dy must be [S,M] and data [E,C,M] of one dtype")
+    S = _check_indloc(indices_locations, top_k)
+    _need(dy.shape[0] == S and gate.dim() == 1 and gate.shape[0] == top_k * S, "dy, gate and indices_locations disagree")
+    E, Cap, M = data.shape
+    if out is None:
+        out = torch.empty_like(data), torch.empty_like(gate)
+    d_data, d_gate = out
+    _need(d_gate.dtype == gate.dtype, "the gate gradient takes the gate's dtype")
+    ws = _workspace(int(lib.lancet_moe_decode_dx_workspace_bytes(E, Cap)), dy.device, workspace)
+    st = lib.lancet_moe_decode_grad(_p(dy), _p(data), _p(gate), _p(indices_locations), S, M, E, Cap, top_k, _dtype_code(dy),
+                                    _gate_code(gate), _p(d_data), _p(d_gate), _p(ws), ws.numel(), _stream())
+    capi.check(st, "lancet_moe_decode_grad")
+    return d_data, d_gate
+
+
 def moe_top2_normalize_gates(raw_gates, merged_indices_locations):
     """Combine weights of the top-2 extension from per-slot raw gate values [2S] and the merged
     indices_locations [2, 2S]."""

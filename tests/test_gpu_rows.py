@@ -60,6 +60,32 @@ def test_rows_of_any_length_and_alignment(pkg, dt, M, offset, k):
     dg = to_np(ops.moe_decode_dg(d_tok, d_buf, d_il, top_k=k))
     bound = mo.moe_decode_dg(np.abs(tok), np.abs(buf), il, k)
     assert (np.abs(dg - mo.moe_decode_dg(tok, buf, il, k)) <= 1e-5 * bound).all()
+    d_rows, d_w = ops.moe_decode_grad(d_tok, d_buf, d_g, d_il, top_k=k, out=(torch.full_like(rows, 7.0), torch.full_like(d_g, 7.0)))
+    near(d_rows, mo.moe_decode_dx(tok, w, il, E, C, k))
+    assert (np.abs(to_np(d_w) - mo.moe_decode_dg(tok, buf, il, k)) <= 1e-5 * bound).all() and not to_np(d_w)[il[0] < 0].any()
     if k == 1:                                  # partition buffers: the same rows, the tail zero-filled again
         merged = ops.moe_redispatch([d_disp], [d_il], out=rows)
         np.testing.assert_array_equal(to_np(merged), disp)
+
+
+@pytest.mark.parametrize("S,k,M,dt,gdt", [(7, 1, 64, "f32", "f32"), (4096, 2, 24, "bf16", "bf16"), (4097, 2, 24, "bf16", "f32"), (8192, 1, 8, "f16", "f16"),
+                                          (8193, 1, 8, "f32", "bf16"), (700, 2, 512, "bf16", "f32"), (700, 2, 1024, "f32", "f32"), (300, 2, 4100, "bf16", "f16")])
+def test_decode_gradients_in_one_pass(pkg, S, k, M, dt, gdt):
+    """moe_decode_grad against the two ops it stands for: rows bit for bit (the same products and roundings), weights within
+    1e-5 of sum|a_i * b_i| plus one rounding to the gate's type.  Sizes on both sides of the 8192 slots up to which the
+    workgroups that clear unowned rows walk the slots themselves; rows of one wave, of several, and longer than a pass."""
+    ops = pkg.ops
+    E = 5
+    gen = torch.Generator(device="cuda").manual_seed(S + M)
+    normal = lambda *shape: torch.empty(shape, device="cuda").normal_(generator=gen).to(_TORCH[dt])  # noqa: E731
+    logits = torch.empty((S, E), device="cuda").normal_(generator=gen) + torch.arange(E, device="cuda")
+    g, il, _, _, disp = ops.moe_encode(normal(S, M), logits.to(_TORCH[gdt]), None, 0.8, top_k=k, gate_is_logits=True)
+    C = disp.shape[1]
+    data, dy = normal(E, C, M), normal(S, M)
+    d_data, d_gate = ops.moe_decode_grad(dy, data, g, il, top_k=k, out=(torch.full_like(data, 7.0), torch.full_like(g, 7.0)))
+    assert torch.equal(d_data, ops.moe_decode_dx(dy, g, il, E, C, top_k=k))
+    want = ops.moe_decode_dg(dy, data, il, top_k=k)
+    bound = ops.moe_decode_dg(dy.abs(), data.abs(), il, top_k=k)
+    ulp = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[gdt]
+    assert d_gate.dtype == _TORCH[gdt]
+    assert bool(((d_gate.float() - want).abs() <= 1e-5 * bound + ulp * want.abs()).all())
