@@ -18,6 +18,29 @@ __device__ __forceinline__ T ld_now(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
+// 2^q lanes share a row: part of a wave, a wave or several.  (Rows of less than a wave used to take a whole one: rows of
+// 512 bytes, 131072 of them, decode top-1 41 -> 24 us, decode_dx 54 -> 30, decode_dg 39 -> 22, scatter 29 -> 23; rows of 1 KB
+// at two granules per lane, 262144 of them, decode 83 -> 69.)  The thread's row, its place among the row's lanes and the
+// distance in granules between the ones it moves.  Neighbouring lanes and waves move neighbouring granules in row order:
+// short waves in row order keep the chip-wide streams close to address order, which the memory system rewards.
+struct RowShare {
+  int r, v, step;
+};
+__device__ __forceinline__ RowShare row_share(int q) {
+  const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kTile + threadIdx.x;
+  RowShare h;
+  h.r = static_cast<int>(t >> q);
+  h.step = 1 << q;
+  h.v = static_cast<int>(static_cast<uint32_t>(t) & static_cast<uint32_t>(h.step - 1));
+  return h;
+}
+// sum over the row's lanes inside a wave
+__device__ __forceinline__ float share_sum(float x, int q) {
+  if (q >= 6) return wave_sum(x);
+  for (int o = 1 << q >> 1; o > 0; o >>= 1) x += __shfl_xor(x, o, kWave);
+  return x;
+}
+
 // How a row is cut into the pieces its lanes move:
 //   kWhole16  16-byte granules, rows and pointers aligned to them;
 //   kAny16    rows of at least 16 bytes that end anywhere and start wherever their elements are aligned: 16-byte
@@ -87,7 +110,7 @@ struct ScatterArgs {
                               // token count when this call moves a token range of a larger mask)
   uint32_t row_bytes;
   int row_vecs;               // granules per row
-  int wpr_shift;              // 2^wpr_shift waves share one token row
+  int q;                      // 2^q lanes share one token row
   int token_blocks;
   int tail_chunks;            // tail workgroups per expert
 };
@@ -96,22 +119,15 @@ template <int MODE, int K, bool DEST = false>
 __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
   typedef Granule<MODE> G;
   typedef typename G::V V;
-  const int w = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
   if (static_cast<int>(blockIdx.x) < a.token_blocks) {
-    // 2^wpr_shift waves share a token row, each moving every 2^wpr_shift-th run of 64 granules: short
-    // waves in row order keep the chip-wide write stream close to address order, which the memory system
-    // rewards (one granule per lane streams ~8 % faster than a wave walking a whole 8 KB row)
-    const uint32_t gw = blockIdx.x * static_cast<uint32_t>(kRowsPerBlock) + w;  // below 2^32: the launcher sees to it
-    const int s = static_cast<int>(gw >> a.wpr_shift);
-    const int part = static_cast<int>(gw & ((1u << a.wpr_shift) - 1u));
+    const RowShare h = row_share(a.q);
+    const int s = h.r, step = h.step;
+    int v = h.v;
     if (s >= a.S) return;
     // The row's granules do not depend on the routing, only their destinations do: the first loads of the row
     // go out before idx / loc are known, so that a wave waits for the longer of the two latencies and not for
     // their sum (a dropped token's row is then read for nothing).  338 -> 333 us at the headline shape.
     const char* src = a.data + static_cast<size_t>(s) * a.row_bytes;
-    const int step = kWave << a.wpr_shift;
-    int v = part * kWave + lane;
     const bool has0 = v < a.row_vecs, has1 = v + step < a.row_vecs;
     const uint32_t o0 = G::at(v, a.row_bytes), o1 = G::at(v + step, a.row_bytes);
     V x0 = G::zero(), x1 = G::zero();
@@ -172,10 +188,12 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
     const int used = a.rows_hi[e] - (a.rows_lo ? a.rows_lo[e] : 0);
     const int first = max(used, 0) + ch * kTailRows;
     const int last = min(first + kTailRows, a.C);
-    for (int r = first + w; r < last; r += kRowsPerBlock) {
-      LANCET_GLOBAL char* row = as_global(a.out + (static_cast<size_t>(e) * a.C + r) * a.row_bytes);
-      for (int v = lane; v < a.row_vecs; v += kWave) G::st(row + G::at(v, a.row_bytes), G::zero());
-    }
+    // the rows lie one behind the other: one run of granules
+    if (first >= last) return;
+    LANCET_GLOBAL char* run = as_global(a.out + (static_cast<size_t>(e) * a.C + first) * a.row_bytes);
+    const uint32_t bytes = static_cast<uint32_t>(last - first) * a.row_bytes;
+    const uint32_t n = (bytes + sizeof(V) - 1) / sizeof(V);
+    for (uint32_t v = threadIdx.x; v < n; v += kTile) G::st(run + G::at(v, bytes), G::zero());
   }
 }
 
@@ -305,19 +323,15 @@ struct DecodeArgs {
   void* out;             // [S, M]
   int S, M, E, C;
   int slot_stride;       // distance between the slots of one token in gates / idx / loc
-  int wpr_shift;         // 2^wpr_shift waves share one token row (each takes every 2^wpr_shift-th run of 64 granules)
+  int q;                 // 2^q lanes share one token row
 };
 
 template <int DT, int K, int MODE, bool DEST = false>
 __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
   typedef Codec<DT> Cd;
-  const int w = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  const uint32_t gw = blockIdx.x * static_cast<uint32_t>(kRowsPerBlock) + w;
-  const int s = static_cast<int>(gw >> a.wpr_shift);
-  const int part = static_cast<int>(gw & ((1u << a.wpr_shift) - 1u));
+  const RowShare h = row_share(a.q);
+  const int s = h.r, step = h.step;
   if (s >= a.S) return;
-  const int step = kWave << a.wpr_shift;
   // Everything a row's addresses and weights come from is asked for at once and without a branch in between: asked
   // for one after the other, each behind the test of the one before, the three words of a slot are three round trips
   // to memory in front of the row's own.
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
 #pragma unroll
     for (int j = 0; j < K; ++j) src[j] = static_cast<const char*>(a.expert_out) + row[j] * row_bytes;
     const u32x4 z = {0u, 0u, 0u, 0u};
-    int v = part * kWave + lane;
+    int v = h.v;
     if (!any) {
       for (; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), z);
       return;
@@ -380,7 +394,7 @@ __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
     float g[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) g[j] = words.weight(j, ok[j]);
-    for (int i = part * kWave + lane; i < a.M; i += step) {
+    for (int i = h.v; i < a.M; i += step) {
 #pragma clang fp contract(off)
       float acc = ok[0] ? mul_rn(g[0], Cd::get(base[row[0] * a.M + i])) : 0.f;
       if (K == 2) acc = add_rn(acc, ok[1] ? mul_rn(g[1], Cd::get(base[row[1] * a.M + i])) : 0.f);
@@ -609,14 +623,11 @@ __global__ __launch_bounds__(kTile) void inverse_map_kernel(const int32_t* idx, 
 template <int DT, int MODE, int K>
 __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, const void* gates, int gd,
                                                                const int32_t* src, void* out, int S, int M,
-                                                               long rows, int wpr_shift) {
+                                                               long rows, int q) {
   typedef Codec<DT> Cd;
-  const int w = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  const uint32_t gw = blockIdx.x * static_cast<uint32_t>(kRowsPerBlock) + w;
-  const long r = gw >> wpr_shift;
-  const int part = static_cast<int>(gw & ((1u << wpr_shift) - 1u));
-  const int step = kWave << wpr_shift;
+  const RowShare h = row_share(q);
+  const long r = h.r;
+  const int step = h.step;
   if (r >= rows) return;
   const int i = src[r];
   // the weight first, then the row: with both asked for at once the reads crowd out the writes here (262144 x 512 bf16
@@ -629,7 +640,7 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
     const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
     LANCET_GLOBAL char* dst = as_global(static_cast<char*>(out) + static_cast<size_t>(r) * row_bytes);
     const u32x4 z = {0u, 0u, 0u, 0u};
-    int v = part * kWave + lane;
+    int v = h.v;
     if (i < 0) {
       for (; v < row_vecs; v += step) G::st(dst + G::at(v, row_bytes), z);
       return;
@@ -652,7 +663,7 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
     typedef typename Cd::S St;
     St* dst = static_cast<St*>(out) + static_cast<size_t>(r) * M;
     const St* sp = static_cast<const St*>(dy) + s * M;
-    for (int k = part * kWave + lane; k < M; k += step)
+    for (int k = h.v; k < M; k += step)
       dst[k] = i >= 0 ? Cd::put(mul_rn(g1[0], Cd::get(sp[k]))) : Cd::put(0.f);
   }
 }
@@ -690,15 +701,14 @@ __device__ __forceinline__ u32x4 drop_bytes(u32x4 x, uint32_t n) {
 template <int DT, int MODE>
 __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const void* expert_out,
                                                           const int32_t* idx, const int32_t* loc, void* out, int gd,
-                                                          int S, int M, int E, int C, int n) {
+                                                          int S, int M, int E, int C, int n, int q) {
   typedef Codec<DT> Cd;
-  const int w = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int i = blockIdx.x * kRowsPerBlock + w;
+  const RowShare h = row_share(q);  // at most a wave
+  const int i = h.r;
   if (i >= n) return;
   const int e = idx[i], l = loc[i];
   if (!((e >= 0) & (e < E) & (l >= 0) & (l < C))) {
-    if (lane == 0) st_gate(out, i, 0.f, gd);
+    if (h.v == 0) st_gate(out, i, 0.f, gd);
     return;
   }
   const size_t s = static_cast<size_t>(i % S);
@@ -710,7 +720,7 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
     const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
     const char* a = static_cast<const char*>(expert_out) + row * row_bytes;
     const char* b = static_cast<const char*>(dy) + s * row_bytes;
-    for (int v = lane; v < row_vecs; v += kWave) {
+    for (int v = h.v; v < row_vecs; v += h.step) {
       const uint32_t o = G::at(v, row_bytes);
       u32x4 x = G::ld(a + o), y = G::ld(b + o);
       if (MODE == kAny16 && o != 16u * static_cast<uint32_t>(v)) x = drop_bytes<DT>(x, 16u * static_cast<uint32_t>(v) - o);
@@ -720,10 +730,10 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
     typedef typename Cd::S St;
     const St* a = static_cast<const St*>(expert_out) + row * M;
     const St* b = static_cast<const St*>(dy) + s * M;
-    for (int k = lane; k < M; k += kWave) acc += Cd::get(a[k]) * Cd::get(b[k]);
+    for (int k = h.v; k < M; k += h.step) acc += Cd::get(a[k]) * Cd::get(b[k]);
   }
-  acc = wave_sum(acc);
-  if (lane == 0) st_gate(out, i, acc, gd);
+  acc = share_sum(acc, q);
+  if (h.v == 0) st_gate(out, i, acc, gd);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -747,7 +757,7 @@ struct DecodeGradArgs {
   int S, E, C, gate_dtype;
   uint32_t row_bytes;
   int row_vecs;            // granules per row
-  int wpr_shift;           // 2^wpr_shift waves of one workgroup share a token
+  int q;                   // 2^q lanes of one workgroup share a token
   int token_blocks;
   int tail_rows;           // rows looked at by one workgroup behind the tokens' (at most 32 * kTile)
   int tail_chunks;         // such workgroups per expert
@@ -775,19 +785,18 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
       }
       __syncthreads();
     }
-    for (int r = first + w; r < last; r += kRowsPerBlock) {
+    const int q = min(a.q, 6);
+    for (int r = first + (static_cast<int>(threadIdx.x) >> q); r < last; r += kTile >> q) {
       const size_t row = static_cast<size_t>(e) * a.C + r;
       const bool owned = a.owner ? a.owner[row] >= 0 : ((s_owned[(r - first) >> 5] >> ((r - first) & 31)) & 1u) != 0;
       if (owned) continue;
       LANCET_GLOBAL char* dst = as_global(a.d_expert_out + row * a.row_bytes);
-      for (int v = lane; v < a.row_vecs; v += kWave) G::st(dst + G::at(v, a.row_bytes), G::zero());
+      for (int v = threadIdx.x & ((1 << q) - 1); v < a.row_vecs; v += 1 << q) G::st(dst + G::at(v, a.row_bytes), G::zero());
     }
     return;
   }
-  const uint32_t gw = blockIdx.x * static_cast<uint32_t>(kRowsPerBlock) + w;
-  const int s = static_cast<int>(gw >> a.wpr_shift);
-  const int part = static_cast<int>(gw & ((1u << a.wpr_shift) - 1u));
-  const int step = kWave << a.wpr_shift;
+  const RowShare h = row_share(a.q);
+  const int s = h.r, step = h.step;
   float acc[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) acc[j] = 0.f;
@@ -807,7 +816,7 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
       any = any || ok[j];
     }
     const char* dy = a.dy + static_cast<size_t>(s) * a.row_bytes;
-    int v = part * kWave + lane;
+    int v = h.v;
     if constexpr (MODE == kWhole16 || MODE == kAny16) {
       // two granules of the token and of each slot's row in flight
       for (; any && v < a.row_vecs; v += 2 * step) {
@@ -815,30 +824,30 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
         const uint32_t o[2] = {G::at(v, a.row_bytes), G::at(v + step, a.row_bytes)};
         u32x4 d[2], x[2][K];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          d[h] = G::zero();
-          if (h == 0 || two) d[h] = G::ld(dy + o[h]);
+        for (int b = 0; b < 2; ++b) {
+          d[b] = G::zero();
+          if (b == 0 || two) d[b] = G::ld(dy + o[b]);
 #pragma unroll
           for (int j = 0; j < K; ++j) {
-            x[h][j] = G::zero();
-            if (ok[j] && (h == 0 || two)) x[h][j] = G::ld(src[j] + o[h]);
+            x[b][j] = G::zero();
+            if (ok[j] && (b == 0 || two)) x[b][j] = G::ld(src[j] + o[b]);
           }
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (h == 1 && !two) break;
-          u32x4 once = d[h];  // without the bytes that another lane has as well
+        for (int b = 0; b < 2; ++b) {
+          if (b == 1 && !two) break;
+          u32x4 once = d[b];  // without the bytes that another lane has as well
           if (MODE == kAny16) {
-            const uint32_t at = 16u * static_cast<uint32_t>(v + h * step);
-            if (o[h] != at) once = drop_bytes<DT>(once, at - o[h]);
+            const uint32_t at = 16u * static_cast<uint32_t>(v + b * step);
+            if (o[b] != at) once = drop_bytes<DT>(once, at - o[b]);
           }
 #pragma unroll
           for (int j = 0; j < K; ++j) {
             if (!ok[j]) continue;
-            const u32x4 dd[1] = {d[h]};
+            const u32x4 dd[1] = {d[b]};
             const float g[1] = {words.weight(j, true)};
-            G::st(dst[j] + o[h], combine_vec<DT, 1>(dd, g));
-            acc[j] = dot_vec<DT>(once, x[h][j], acc[j]);
+            G::st(dst[j] + o[b], combine_vec<DT, 1>(dd, g));
+            acc[j] = dot_vec<DT>(once, x[b][j], acc[j]);
           }
         }
       }
@@ -856,22 +865,22 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
     }
   }
 #pragma unroll
-  for (int j = 0; j < K; ++j) acc[j] = wave_sum(acc[j]);
-  if (a.wpr_shift > 0) {  // the token's waves, all of this workgroup, in order
+  for (int j = 0; j < K; ++j) acc[j] = share_sum(acc[j], a.q);
+  if (a.q > 6) {  // the token's waves, all of this workgroup, in order
     if (lane == 0) {
 #pragma unroll
       for (int j = 0; j < K; ++j) s_dot[w][j] = acc[j];
     }
     __syncthreads();
-    if (part == 0) {
+    if (h.v == 0) {
 #pragma unroll
       for (int j = 0; j < K; ++j) {
         acc[j] = 0.f;
-        for (int q = 0; q < (1 << a.wpr_shift); ++q) acc[j] += s_dot[w + q][j];
+        for (int k = 0; k < (step / kWave); ++k) acc[j] += s_dot[w + k][j];
       }
     }
   }
-  if (s < a.S && part == 0 && lane == 0) {
+  if (s < a.S && h.v == 0) {
 #pragma unroll
     for (int j = 0; j < K; ++j) st_gate(a.d_gates, static_cast<size_t>(j) * a.S + s, acc[j], a.gate_dtype);
   }
@@ -882,18 +891,15 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
 // ---------------------------------------------------------------------------------------
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// log2 of the number of waves that share one row of `units` granules: a power of two (the kernels split the wave
-// index with a shift), per_lane granules per lane where the grid allows it, at most 16 waves.  Measured at 8 KB
-// rows: the scatter is fastest with one granule per lane (8 waves a row), the gather-combine with two (4 waves).
-static inline int split_waves(long units, long rows, int per_lane = 1) {
-  const long span = static_cast<long>(kWave) * per_lane;
-  const long want = std::max<long>((units + span - 1) / span, 1);
-  int shift = 0;
-  while (shift < 4 && (1L << shift) < want) ++shift;
-  // the grid stays below 2^30 workgroups and the wave index below 2^32
-  while (shift > 0 && ((rows << shift) + kRowsPerBlock - 1) / kRowsPerBlock > 0x3fffffffL) --shift;
-  return shift;
+// log2 of the number of lanes that share one row of `units` granules: as few as leave per_lane granules to each, at most
+// 2^max_q, so few that the grid stays below 2^30 workgroups.
+static inline int row_lanes(long units, long rows, int per_lane, int max_q = 10) {
+  int q = 0;
+  while (q < max_q && (static_cast<long>(per_lane) << q) < units) ++q;
+  while (q > 0 && ((rows << q) + kTile - 1) / kTile > 0x3fffffffL) --q;
+  return q;
 }
+static inline long row_blocks(long rows, int q) { return ((rows << q) + kTile - 1) / kTile; }
 
 // the way rows of row_bytes bytes in arrays at the given addresses are cut
 static inline RowMode row_mode(size_t row_bytes, int elem_bytes, bool aligned) {
@@ -951,8 +957,8 @@ hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, con
   a.slot_stride = slot_stride < 0 ? S : slot_stride;
   a.row_bytes = static_cast<uint32_t>(row_bytes);  // M < 2^30
   a.row_vecs = row_granules(mode, row_bytes, elem_bytes);
-  a.wpr_shift = split_waves(a.row_vecs, S);
-  a.token_blocks = static_cast<int>(((static_cast<long>(S) << a.wpr_shift) + kRowsPerBlock - 1) / kRowsPerBlock);
+  a.q = row_lanes(a.row_vecs, S, 1);
+  a.token_blocks = static_cast<int>(row_blocks(S, a.q));
   a.tail_chunks = rows_hi ? (C + kTailRows - 1) / kTailRows : 0;
   const long blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_chunks) * E;
   if (blocks == 0) return hipSuccess;
@@ -992,8 +998,9 @@ hipError_t run_zero_bytes(void* p, size_t nbytes, hipStream_t st) {
 template <int DT>
 static hipError_t decode_launch(DecodeArgs a, int K, RowMode mode, hipStream_t st) {
   if (a.S == 0 || a.M == 0) return hipSuccess;
-  a.wpr_shift = split_waves(row_granules(mode, static_cast<size_t>(a.M) * sizeof(typename Codec<DT>::S), sizeof(typename Codec<DT>::S)), a.S, K == 1 ? 2 : 1);
-  const unsigned blocks = static_cast<unsigned>(((static_cast<long>(a.S) << a.wpr_shift) + kRowsPerBlock - 1) / kRowsPerBlock);
+  constexpr int eb = sizeof(typename Codec<DT>::S);
+  a.q = row_lanes(row_granules(mode, static_cast<size_t>(a.M) * eb, eb), a.S, K == 1 ? 2 : 1);
+  const unsigned blocks = static_cast<unsigned>(row_blocks(a.S, a.q));
   if (a.dest) {
     if (mode != kWhole16) return hipErrorInvalidValue;
     if (K == 1) decode_rows_kernel<DT, 1, kWhole16, true><<<blocks, kTile, 0, st>>>(a);
@@ -1056,7 +1063,7 @@ hipError_t run_redispatch_rows(const PtrTable& bufs, int P, int M, int C, int E,
   for (int p = 0; p < P; ++p) aligned = aligned && aligned16(bufs.p[p]);
   const RowMode mode = row_mode(row_bytes, elem_bytes, aligned);
   const int units = row_granules(mode, row_bytes, elem_bytes);
-  const int shift = split_waves(units, rows, 2);  // two granules per lane: 426 -> 408 us
+  const int shift = std::max(row_lanes(units, rows, 2), 6) - 6;  // whole waves per row, two granules per lane: 426 -> 408 us
   const unsigned blocks = static_cast<unsigned>(((rows << shift) + kRowsPerBlock - 1) / kRowsPerBlock);
   LANCET_ROW_SWITCH(mode, (redispatch_rows_kernel<MODE><<<blocks, kTile, 0, st>>>(
                               bufs, P, E, C, static_cast<uint32_t>(row_bytes), units, shift, counts, static_cast<char*>(out))))
@@ -1076,11 +1083,11 @@ template <int DT>
 static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, void* out, int S, int M,
                                    long rows, int K, RowMode mode, hipStream_t st) {
   constexpr int eb = sizeof(typename Codec<DT>::S);
-  const int shift = split_waves(row_granules(mode, static_cast<size_t>(M) * eb, eb), rows, 2);  // two granules per lane: 442 -> 408 us
-  const unsigned blocks = static_cast<unsigned>(((rows << shift) + kRowsPerBlock - 1) / kRowsPerBlock);
+  const int q = row_lanes(row_granules(mode, static_cast<size_t>(M) * eb, eb), rows, 2);  // two granules per lane: 442 -> 408 us
+  const unsigned blocks = static_cast<unsigned>(row_blocks(rows, q));
   LANCET_CODED_ROW_SWITCH(DT, mode,
-    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift);
-    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, shift))
+    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, q);
+    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, q))
   return hipGetLastError();
 }
 
@@ -1117,14 +1124,19 @@ static hipError_t decode_grad_launch(DecodeGradArgs a, int K, int M, RowMode mod
   constexpr int eb = sizeof(typename Codec<DT>::S);
   a.row_bytes = static_cast<uint32_t>(M) * eb;
   a.row_vecs = row_granules(mode, a.row_bytes, eb);
-  a.wpr_shift = std::min(split_waves(a.row_vecs, a.S, 2), 2);
-  a.token_blocks = static_cast<int>(((static_cast<long>(a.S) << a.wpr_shift) + kRowsPerBlock - 1) / kRowsPerBlock);
+  // The waves of a token are of one workgroup.  Granules per lane, one / two: 65536 x 1024 bf16 top-2 132 / 139 us, rows of
+  // 384 60 / 56, 262144 x 512 top-1 114 / 93, rows of 4096 the same; 10007 x 1003 top-2 (unaligned) 26 / 23.
+  a.q = row_lanes(a.row_vecs, a.S, K == 2 && a.row_vecs > kWave && mode == kWhole16 ? 1 : 2, 8);
+  a.token_blocks = static_cast<int>(row_blocks(a.S, a.q));
   a.tail_rows = a.owner ? kGradTailRows : kGradScanRows;
   a.tail_chunks = (a.C + a.tail_rows - 1) / a.tail_rows;
   const unsigned blocks = static_cast<unsigned>(a.token_blocks + static_cast<long>(a.tail_chunks) * a.E);
   if (blocks == 0) return hipSuccess;
+  // top-1 rows of several waves: as in the scatter, 317 against 329 us at 65536 x 4096 bf16 (top-2 577 / 581, 52 / 51 at
+  // 16384 x 1024 fp32; rows of one wave 182 / 151)
+  const size_t lds = K == 1 && a.q > 6 ? kScatterLds : 0;
   LANCET_CODED_ROW_SWITCH(DT, mode,
-    if (K == 1) decode_grad_kernel<DT, 1, MODE><<<blocks, kTile, 0, st>>>(a);
+    if (K == 1) decode_grad_kernel<DT, 1, MODE><<<blocks, kTile, lds, st>>>(a);
     else decode_grad_kernel<DT, 2, MODE><<<blocks, kTile, 0, st>>>(a))
   return hipGetLastError();
 }
@@ -1162,8 +1174,12 @@ hipError_t run_decode_grad(const void* dy, const void* expert_out, const void* g
 template <int DT>
 static hipError_t decode_dg_launch(const void* dy, const void* expert_out, const int32_t* idx, const int32_t* loc,
                                    void* out, int gd, int S, int M, int E, int C, int n, RowMode mode, hipStream_t st) {
-  const int blocks = (n + kRowsPerBlock - 1) / kRowsPerBlock;
-  LANCET_CODED_ROW_SWITCH(DT, mode, (decode_dg_kernel<DT, MODE><<<blocks, kTile, 0, st>>>(dy, expert_out, idx, loc, out, gd, S, M, E, C, n)))
+  constexpr int eb = sizeof(typename Codec<DT>::S);
+  // two granules per lane from 512 bytes on (262144 x 512 bf16 top-1 53 -> 43 us, 65536 x 384 top-2 44 -> 33), one in
+  // shorter rows (200000 x 64: 10.6 against 15.5)
+  const int units = row_granules(mode, static_cast<size_t>(M) * eb, eb);
+  const int q = row_lanes(units, n, units >= 32 ? 2 : 1, 6);
+  LANCET_CODED_ROW_SWITCH(DT, mode, (decode_dg_kernel<DT, MODE><<<static_cast<unsigned>(row_blocks(n, q)), kTile, 0, st>>>(dy, expert_out, idx, loc, out, gd, S, M, E, C, n, q)))
   return hipGetLastError();
 }
 
