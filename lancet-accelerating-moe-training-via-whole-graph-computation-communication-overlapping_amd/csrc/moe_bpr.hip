@@ -8,7 +8,7 @@ namespace lancet {
 
 // ---------------------------------------------------------------------------------------
 // Batch-prioritised routing.
-//   bpr_select_kernel : one workgroup per expert.  Finds, with a 4 x 8-bit radix select on the
+//   bpr_select_kernel : one workgroup per expert.  Finds, with a radix select of 10-bit digits on the
 //                       order-preserving integer image of the fp32 priority, the C-th largest
 //                       priority among the expert's tokens (threshold), how many ties at the
 //                       threshold may stay (quota, lowest token ids first) and how many ties
@@ -117,41 +117,12 @@ __global__ __launch_bounds__(kTile) void bpr_prepare_kernel(const void* gate, in
   }
 }
 
-// One descending step of the radix select, by the first wave of the workgroup: the digit that holds the need-th
-// largest key among the keys counted in hist[256], and what is still needed inside that digit.  Lane l owns the
-// digits 255 - 4l .. 252 - 4l; a wave scan of the lanes' sums finds the lane, the lane finds the digit.  (A single
-// thread walking the 256 counters is a chain of dependent LDS reads: it was most of this kernel's time.)
-__device__ __forceinline__ void select_digit(const uint32_t* hist, uint32_t prefix, uint32_t* s_prefix, uint32_t* s_need) {
-  const int lane = threadIdx.x;  // called with threadIdx.x < kWave
-  const uint32_t need = *s_need;
-  uint32_t h[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) h[j] = hist[255 - (4 * lane + j)];
-  const uint32_t mine = h[0] + h[1] + h[2] + h[3];
-  uint32_t inc = mine;
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t v = __shfl_up(inc, off, kWave);
-    if (lane >= off) inc += v;
-  }
-  uint32_t run = inc - mine;  // keys in digits above this lane's
-  if (run < need && need <= inc) {
-    int j = 0;
-    for (; j < 3; ++j) {
-      if (need <= run + h[j]) break;
-      run += h[j];
-    }
-    *s_need = need - run;
-    *s_prefix = (prefix << 8) | static_cast<uint32_t>(255 - (4 * lane + j));
-  } else if (lane == kWave - 1 && inc < need) {
-    // fewer keys than needed (does not happen with consistent counts): digit 0 takes what is left
-    *s_need = need - (inc - h[3]);
-    *s_prefix = prefix << 8;
-  }
-}
-
-constexpr int kSelectKeys = 10240;  // keys of one expert kept in LDS (40 KB)
+// Keys of one expert kept in LDS (128 KB): the largest power of two that leaves room for the tiles' positions.  An
+// expert that half of a batch of 65536 tokens chose still fits.
+constexpr int kSelectKeys = 32768;
 constexpr int kSelectTiles = 4096;  // tiles whose group positions fit in LDS (16 KB): batches up to 1M tokens
+constexpr int kSelectBits = 10;     // digit of the radix select: one histogram bin per thread
+static_assert((1 << kSelectBits) == kSelectThreads, "a thread owns one bin");
 
 // exclusive scan over the kSelectThreads values of a workgroup; *total = their sum.  s_wave: 16 words of LDS.
 __device__ __forceinline__ uint32_t select_block_scan(uint32_t v, uint32_t* s_wave, uint32_t* total) {
@@ -176,24 +147,42 @@ __device__ __forceinline__ uint32_t select_block_scan(uint32_t v, uint32_t* s_wa
   return before + inc - v;
 }
 
-// the i-th key of the expert in token order: its tile by bisection over the tiles' positions (s_pos: position of
-// the tile's first key in the low 22 bits, start of the expert's group inside the tile above them)
-__device__ __forceinline__ uint32_t select_gather(const BprArgs& a, const uint32_t* s_pos, uint32_t i) {
-  int lo = 0, hi = a.ntiles0 - 1;  // last tile whose position is <= i
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if ((s_pos[mid] & 0x3fffffu) <= i) lo = mid; else hi = mid - 1;
+// f(key, position) for every key of the expert, position = its place in token order, from the prepare kernel's groups.
+// A group is read by 2^q neighbouring lanes, q by the expert's mean keys per tile, four loads of a lane in flight:
+// s_pos holds the position of a tile's first key in the low 22 bits and the start of its group inside the tile above
+// them, so nothing is searched for.  (A lane that found the tile of its key by bisection over the positions spent most of
+// the kernel on it: 12 dependent LDS reads per key.)
+template <typename F>
+__device__ __forceinline__ void walk_groups(const BprArgs& a, const uint32_t* s_pos, uint32_t count, int q, F f) {
+  const uint32_t width = 1u << q;
+  const uint32_t sub = threadIdx.x & (width - 1u);
+  for (int t = static_cast<int>(threadIdx.x >> q); t < a.ntiles0; t += kSelectThreads >> q) {
+    const uint32_t w = s_pos[t];
+    const uint32_t pos = w & 0x3fffffu;
+    const uint32_t n = (t + 1 < a.ntiles0 ? s_pos[t + 1] & 0x3fffffu : count) - pos;
+    const uint64_t* group = a.keys + static_cast<size_t>(t) * kTile + (w >> 22);
+    for (uint32_t i = sub; i < n; i += 4u * width) {
+      uint64_t k[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) k[j] = i + j * width < n ? group[i + j * width] : 0ull;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + j * width < n) f(static_cast<uint32_t>(k[j]), pos + i + j * width);
+    }
   }
-  const uint32_t w = s_pos[lo];
-  return static_cast<uint32_t>(a.keys[static_cast<size_t>(lo) * kTile + (w >> 22) + (i - (w & 0x3fffffu))]);
 }
 
+// One workgroup per expert; what bounds it is the one expert that most tokens chose, whose keys a single CU reads and
+// counts.  The digits start below the leading bits that all keys share (probabilities have two or three exponents, so a
+// digit that starts at bit 31 puts every key into the same few bins, whose LDS atomics then run one after the other),
+// and passes end with the lowest bit in which keys differ.  32768 tokens on 64 experts of which a few are hot (top-1,
+// most keys on one expert): 78 -> 18.5 us.
 __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
   __shared__ uint32_t s_keys[kSelectKeys];
   __shared__ uint32_t s_pos[kSelectTiles];
-  __shared__ uint32_t hist[256];
+  __shared__ uint32_t hist[1 << kSelectBits];
   __shared__ uint32_t s_wave[kSelectThreads / kWave];
-  __shared__ uint32_t s_prefix, s_need, s_count;
+  __shared__ uint32_t s_prefix, s_need, s_count, s_min, s_max;
   const int e = blockIdx.x;
   const int tid = threadIdx.x;
   // The expert's keys, in token order.  Up to kSelectTiles tiles, the prepare kernel's groups say where they are:
@@ -201,9 +190,15 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
   // in every pass).  Longer batches are read whole, once per pass.
   const bool grouped = a.ntiles0 <= kSelectTiles;
   uint32_t count = 0, nfront = 0;
+  if (tid == 0) {
+    s_count = 0;
+    s_min = 0xffffffffu;
+    s_max = 0u;
+  }
   if (grouped) {
     uint32_t carry = 0;
     const int tstart = a.part_lo / kTile;  // the tile that holds the partition's first token
+    const uint32_t early = a.S0 > 0 ? par_value(a.par + 3 * a.E + e) : 0u;
     for (int base = 0; base < a.ntiles0; base += kSelectThreads) {
       const int t = base + tid;
       const uint32_t g = t < a.ntiles0 ? static_cast<uint32_t>(a.groups[static_cast<size_t>(e) * a.ntiles0 + t]) : 0u;
@@ -214,9 +209,8 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
     }
     __syncthreads();
     count = carry;
-    nfront = a.S0 > 0 ? (s_pos[tstart] & 0x3fffffu) + par_value(a.par + 3 * a.E + e) : 0u;
+    nfront = a.S0 > 0 ? (s_pos[tstart] & 0x3fffffu) + early : 0u;
   } else {
-    if (tid == 0) s_count = 0;
     __syncthreads();
     uint32_t local = 0;
     for (int s = tid; s < a.S0; s += kSelectThreads) local += (tok_expert(a.tok[s]) == e);
@@ -243,54 +237,84 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
     return;
   }
   const bool in_lds = grouped && count <= kSelectKeys;
-  if (in_lds) {
-    for (uint32_t i = tid; i < count; i += kSelectThreads) s_keys[i] = select_gather(a, s_pos, i);
-  }
-  if (tid == 0) {
-    s_prefix = 0;
-    s_need = static_cast<uint32_t>(a.C);
-  }
-  for (int pass = 0; pass < 4; ++pass) {
-    const int shift = 24 - 8 * pass;
-    if (tid < 256) hist[tid] = 0;
-    __syncthreads();
-    const uint32_t prefix = s_prefix;
-    if (grouped) {
-      for (uint32_t i = tid; i < count; i += kSelectThreads) {
-        const uint32_t k = in_lds ? s_keys[i] : select_gather(a, s_pos, i);
-        if (pass == 0 || (k >> (shift + 8)) == prefix) atomicAdd(&hist[(k >> shift) & 0xffu], 1u);
-      }
+  int q = 0;
+  while (q < 6 && static_cast<uint64_t>(a.ntiles0) << q < count) ++q;
+  // f(key, whether its token lies before the partition) for all keys
+  const auto every_key = [&](auto f) {
+    if (in_lds) {
+      for (uint32_t i = tid; i < count; i += kSelectThreads) f(s_keys[i], i < nfront);
+    } else if (grouped) {
+      walk_groups(a, s_pos, count, q, [&](uint32_t k, uint32_t pos) { f(k, pos < nfront); });
     } else {
       for (int s = tid; s < a.S0; s += kSelectThreads) {
         const uint64_t t = a.tok[s];
-        if (tok_expert(t) != e) continue;
-        const uint32_t k = order_key(tok_prio(t));
-        if (pass == 0 || (k >> (shift + 8)) == prefix) atomicAdd(&hist[(k >> shift) & 0xffu], 1u);
+        if (tok_expert(t) == e) f(order_key(tok_prio(t)), s < a.part_lo);
       }
     }
-    __syncthreads();
-    if (tid < kWave) select_digit(hist, prefix, &s_prefix, &s_need);
-    __syncthreads();
-  }
-  const uint32_t thr = s_prefix;
-  // ties that precede the partition
-  if (tid == 0) s_count = 0;
-  __syncthreads();
-  uint32_t local = 0;
-  if (grouped) {
-    for (uint32_t i = tid; i < nfront; i += kSelectThreads) local += ((in_lds ? s_keys[i] : select_gather(a, s_pos, i)) == thr);
+  };
+  uint32_t lo = 0xffffffffu, hi = 0u;
+  if (in_lds) {
+    walk_groups(a, s_pos, count, q, [&](uint32_t k, uint32_t pos) {
+      s_keys[pos] = k;
+      lo = min(lo, k), hi = max(hi, k);
+    });
   } else {
-    for (int s = tid; s < a.part_lo; s += kSelectThreads) {
-      const uint64_t t = a.tok[s];
-      local += (tok_expert(t) == e && order_key(tok_prio(t)) == thr);
-    }
+    every_key([&](uint32_t k, bool) { lo = min(lo, k), hi = max(hi, k); });
   }
-  if (local) atomicAdd(&s_count, local);
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    lo = min(lo, static_cast<uint32_t>(__shfl_xor(lo, off, kWave)));
+    hi = max(hi, static_cast<uint32_t>(__shfl_xor(hi, off, kWave)));
+  }
+  if (lane_id() == 0) {
+    atomicMin(&s_min, lo);
+    atomicMax(&s_max, hi);
+  }
+  if (tid == 0) s_need = static_cast<uint32_t>(a.C);
   __syncthreads();
+  // digits from the highest bit in which two keys differ; `left` bits are still to be found
+  int left = s_min == s_max ? 0 : 32 - __clz(s_min ^ s_max);
+  uint32_t prefix = left == 32 ? 0u : s_min >> left;
+  while (left > 0) {
+    const int bits = min(left, kSelectBits);
+    const int shift = left - bits;
+    const uint32_t digits = (1u << bits) - 1u;
+    hist[tid] = 0;
+    __syncthreads();
+    const uint32_t need = s_need;
+    every_key([&](uint32_t k, bool) {
+      if (left == 32 || (k >> left) == prefix) atomicAdd(&hist[(k >> shift) & digits], 1u);
+    });
+    __syncthreads();
+    // the digit that holds the need-th largest of the keys counted, and what is needed inside it: bins in descending
+    // order, one per thread
+    const uint32_t bin = static_cast<uint32_t>(kSelectThreads - 1 - tid);
+    const uint32_t h = hist[bin];
+    uint32_t total;
+    const uint32_t above = select_block_scan(h, s_wave, &total);
+    // (fewer keys than needed does not happen with consistent counts: digit 0 takes what is left)
+    if ((above < need && need <= above + h) || (bin == 0u && total < need)) {
+      s_need = need - above;
+      s_prefix = (left == 32 ? 0u : prefix << bits) | bin;
+    }
+    __syncthreads();
+    prefix = s_prefix;
+    left = shift;
+  }
+  const uint32_t thr = prefix;
+  // ties that precede the partition
+  if (a.part_lo > 0) {
+    uint32_t local = 0;
+    every_key([&](uint32_t k, bool early) { local += early && k == thr; });
+    if (!grouped && tid == 0) s_count = 0;  // held the expert's count
+    __syncthreads();
+    if (local) atomicAdd(&s_count, local);
+    __syncthreads();
+  }
   if (tid == 0) {
     a.par[e] = foreign_word(0u, thr);
     a.par[a.E + e] = foreign_word(0u, s_need);
-    a.par[2 * a.E + e] = foreign_word(0u, s_count);
+    a.par[2 * a.E + e] = foreign_word(0u, a.part_lo > 0 ? s_count : 0u);
   }
 }
 

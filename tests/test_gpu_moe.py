@@ -1020,3 +1020,38 @@ def test_default_workspaces_are_kept_per_stream(pkg):
         np.testing.assert_array_equal(to_np(got[1]), want[1])
         np.testing.assert_array_equal(to_np(got[4]), want[4])
     assert ops.scan_errors() == 0
+
+
+@pytest.mark.parametrize("S0,E,P,kind", [(70000, 4, 2, "hot"), (40000, 3, 1, "hot"), (5000, 2, 2, "equal"), (5001, 2, 1, "one_bit"),
+                                         (20000, 70, 4, "signs"), (33000, 5, 3, "bf16"), (4500, 300, 1, "signs")])
+def test_bpr_select_over_key_ranges(pkg, S0, E, P, kind):
+    """The radix select where its parts can go wrong: more keys of one expert than LDS holds (70000 tokens, nearly all on
+    one expert) and nearly as many, keys that all agree (no digit), that differ in the lowest bit alone, of both signs
+    with infinities (no common leading bits, digits of 10, 10, 10 and 2 bits), massive ties of a 16-bit gate; partitions
+    that do not start on a tile.  Routing is bit-exact."""
+    rng = np.random.default_rng(S0 + E)
+    gate = rng.random((S0, E), dtype=np.float32) * 0.5
+    if kind == "hot":
+        gate[:, 1] += 0.45
+    elif kind == "equal":
+        gate[:] = 0.25
+    elif kind == "one_bit":
+        gate[:] = 0.25
+        gate[:, 0] = np.where(rng.random(S0) < 0.5, np.float32(0.25), np.nextafter(np.float32(0.25), np.float32(1)))
+    elif kind == "signs":
+        gate = rng.standard_normal((S0, E), dtype=np.float32) - 2.0
+        gate[::97, E // 2] = np.inf
+        gate[5::89, :] = -np.inf
+    elif kind == "bf16":
+        gate = mo.round_to_bf16(gate)
+    data = rng.standard_normal((S0, 4), dtype=np.float32)
+    d_gate = dev(gate).to(torch.bfloat16) if kind == "bf16" else dev(gate)
+    dropped = 0
+    for pid in range(P):
+        want = mo.moe_encode_bpr(data, gate, P, pid, 0.7, fast_scatter=True)
+        got = pkg.ops.moe_encode_batch_prioritized(dev(data), d_gate, P, pid, 0.7)
+        np.testing.assert_array_equal(to_np(got[1]), want[1])
+        np.testing.assert_array_equal(to_np(got[2]), want[2])
+        np.testing.assert_array_equal(to_np(got[4]), want[4])
+        dropped += int((want[1][0] < 0).sum())
+    assert dropped > 0
