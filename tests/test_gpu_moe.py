@@ -1055,3 +1055,34 @@ def test_bpr_select_over_key_ranges(pkg, S0, E, P, kind):
         np.testing.assert_array_equal(to_np(got[4]), want[4])
         dropped += int((want[1][0] < 0).sum())
     assert dropped > 0
+
+
+@pytest.mark.parametrize("dt,dims", [("bf16", (3, 70, 401)), ("f32", (70, 3, 4096)), ("bf16", (2, 50, 1024)), ("f16", (5, 3, 2731))])
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("base", [0, 1])
+def test_sparse_copies_of_several_tiles_at_any_alignment(pkg, dt, dims, axis, base):
+    """Blocks longer than a workgroup's tile of 1024 granules, more than 64 of them (counts added up in two rounds), ranges
+    that start and end inside a granule, arrays that are not aligned to one (base = elements past an allocation's start).
+    Both directions and the fill are bit-exact."""
+    ops = pkg.ops
+    rng = np.random.default_rng(sum(dims) + axis + base)
+    nb, run = dims[axis], int(np.prod(dims)) // dims[axis]
+    at = lambda x: torch.cat([torch.zeros(base, dtype=x.dtype, device="cuda"), x.reshape(-1)])[base:].view(x.shape)  # noqa: E731
+    starts = rng.integers(0, run // 3 + 1, nb).astype(np.uint64)
+    if axis == 1:
+        starts[::2] = starts[::2] // 8 * 8
+    counts = (rng.integers(0, run + 1, nb) * (rng.random(nb) < 0.8)).astype(np.uint64)
+    counts = np.minimum(counts, run - starts)
+    counts[-1] = run - starts[-1]
+    total = int(counts.sum())
+    src = rows_as_oracle(rng.standard_normal(dims, dtype=np.float32), dt)
+    d_c, d_s = dev(counts.astype(np.int64)), dev(starts.astype(np.int64))
+    wire = ops.memcpy_sparse_ranges_to_cont_3d(at(rows_to_torch(src, dt)), at(rows_to_torch(np.zeros(total, np.float32), dt)),
+                                               d_c, d_s, axis=axis)
+    want = mo.memcpy_sparse_ranges_to_cont_3d(src, np.zeros(total, np.float32), counts, starts, axis=axis)
+    np.testing.assert_array_equal(to_np(wire), want)
+    nines = np.full(dims, 9.0, np.float32)
+    back = ops.memcpy_cont_to_sparse_ranges_3d(wire, at(rows_to_torch(nines, dt)), d_c, d_s, axis=axis)
+    np.testing.assert_array_equal(to_np(back), mo.memcpy_cont_to_sparse_ranges_3d(want, nines.copy(), counts, starts, axis=axis))
+    filled = ops.memcpy_cont_to_sparse_3d(wire, at(rows_to_torch(nines, dt)), d_c, axis=axis, zero_tail=True)
+    np.testing.assert_array_equal(to_np(filled), mo.memcpy_cont_to_sparse_3d(want, nines.copy(), counts, axis=axis, zero_tail=True))
