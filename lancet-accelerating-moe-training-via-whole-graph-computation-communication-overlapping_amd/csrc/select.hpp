@@ -2,6 +2,7 @@
 // batch-prioritised routing (moe_bpr.hip).
 #pragma once
 #include "scan.hpp"
+#include <type_traits>
 #include "../../include/lancet_hip.h"
 
 namespace lancet {
@@ -160,15 +161,194 @@ __device__ __forceinline__ Routed route_token(const void* __restrict__ row, cons
   return r;
 }
 
-// ---- rows longer than a cache line: staged through LDS ------------------------------------------------------
+// ---- rows held in registers ---------------------------------------------------------------------------------
+// A row of up to kHeldGranules 16-byte granules is taken by 2^q neighbouring lanes, four granules each, all loads in
+// flight together and the next rows' behind them; what the lanes chose is merged by shuffles, and the exponentials are
+// summed from the registers once the row's maximum is known.  The kernel is bound by its vector instructions (262144
+// tokens x 64 fp32 experts: 67 MB, which memory delivers in 11 us), so nothing is decided per element that can be decided
+// per row: the running choice starts from "none" at -inf, and the rows that this does not describe (a NaN, a row whose
+// choice is -inf, an infinite sum) are told by their outcome and walked again one by one by route_token.
+// First routing kernel, before (rows walked by one lane each, through LDS where they are longer than a line, element by
+// element where they are not whole granules) and after, us: 262144 x 64 fp32 top-1 27.0 -> 17.7, 65536 x 32 fp32 top-2
+// 9.6 -> 8.5, 10007 x 60 bf16 top-2 21 -> 8.3.  The sum is formed from 16 terms (32 of 16 bits) per lane and then over the
+// lanes: largest relative error of a gate value at 64 / 256 experts 6.4e-7 / 1.2e-6 before, 3.6e-7 / 2.3e-7 after.
+constexpr int kHeldPerLane = 4;
+constexpr int kHeldGranules = 16 * kHeldPerLane;
+typedef u32x4 u32x4_gate __attribute__((aligned(2)));
+
+// Rows of 3 to 64 granules.  Two granules are as fast walked by their lane (16 tiles x 8 fp32 experts: 7.4 us, held 7.8).
+// Without the softmax the walk is a few compares per value and has no serial rounds, which short launches on aligned rows
+// notice (32 tiles x 32 experts 8.4 us, held 8.8; 128 x 64 6.9, held 7.5): they keep it.  The choice is the same either way.
+constexpr int kHeldMinTiles = 256;
+__host__ __device__ inline bool rows_are_held(const void* gate, const void* noise, int S, int E, int gb, bool is_logits) {
+  const int bytes = E * gb;
+  if (noise != nullptr || bytes <= 32 || bytes > 16 * kHeldGranules) return false;
+  return is_logits || (S + kTile - 1) / kTile >= kHeldMinTiles || bytes % 16 != 0 || (reinterpret_cast<uintptr_t>(gate) & 15u) != 0;
+}
+
+// f(x, i) for the values of a granule as fp32; i is the value's place in it
+template <int GD, typename F>
+__device__ __forceinline__ void each_value(const u32x4& x, F f) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (GD == LANCET_F32) {
+      f(__uint_as_float(x[w]), w);
+    } else {
+      f(half_word<GD>(x[w] & 0xffffu), 2 * w);
+      f(half_word<GD>(x[w] >> 16), 2 * w + 1);
+    }
+  }
+}
+
+constexpr int kNoExpert = 0x7fffffff;
+
+// The value of the partner in merge step 0 .. 3 of a group of up to 16 lanes that agree inside their half of it: the
+// neighbour, the pair's, the quad's and the half row's mirror image.  (Register moves: a shuffle goes through LDS, and the
+// merges of a round are a serial chain; selection of 32768 x 64 8.0 -> 7.5 us.)
+template <int STEP>
+__device__ __forceinline__ int merge_partner(int x) {
+  constexpr int ctrl = STEP == 0 ? 0xb1 : STEP == 1 ? 0x4e : STEP == 2 ? 0x141 : 0x140;
+  return __builtin_amdgcn_update_dpp(0, x, ctrl, 0xf, 0xf, false);
+}
+template <int STEP>
+__device__ __forceinline__ float merge_partner(float x) {
+  return __int_as_float(merge_partner<STEP>(__float_as_int(x)));
+}
+// f(step) for the merge steps of a group of 2^q lanes
+template <typename F>
+__device__ __forceinline__ void merge_steps(int q, F f) {
+  if (q > 0) f(std::integral_constant<int, 0>());
+  if (q > 1) f(std::integral_constant<int, 1>());
+  if (q > 2) f(std::integral_constant<int, 2>());
+  if (q > 3) f(std::integral_constant<int, 3>());
+}
+
+// what route_token returns, for the lane's token of the wave's nrows <= 64 consecutive ones from `rows` on (lanes past
+// them: anything).  All lanes of the wave, uniform control flow.
+template <int K, int GD>
+__device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, int E, bool is_logits) {
+  constexpr int gb = GD == LANCET_F32 ? 4 : 2;
+  constexpr int V = 16 / gb;
+  const int lane = lane_id();
+  const uint32_t row_bytes = static_cast<uint32_t>(E) * gb;
+  const int n = static_cast<int>((row_bytes + 15u) / 16u);
+  int q = 0;
+  while (kHeldPerLane << q < n) ++q;
+  const int width = 1 << q, per_round = kWave >> q;  // lanes per row, rows per round
+  const int sub = lane & (width - 1);
+  // where the lane's granules lie in a row; the last of a row that is not whole granules is drawn back to end with it, and
+  // the values it shares with the one before (the first `dup`) count as -inf
+  uint32_t at[kHeldPerLane];
+  int dup[kHeldPerLane];
+#pragma unroll
+  for (int k = 0; k < kHeldPerLane; ++k) {
+    const int g = k * width + sub;
+    at[k] = min(16u * static_cast<uint32_t>(g), row_bytes - 16u);
+    dup[k] = g < n ? static_cast<int>(16u * static_cast<uint32_t>(g) - at[k]) / gb : V;
+  }
+  const bool ragged = n * 16 != static_cast<int>(row_bytes) || n != kHeldPerLane * width;
+  const auto load = [&](int r, u32x4 (&x)[kHeldPerLane]) {
+    const int row = r * per_round + (lane >> q);
+    const char* p = rows + static_cast<size_t>(min(row, nrows - 1)) * row_bytes;
+#pragma unroll
+    for (int k = 0; k < kHeldPerLane; ++k) x[k] = *reinterpret_cast<const u32x4_gate*>(p + at[k]);
+  };
+  const int rounds = (nrows + per_round - 1) / per_round;
+  float v1 = 0.f, v2 = 0.f, sum = 0.f;  // the lane's own token
+  int i1 = 0, i2 = 0;
+  u32x4 x[kHeldPerLane], nx[kHeldPerLane];
+  load(0, x);
+  for (int r = 0; r < rounds; ++r) {
+    if (r + 1 < rounds) load(r + 1, nx);
+    float f[kHeldPerLane][V];
+#pragma unroll
+    for (int k = 0; k < kHeldPerLane; ++k) each_value<GD>(x[k], [&](float val, int i) { f[k][i] = val; });
+    if (ragged) {
+#pragma unroll
+      for (int k = 0; k < kHeldPerLane; ++k)
+#pragma unroll
+        for (int i = 0; i < V; ++i) f[k][i] = i < dup[k] ? -INFINITY : f[k][i];
+    }
+    float a1 = -INFINITY, a2 = -INFINITY;
+    int j1 = kNoExpert, j2 = kNoExpert;
+#pragma unroll
+    for (int k = 0; k < kHeldPerLane; ++k) {
+      const int j0 = static_cast<int>(at[k] / gb);
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const float val = f[k][i];
+        const bool first = val > a1;
+        if (K == 2) {
+          const bool second = val > a2;
+          a2 = first ? a1 : (second ? val : a2);
+          j2 = first ? j1 : (second ? j0 + i : j2);
+        }
+        a1 = first ? val : a1;
+        j1 = first ? j0 + i : j1;
+      }
+    }
+    merge_steps(q, [&](auto step) {
+      const float b1 = merge_partner<step.value>(a1);
+      const int k1 = merge_partner<step.value>(j1);
+      const bool theirs = (b1 > a1) | ((b1 == a1) & (k1 < j1));  // equal values: the first expert
+      if (K == 2) {
+        const float b2 = merge_partner<step.value>(a2);
+        const int k2 = merge_partner<step.value>(j2);
+        // the second choice is the loser of the two firsts or the winner's own second
+        const float c = theirs ? a1 : b1, d = theirs ? b2 : a2;
+        const int cj = theirs ? j1 : k1, dj = theirs ? k2 : j2;
+        const bool loser = (c > d) | ((c == d) & (cj < dj));
+        a2 = loser ? c : d;
+        j2 = loser ? cj : dj;
+      }
+      a1 = theirs ? b1 : a1;
+      j1 = theirs ? k1 : j1;
+    });
+    float part = 0.f;
+#pragma unroll
+    for (int k = 0; k < kHeldPerLane; ++k)
+#pragma unroll
+      for (int i = 0; i < V; ++i) part += is_logits ? __expf(f[k][i] - a1) : f[k][i];
+    merge_steps(q, [&](auto step) { part += merge_partner<step.value>(part); });
+    // the round's tokens to their lanes
+    const int from = (lane & (per_round - 1)) << q;
+    const bool mine = lane / per_round == r;
+    const float t1 = __shfl(a1, from, kWave), ts = __shfl(part, from, kWave);
+    const int u1 = __shfl(j1, from, kWave);
+    v1 = mine ? t1 : v1;
+    i1 = mine ? u1 : i1;
+    sum = mine ? ts : sum;
+    if (K == 2) {
+      const float t2 = __shfl(a2, from, kWave);
+      const int u2 = __shfl(j2, from, kWave);
+      v2 = mine ? t2 : v2;
+      i2 = mine ? u2 : i2;
+    }
+#pragma unroll
+    for (int k = 0; k < kHeldPerLane; ++k) x[k] = nx[k];
+  }
+  Routed res;
+  const bool plain = sum == sum && i1 != kNoExpert && (K == 1 || i2 != kNoExpert);
+  if (plain || lane >= nrows) {
+    res.e0 = i1;
+    res.p0 = is_logits ? 1.f / sum : v1;
+    res.e1 = K == 2 ? i2 : -1;
+    res.p1 = K == 2 ? (is_logits ? expf(v2 - v1) / sum : v2) : 0.f;
+  } else {
+    res = route_token<K, GD>(rows + static_cast<size_t>(lane) * row_bytes, nullptr, E, is_logits);
+  }
+  return res;
+}
+
+// ---- rows longer than registers hold: staged through LDS ----------------------------------------------------
 // A lane that walks its own row touches each 128-byte line of it in eight loads, and every load of the wave
 // touches 64 different lines; with rows of several lines and many waves on a CU the lines are evicted between a
-// lane's visits and fetched again (1M tokens x 64 fp32 experts: 0.55 TB/s).  Such rows are therefore read the way
-// they lie in memory, a wave's 64 rows 128 bytes at a time (eight lanes per row and line, every line whole in one
-// load), passed through LDS and walked from there, each lane its own row as before: the values and their order
-// are the same, so is the result.  It pays from about two workgroups per CU on (512 tiles: routing of 1M tokens x
-// 64 experts 482 -> 98 us, 262144 x 256 274 -> 92); launches of fewer tiles keep the direct walk, whose lines survive
-// in the cache (65536 x 256 top-2: 50 against 64 us).
+// lane's visits and fetched again.  Rows of more than 64 granules are therefore read the way they lie in memory, a wave's
+// 64 rows 128 bytes at a time (eight lanes per row and line, every line whole in one load), passed through LDS and walked
+// from there, each lane its own row as before: the values and their order are the same, so is the result.  It pays from
+// about two workgroups per CU on (512 tiles); launches of fewer tiles keep the direct walk, whose lines survive in the
+// cache (both measured with rows of 256 fp32 experts, which are held in registers now: 262144 rows 274 -> 92 us, 65536 rows
+// top-2 50 against 64).
 constexpr int kStageMinTiles = 512;
 constexpr int kStageChunk = 128;                   // bytes of a row staged at a time
 constexpr int kStageRow = kStageChunk + 16;        // row pitch in LDS (the pad spreads the lanes' reads over the banks)
@@ -178,7 +358,7 @@ constexpr int kStageBytes = kWavesPerTile * kStageWave;
 template <int GD>
 __host__ __device__ inline bool rows_are_staged(const void* gate, const void* noise, int S, int E) {
   constexpr int gb = GD == LANCET_F32 ? 4 : 2;
-  return noise == nullptr && (S + kTile - 1) / kTile >= kStageMinTiles && E * gb > kStageChunk && (E * gb) % 16 == 0 &&
+  return noise == nullptr && (S + kTile - 1) / kTile >= kStageMinTiles && E * gb > 16 * kHeldGranules && (E * gb) % 16 == 0 &&
          (reinterpret_cast<uintptr_t>(gate) & 15u) == 0;
 }
 
@@ -262,6 +442,15 @@ __device__ __forceinline__ Routed route_tile_token(const void* gate, const void*
                                                    void* lds) {
   constexpr size_t gb = GD == LANCET_F32 ? 4 : 2;
   Routed r = {-1, -1, 0.f, 0.f};
+  if (rows_are_held(gate, noise, S, E, static_cast<int>(gb), is_logits)) {
+    const int first = s - lane_id();  // the wave's first token
+    if (first < S) {
+      const Routed held = route_rows_held<K, GD>(static_cast<const char*>(gate) + static_cast<size_t>(first) * E * gb,
+                                                 min(S - first, kWave), E, is_logits);
+      if (s < S) r = held;
+    }
+    return r;
+  }
   if (!rows_are_staged<GD>(gate, noise, S, E)) {
     if (s < S) {
       const size_t off = static_cast<size_t>(s) * E * gb;

@@ -1086,3 +1086,45 @@ def test_sparse_copies_of_several_tiles_at_any_alignment(pkg, dt, dims, axis, ba
     np.testing.assert_array_equal(to_np(back), mo.memcpy_cont_to_sparse_ranges_3d(want, nines.copy(), counts, starts, axis=axis))
     filled = ops.memcpy_cont_to_sparse_3d(wire, at(rows_to_torch(nines, dt)), d_c, axis=axis, zero_tail=True)
     np.testing.assert_array_equal(to_np(filled), mo.memcpy_cont_to_sparse_3d(want, nines.copy(), counts, axis=axis, zero_tail=True))
+
+
+@pytest.mark.parametrize("gd", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("E", [2, 3, 4, 5, 7, 8, 9, 16, 31, 60, 64, 65, 128, 255, 256, 257, 511, 512])
+def test_selection_at_every_row_length(pkg, gd, E):
+    """Rows taken by 1 to 16 lanes, with a last granule that is drawn back, one granule short of a lane's four or beyond
+    what is held in registers; ties everywhere (16-bit values, copied columns), rows of -inf but for one or two entries.
+    Selection is exact (first maximum); values against a 64-bit softmax: its sum has up to 512 terms of relative error
+    2^-22 each (hardware exponential) and is rounded at most 512 times, and a 16-bit value is rounded once more."""
+    ops = pkg.ops
+    S = 700
+    rng = np.random.default_rng(E)
+    x = rng.standard_normal((S, E)).astype(np.float32) * 2
+    x[:, -1] = x[:, 0]                       # ties between the first and the last lane
+    x[::7, E // 2] = x[::7, 0]
+    x[3::50] = 0.5
+    x[5::50] = -np.inf
+    x[5::50, E // 2] = 1.0                   # second choice: the first of the entries at -inf
+    x[6::50] = -np.inf
+    x[6::50, E - 1] = 1.0
+    x[6::50, 0] = -2.0
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[gd]
+    gate = torch.from_numpy(x).to(tdt)
+    x = gate.float().numpy().astype(np.float64)
+    order = np.argsort(-x, axis=1, kind="stable")
+    p = np.exp(x - x.max(axis=1, keepdims=True))
+    p /= p.sum(axis=1, keepdims=True)
+    eps = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -10}[gd]
+    tol = 520 * 2.0 ** -22 if E > 64 else 70 * 2.0 ** -22
+    for k in (1, 2):
+        for logits in (True, False):
+            g, il, _, _ = ops.moe_route(gate.cuda(), None, 1, top_k=k, gate_is_logits=logits, capacity=S * k)
+            idx = to_np(il)[0].reshape(k, S)
+            np.testing.assert_array_equal(idx, order[:, :k].T)
+            if not logits and k == 2:
+                continue                     # weights of raw values of either sign are not meaningful
+            val = np.take_along_axis(p if logits else x, order[:, :k], 1).T
+            if k == 2:                       # raw values are stored rounded, then normalised and rounded again
+                val = val / val.sum(axis=0)
+            bound = (2 * tol + (3 if k == 2 else 1) * eps if logits else 0.0) * np.abs(val) + (2.0 ** -24 if gd == "f16" else 0.0) * k
+            got = to_np(g.float()).astype(np.float64).reshape(k, S)
+            assert (np.abs(got - val) <= bound).all(), np.abs(got - val).max()
