@@ -430,6 +430,30 @@ __global__ __launch_bounds__(kTile) void count_experts_kernel(PtrTable t, int S,
     if (hist[c]) atomicAdd(counts + static_cast<size_t>(p) * E + c, hist[c]);
 }
 
+// Partitions of up to kCountWhole tokens: one workgroup counts a partition alone, sixteen tokens a thread at most, so that
+// nothing has to be cleared first and no counter is shared: four partitions of 8192 tokens 1.4 + 3.1 us in two launches, 2.8 in
+// one; the partitioned chain of 32768 x 2048 tokens, which counts twice, 201 -> 198 us.
+constexpr int kCountWhole = 16384;
+constexpr int kCountThreads = 1024;
+__global__ __launch_bounds__(kCountThreads) void count_experts_whole_kernel(PtrTable t, int S, int E, uint32_t* counts) {
+  extern __shared__ uint32_t hist[];
+  const int p = blockIdx.x;
+  const int32_t* idx = static_cast<const int32_t*>(t.p[p]);
+  for (int c = threadIdx.x; c < E; c += kCountThreads) hist[c] = 0;
+  __syncthreads();
+  constexpr int kBatch = 8;  // loads in flight per thread
+  for (int i = threadIdx.x; i < S; i += kBatch * kCountThreads) {
+    int e[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) e[k] = i + k * kCountThreads < S ? idx[i + k * kCountThreads] : -1;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k)
+      if (e[k] >= 0 && e[k] < E) atomicAdd(&hist[e[k]], 1u);
+  }
+  __syncthreads();
+  for (int c = threadIdx.x; c < E; c += kCountThreads) counts[static_cast<size_t>(p) * E + c] = hist[c];
+}
+
 // out[0, p*S+i] = idx, out[1, p*S+i] = loc + sum_{q<p} kept[q][idx]; dropped -> (-1,-1)
 // (tutel_moe_dispatch.cu:214-236).
 __global__ __launch_bounds__(kTile) void merge_masks_kernel(PtrTable t, int P, int S, int E,
@@ -1039,8 +1063,13 @@ hipError_t run_decode_rows(const void* expert_out, const void* gates, int gate_d
 }
 
 hipError_t run_count_experts(const PtrTable& indlocs, int P, int S, int E, uint32_t* counts, hipStream_t st) {
+  if (S <= kCountWhole) {
+    if (P == 0 || E == 0) return hipSuccess;
+    count_experts_whole_kernel<<<P, kCountThreads, E * sizeof(uint32_t), st>>>(indlocs, S, E, counts);
+    return hipGetLastError();
+  }
   hipError_t err = run_fill_u32(counts, static_cast<size_t>(P) * E, 0u, st);
-  if (err != hipSuccess || S == 0) return err;
+  if (err != hipSuccess) return err;
   dim3 grid((S + kTile * kCountPerThread - 1) / (kTile * kCountPerThread), P);
   count_experts_kernel<<<grid, kTile, E * sizeof(uint32_t), st>>>(indlocs, S, E, counts);
   return hipGetLastError();

@@ -89,3 +89,21 @@ def test_decode_gradients_in_one_pass(pkg, S, k, M, dt, gdt):
     ulp = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[gdt]
     assert d_gate.dtype == _TORCH[gdt]
     assert bool(((d_gate.float() - want).abs() <= 1e-5 * bound + ulp * want.abs()).all())
+
+
+@pytest.mark.parametrize("S", [1, 1023, 8193, 16384, 16385])
+@pytest.mark.parametrize("P,E", [(1, 1), (3, 70), (2, 512)])
+def test_partition_counts_at_the_limits_of_one_workgroup(pkg, S, P, E):
+    """moe_merge_masks on partitions that one workgroup counts alone (up to 16384 tokens) and on longer ones; exact."""
+    rng = np.random.default_rng(S + E)
+    masks = []
+    for _ in range(P):
+        e = rng.integers(-1, E, S).astype(np.int32)
+        masks.append(np.stack([e, rng.integers(0, 50, S).astype(np.int32)]))
+    got = to_np(pkg.ops.moe_merge_masks([dev(m) for m in masks], E))
+    before = np.zeros(E, np.int64)
+    for p, (e, l) in enumerate(masks):
+        part = got[:, p * S:(p + 1) * S]
+        np.testing.assert_array_equal(part[0], e)
+        np.testing.assert_array_equal(part[1], np.where(e >= 0, l + before[np.maximum(e, 0)], -1))
+        before += np.bincount(e[e >= 0], minlength=E)
