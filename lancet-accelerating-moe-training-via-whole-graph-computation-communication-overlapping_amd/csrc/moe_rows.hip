@@ -708,7 +708,7 @@ __device__ __forceinline__ float dot_vec(const u32x4& x, const u32x4& y, float a
   return acc;
 }
 // a granule with its first n bytes (whole elements) as zeros: the last granule of a row that was drawn back over bytes
-// another lane has already counted
+// another lane has already counted.  (Of both factors of a product: zero times infinity is no zero.)
 template <int DT>
 __device__ __forceinline__ u32x4 drop_bytes(u32x4 x, uint32_t n) {
 #pragma unroll
@@ -747,7 +747,11 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
     for (int v = h.v; v < row_vecs; v += h.step) {
       const uint32_t o = G::at(v, row_bytes);
       u32x4 x = G::ld(a + o), y = G::ld(b + o);
-      if (MODE == kAny16 && o != 16u * static_cast<uint32_t>(v)) x = drop_bytes<DT>(x, 16u * static_cast<uint32_t>(v) - o);
+      if (MODE == kAny16 && o != 16u * static_cast<uint32_t>(v)) {
+        const uint32_t n = 16u * static_cast<uint32_t>(v) - o;
+        x = drop_bytes<DT>(x, n);
+        y = drop_bytes<DT>(y, n);
+      }
       acc = dot_vec<DT>(x, y, acc);
     }
   } else {
@@ -860,10 +864,15 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
           if (b == 1 && !two) break;
-          u32x4 once = d[b];  // without the bytes that another lane has as well
+          // for the dot products: without the bytes that another lane has as well
+          u32x4 once = d[b];
           if (MODE == kAny16) {
             const uint32_t at = 16u * static_cast<uint32_t>(v + b * step);
-            if (o[b] != at) once = drop_bytes<DT>(once, at - o[b]);
+            if (o[b] != at) {
+              once = drop_bytes<DT>(once, at - o[b]);
+#pragma unroll
+              for (int j = 0; j < K; ++j) x[b][j] = drop_bytes<DT>(x[b][j], at - o[b]);
+            }
           }
 #pragma unroll
           for (int j = 0; j < K; ++j) {

@@ -107,3 +107,26 @@ def test_partition_counts_at_the_limits_of_one_workgroup(pkg, S, P, E):
         np.testing.assert_array_equal(part[0], e)
         np.testing.assert_array_equal(part[1], np.where(e >= 0, l + before[np.maximum(e, 0)], -1))
         before += np.bincount(e[e >= 0], minlength=E)
+
+
+@pytest.mark.parametrize("dt,M,offset", [("f32", 5, 0), ("f32", 9, 0), ("f32", 255, 0), ("f32", 12, 1), ("bf16", 9, 0), ("bf16", 15, 1), ("f16", 1003, 0),
+                                         ("bf16", 64, 3)])
+def test_weight_gradients_of_rows_with_an_infinity(pkg, dt, M, offset):
+    """One infinity per row, at every place among the last 24 elements (two granules and more: also those that the
+    drawn-back granule reads a second time), in the token row or in the expert's.  The other factor is not zero, so the
+    weight gradient is that infinity with the factor's sign, from moe_decode_dg and moe_decode_grad alike."""
+    ops = pkg.ops
+    S = min(M, 24)
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    rows = lambda: (torch.rand((S, M), device="cuda", generator=gen) + 0.5) * (torch.randint(0, 2, (S, M), device="cuda", generator=gen) * 2 - 1)  # noqa: E731
+    il = torch.stack([torch.zeros(S, dtype=torch.int32, device="cuda"), torch.arange(S, dtype=torch.int32, device="cuda")])
+    weights = torch.ones(S, device="cuda")
+    at = torch.arange(M - S, M, device="cuda")
+    here = torch.arange(S, device="cuda")
+    for infinite in (0, 1):
+        pair = [rows(), rows()]
+        pair[infinite][here, at] = float("inf")
+        want = pair[1 - infinite][here, at].sign() * float("inf")
+        tok, buf = (_at(x.to(_TORCH[dt]), offset) for x in pair)
+        assert torch.equal(ops.moe_decode_dg(tok, buf.view(1, S, M), il), want)
+        assert torch.equal(ops.moe_decode_grad(tok, buf.view(1, S, M), weights, il)[1], want)
