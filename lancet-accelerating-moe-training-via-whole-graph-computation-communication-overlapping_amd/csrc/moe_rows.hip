@@ -692,20 +692,38 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
   }
 }
 
-// acc + the products of the elements of two granules, in order
+// acc + the products of the elements of two granules, in order, one rounding per element.  (Spelled out: left to itself
+// the compiler moves sums into the chains it finds, or takes fp16 elements two at a time.)
 template <int DT>
 __device__ __forceinline__ float dot_vec(const u32x4& x, const u32x4& y, float acc) {
+#pragma clang fp contract(off)
   typedef Codec<DT> Cd;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     if (Cd::kPerVec == 4) {
-      acc += Cd::get(x[k]) * Cd::get(y[k]);
+      acc = __builtin_fmaf(Cd::get(x[k]), Cd::get(y[k]), acc);
     } else {
-      acc += Cd::get(static_cast<typename Cd::S>(x[k] & 0xffffu)) * Cd::get(static_cast<typename Cd::S>(y[k] & 0xffffu));
-      acc += Cd::get(static_cast<typename Cd::S>(x[k] >> 16)) * Cd::get(static_cast<typename Cd::S>(y[k] >> 16));
+      acc = __builtin_fmaf(Cd::get(static_cast<typename Cd::S>(x[k] & 0xffffu)), Cd::get(static_cast<typename Cd::S>(y[k] & 0xffffu)), acc);
+      acc = __builtin_fmaf(Cd::get(static_cast<typename Cd::S>(x[k] >> 16)), Cd::get(static_cast<typename Cd::S>(y[k] >> 16)), acc);
     }
   }
   return acc;
+}
+// The sum of the products of two granules.  Where a lane takes several granules of a row, each has a sum of its own (one
+// chain over both has up to a fifth more error against 64 bits: rows of 256 fp16 values 8.5e-8, so 7.6e-8), which makes the
+// sum over a row of up to 64 granules the same tree however many a lane takes.  Granules of rows that end inside one are
+// summed in pairs, as such rows have long been walked by a lane per element, without a chain.
+template <int DT, int MODE>
+__device__ __forceinline__ float dot_granule(const u32x4& x, const u32x4& y) {
+  if (MODE == kWhole16) return dot_vec<DT>(x, y, 0.f);
+  typedef Codec<DT> Cd;
+  const auto pair = [&](int k) {  // both elements of word k (fp32: of words k and k + 1)
+    if (Cd::kPerVec == 4) return __builtin_fmaf(Cd::get(x[k]), Cd::get(y[k]), mul_rn(Cd::get(x[k + 1]), Cd::get(y[k + 1])));
+    return __builtin_fmaf(Cd::get(static_cast<typename Cd::S>(x[k] & 0xffffu)), Cd::get(static_cast<typename Cd::S>(y[k] & 0xffffu)),
+                          mul_rn(Cd::get(static_cast<typename Cd::S>(x[k] >> 16)), Cd::get(static_cast<typename Cd::S>(y[k] >> 16))));
+  };
+  if (Cd::kPerVec == 4) return add_rn(pair(0), pair(2));
+  return add_rn(add_rn(pair(0), pair(1)), add_rn(pair(2), pair(3)));
 }
 // a granule with its first n bytes (whole elements) as zeros: the last granule of a row that was drawn back over bytes
 // another lane has already counted.  (Of both factors of a product: zero times infinity is no zero.)
@@ -744,15 +762,22 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
     const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
     const char* a = static_cast<const char*>(expert_out) + row * row_bytes;
     const char* b = static_cast<const char*>(dy) + s * row_bytes;
-    for (int v = h.v; v < row_vecs; v += h.step) {
-      const uint32_t o = G::at(v, row_bytes);
-      u32x4 x = G::ld(a + o), y = G::ld(b + o);
-      if (MODE == kAny16 && o != 16u * static_cast<uint32_t>(v)) {
-        const uint32_t n = 16u * static_cast<uint32_t>(v) - o;
-        x = drop_bytes<DT>(x, n);
-        y = drop_bytes<DT>(y, n);
+    if (MODE == kWhole16 && h.step == kWave) {  // many granules per lane: its sum goes on from one to the next
+      for (int v = h.v; v < row_vecs; v += kWave) {
+        const uint32_t o = G::at(v, row_bytes);
+        acc = dot_vec<DT>(G::ld(a + o), G::ld(b + o), acc);
       }
-      acc = dot_vec<DT>(x, y, acc);
+    } else {
+      for (int v = h.v; v < row_vecs; v += h.step) {
+        const uint32_t o = G::at(v, row_bytes);
+        u32x4 x = G::ld(a + o), y = G::ld(b + o);
+        if (MODE == kAny16 && o != 16u * static_cast<uint32_t>(v)) {
+          const uint32_t n = 16u * static_cast<uint32_t>(v) - o;
+          x = drop_bytes<DT>(x, n);
+          y = drop_bytes<DT>(y, n);
+        }
+        acc = add_rn(acc, dot_granule<DT, MODE>(x, y));
+      }
     }
   } else {
     typedef typename Cd::S St;
@@ -768,7 +793,8 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
 // decode_dx and decode_dg of one decode in one pass: a token's row of dy is read once, multiplied with the expert rows
 // its slots came from (the weights' gradients) and, times each weight, written to the same rows of the gradient.  As two
 // ops the row is read four times for top-2: 3.0 instead of 4.6 GB at 65536 x 4096 bf16 top-2, 32 experts.
-// Same products and roundings as decode_dx; the dot products are summed in another order than decode_dg's.
+// Same products and roundings as decode_dx; the dot products of rows of more than 64 granules are summed in another order
+// than decode_dg's.
 // Workgroups behind the tokens' clear the rows no slot owns.  Which those are, they look up in the inverse map
 // (decode_dx) or, in short batches, find out themselves by walking all slots, which saves the two launches that make
 // the map (kScanSlots below).
@@ -880,7 +906,7 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
             const u32x4 dd[1] = {d[b]};
             const float g[1] = {words.weight(j, true)};
             G::st(dst[j] + o[b], combine_vec<DT, 1>(dd, g));
-            acc[j] = dot_vec<DT>(once, x[b][j], acc[j]);
+            acc[j] = add_rn(acc[j], dot_granule<DT, MODE>(once, x[b][j]));
           }
         }
       }

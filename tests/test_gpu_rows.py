@@ -130,3 +130,43 @@ def test_weight_gradients_of_rows_with_an_infinity(pkg, dt, M, offset):
         tok, buf = (_at(x.to(_TORCH[dt]), offset) for x in pair)
         assert torch.equal(ops.moe_decode_dg(tok, buf.view(1, S, M), il), want)
         assert torch.equal(ops.moe_decode_grad(tok, buf.view(1, S, M), weights, il)[1], want)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M", [5, 8, 24, 64, 120, 256, 264, 512, 9, 60, 100, 257, 383, 500, 511])
+def test_weight_gradients_are_sums_of_granules(pkg, dt, M):
+    """Rows of up to 64 granules: a weight gradient is the sum over the granules' own sums, added up as a tree, however many
+    granules a lane takes.  Products of 16-bit values are exact in fp32, so that the order of the additions says every bit:
+    inside a granule in order where rows are whole granules, in pairs where they end inside one."""
+    ops = pkg.ops
+    S = 64
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    tok, buf = (torch.empty((S, M), device="cuda").normal_(generator=gen).to(_TORCH[dt]) for _ in range(2))
+    il = torch.stack([torch.zeros(S, dtype=torch.int32, device="cuda"), torch.arange(S, dtype=torch.int32, device="cuda")])
+    prod = to_np(tok) * to_np(buf)
+    if M < 8:
+        parts = prod                                             # a lane per element
+    else:
+        n = (M + 7) // 8
+        padded = np.zeros((S, n * 8), np.float32)
+        padded[:, :M] = prod
+        if M % 8:                                                # drawn back: zeros in front
+            padded[:, n * 8 - 8:] = 0
+            padded[:, n * 8 - (M - (n - 1) * 8):] = prod[:, (n - 1) * 8:]
+        p = padded.reshape(S, n, 8)
+        if M % 8 == 0:
+            parts = p[:, :, 0].copy()
+            for i in range(1, 8):
+                parts = parts + p[:, :, i]
+        else:
+            q = p[:, :, 0::2] + p[:, :, 1::2]
+            parts = (q[:, :, 0] + q[:, :, 1]) + (q[:, :, 2] + q[:, :, 3])
+    lanes = np.zeros((S, 64), np.float32)
+    lanes[:, :parts.shape[1]] = parts
+    o = 32
+    while o:
+        lanes = lanes[:, :o] + lanes[:, o:2 * o]
+        o //= 2
+    want = lanes[:, 0]
+    np.testing.assert_array_equal(to_np(ops.moe_decode_dg(tok, buf.view(1, S, M), il)), want)
+    np.testing.assert_array_equal(to_np(ops.moe_decode_grad(tok, buf.view(1, S, M), torch.ones(S, device="cuda"), il)[1]), want)
