@@ -188,12 +188,14 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
     const int used = a.rows_hi[e] - (a.rows_lo ? a.rows_lo[e] : 0);
     const int first = max(used, 0) + ch * kTailRows;
     const int last = min(first + kTailRows, a.C);
-    // the rows lie one behind the other: one run of granules
-    if (first >= last) return;
-    LANCET_GLOBAL char* run = as_global(a.out + (static_cast<size_t>(e) * a.C + first) * a.row_bytes);
-    const uint32_t bytes = static_cast<uint32_t>(last - first) * a.row_bytes;
-    const uint32_t n = (bytes + sizeof(V) - 1) / sizeof(V);
-    for (uint32_t v = threadIdx.x; v < n; v += kTile) G::st(run + G::at(v, bytes), G::zero());
+    // the rows lie one behind the other: one run of granules, or one per row where the run's length takes more than 32 bits
+    const int rows = a.row_bytes <= 0xffffffffu / kTailRows ? kTailRows : 1;
+    for (int r = first; r < last; r += rows) {
+      LANCET_GLOBAL char* run = as_global(a.out + (static_cast<size_t>(e) * a.C + r) * a.row_bytes);
+      const uint32_t bytes = static_cast<uint32_t>(min(rows, last - r)) * a.row_bytes;
+      const uint32_t n = static_cast<uint32_t>((bytes + sizeof(V) - 1) / sizeof(V));
+      for (uint32_t v = threadIdx.x; v < n; v += kTile) G::st(run + G::at(v, bytes), G::zero());
+    }
   }
 }
 

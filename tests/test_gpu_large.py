@@ -125,3 +125,18 @@ def test_pack_and_unpack_rebuild_the_buffer(big):
     back = torch.full_like(disp, 3.0)
     ops.memcpy_cont_to_sparse_3d(wire, back, elems, axis=0, zero_tail=True)
     assert torch.equal(_bits(back), _bits(disp))
+
+
+def test_zero_tail_of_rows_of_256_mib(pkg):
+    """Sixteen unused rows of 2^28 bytes each, the run one workgroup clears, are 2^32 bytes: more than 32 bits count."""
+    ops = pkg.ops
+    if torch.cuda.mem_get_info()[0] < 8 << 30:
+        pytest.skip("needs 8 GiB of free device memory")
+    M, C = 1 << 26, 17
+    data = torch.ones((1, M), device="cuda")
+    buf = torch.full((1, C, M), 7.0, device="cuda")
+    il = torch.zeros((2, 1), dtype=torch.int32, device="cuda")
+    ops.moe_scatter(data, il, None, torch.ones(1, dtype=torch.int32, device="cuda"), 1, C, out=buf)
+    assert bool((buf[0, 0] == 1).all())
+    for r in range(1, C):
+        assert not bool(buf[0, r].any())
