@@ -75,6 +75,8 @@ struct Granule<kAny16> {
   static __device__ __forceinline__ void st(LANCET_GLOBAL char* p, V x) { *(LANCET_GLOBAL u32x4_any*)p = x; }
   static __device__ __forceinline__ V zero() { return u32x4{0u, 0u, 0u, 0u}; }
 };
+// 16-byte granules of a row of 16 bytes or more (up to 4 GB, where adding first would wrap)
+__device__ __forceinline__ int granules_of(uint32_t row_bytes) { return static_cast<int>((row_bytes - 1u) / 16u + 1u); }
 template <typename E>
 struct GranuleElem {
   typedef E V;
@@ -357,7 +359,7 @@ __global__ __launch_bounds__(kTile) void decode_rows_kernel(DecodeArgs a) {
   if constexpr (MODE == kWhole16 || MODE == kAny16) {
     typedef Granule<MODE> G;
     const uint32_t row_bytes = static_cast<uint32_t>(a.M) * static_cast<uint32_t>(sizeof(typename Cd::S));
-    const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
+    const int row_vecs = granules_of(row_bytes);
     LANCET_GLOBAL char* dst = as_global(static_cast<char*>(a.out) + static_cast<size_t>(s) * row_bytes);
     const char* src[K];
 #pragma unroll
@@ -663,7 +665,7 @@ __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, c
   if constexpr (MODE == kWhole16 || MODE == kAny16) {
     typedef Granule<MODE> G;
     const uint32_t row_bytes = static_cast<uint32_t>(M) * static_cast<uint32_t>(sizeof(typename Cd::S));
-    const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
+    const int row_vecs = granules_of(row_bytes);
     LANCET_GLOBAL char* dst = as_global(static_cast<char*>(out) + static_cast<size_t>(r) * row_bytes);
     const u32x4 z = {0u, 0u, 0u, 0u};
     int v = h.v;
@@ -761,7 +763,7 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
   if constexpr (MODE == kWhole16 || MODE == kAny16) {
     typedef Granule<MODE> G;
     const uint32_t row_bytes = static_cast<uint32_t>(M) * static_cast<uint32_t>(sizeof(typename Cd::S));
-    const int row_vecs = static_cast<int>((row_bytes + 15u) / 16u);
+    const int row_vecs = granules_of(row_bytes);
     const char* a = static_cast<const char*>(expert_out) + row * row_bytes;
     const char* b = static_cast<const char*>(dy) + s * row_bytes;
     if (MODE == kWhole16 && h.step == kWave) {  // many granules per lane: its sum goes on from one to the next

@@ -140,3 +140,35 @@ def test_zero_tail_of_rows_of_256_mib(pkg):
     assert bool((buf[0, 0] == 1).all())
     for r in range(1, C):
         assert not bool(buf[0, r].any())
+
+
+def test_rows_of_almost_4_gib(pkg):
+    """The longest rows the library takes, 2^30 - 1 fp32 values: the number of their granules, rounded up, must not wrap.
+    Rows are zero but for values at both ends, whose products are exact."""
+    ops = pkg.ops
+    if torch.cuda.mem_get_info()[0] < 20 << 30:
+        pytest.skip("needs 20 GiB of free device memory")
+    M = (1 << 30) - 1
+    places = torch.tensor([0, 1, 5, M // 2, M - 6, M - 4, M - 3, M - 2, M - 1], device="cuda")
+    at = places.tolist()
+    x, y = torch.zeros(M, device="cuda"), torch.zeros(M, device="cuda")
+    x[places] = torch.arange(1.0, 1.0 + len(at), device="cuda")
+    y[places] = 2.0
+    il = torch.zeros((2, 1), dtype=torch.int32, device="cuda")
+    g = torch.full((1,), 3.0, device="cuda")
+
+    def is_3x(t):
+        t = t.view(-1)
+        return bool((t[places] == 3 * x[places]).all()) and int(t[:M // 2].count_nonzero() + t[M // 2:].count_nonzero()) == len(at)
+
+    out = torch.full((1, M), 7.0, device="cuda")
+    ops.moe_decode(x.view(1, 1, M), g, il, out=out)
+    assert is_3x(out)
+    out.fill_(7.0)
+    ops.moe_decode_dx(x.view(1, M), g, il, 1, 1, out=out.view(1, 1, M))
+    assert is_3x(out)
+    out.fill_(7.0)
+    dot = 2.0 * sum(range(1, 1 + len(at)))
+    _, dg = ops.moe_decode_grad(x.view(1, M), y.view(1, 1, M), g, il, out=(out.view(1, 1, M), torch.zeros_like(g)))
+    assert is_3x(out) and float(dg) == dot
+    assert float(ops.moe_decode_dg(x.view(1, M), y.view(1, 1, M), il)) == dot
