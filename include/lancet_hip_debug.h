@@ -27,8 +27,8 @@ int64_t lancet_lans_debug_chunk_table(const int64_t* numels, int T, int resident
 int lancet_lans_plan_debug(lancet_lans_plan_t plan, unsigned spin_limit, unsigned flags);
 
 /* *slots = chunk slots the resident kernel handed out in the plan's last lancet_lans_step, 0 when that step
- * went through the sweeps alone (schedule, no tensor that fits, or a resident tensor whose arrays were not
- * 16-byte aligned).  Lets a test tell which kernels it has exercised. */
+ * went through the sweeps alone (schedule, no tensor that fits, or a tensor of whole chunks whose arrays were not
+ * aligned to four elements).  Lets a test tell which kernels it has exercised. */
 int lancet_lans_plan_debug_last_resident(lancet_lans_plan_t plan, int* slots);
 
 /* Test hook: number of polls a workgroup of the position scan waits for a predecessor's word before it gives

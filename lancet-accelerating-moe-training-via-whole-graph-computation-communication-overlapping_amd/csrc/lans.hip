@@ -1288,6 +1288,9 @@ __global__ __launch_bounds__(kLansThreads, kResidentWavesPerSimd) void lans_resi
 // ---------------------------------------------------------------------------------------
 using namespace lancet;
 
+// the resident kernel's groups of tensors (see the plan's own order): none of them, whole chunks, ragged
+enum : char { kResNone, kResWhole, kResRagged };
+
 struct lancet_lans_plan {
   uint32_t magic;
   int device;
@@ -1312,7 +1315,7 @@ struct lancet_lans_plan {
   int n_res_slots;        // ... and of the ragged ones behind them
   int big_slot, ragged_slot, small_slot;  // first chunk slot of each group in the table of all tensors
   std::vector<int32_t> order;  // plan position -> position in the caller's lists
-  std::vector<char> is_resident;  // by position in the caller's lists: the resident kernel takes this tensor
+  std::vector<char> res_group;  // by position in the caller's lists: which of the resident kernel's groups the tensor is of
   size_t words_bytes;
   uint32_t spin_limit;
   int last_resident_slots;  // chunk slots the resident kernel of the last step handed out (0: it did not run)
@@ -1488,9 +1491,9 @@ extern "C" int lancet_lans_plan_create(const int64_t* numels, int T, lancet_lans
   pl->n_res_slots = static_cast<int>(L.res_tensor.size());
   pl->nchunks = static_cast<int>(L.ctensor.size());
   if (pl->n_res_slots > 0) pl->schedule = LANCET_LANS_RESIDENT;
-  pl->is_resident.assign(T, 0);
-  for (int k = 0; k < pl->small_first; ++k)
-    if (k < pl->big_first || k >= pl->ragged_first) pl->is_resident[pl->order[k]] = 1;
+  pl->res_group.assign(T, kResNone);
+  for (int k = 0; k < pl->big_first; ++k) pl->res_group[pl->order[k]] = kResWhole;
+  for (int k = pl->ragged_first; k < pl->small_first; ++k) pl->res_group[pl->order[k]] = kResRagged;
   // device block layout
   const size_t n = static_cast<size_t>(pl->nchunks);
   const size_t n1 = n ? n : 1;
@@ -1611,14 +1614,16 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   const uintptr_t g_elem = g_dtype == LANCET_F32 ? 3u : 1u;   // alignment masks: one element, four elements
   const uintptr_t g_vec = g_dtype == LANCET_F32 ? 15u : 7u;
   bool changed = false;
-  bool aligned16 = true;  // the resident kernel moves four elements per access: a step in which one of its tensors is not aligned to that runs as sweeps
+  // The resident kernel moves four elements per access: a step in which one of its whole tensors is not aligned to that
+  // runs as sweeps, one in which a ragged tensor is not leaves the ragged ones to the sweeps.
+  bool aligned[3] = {true, true, true};  // by group
   for (int i = 0; i < T; ++i) {
     void* const lo = p_lowp ? p_lowp[i] : nullptr;
     if (pl->numels[i] > 0 && (!g[i] || !p[i] || !m[i] || !v[i] || (p_lowp && !lo))) return LANCET_ERR_NULL;
     const uintptr_t bits = reinterpret_cast<uintptr_t>(p[i]) | reinterpret_cast<uintptr_t>(m[i]) | reinterpret_cast<uintptr_t>(v[i]);
     const uintptr_t gbits = reinterpret_cast<uintptr_t>(g[i]), lbits = reinterpret_cast<uintptr_t>(lo);
     if ((bits & 3u) || (gbits & g_elem) || (lbits & 1u)) return LANCET_ERR_ALIGN;
-    aligned16 = aligned16 && (!pl->is_resident[i] || ((bits & 15u) == 0 && (gbits & g_vec) == 0 && (lbits & 7u) == 0));
+    if ((bits & 15u) != 0 || (gbits & g_vec) != 0 || (lbits & 7u) != 0) aligned[static_cast<int>(pl->res_group[i])] = false;
     changed = changed || pl->shadow[i] != g[i] || pl->shadow[T + i] != p[i] ||
               pl->shadow[2 * T + i] != m[i] || pl->shadow[3 * T + i] != v[i] || pl->shadow[4 * T + i] != lo;
   }
@@ -1666,10 +1671,11 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   sc.spin_limit = pl->spin_limit;
   sc.epoch = 0;
   // The resident kernel takes the whole and the ragged tensors, the sweeps the large ones; under the sweeps schedule,
-  // and in a step whose arrays are not aligned, the sweeps take all three groups.  Its ragged chunks are padded with
-  // zeros, whose updates are 0 / eps: a step with an eps whose reciprocal is not safely finite leaves them to the sweeps.
-  const bool resident = pl->schedule == LANCET_LANS_RESIDENT && pl->n_res_slots > 0 && aligned16;
-  const bool ragged = resident && h->eps >= 1e-30f;
+  // and in a step whose whole tensors are not aligned, the sweeps take all three groups.  Its ragged chunks are padded with
+  // zeros, whose updates are 0 / eps: a step with an eps whose reciprocal is not safely finite leaves them to the sweeps,
+  // as does one in which a ragged tensor is not aligned.
+  const bool resident = pl->schedule == LANCET_LANS_RESIDENT && pl->n_res_slots > 0 && aligned[kResWhole];
+  const bool ragged = resident && aligned[kResRagged] && h->eps >= 1e-30f;
   t.nres = !resident ? 0 : ragged ? pl->n_res_slots : pl->n_whole_slots;
   pl->last_resident_slots = t.nres;
   const int sweep_tensor = resident ? pl->big_first : 0, sweep_slot = resident ? pl->big_slot : 0;

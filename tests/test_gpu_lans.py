@@ -589,3 +589,45 @@ def test_lans_norms_of_tensors_with_many_partial_sums(pkg):
             want = float(t.norm())
             assert abs(float(norms[k, i]) - want) <= 1.2e-6 * want
     plan.close()
+
+
+@pytest.mark.parametrize("gdt,which", [("f32", "p"), ("f32", "g"), ("bf16", "g"), ("bf16", "low")])
+def test_an_unaligned_ragged_tensor_leaves_the_whole_ones_alone(pkg, gdt, which):
+    """Tensors of whole chunks beside ragged ones, one of which has an array that is not aligned to four elements (a slice of
+    a flat bucket): the whole tensors stay in the resident kernel (its slots are theirs alone), the ragged ones go through
+    the sweeps, and the values are the oracle's.  With every array aligned the kernel takes both groups."""
+    capi = pkg.capi
+    numels = [5 * 8192, 20001, 3 * 8192, 16384 + 3]
+    rng, p, m, v = make_state(7, [(n,) for n in numels])
+    low = [torch.zeros(n, dtype=torch.bfloat16, device="cuda") for n in numels] if which == "low" else None
+    dp, dm, dv = [dev(a) for a in p], [dev(a) for a in m], [dev(a) for a in v]
+
+    def shifted(t):                       # t's values one element into an allocation
+        buf = torch.cat([t[:1], t])
+        return buf[1:]
+
+    if which == "p":
+        dp[1] = shifted(dp[1])
+    elif which == "low":
+        low[1] = shifted(low[1])
+    whole, ragged = 8, 3 + 3
+    plan = pkg.ops.LansPlan(numels)
+    for step in range(1, 4):
+        g = [_rounder(gdt)(rng.normal(0, 1e-3, n).astype(np.float32)).astype(np.float32) for n in numels]
+        lo.lans_step(g, p, m, v, step)
+        dg = [dev(a).to(_TORCH[gdt]) for a in g]
+        if which == "g":
+            dg[1] = shifted(dg[1])
+        plan.step(dg, dp, dm, dv, step, capi.LansHyper(1e-3, 0.9, 0.999, 1e-6, 1, 0.01, 1, 1, 1), p_lowp=low)
+        assert plan.last_resident_slots() == whole
+    for i in range(len(numels)):
+        assert_close_scaled(to_np(dp[i]), p[i], P_RTOL, "p[%d]" % i)
+        assert_close_scaled(to_np(dm[i]), m[i], 1e-5, "m[%d]" % i)
+        assert_close_scaled(to_np(dv[i]), v[i], 1e-5, "v[%d]" % i)
+        if low:
+            assert torch.equal(low[i], dp[i].to(torch.bfloat16))
+    same = lambda lst: [t.clone() for t in lst]  # noqa: E731
+    plan.step(same(dg), same(dp), same(dm), same(dv), 4, capi.LansHyper(1e-3, 0.9, 0.999, 1e-6, 1, 0.01, 1, 1, 1),
+              p_lowp=same(low) if low else None)
+    assert plan.last_resident_slots() == whole + ragged and plan.error() == 0
+    plan.close()
