@@ -418,7 +418,7 @@ int lancet_lans_step_mixed(lancet_lans_plan_t plan, const void* const* g, int g_
  * lancet_lans_plan_resident_capacity() chunks (the last chunk of a tensor may be a partial one); larger tensors of the
  * plan take the three sweeps in the same step.  So does every tensor of a step in which an array of a tensor of whole
  * chunks is not aligned to four elements, and every tensor with a partial chunk of a step in which an array of one of
- * those is not, or with eps < 1e-30.  Tensors of at most two chunks that are not whole chunks are updated by one
+ * those is not, with eps < 1e-30, or with a beta2 of 1 under bias correction.  Tensors of at most two chunks that are not whole chunks are updated by one
  * workgroup each, under either schedule.
  * Contract of this schedule: its workgroups wait for one another (for chunks of the same tensor only), so
  * at least half of them must be running on the device at the same time.  The grid is sized to what an

@@ -1672,10 +1672,12 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   sc.epoch = 0;
   // The resident kernel takes the whole and the ragged tensors, the sweeps the large ones; under the sweeps schedule,
   // and in a step whose whole tensors are not aligned, the sweeps take all three groups.  Its ragged chunks are padded with
-  // zeros, whose updates are 0 / eps: a step with an eps whose reciprocal is not safely finite leaves them to the sweeps,
+  // zeros, whose updates are 0 / (sqrt(0 / bc2) + eps): a step with an eps whose reciprocal is not safely finite, or with
+  // a second bias correction of zero (beta2 = 1; real elements are divided by infinity there), leaves them to the sweeps,
   // as does one in which a ragged tensor is not aligned.
   const bool resident = pl->schedule == LANCET_LANS_RESIDENT && pl->n_res_slots > 0 && aligned[kResWhole];
-  const bool ragged = resident && aligned[kResRagged] && h->eps >= 1e-30f;
+  const bool padding_is_zero = h->eps >= 1e-30f && !(h->bias_correction && (h->beta2 == 1.f || h->beta2 == -1.f));
+  const bool ragged = resident && aligned[kResRagged] && padding_is_zero;
   t.nres = !resident ? 0 : ragged ? pl->n_res_slots : pl->n_whole_slots;
   pl->last_resident_slots = t.nres;
   const int sweep_tensor = resident ? pl->big_first : 0, sweep_slot = resident ? pl->big_slot : 0;

@@ -631,3 +631,26 @@ def test_an_unaligned_ragged_tensor_leaves_the_whole_ones_alone(pkg, gdt, which)
               p_lowp=same(low) if low else None)
     assert plan.last_resident_slots() == whole + ragged and plan.error() == 0
     plan.close()
+
+
+@pytest.mark.parametrize("beta2", [1.0, -1.0])
+def test_a_second_bias_correction_of_zero(pkg, beta2):
+    """beta2 = 1 (or -1 in an even step) with bias correction: 1 - beta2^step is zero, v / 0 infinite and the update zero but
+    for the weight decay.  A last chunk padded with zeros would make 0 / 0 of it: tensors that end inside a chunk take the
+    other schedule, with the same finite values as a plan that runs the sweeps alone."""
+    capi = pkg.capi
+    numels = [3 * 8192, 16385, 3 * 8192 - 1, 1000]
+    out, slots = [], []
+    for schedule in (None, capi.LANS_SWEEPS):
+        g, p, m, v = _fresh_state(numels, 5)
+        v = [t + (1e-6 if beta2 == 1 else 0) for t in v]          # every new second moment is positive
+        plan = pkg.ops.LansPlan(numels, schedule=schedule)
+        plan.step(g, p, m, v, 2, capi.LansHyper(1e-3, 0.9, beta2, 1e-6, 1, 0.01, 1, 1, 1))
+        assert plan.error() == 0
+        slots.append(plan.last_resident_slots())
+        plan.close()
+        out.append(p + m + v)
+    for a, b in zip(*out):
+        assert bool(torch.isfinite(b).all())
+        assert_close_scaled(to_np(a), to_np(b), P_RTOL, "p, m or v")
+    assert slots == [3, 0]                            # the tensor of whole chunks alone
