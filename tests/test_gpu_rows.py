@@ -170,3 +170,19 @@ def test_weight_gradients_are_sums_of_granules(pkg, dt, M):
     want = lanes[:, 0]
     np.testing.assert_array_equal(to_np(ops.moe_decode_dg(tok, buf.view(1, S, M), il)), want)
     np.testing.assert_array_equal(to_np(ops.moe_decode_grad(tok, buf.view(1, S, M), torch.ones(S, device="cuda"), il)[1]), want)
+
+
+def test_decode_gradient_outputs_are_checked(pkg):
+    """moe_decode_grad writes E * C * M elements and k * S weights: outputs that do not hold them are refused on the host."""
+    ops = pkg.ops
+    S, E, C, M = 8, 2, 4, 16
+    data, dy, gate = torch.ones((E, C, M), device="cuda"), torch.ones((S, M), device="cuda"), torch.ones(S, device="cuda")
+    il = torch.stack([torch.arange(S, device="cuda") // C, torch.arange(S, device="cuda") % C]).int()
+    rows, weights = torch.empty_like(data), torch.empty_like(gate)
+    for out in ((rows[:, :3].contiguous(), weights), (rows.half(), weights), (rows.transpose(0, 1).contiguous().transpose(0, 1), weights),
+                (rows.cpu(), weights), (rows, weights[:7]), (rows, weights.half()), (rows, torch.empty(2 * S, device="cuda")[::2]),
+                (rows, weights.cpu())):
+        with pytest.raises(ValueError):
+            ops.moe_decode_grad(dy, data, gate, il, out=out)
+    ops.moe_decode_grad(dy, data, gate, il, out=(rows, weights))
+    assert bool((rows == 1).all()) and bool((weights == M).all())
