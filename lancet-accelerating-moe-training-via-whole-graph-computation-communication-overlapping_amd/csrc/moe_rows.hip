@@ -435,27 +435,40 @@ __global__ __launch_bounds__(kTile) void count_experts_kernel(PtrTable t, int S,
 }
 
 // Partitions of up to kCountWhole tokens: one workgroup counts a partition alone, sixteen tokens a thread at most, so that
-// nothing has to be cleared first and no counter is shared: four partitions of 8192 tokens 1.4 + 3.1 us in two launches, 2.8 in
-// one; the partitioned chain of 32768 x 2048 tokens, which counts twice, 201 -> 198 us.
+// nothing has to be cleared first and no counter is shared between workgroups.  Bound by the LDS atomics of its one CU,
+// which run one after the other where they meet in a counter: every counter has kCountCopies copies side by side, one per
+// lane modulo their number.  moe_merge_masks, four partitions, 64 experts, in us: clearing and counting in several
+// workgroups / one workgroup with one copy / with sixteen
+//   8192 tokens, even 6.4 / 5.2 / 5.1, seven in ten on one expert 6.6 / 9.4 / 5.4
+//   16384 tokens, even 6.4 / 5.9 / 5.9, all on one expert 6.8 / 18.5 / 5.9
+// (8 copies are up to 8 % slower there, 32 the same).  Beyond kCountWhole the one CU's share grows and the launches' does not.
 constexpr int kCountWhole = 16384;
 constexpr int kCountThreads = 1024;
+constexpr int kCountCopies = 16;
+static_assert(LANCET_MAX_EXPERTS * kCountCopies * sizeof(uint32_t) <= 32768, "LDS a launch may have by default, twice over");
 __global__ __launch_bounds__(kCountThreads) void count_experts_whole_kernel(PtrTable t, int S, int E, uint32_t* counts) {
   extern __shared__ uint32_t hist[];
   const int p = blockIdx.x;
   const int32_t* idx = static_cast<const int32_t*>(t.p[p]);
-  for (int c = threadIdx.x; c < E; c += kCountThreads) hist[c] = 0;
+  for (int c = threadIdx.x; c < E * kCountCopies; c += kCountThreads) hist[c] = 0;
   __syncthreads();
   constexpr int kBatch = 8;  // loads in flight per thread
+  const int copy = threadIdx.x % kCountCopies;
   for (int i = threadIdx.x; i < S; i += kBatch * kCountThreads) {
     int e[kBatch];
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) e[k] = i + k * kCountThreads < S ? idx[i + k * kCountThreads] : -1;
 #pragma unroll
     for (int k = 0; k < kBatch; ++k)
-      if (e[k] >= 0 && e[k] < E) atomicAdd(&hist[e[k]], 1u);
+      if (e[k] >= 0 && e[k] < E) atomicAdd(&hist[e[k] * kCountCopies + copy], 1u);
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < E; c += kCountThreads) counts[static_cast<size_t>(p) * E + c] = hist[c];
+  for (int c = threadIdx.x; c < E; c += kCountThreads) {
+    uint32_t n = 0;
+#pragma unroll
+    for (int k = 0; k < kCountCopies; ++k) n += hist[c * kCountCopies + (k + c) % kCountCopies];  // (neighbours in other banks)
+    counts[static_cast<size_t>(p) * E + c] = n;
+  }
 }
 
 // out[0, p*S+i] = idx, out[1, p*S+i] = loc + sum_{q<p} kept[q][idx]; dropped -> (-1,-1)
@@ -1104,7 +1117,7 @@ hipError_t run_decode_rows(const void* expert_out, const void* gates, int gate_d
 hipError_t run_count_experts(const PtrTable& indlocs, int P, int S, int E, uint32_t* counts, hipStream_t st) {
   if (S <= kCountWhole) {
     if (P == 0 || E == 0) return hipSuccess;
-    count_experts_whole_kernel<<<P, kCountThreads, E * sizeof(uint32_t), st>>>(indlocs, S, E, counts);
+    count_experts_whole_kernel<<<P, kCountThreads, E * kCountCopies * sizeof(uint32_t), st>>>(indlocs, S, E, counts);
     return hipGetLastError();
   }
   hipError_t err = run_fill_u32(counts, static_cast<size_t>(P) * E, 0u, st);

@@ -186,3 +186,17 @@ def test_decode_gradient_outputs_are_checked(pkg):
             ops.moe_decode_grad(dy, data, gate, il, out=out)
     ops.moe_decode_grad(dy, data, gate, il, out=(rows, weights))
     assert bool((rows == 1).all()) and bool((weights == M).all())
+
+
+@pytest.mark.parametrize("S,E", [(16384, 1), (16384, 512), (16383, 64), (40, 512)])
+@pytest.mark.parametrize("kind", ["one", "two", "sorted"])
+def test_partition_counts_of_few_experts(pkg, S, E, kind):
+    """Tokens that meet in one counter, in two, or expert by expert in token order: every lane counts in a copy of its own
+    modulo their number.  The second partition's locations are the first one's counts; exact."""
+    e = {"one": np.full(S, E - 1), "two": np.arange(S) % 2 * (E - 1), "sorted": np.arange(S) * E // S}[kind].astype(np.int32)
+    e[::13] = -1
+    mask = dev(np.stack([e, np.zeros(S, np.int32)]))
+    got = to_np(pkg.ops.moe_merge_masks([mask, mask], E))
+    np.testing.assert_array_equal(got[0], np.concatenate([e, e]))
+    counts = np.bincount(e[e >= 0], minlength=E)
+    np.testing.assert_array_equal(got[1, S:], np.where(e >= 0, counts[np.maximum(e, 0)], -1))
