@@ -28,7 +28,7 @@ struct RouteArgs {
 // K = 2: ranks of both slots are produced in one pass (2E counters); slot-2 locations need the
 //        slot-1 totals of all tiles, so raw (expert, rank, value) are left in the output arrays
 //        and finalize_top2_kernel completes them.
-template <int K, int GD>
+template <int K, int GD, bool HELD>
 __global__ __launch_bounds__(kTile) void route_scan_kernel(RouteArgs a) {
   extern __shared__ uint32_t s_cnt[];
   const int tid = threadIdx.x;
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kTile) void route_scan_kernel(RouteArgs a) {
       e[0] = (x >= 0 && x < a.E) ? x : -1;
     }
   } else {
-    const Routed r = route_tile_token<K, GD>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
+    const Routed r = route_tile_token<K, GD, HELD>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
     if (valid) {
       e[0] = r.e0;
       p[0] = r.p0;
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kTile) void route_scan_kernel(RouteArgs a) {
 // ---- the same routing as two or three kernels that wait for nothing (scan_form) ------------------------------
 // route_count_kernel: selection, ranks inside the tile, the tile's counts -> table.  Leaves expert, rank inside the
 // tile and raw gate value in idx_out / loc_out / gates_s (idx_out is not written when the experts are given).
-template <int K, int GD>
+template <int K, int GD, bool HELD>
 __global__ __launch_bounds__(kTile) void route_count_kernel(RouteArgs a) {
   extern __shared__ uint32_t s_cnt[];
   const int tid = threadIdx.x;
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(kTile) void route_count_kernel(RouteArgs a) {
       e[0] = (x >= 0 && x < a.E) ? x : -1;
     }
   } else {
-    const Routed r = route_tile_token<K, GD>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
+    const Routed r = route_tile_token<K, GD, HELD>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
     if (valid) {
       e[0] = r.e0;
       p[0] = r.p0;
@@ -296,12 +296,12 @@ __global__ __launch_bounds__(kTile) void finalize_top2_kernel(RouteArgs a) {
 }
 
 // Selection only (no scan).
-template <int K, int GD>
+template <int K, int GD, bool HELD>
 __global__ __launch_bounds__(kTile) void gate_topk_kernel(const void* gate, const void* noise, int S, int E,
                                                           int is_logits, int32_t* idx, void* val) {
   extern __shared__ uint32_t s_stage[];
   const int s = blockIdx.x * kTile + threadIdx.x;
-  const Routed r = route_tile_token<K, GD>(gate, noise, s, S, E, is_logits != 0, s_stage);
+  const Routed r = route_tile_token<K, GD, HELD>(gate, noise, s, S, E, is_logits != 0, s_stage);
   if (s >= S) return;
   idx[s] = r.e0;
   st_gate(val, s, r.p0, GD);
@@ -396,10 +396,10 @@ hipError_t run_gate_topk(const void* gate, const void* noise, int S, int E, int 
                          int32_t* idx, void* val, hipStream_t st) {
   if (S == 0) return hipSuccess;
   const int blocks = (S + kTile - 1) / kTile;
-  const size_t lds = stage_lds_bytes(gate_dtype, gate, K == 2 ? noise : nullptr, S, E);
-  LANCET_GATE_SWITCH(gate_dtype,
-    if (K == 1) gate_topk_kernel<1, GD><<<blocks, kTile, lds, st>>>(gate, nullptr, S, E, is_logits, idx, val);
-    else gate_topk_kernel<2, GD><<<blocks, kTile, lds, st>>>(gate, noise, S, E, is_logits, idx, val))
+  const SelectLaunch sel = select_launch(gate_dtype, gate, K == 2 ? noise : nullptr, S, E, is_logits);
+  LANCET_SELECT_SWITCH(gate_dtype, sel.held,
+    if (K == 1) gate_topk_kernel<1, GD, HELD><<<blocks, kTile, sel.lds, st>>>(gate, nullptr, S, E, is_logits, idx, val);
+    else gate_topk_kernel<2, GD, HELD><<<blocks, kTile, sel.lds, st>>>(gate, noise, S, E, is_logits, idx, val))
   return hipGetLastError();
 }
 
@@ -427,16 +427,17 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
   a.ws = scan_ws_view(ws);
   a.seg_rows = 0;
   hipError_t err = hipSuccess;
-  const size_t lds = std::max(scan_lds_bytes(K * E), idx_in ? size_t(0) : stage_lds_bytes(gate_dtype, gate, a.noise, S, E));
+  const SelectLaunch sel = idx_in ? SelectLaunch{false, 0} : select_launch(gate_dtype, gate, a.noise, S, E, is_logits);
+  const size_t lds = std::max(scan_lds_bytes(K * E), sel.lds);
   const ScanForm form = scan_form(a.ntiles, static_cast<int64_t>(K) * E, K, force_lookback);
   if (form != kScanLookback) {
     // two or three kernels that wait for nothing instead of a look-back between tiles that all run at once
     const int NC = K * E;
     const size_t lds2 = 2 * static_cast<size_t>(NC) * sizeof(uint32_t);
     if (K == 1) {
-      LANCET_GATE_SWITCH(gate_dtype, (route_count_kernel<1, GD><<<a.ntiles, kTile, lds, st>>>(a)))
+      LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_count_kernel<1, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
     } else {
-      LANCET_GATE_SWITCH(gate_dtype, (route_count_kernel<2, GD><<<a.ntiles, kTile, lds, st>>>(a)))
+      LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_count_kernel<2, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
     }
     err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -450,9 +451,9 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
     return hipGetLastError();
   }
   if (K == 1) {
-    LANCET_GATE_SWITCH(gate_dtype, (route_scan_kernel<1, GD><<<a.ntiles, kTile, lds, st>>>(a)))
+    LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_scan_kernel<1, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
   } else {
-    LANCET_GATE_SWITCH(gate_dtype, (route_scan_kernel<2, GD><<<a.ntiles, kTile, lds, st>>>(a)))
+    LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_scan_kernel<2, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     finalize_top2_kernel<<<a.ntiles, kTile, 0, st>>>(a);

@@ -176,14 +176,35 @@ constexpr int kHeldPerLane = 4;
 constexpr int kHeldGranules = 16 * kHeldPerLane;
 typedef u32x4 u32x4_gate __attribute__((aligned(2)));
 
-// Rows of 3 to 64 granules.  Two granules are as fast walked by their lane (16 tiles x 8 fp32 experts: 7.4 us, held 7.8).
-// Without the softmax the walk is a few compares per value and has no serial rounds, which short launches on aligned rows
-// notice (32 tiles x 32 experts 8.4 us, held 8.8; 128 x 64 6.9, held 7.5): they keep it.  The choice is the same either way.
-constexpr int kHeldMinTiles = 256;
-__host__ __device__ inline bool rows_are_held(const void* gate, const void* noise, int S, int E, int gb, bool is_logits) {
-  const int bytes = E * gb;
+// Which rows are held (`gate` values of gb bytes, no noise).  Rows of 3 to 64 granules that are not whole granules or not
+// aligned to them: all, whatever the batch (the walk takes them value by value: 2048 x 31 fp32 13.6 us, held 7.5).  Aligned
+// rows of whole granules, where the walk is a load per granule (walked / held, top-1, us):
+//   * the lanes of a row take n = 4, 8, 16, 32 or 64 granules and do the work of all whether the row has them or not, so
+//     that a row of 36 costs as much as one of 64: 16384 x 144 fp32 logits 18.0 / 25.6, x 256 22.6 / 22.7.  In short launches
+//     only full lanes pay, and rows of up to 16 granules of which one in eight is missing (2048 x 60 fp32 9.9 / 9.5, x 52
+//     9.2 / 9.5; in less than a tile a tenth slower).  From 384 tiles on, where the walk's lines no longer survive in the cache
+//     from one load to the next, three quarters are enough (98304 x 96 fp32 27.7 / 23.6, 65536 of them 30.1 / 30.2), and
+//     from 512 tiles on any row of more than the line that a walk reads at once (131072 x 144 fp32 42.9 / 35.9);
+//   * fp32 rows of more than 16 granules in less than a tile: a wave has 16 and more rounds of them to itself, one after
+//     the other, where the walk has one (64 x 256 logits 13.4 / 16.1);
+//   * without the softmax the walk is a few compares per value, and only the cache decides: from 512 tiles and a whole line
+//     on (131072 x 64 fp32 19.1 / 15.0; 98304 x 128 18.9 / 21.0).
+// The choice is the same either way.
+constexpr int kStageMinTiles = 512;
+constexpr int kHeldPackedTiles = 384;
+inline bool rows_are_held(const void* gate, const void* noise, int S, int E, int gb, bool is_logits) {
+  const int bytes = E * gb, n = bytes / 16;
   if (noise != nullptr || bytes <= 32 || bytes > 16 * kHeldGranules) return false;
-  return is_logits || (S + kTile - 1) / kTile >= kHeldMinTiles || bytes % 16 != 0 || (reinterpret_cast<uintptr_t>(gate) & 15u) != 0;
+  if (bytes % 16 != 0 || (reinterpret_cast<uintptr_t>(gate) & 15u) != 0) return true;
+  const int tiles = (S + kTile - 1) / kTile;
+  int taken = kHeldPerLane;
+  while (taken < n) taken *= 2;
+  const bool packed = 4 * n >= 3 * taken;
+  if (!is_logits) return tiles >= kStageMinTiles && n >= 8 && packed;
+  if (tiles >= kStageMinTiles) return n > 8 || packed;
+  if (tiles >= kHeldPackedTiles) return packed;
+  if (n < taken) return n <= 16 && 8 * n >= 7 * taken && tiles >= 4;
+  return n <= 16 || gb == 2 || S >= kTile;
 }
 
 // f(x, i) for the values of a granule as fp32; i is the value's place in it
@@ -340,16 +361,14 @@ __device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, i
   return res;
 }
 
-// ---- rows longer than registers hold: staged through LDS ----------------------------------------------------
+// ---- rows longer than a cache line: staged through LDS ------------------------------------------------------
 // A lane that walks its own row touches each 128-byte line of it in eight loads, and every load of the wave
 // touches 64 different lines; with rows of several lines and many waves on a CU the lines are evicted between a
-// lane's visits and fetched again.  Rows of more than 64 granules are therefore read the way they lie in memory, a wave's
-// 64 rows 128 bytes at a time (eight lanes per row and line, every line whole in one load), passed through LDS and walked
-// from there, each lane its own row as before: the values and their order are the same, so is the result.  It pays from
-// about two workgroups per CU on (512 tiles); launches of fewer tiles keep the direct walk, whose lines survive in the
-// cache (both measured with rows of 256 fp32 experts, which are held in registers now: 262144 rows 274 -> 92 us, 65536 rows
-// top-2 50 against 64).
-constexpr int kStageMinTiles = 512;
+// lane's visits and fetched again.  Such rows, where they are not held in registers, are therefore read the way they lie in
+// memory, a wave's 64 rows 128 bytes at a time (eight lanes per row and line, every line whole in one load), passed through
+// LDS and walked from there, each lane its own row as before: the values and their order are the same, so is the result.  It
+// pays from about two workgroups per CU on (kStageMinTiles: 262144 rows of 256 fp32 experts 274 -> 92 us); launches of fewer
+// tiles keep the direct walk, whose lines survive in the cache (65536 of them, top-2, 50 against 64).
 constexpr int kStageChunk = 128;                   // bytes of a row staged at a time
 constexpr int kStageRow = kStageChunk + 16;        // row pitch in LDS (the pad spreads the lanes' reads over the banks)
 constexpr int kStageWave = kWave * kStageRow;      // bytes per wave
@@ -358,7 +377,7 @@ constexpr int kStageBytes = kWavesPerTile * kStageWave;
 template <int GD>
 __host__ __device__ inline bool rows_are_staged(const void* gate, const void* noise, int S, int E) {
   constexpr int gb = GD == LANCET_F32 ? 4 : 2;
-  return noise == nullptr && (S + kTile - 1) / kTile >= kStageMinTiles && E * gb > 16 * kHeldGranules && (E * gb) % 16 == 0 &&
+  return noise == nullptr && (S + kTile - 1) / kTile >= kStageMinTiles && E * gb > kStageChunk && (E * gb) % 16 == 0 &&
          (reinterpret_cast<uintptr_t>(gate) & 15u) == 0;
 }
 
@@ -435,14 +454,15 @@ __device__ __forceinline__ F walk_rows_staged(const char* rows, int nrows, int E
 }
 
 // Selection for token s of a workgroup whose thread t holds token s = first + t (kTile consecutive tokens): what
-// route_token gives, by the direct walk or through LDS.  All kTile threads, uniform control flow; lds = at least
-// kStageBytes when rows_are_staged (it may be reused after the call).  Threads with s >= S get {-1, -1, 0, 0}.
-template <int K, int GD>
+// route_token gives, from registers (HELD: rows_are_held), by the direct walk or through LDS.  All kTile threads, uniform
+// control flow; lds = at least kStageBytes when rows_are_staged (it may be reused after the call).  Threads with s >= S get
+// {-1, -1, 0, 0}.
+template <int K, int GD, bool HELD>
 __device__ __forceinline__ Routed route_tile_token(const void* gate, const void* noise, int s, int S, int E, bool is_logits,
                                                    void* lds) {
   constexpr size_t gb = GD == LANCET_F32 ? 4 : 2;
   Routed r = {-1, -1, 0.f, 0.f};
-  if (rows_are_held(gate, noise, S, E, static_cast<int>(gb), is_logits)) {
+  if (HELD) {
     const int first = s - lane_id();  // the wave's first token
     if (first < S) {
       const Routed held = route_rows_held<K, GD>(static_cast<const char*>(gate) + static_cast<size_t>(first) * E * gb,
@@ -492,11 +512,21 @@ __device__ __forceinline__ Routed route_tile_token(const void* gate, const void*
     default: { constexpr int GD = LANCET_F32; __VA_ARGS__; } break;           \
   }
 
-// LDS a selecting kernel needs for the rows it stages (0: it walks them directly)
-inline size_t stage_lds_bytes(int gate_dtype, const void* gate, const void* noise, int S, int E) {
-  bool staged = false;
-  LANCET_GATE_SWITCH(gate_dtype, staged = rows_are_staged<GD>(gate, noise, S, E))
-  return staged ? kStageBytes : 0;
+// GD and HELD as compile-time constants inside `...`
+#define LANCET_SELECT_SWITCH(gd, held, ...)                         \
+  LANCET_GATE_SWITCH(gd, if (held) { constexpr bool HELD = true; __VA_ARGS__; } else { constexpr bool HELD = false; __VA_ARGS__; })
+
+// how a kernel that selects is launched: its variant, and the LDS it needs for the rows it stages
+struct SelectLaunch {
+  bool held;
+  size_t lds;
+};
+inline SelectLaunch select_launch(int gate_dtype, const void* gate, const void* noise, int S, int E, bool is_logits) {
+  SelectLaunch l = {rows_are_held(gate, noise, S, E, gate_dtype == LANCET_F32 ? 4 : 2, is_logits), 0};
+  if (!l.held) {
+    LANCET_GATE_SWITCH(gate_dtype, l.lds = rows_are_staged<GD>(gate, noise, S, E) ? kStageBytes : 0)
+  }
+  return l;
 }
 
 }  // namespace lancet

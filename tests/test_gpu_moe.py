@@ -1128,3 +1128,34 @@ def test_selection_at_every_row_length(pkg, gd, E):
             bound = (2 * tol + (3 if k == 2 else 1) * eps if logits else 0.0) * np.abs(val) + (2.0 ** -24 if gd == "f16" else 0.0) * k
             got = to_np(g.float()).astype(np.float64).reshape(k, S)
             assert (np.abs(got - val) <= bound).all(), np.abs(got - val).max()
+
+
+@pytest.mark.parametrize("gd,E", [("f32", 16), ("f32", 20), ("f32", 24), ("f32", 36), ("f32", 96), ("f32", 144), ("f32", 256), ("bf16", 24), ("bf16", 48),
+                                  ("bf16", 72), ("bf16", 96), ("f16", 288), ("bf16", 512)])
+def test_selection_of_long_batches_and_their_pieces(pkg, gd, E):
+    """Aligned rows are held in registers, walked or staged by the length of the batch and by how full their lanes are: at
+    383, 384, 511 and 512 tiles the choice is that of the same rows in pieces of 64 and 256 tiles, and of a piece that
+    starts at an unaligned address (always held); the values are the same to the sums' rounding (E terms: E * 2^-23)."""
+    ops = pkg.ops
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[gd]
+    gen = torch.Generator(device="cuda").manual_seed(E)
+    S = 512 * 256
+    x = torch.empty((S, E), device="cuda").normal_(generator=gen).to(tdt)
+    x[::5, E - 1] = x[::5, 0]                    # ties between the first and the last lane
+    x[3::77] = -float("inf")
+    x[3::77, E // 2] = 1.0
+    for k in (1, 2):
+        for logits in (True, False):
+            gate = x if logits else x.float().exp().to(tdt)
+            def route(g):
+                v, il, _, _ = ops.moe_route(g, None, 1, top_k=k, gate_is_logits=logits, capacity=k * g.shape[0])
+                return il[0].view(k, -1), v.view(k, -1).float()
+            odd = torch.empty(1 + 4096 * E, dtype=tdt, device="cuda")[1:].view(4096, E)
+            odd.copy_(gate[:4096])
+            idx, val = route(gate)
+            bound = (2 * E * 2.0 ** -23 + (0 if gd == "f32" else 2.0 ** (-7 if gd == "bf16" else -9))) * val
+            for n in (383 * 256, 384 * 256 - 1, 511 * 256, 511 * 256 + 1, 64 * 256, 256 * 256):
+                a, b = route(gate[:n])
+                assert torch.equal(a, idx[:, :n]) and bool(((b - val[:, :n]).abs() <= bound[:, :n]).all())
+            a, b = route(odd)
+            assert torch.equal(a, idx[:, :4096]) and bool(((b - val[:, :4096]).abs() <= bound[:, :4096]).all())
