@@ -172,17 +172,20 @@ __device__ __forceinline__ void walk_groups(const BprArgs& a, const uint32_t* s_
   }
 }
 
-// One workgroup per expert; what bounds it is the one expert that most tokens chose, whose keys a single CU reads and
-// counts.  The digits start below the leading bits that all keys share (probabilities have two or three exponents, so a
-// digit that starts at bit 31 puts every key into the same few bins, whose LDS atomics then run one after the other),
-// and passes end with the lowest bit in which keys differ.  32768 tokens on 64 experts of which a few are hot (top-1,
-// most keys on one expert): 78 -> 18.5 us.
+// One workgroup per expert.  What bounds it is, in long batches, the one expert that most tokens chose, whose keys a single
+// CU reads and counts; in short ones the barriers of its 1024 threads, of which a digit takes six.  The digits start below
+// the leading bits that all keys share (probabilities have two or three exponents, so a digit that starts at bit 31 puts
+// every key into the same few bins, whose LDS atomics then run one after the other).  As soon as no more keys than a wave has
+// lanes share what is found of the threshold, which is mostly after one digit, they are compared with one another.  32768
+// tokens on 64 experts of which a few are hot (top-1, most keys on one expert): four 8-bit digits from bit 31 on 78 us, three
+// of 10 bits 18.5.  moe_encode_batch_prioritized as a whole, the same two and with the keys compared after the first digit:
+// 256 tokens on 16 experts 17.1 / 18.2 / 15.6 us, 1024 on 64 20.5 / 21.4 / 18.7.
 __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
   __shared__ uint32_t s_keys[kSelectKeys];
   __shared__ uint32_t s_pos[kSelectTiles];
   __shared__ uint32_t hist[1 << kSelectBits];
   __shared__ uint32_t s_wave[kSelectThreads / kWave];
-  __shared__ uint32_t s_prefix, s_need, s_count, s_min, s_max;
+  __shared__ uint32_t s_prefix, s_need, s_count, s_min, s_max, s_bin, s_few;
   const int e = blockIdx.x;
   const int tid = threadIdx.x;
   // The expert's keys, in token order.  Up to kSelectTiles tiles, the prepare kernel's groups say where they are:
@@ -192,6 +195,7 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
   uint32_t count = 0, nfront = 0;
   if (tid == 0) {
     s_count = 0;
+    s_few = 0;
     s_min = 0xffffffffu;
     s_max = 0u;
   }
@@ -275,7 +279,8 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
   // digits from the highest bit in which two keys differ; `left` bits are still to be found
   int left = s_min == s_max ? 0 : 32 - __clz(s_min ^ s_max);
   uint32_t prefix = left == 32 ? 0u : s_min >> left;
-  while (left > 0) {
+  uint32_t open = count;  // keys that share what is found of the threshold
+  while (left > 0 && open > kWave) {
     const int bits = min(left, kSelectBits);
     const int shift = left - bits;
     const uint32_t digits = (1u << bits) - 1u;
@@ -296,10 +301,40 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
     if ((above < need && need <= above + h) || (bin == 0u && total < need)) {
       s_need = need - above;
       s_prefix = (left == 32 ? 0u : prefix << bits) | bin;
+      s_bin = h;
     }
     __syncthreads();
     prefix = s_prefix;
+    open = s_bin;
     left = shift;
+  }
+  if (left > 0) {
+    // no more keys than a wave has lanes: it compares them with one another, and counts the threshold's equals that
+    // precede the partition on the way
+    every_key([&](uint32_t k, bool early) {
+      if (left == 32 || (k >> left) == prefix) {
+        const uint32_t at = atomicAdd(&s_few, 1u);
+        hist[at] = k;
+        hist[kWave + at] = early;
+      }
+    });
+    __syncthreads();
+    if (tid < static_cast<int>(open)) {
+      const uint32_t mine = hist[tid];
+      uint32_t above = 0, same = 0, front = 0;
+      for (uint32_t i = 0; i < open; ++i) {
+        above += hist[i] > mine;
+        same += hist[i] == mine;
+        front += (hist[i] == mine) & hist[kWave + i];
+      }
+      const uint32_t need = s_need;
+      if (above < need && need <= above + same) {  // equal keys write the same words
+        a.par[e] = foreign_word(0u, mine);
+        a.par[a.E + e] = foreign_word(0u, need - above);
+        a.par[2 * a.E + e] = foreign_word(0u, front);
+      }
+    }
+    return;
   }
   const uint32_t thr = prefix;
   // ties that precede the partition

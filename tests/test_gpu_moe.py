@@ -1159,3 +1159,28 @@ def test_selection_of_long_batches_and_their_pieces(pkg, gd, E):
                 assert torch.equal(a, idx[:, :n]) and bool(((b - val[:, :n]).abs() <= bound[:, :n]).all())
             a, b = route(odd)
             assert torch.equal(a, idx[:, :4096]) and bool(((b - val[:, :4096]).abs() <= bound[:, :4096]).all())
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 700])
+@pytest.mark.parametrize("kind", ["distinct", "ties", "equal", "two_bins"])
+@pytest.mark.parametrize("P", [1, 2])
+def test_bpr_select_of_few_keys(pkg, n, kind, P):
+    """n keys on one of two experts, of which a part fits: around the 64 that a wave compares with one another, at once or
+    after a digit that leaves as many (keys in two narrow groups) or more (ties); ties that precede the second partition.
+    Routing is bit-exact."""
+    rng = np.random.default_rng(n)
+    S0 = 2 * n + (2 * n) % P
+    gate = np.full((S0, 2), 0.125, np.float32)
+    mine = rng.permutation(S0)[:n]
+    gate[:, 1] = 0.25
+    values = {"distinct": 0.5 + rng.permutation(n) / (4.0 * n), "ties": 0.5 + rng.integers(0, 3, n) / 8.0, "equal": np.full(n, 0.5),
+              "two_bins": np.where(rng.random(n) < 0.5, 0.5, 0.75) + rng.permutation(n) * 2.0 ** -20}[kind]
+    gate[mine, 0] = values.astype(np.float32)
+    data = rng.standard_normal((S0, 4), dtype=np.float32)
+    for cf in (0.3, 0.9):
+        for pid in range(P):
+            want = mo.moe_encode_bpr(data, gate, P, pid, cf, fast_scatter=True)
+            got = pkg.ops.moe_encode_batch_prioritized(dev(data), dev(gate), P, pid, cf)
+            np.testing.assert_array_equal(to_np(got[1]), want[1])
+            np.testing.assert_array_equal(to_np(got[2]), want[2])
+            np.testing.assert_array_equal(to_np(got[4]), want[4])
