@@ -316,7 +316,9 @@ struct RowWords {
 };
 
 // (Granules per lane: one for top-2, two for top-1, so that a wave has two row loads in flight either way.  65536 x 4096
-// bf16: top-2 264 us with one, 270 with two, 273 with four; top-1 193 / 177 / 188.)
+// bf16: top-2 264 us with one, 270 with two, 273 with four; top-1 193 / 177 / 188.  Two for top-2 as well where a row of
+// more than a wave would leave lanes idle, which is to say where it has no power of two of granules: 32768 x 2560 bf16 105.1
+// with one, 83.6 with two, 32768 x 3072 113.0 and 98.3, 32768 x 4096 130.0 and 132.3.)
 struct DecodeArgs {
   const void* expert_out;
   const void* gates;     // [K*S] of gate_dtype; null = all ones (moe_encode_dx)
@@ -975,6 +977,10 @@ static inline int row_lanes(long units, long rows, int per_lane, int max_q = 10)
   while (q > 0 && ((rows << q) + kTile - 1) / kTile > 0x3fffffffL) --q;
   return q;
 }
+// Few granules in all: the launch is over when its first loads are back, and a second granule per lane only makes the waves
+// longer (rows of at most a wave, decode top-1, two / one: 1024 x 192 bf16 2.9 / 2.5 us, 8192 x 128 3.2 / 2.9; 4096 x 384 with
+// half as many again 3.4 / 3.7).
+static inline bool few_granules(long units, long rows) { return units * rows <= 131072; }
 static inline long row_blocks(long rows, int q) { return ((rows << q) + kTile - 1) / kTile; }
 
 // the way rows of row_bytes bytes in arrays at the given addresses are cut
@@ -1075,7 +1081,10 @@ template <int DT>
 static hipError_t decode_launch(DecodeArgs a, int K, RowMode mode, hipStream_t st) {
   if (a.S == 0 || a.M == 0) return hipSuccess;
   constexpr int eb = sizeof(typename Codec<DT>::S);
-  a.q = row_lanes(row_granules(mode, static_cast<size_t>(a.M) * eb, eb), a.S, K == 1 ? 2 : 1);
+  const int units = row_granules(mode, static_cast<size_t>(a.M) * eb, eb);
+  const bool few = few_granules(units, a.S);
+  const bool spare = units > kWave && (units & (units - 1)) != 0 && !few;
+  a.q = row_lanes(units, a.S, K == 1 ? (few && units <= kWave ? 1 : 2) : (spare ? 2 : 1));
   const unsigned blocks = static_cast<unsigned>(row_blocks(a.S, a.q));
   if (a.dest) {
     if (mode != kWhole16) return hipErrorInvalidValue;
@@ -1164,7 +1173,8 @@ template <int DT>
 static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, void* out, int S, int M,
                                    long rows, int K, RowMode mode, hipStream_t st) {
   constexpr int eb = sizeof(typename Codec<DT>::S);
-  const int q = row_lanes(row_granules(mode, static_cast<size_t>(M) * eb, eb), rows, 2);  // two granules per lane: 442 -> 408 us
+  const int units = row_granules(mode, static_cast<size_t>(M) * eb, eb);
+  const int q = row_lanes(units, rows, few_granules(units, rows) && units <= kWave ? 1 : 2);  // two granules per lane: 442 -> 408 us
   const unsigned blocks = static_cast<unsigned>(row_blocks(rows, q));
   LANCET_CODED_ROW_SWITCH(DT, mode,
     if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, q);
@@ -1257,9 +1267,10 @@ static hipError_t decode_dg_launch(const void* dy, const void* expert_out, const
                                    void* out, int gd, int S, int M, int E, int C, int n, RowMode mode, hipStream_t st) {
   constexpr int eb = sizeof(typename Codec<DT>::S);
   // two granules per lane from 512 bytes on (262144 x 512 bf16 top-1 53 -> 43 us, 65536 x 384 top-2 44 -> 33), one in
-  // shorter rows (200000 x 64: 10.6 against 15.5)
+  // shorter rows (200000 x 64: 10.6 against 15.5) and, with rows of at most a wave, in launches of up to 262144 granules
+  // (4096 x 512 bf16 top-1 3.2 against 3.7)
   const int units = row_granules(mode, static_cast<size_t>(M) * eb, eb);
-  const int q = row_lanes(units, n, units >= 32 ? 2 : 1, 6);
+  const int q = row_lanes(units, n, units >= 32 && !few_granules(units, n / 2) ? 2 : 1, 6);
   LANCET_CODED_ROW_SWITCH(DT, mode, (decode_dg_kernel<DT, MODE><<<static_cast<unsigned>(row_blocks(n, q)), kTile, 0, st>>>(dy, expert_out, idx, loc, out, gd, S, M, E, C, n, q)))
   return hipGetLastError();
 }

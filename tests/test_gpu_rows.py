@@ -200,3 +200,30 @@ def test_partition_counts_of_few_experts(pkg, S, E, kind):
     np.testing.assert_array_equal(got[0], np.concatenate([e, e]))
     counts = np.bincount(e[e >= 0], minlength=E)
     np.testing.assert_array_equal(got[1, S:], np.where(e >= 0, counts[np.maximum(e, 0)], -1))
+
+
+@pytest.mark.parametrize("dt,M,S", [("bf16", 768, 1365), ("bf16", 768, 1366), ("f32", 520, 1100), ("bf16", 1003, 1100), ("f16", 520, 2017), ("f32", 256, 2049), ("bf16", 24, 43691)])
+@pytest.mark.parametrize("k", [1, 2])
+def test_gathers_of_one_and_two_granules_per_lane(pkg, dt, M, S, k):
+    """Lanes take one or two granules of a row by the number of granules in all (131072) and by whether a row fills its
+    lanes: sizes on both sides of the line, rows of 96 and 126 granules among them.  Bit for bit in fp32, 16-bit sums
+    within one unit in the last place."""
+    ops = pkg.ops
+    E = 4
+    data, logits = make_inputs(S + M, S, M, E)
+    x = rows_as_oracle(data, dt)
+    d_g, d_il, _, _, _ = ops.moe_encode(rows_to_torch(data[:, :1], dt), dev(logits), None, 0.9, top_k=k, gate_is_logits=True)
+    C = ops.moe_capacity(S, E, 0.9 * k)
+    il, w = to_np(d_il), to_np(d_g)
+    buf = rows_as_oracle(np.random.default_rng(S).standard_normal((E, C, M), dtype=np.float32), dt)
+    d_buf = rows_to_torch(buf, dt)
+
+    def near(got, want):
+        if dt == "f32":
+            np.testing.assert_array_equal(to_np(got), want)
+        else:
+            assert ulp_distance(got, torch.from_numpy(want).to(_TORCH[dt]).cuda()) <= 1
+
+    near(ops.moe_decode(d_buf, d_g, d_il, top_k=k), mo.moe_decode(buf, w, il, k=k))
+    near(ops.moe_encode_dx(d_buf, d_il, top_k=k), mo.moe_encode_dx(buf, il, k))
+    near(ops.moe_decode_dx(rows_to_torch(data, dt), d_g, d_il, E, C, top_k=k), mo.moe_decode_dx(x, w, il, E, C, k))
