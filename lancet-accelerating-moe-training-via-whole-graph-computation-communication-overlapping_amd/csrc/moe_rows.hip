@@ -1011,7 +1011,8 @@ static inline int row_granules(RowMode mode, size_t row_bytes, int elem_bytes) {
 // workgroups on a CU instead of 8: with all wave slots taken its reads crowd out its writes.  8 / 6 / 5 / 4 / 3 workgroups:
 // 344 / 337 / 324 / 350 / 420 us at 65536 x 4096 bf16 top-2, 206 / 208 / 200 / 221 / 243 top-1, 165 against 160 at rows of
 // 2048.  Rows of one wave want every slot: 90 / 92 / 99 / 108 us at 262144 x 512.  The gather kernels do not gain.
-constexpr size_t kScatterLds = 27000;
+constexpr size_t kCuLds = 160 * 1024;
+constexpr size_t kScatterLds = kCuLds / 6 + 1;  // six do not fit, however LDS is rounded up; five do
 
 hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, const int32_t* loc,
                             const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
@@ -1205,10 +1206,14 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
   }
 }
 
-// Slots up to which the clearing workgroups of decode_grad_kernel walk all of them themselves (64 KB of indices each).
+// Slots up to which the clearing workgroups of decode_grad_kernel walk all of them themselves instead of looking rows up in
+// a map that two launches before it make.  Map / walk by workgroups of 64 rows, us: 1024 slots, 4 to 512 experts, rows of 64
+// bf16 6.3 / 3.0; 4096 slots 6.6 / 4.5, rows of 2048 14.6 / 14.5 with 4 experts and 14.6 / 12.1 with 512; 8192 slots 7.0 / 7.1,
+// rows of 2048 23.3 / 24.7 and 24.0 / 23.3; 12000 slots 7.2 / 9.6.  (128 rows per workgroup: those that have rows to clear
+// become the launch's end, 18.1 us for the 14.5 above.)
 constexpr int kScanSlots = 8192;
-constexpr int kGradTailRows = 16;   // rows per clearing workgroup with the inverse map
-constexpr int kGradScanRows = 128;  // ... that walks the slots: enough for the walk to be worth it
+constexpr int kGradTailRows = 16;  // rows per clearing workgroup with the inverse map
+constexpr int kGradScanRows = 64;  // ... that walks the slots
 
 template <int DT>
 static hipError_t decode_grad_launch(DecodeGradArgs a, int K, int M, RowMode mode, hipStream_t st) {
