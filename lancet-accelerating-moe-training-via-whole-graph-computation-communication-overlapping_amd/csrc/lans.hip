@@ -191,8 +191,9 @@ __device__ __forceinline__ LansElem make_elem(const LansScalars& sc, float gn, f
 
 // bias corrections 1 - beta^step (src/op/dialect/cuda/lans.cc:108-113), from a host step or
 // from the fp32 step scalar in device memory (no host synchronisation, unlike lans.cc:102-107)
-// (The powers by repeated squaring in double: at most 62 products, 1e-14 relative, where the float result has 6e-8;
-// the general pow takes several microseconds on its one lane, which every step waits for.)
+// (The powers by repeated squaring in double.  A squaring doubles the relative error, so that beta^step carries step * 2^-53
+// of it; of 1 - beta^step that is at most 2^-53 / (1 - beta), 2e-9 for the largest float below 1, where the float result is
+// rounded to 6e-8.  The general pow takes several microseconds on its one lane, which every step waits for.)
 __device__ __forceinline__ void bias_corrections(const LansScalars& sc, float& bc1, float& bc2) {
   int step = sc.step_host;
   if (sc.step_dev) step = static_cast<int>(*sc.step_dev);
@@ -1213,7 +1214,7 @@ __device__ __forceinline__ void small_step(const LansTables& t, const LansScalar
 }
 
 // Workgroup 0 begins the step: clears the resident kernel's ticket, moves the step epoch on, decides whether the step
-// runs at all (step_is_skipped), forms the two bias corrections (pow in double: kept out of the resident kernel, whose
+// runs at all (step_is_skipped), forms the two bias corrections (in double: kept out of the resident kernel, whose
 // registers are all spoken for) and brings the caller's gradient norms into the plan's order.  The epoch lives on the
 // device so that a step recorded in a graph tags every replay differently; when it wraps (2^31 steps) every word of
 // earlier steps is forgotten.  The error word is left alone.

@@ -1,6 +1,7 @@
 // Row movers: scatter of token rows into the [E,C,M] expert buffer, weighted gather-combine
-// back, partition merge of masks and buffers.  All are pure HBM streaming: one wave per row,
-// 16-byte accesses, streaming (non-temporal) loads and stores, every output byte written once.
+// back, partition merge of masks and buffers, and the gradients of both.  All are pure HBM streaming: rows
+// shared by part of a wave, a wave or several, 16-byte accesses, every output byte written once (but for the
+// bytes that two granules of a row share which ends inside one: written twice, with the same value).
 #include "launchers.hpp"
 #include "common.hpp"
 #include "../../include/lancet_hip.h"
@@ -757,8 +758,8 @@ __device__ __forceinline__ u32x4 drop_bytes(u32x4 x, uint32_t n) {
 }
 
 // grad_gates_s[i] = <expert_out[idx, loc, :], dy[s, :]> for slot-token i, 0 when the slot is dropped
-// (decode_backward_gate_kernel, tutel_moe_dispatch.cu:126-157): one wave per slot-token, fp32 partial
-// sums per lane, xor-tree over the wave.
+// (decode_backward_gate_kernel, tutel_moe_dispatch.cu:126-157): at most a wave per slot-token, fp32 partial
+// sums per lane, xor-tree over its lanes.
 template <int DT, int MODE>
 __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const void* expert_out,
                                                           const int32_t* idx, const int32_t* loc, void* out, int gd,
