@@ -954,7 +954,7 @@ def main():
                                "(BASELINE config 4 shape, headline)" % (S, M, E, Cap),
                    "tokens": S, "hidden": M, "experts": E, "capacity": Cap, "top_k": K,
                    "kept_slots": kept, "gate": "fp32 logits, softmax fused"},
-        "roofline": {"bound": "hbm", "kernel": "scatter_rows_kernel<u32x4,2> (encode_forward)",
+        "roofline": {"bound": "hbm", "kernel": "scatter_rows_kernel<kWhole16,2> (encode_forward)",
                      "achieved": round(scatter_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(scatter_gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": "profiles/scatter_rows_headline_traffic.json: HBM bytes per launch from rocprofv3 --pmc "
