@@ -409,14 +409,14 @@ int lancet_lans_step_mixed(lancet_lans_plan_t plan, const void* const* g, int g_
  * replay is a new step.  The pointer tables are uploaded (one host-to-device copy) by the first call that
  * sees a new set of pointers: make that call once before recording. */
 /* Schedules of the step.
- * LANCET_LANS_RESIDENT (what a new plan has when the kernel takes at least one of its tensors): one persistent kernel that
+ * LANCET_LANS_RESIDENT (what a new plan has when at least one tensor fits it: at most the capacity in chunks, and either whole chunks
+ * or more than two): one persistent kernel that
  * reads and writes every array once (28 B/param).  Each workgroup runs a three-stage pipeline over chunks of
  * 8192 parameters (sum of g^2 / moments and the two updates / parameter write) and keeps a chunk on chip
  * between the stages; it publishes the sums of its chunks and forms the norms it needs from the published
  * sums of all the tensor's chunks.  The kernel takes the tensors of at most
- * lancet_lans_plan_resident_capacity() chunks.  The last chunk of a tensor may be a partial one if the tensor has more than
- * two; a plan without tensors of whole chunks sweeps these unless they have more than one and a half times the capacity
- * in chunks.  Larger tensors of the plan take the three sweeps in the same step.  So does every tensor of a step in which an array of a tensor of whole
+ * lancet_lans_plan_resident_capacity() chunks (the last chunk of a tensor may be a partial one); larger tensors of the
+ * plan take the three sweeps in the same step.  So does every tensor of a step in which an array of a tensor of whole
  * chunks is not aligned to four elements, and every tensor with a partial chunk of a step in which an array of one of
  * those is not, with eps < 1e-30, or with a beta2 of 1 under bias correction.  Tensors of at most two chunks that are not whole chunks are updated by one
  * workgroup each, under either schedule.

@@ -1369,20 +1369,6 @@ static ChunkLayout chunk_layout(const int64_t* numels, int T, int limit, int rou
     else if (k <= limit) ragged.push_back(i);
     else big.push_back(i);
   }
-  // Ragged tensors by themselves fill the kernel's pipeline for more than a round and a half, or the sweeps are the
-  // shorter way (30 of 66666 parameters, bf16 gradients and copies, 270 chunks: 29.4 us swept, 34.2 resident; 4 of 1048577, 516
-  // chunks: 46.3 and 49.4; 12 of 589825, 876 chunks: 70.1 and 58.0).  Beside whole tensors, whose kernel runs anyway, they cost
-  // less there than in launches of their own.
-  const auto chunks_in = [&](const std::vector<int32_t>& group) {
-    int64_t n = 0;
-    for (int i : group) n += chunks_of(numels[i]);
-    return n;
-  };
-  if (chunks_in(whole) == 0 && 2 * chunks_in(ragged) <= 3 * static_cast<int64_t>(std::max(round, 1))) {
-    big.insert(big.end(), ragged.begin(), ragged.end());
-    std::sort(big.begin(), big.end());
-    ragged.clear();
-  }
   const auto larger = [&](int a, int b) { return chunks_of(numels[a]) > chunks_of(numels[b]); };
   std::stable_sort(whole.begin(), whole.end(), larger);
   if (round < 1) round = 1;

@@ -660,31 +660,3 @@ def test_a_second_bias_correction_of_zero(pkg, beta2):
         assert bool(torch.isfinite(b).all())
         assert_close_scaled(to_np(a), to_np(b), P_RTOL, "p, m or v")
     assert slots == [3, 0]                            # the tensor of whole chunks alone
-
-
-def test_ragged_tensors_alone_are_swept_until_they_fill_the_kernel(pkg):
-    """A plan of ragged tensors only: swept up to one and a half rounds of the resident kernel, resident beyond; with a tensor
-    of whole chunks beside them they are resident however few they are.  The values are the same to the sums' rounding."""
-    capi = pkg.capi
-    grid = pkg.ops.LansPlan([3 * 8192]).resident_capacity()[0]
-    n, chunks = 20 * 8192 + 5, 21
-    few, many = 3 * grid // 2 // chunks, 3 * grid // 2 // chunks + 1
-    for numels, slots in (([n] * few, 0), ([n] * many, chunks * many), ([8192] + [n] * 2, 1 + 2 * chunks)):
-        plan, sweeps = pkg.ops.LansPlan(numels), pkg.ops.LansPlan(numels, schedule=capi.LANS_SWEEPS)
-        assert plan.schedule() == (capi.LANS_RESIDENT if slots else capi.LANS_SWEEPS)
-        if not slots:
-            with pytest.raises(capi.LancetError):
-                plan.set_schedule(capi.LANS_RESIDENT)
-        out = []
-        for each in (plan, sweeps):
-            state = _fresh_state(numels, 3)
-            for step in (1, 2):
-                each.step(*state, step, capi.LansHyper(1e-3, 0.9, 0.999, 1e-6, 1, 0.01, 1, 1, 1))
-            out.append(state[1] + state[2] + state[3])
-        # (a round is not split over two: padding behind the last tensor that fits counts as slots)
-        assert plan.last_resident_slots() >= slots and bool(plan.last_resident_slots()) == bool(slots)
-        assert plan.error() == 0 and sweeps.last_resident_slots() == 0
-        for a, b in zip(*out):
-            assert_close_scaled(to_np(a), to_np(b), P_RTOL, "p, m or v")
-        plan.close()
-        sweeps.close()
