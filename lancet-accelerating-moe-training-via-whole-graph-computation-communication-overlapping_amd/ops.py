@@ -456,11 +456,12 @@ def moe_decode_grad(dy, data, gate, indices_locations, top_k=1, workspace=None, 
     _need(dy.shape[0] == S and gate.dim() == 1 and gate.shape[0] == top_k * S, "dy, gate and indices_locations disagree")
     E, Cap, M = data.shape
     if out is None:
-        out = torch.empty_like(data), torch.empty_like(gate)
-    d_data, d_gate = out
-    _dev(d_data, "the expert rows' gradient"), _dev(d_gate, "the gate gradient")
-    _need(d_data.shape == data.shape and d_data.dtype == data.dtype, "the expert rows' gradient has the rows' shape and dtype")
-    _need(d_gate.shape == gate.shape and d_gate.dtype == gate.dtype, "the gate gradient has the gate's shape and dtype")
+        d_data, d_gate = torch.empty_like(data), torch.empty_like(gate)
+    else:
+        d_data, d_gate = out
+        _dev(d_data, "the expert rows' gradient"), _dev(d_gate, "the gate gradient")
+        _need(d_data.shape == data.shape and d_data.dtype == data.dtype, "the expert rows' gradient has the rows' shape and dtype")
+        _need(d_gate.shape == gate.shape and d_gate.dtype == gate.dtype, "the gate gradient has the gate's shape and dtype")
     ws = _workspace(int(lib.lancet_moe_decode_dx_workspace_bytes(E, Cap)), dy.device, workspace)
     st = lib.lancet_moe_decode_grad(_p(dy), _p(data), _p(gate), _p(indices_locations), S, M, E, Cap, top_k, _dtype_code(dy),
                                     _gate_code(gate), _p(d_data), _p(d_gate), _p(ws), ws.numel(), _stream())
