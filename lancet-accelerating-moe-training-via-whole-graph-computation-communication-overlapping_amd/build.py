@@ -2,6 +2,7 @@
 
 liblancet_hip.so      HIP kernels + the C ABI declared in include/lancet_hip.h
 liblancet_raf_ops.so  C++ op layer (RAF OpEnv / dialect vocabulary) on top of the C ABI
+lancet_torch_host.so  host path of the operators over torch tensors (a Python extension on top of the C ABI)
 
 Run `python build.py` (or __graft_entry__.build()).  hipcc cross-compiles without a GPU.
 """
@@ -64,10 +65,22 @@ def build_ops():
     return out
 
 
+def build_torch_host():
+    """The native host path of the operators: a Python extension over the C ABI and torch's own libraries."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    out = os.path.join(LIBDIR, "lancet_torch_host.so")
+    include = [sysconfig.get_paths()["include"]] + cpp_extension.include_paths() + ["/opt/rocm/include"]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"] +
+         [x for d in include for x in ("-isystem", d)] +
+         ["-o", out, os.path.join(HERE, "torch_host", "torch_host.cc")] +
+         [x for d in cpp_extension.library_paths() for x in ("-L", d)] +
+         ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-L", LIBDIR, "-llancet_hip", "-Wl,-rpath,$ORIGIN"])
+    return out
+
+
 def build_all():
-    a = build_hip()
-    b = build_ops()
-    return [p for p in (a, b) if p]
+    return [p for p in (build_hip(), build_ops(), build_torch_host()) if p]
 
 
 if __name__ == "__main__":

@@ -4,6 +4,7 @@ The library is loaded from <package>/lib/liblancet_hip.so (built in-tree by buil
 There is no fallback: a missing library raises.
 """
 import ctypes as C
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -132,6 +133,29 @@ def load():
         raise RuntimeError("liblancet_hip.so has ABI version %d, expected %d" % (got, ABI_VERSION))
     _lib = lib
     return lib
+
+
+HOST_NAME = "lancet_torch_host"
+_host = None
+
+
+def host():
+    """The native host path of the operators (torch_host/): argument checks, allocation and launch in one call each.
+    Raises if it was not built."""
+    global _host
+    if _host is None or _lib is None:
+        load()
+        path = os.path.join(os.path.dirname(LIB_PATH), HOST_NAME + ".so")
+        if not os.path.exists(path):
+            raise RuntimeError("%s.so is not built (%s). Run `python %s` first; there is no fallback path."
+                               % (HOST_NAME, path, os.path.join(HERE, "build.py")))
+        spec = importlib.util.spec_from_file_location(HOST_NAME, path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        from . import ops
+        module.bind(LancetError, ops._scan_pool, ops._scan_workspace)
+        _host = module
+    return _host
 
 
 def status_string(status):

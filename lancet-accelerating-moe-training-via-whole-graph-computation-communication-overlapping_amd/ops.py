@@ -59,14 +59,6 @@ def _dev(t, name):
     _need(t.is_contiguous(), "%s must be contiguous" % name)
 
 
-def _workspace(nbytes, device, given):
-    if given is not None:
-        _need(given.is_cuda and given.dtype == torch.uint8 and given.numel() >= nbytes,
-              "workspace must be a uint8 GPU tensor of at least %d bytes" % nbytes)
-        return given
-    return torch.empty(max(int(nbytes), 4), dtype=torch.uint8, device=device)
-
-
 class ScanWorkspace:
     """Device memory of the position scan (moe_encode, moe_route, moe_encode_batch_prioritized, gen_location).
 
@@ -130,15 +122,6 @@ def moe_capacity(S, E, capacity_factor):
     return int(capi.load().lancet_moe_capacity(int(S), int(E), float(capacity_factor)))
 
 
-def _check_encode_inputs(data, gate):
-    _dev(data, "data"), _dev(gate, "gate")
-    _need(data.dim() == 2, "Expected input data to be 2D.")
-    _need(gate.dim() == 2, "Expected input gate to be 2D.")
-    _need(data.shape[0] == gate.shape[0], "Input data and gate should have matching shape in dim 0.")
-    _gate_code(gate)
-    return _dtype_code(data)
-
-
 @functools.lru_cache(maxsize=256)
 def moe_encode_workspace_bytes(S, E, top_k=1):
     return int(capi.load().lancet_moe_encode_workspace_bytes(int(S), int(E), int(top_k)))
@@ -147,14 +130,6 @@ def moe_encode_workspace_bytes(S, E, top_k=1):
 def _flags(gate_is_logits, zero_tail, rows_at_used=False, scan_lookback=False):
     return ((capi.GATE_IS_LOGITS if gate_is_logits else 0) | (0 if zero_tail else capi.NO_TAIL_ZERO) |
             (capi.ROWS_AT_USED if rows_at_used else 0) | (capi.SCAN_LOOKBACK if scan_lookback else 0))
-
-
-def _check_noise(gate2_noise, gate, top_k):
-    if gate2_noise is None:
-        return
-    _dev(gate2_noise, "gate2_noise")
-    _need(top_k == 2, "gate2_noise only exists for the second choice (top_k = 2)")
-    _need(gate2_noise.shape == gate.shape and gate2_noise.dtype == gate.dtype, "gate2_noise must have the gate's shape and dtype")
 
 
 def moe_encode(data, gate, used_capacity, capacity_factor=1.0, top_k=1, gate_is_logits=False,
@@ -175,35 +150,8 @@ def moe_encode(data, gate, used_capacity, capacity_factor=1.0, top_k=1, gate_is_
     int(2 * capacity_factor * ceil(S / E)) when E does not divide S or the factor is fractional
     (S = 300, E = 8, factor 1: 75 against 76).  scan_lookback=True runs the position scan as one kernel with a
     look-back between its tiles whatever the size (LANCET_SCAN_LOOKBACK)."""
-    lib = capi.load()
-    dt = _check_encode_inputs(data, gate)
-    S, M = data.shape
-    E = gate.shape[1]
-    _need(top_k in (1, 2), "top_k must be 1 or 2")
-    _check_noise(gate2_noise, gate, top_k)
-    cf = float(capacity_factor) * (2.0 if top_k == 2 else 1.0)
-    Cap = moe_capacity(S, E, cf) if capacity is None else int(capacity)
-    _need(Cap >= 0, "capacity must not be negative")
-    if used_capacity is not None:
-        _dev(used_capacity, "used_capacity")
-        _need(used_capacity.dim() == 1 and used_capacity.numel() == E and used_capacity.dtype == torch.int32,
-              "Input used_capacity should be 1-D int32 of length E.")
-    dev = data.device
-    if out is None:
-        gates_s = torch.empty(top_k * S, dtype=gate.dtype, device=dev)
-        indloc = torch.empty((2, top_k * S), dtype=torch.int32, device=dev)
-        used_out = torch.empty(E, dtype=torch.int32, device=dev)
-        elems = torch.empty(E, dtype=torch.int64, device=dev)
-        disp = torch.empty((E, Cap, M), dtype=data.dtype, device=dev)
-    else:
-        gates_s, indloc, used_out, elems, disp = out
-    ws = _scan_workspace(moe_encode_workspace_bytes(S, E, top_k), dev, workspace)
-    _need(gates_s.dtype == gate.dtype, "gates_s takes the gate's dtype")
-    st = lib.lancet_moe_encode(_p(data), _p(gate), _p(gate2_noise), _p(used_capacity), S, M, E, Cap, top_k, dt,
-                               _gate_code(gate), _flags(gate_is_logits, zero_tail, rows_at_used, scan_lookback), _p(gates_s), _p(indloc),
-                               _p(used_out), _p(elems), _p(disp), _p(ws.buf), ws.nbytes, _stream())
-    capi.check(st, "lancet_moe_encode")
-    return gates_s, indloc, used_out, elems.view(torch.uint64) if elems.dtype == torch.int64 else elems, disp
+    return capi.host().moe_encode(data, gate, gate2_noise, used_capacity, capacity_factor, None if capacity is None else int(capacity),
+                                  top_k, _flags(gate_is_logits, zero_tail, rows_at_used, scan_lookback), workspace, out)
 
 
 def moe_route(gate, used_capacity, M, capacity_factor=1.0, top_k=1, gate_is_logits=False, gate2_noise=None,
@@ -211,26 +159,8 @@ def moe_route(gate, used_capacity, M, capacity_factor=1.0, top_k=1, gate_is_logi
     """The routing half of moe_encode (selection + position scan, src/op/dialect/cuda/moe.cc:366-380), so that
     a caller can run it ahead of, or beside, the row movement of another partition.  M only scales
     elements_per_expert.  Returns (gates_s, indices_locations, used_capacity, elements_per_expert)."""
-    lib = capi.load()
-    _dev(gate, "gate")
-    _need(gate.dim() == 2, "gate must be 2-D")
-    gd = _gate_code(gate)
-    S, E = gate.shape
-    _need(top_k in (1, 2), "top_k must be 1 or 2")
-    _check_noise(gate2_noise, gate, top_k)
-    Cap = moe_capacity(S, E, float(capacity_factor) * (2.0 if top_k == 2 else 1.0)) if capacity is None else int(capacity)
-    dev = gate.device
-    if out is None:
-        out = (torch.empty(top_k * S, dtype=gate.dtype, device=dev),
-               torch.empty((2, top_k * S), dtype=torch.int32, device=dev),
-               torch.empty(E, dtype=torch.int32, device=dev), torch.empty(E, dtype=torch.int64, device=dev))
-    gates_s, indloc, used_out, elems = out[:4]
-    ws = _scan_workspace(moe_encode_workspace_bytes(S, E, top_k), dev, workspace)
-    _need(gates_s.dtype == gate.dtype, "gates_s takes the gate's dtype")
-    st = lib.lancet_moe_route(_p(gate), _p(gate2_noise), _p(used_capacity), S, int(M), E, Cap, top_k, gd, _flags(gate_is_logits, True, False, scan_lookback),
-                              _p(gates_s), _p(indloc), _p(used_out), _p(elems), _p(ws.buf), ws.nbytes, _stream())
-    capi.check(st, "lancet_moe_route")
-    return gates_s, indloc, used_out, elems
+    return capi.host().moe_route(gate, gate2_noise, used_capacity, int(M), capacity_factor, None if capacity is None else int(capacity),
+                                 top_k, _flags(gate_is_logits, True, False, scan_lookback), workspace, out, None)
 
 
 def moe_scatter(data, indices_locations, used_in, used_out, n_experts, capacity, top_k=1, zero_tail=True,
@@ -259,38 +189,14 @@ def moe_scatter_tokens(data, indices_locations, used_in, used_out, token_first, 
     buffer and the rows go to their final places.  The calls of all token ranges together give the buffer of
     one moe_encode over the batch; one of them passes zero_tail=True, the others False.  used_in / used_out are
     what the routing call took and returned (used_in None = zeros)."""
-    lib = capi.load()
-    _dev(data, "data")
-    _need(data.dim() == 2, "Expected input data to be 2D.")
-    S_total = _check_indloc(indices_locations, top_k)
-    n, M = data.shape
-    _need(0 <= token_first and token_first + n <= S_total, "token range outside the routed batch")
-    if out is None:
-        out = torch.empty((n_experts, capacity, M), dtype=data.dtype, device=data.device)
-    st = lib.lancet_moe_scatter_tokens(_p(data), _p(indices_locations), _p(used_in), _p(used_out), S_total, int(token_first), n, M,
-                                       int(n_experts), int(capacity), top_k, _dtype_code(data),
-                                       _flags(False, zero_tail), _p(out), _stream())
-    capi.check(st, "lancet_moe_scatter_tokens")
-    return out
+    return capi.host().moe_scatter_tokens(data, indices_locations, used_in, used_out, int(token_first), int(n_experts), int(capacity),
+                                          top_k, _flags(False, zero_tail), out, None)
 
 
 def moe_decode_tokens(data, gate, indices_locations, token_first, n_tokens, top_k=1, out=None):
     """moe_decode of tokens [token_first, token_first + n_tokens) of a whole-batch routing: gate [k*S_total] and
     indices_locations [2, k*S_total] cover the batch, the result is [n_tokens, M]."""
-    lib = capi.load()
-    _dev(data, "data"), _dev(gate, "gate")
-    _need(data.dim() == 3, "Expected input data to be 3D.")
-    _need(gate.dim() == 1, "gate must be 1-D")
-    S_total = _check_indloc(indices_locations, top_k)
-    _need(gate.shape[0] == top_k * S_total, "gate and indices_locations disagree on the token count")
-    _need(0 <= token_first and 0 <= n_tokens and token_first + n_tokens <= S_total, "token range outside the routed batch")
-    E, Cap, M = data.shape
-    if out is None:
-        out = torch.empty((n_tokens, M), dtype=data.dtype, device=data.device)
-    st = lib.lancet_moe_decode_tokens(_p(data), _p(gate), _p(indices_locations), S_total, int(token_first),
-                                      int(n_tokens), M, E, Cap, top_k, _dtype_code(data), _gate_code(gate), _p(out), _stream())
-    capi.check(st, "lancet_moe_decode_tokens")
-    return out
+    return capi.host().moe_decode_tokens(data, gate, indices_locations, int(token_first), int(n_tokens), top_k, out, None)
 
 
 @functools.lru_cache(maxsize=256)
@@ -303,52 +209,13 @@ def moe_encode_batch_prioritized(data, gate, n_partitions=1, partition_id=0, cap
     """raf.op.moe_encode_batch_prioritized(data, gate, n_partitions=1, partition_id=0,
     capacity_factor=1.0): data/gate are the whole batch, the outputs cover partition
     partition_id (S = S0 / n_partitions tokens)."""
-    lib = capi.load()
-    dt = _check_encode_inputs(data, gate)
-    S0, M = data.shape
-    E = gate.shape[1]
-    _need(n_partitions > 0, "n_partitions should be greater than 0.")
-    _need(0 <= partition_id < n_partitions, "partition_id should be less than n_partitions.")
-    S = S0 // n_partitions
-    Cap = moe_capacity(S, E, capacity_factor)
-    dev = data.device
-    if out is None:
-        gates_s = torch.empty(S, dtype=gate.dtype, device=dev)
-        indloc = torch.empty((2, S), dtype=torch.int32, device=dev)
-        used_out = torch.empty(E, dtype=torch.int32, device=dev)
-        elems = torch.empty(E, dtype=torch.int64, device=dev)
-        disp = torch.empty((E, Cap, M), dtype=data.dtype, device=dev)
-    else:
-        gates_s, indloc, used_out, elems, disp = out
-    ws = _scan_workspace(moe_encode_bpr_workspace_bytes(S0, E, n_partitions), dev, workspace)
-    _need(gates_s.dtype == gate.dtype, "gates_s takes the gate's dtype")
-    st = lib.lancet_moe_encode_bpr(_p(data), _p(gate), S0, M, E, Cap, n_partitions, partition_id, dt, _gate_code(gate),
-                                   _flags(gate_is_logits, zero_tail, False, scan_lookback), _p(gates_s), _p(indloc),
-                                   _p(used_out), _p(elems), _p(disp), _p(ws.buf), ws.nbytes, _stream())
-    capi.check(st, "lancet_moe_encode_bpr")
-    return gates_s, indloc, used_out, elems.view(torch.uint64) if elems.dtype == torch.int64 else elems, disp
+    return capi.host().moe_encode_bpr(data, gate, n_partitions, partition_id, capacity_factor,
+                                      _flags(gate_is_logits, zero_tail, False, scan_lookback), workspace, out)
 
 
 def moe_decode(data, gate, indices_locations, top_k=1, out=None):
     """raf.op.moe_decode(data [E,C,M], gate [k*S], indices_locations [2, k*S]) -> [S, M]."""
-    lib = capi.load()
-    _dev(data, "data"), _dev(gate, "gate"), _dev(indices_locations, "indices_locations")
-    _need(data.dim() == 3, "Expected input data to be 3D.")
-    _need(gate.dim() == 1, "Expected input gate to be 1D.")
-    gd = _gate_code(gate)
-    _need(indices_locations.dtype == torch.int32 and indices_locations.dim() == 2 and
-          indices_locations.shape[0] == 2 and indices_locations.shape[1] == gate.shape[0],
-          "indices_locations must be int32 [2, k*S]")
-    dt = _dtype_code(data)
-    E, Cap, M = data.shape
-    _need(gate.shape[0] % top_k == 0, "gate length must be a multiple of top_k")
-    S = gate.shape[0] // top_k
-    if out is None:
-        out = torch.empty((S, M), dtype=data.dtype, device=data.device)
-    st = lib.lancet_moe_decode(_p(data), _p(gate), _p(indices_locations), S, M, E, Cap, top_k, dt, gd, _p(out),
-                               _stream())
-    capi.check(st, "lancet_moe_decode")
-    return out
+    return capi.host().moe_decode(data, gate, indices_locations, top_k, out)
 
 
 def _check_indloc(indices_locations, top_k):
@@ -361,31 +228,12 @@ def _check_indloc(indices_locations, top_k):
 
 def moe_encode_dx(dy, indices_locations, top_k=1, out=None):
     """raf.op.moe_encode_dx(dy [E,C,M], indices_locations [2, k*S]) -> [S, M]."""
-    lib = capi.load()
-    _dev(dy, "dy")
-    _need(dy.dim() == 3, "Input dy should be 3-D.")
-    S = _check_indloc(indices_locations, top_k)
-    E, Cap, M = dy.shape
-    if out is None:
-        out = torch.empty((S, M), dtype=dy.dtype, device=dy.device)
-    st = lib.lancet_moe_encode_dx(_p(dy), _p(indices_locations), S, M, E, Cap, top_k, _dtype_code(dy), _p(out), _stream())
-    capi.check(st, "lancet_moe_encode_dx")
-    return out
+    return capi.host().moe_encode_dx(dy, indices_locations, top_k, out)
 
 
 def moe_encode_dg(dy, indices_locations, n_experts, top_k=1, out=None):
     """raf.op.moe_encode_dg(dy [k*S], indices_locations, n_experts) -> [S, E] of dy's dtype."""
-    lib = capi.load()
-    _dev(dy, "dy")
-    _need(dy.dim() == 1, "Input dy should be 1-D.")
-    S = _check_indloc(indices_locations, top_k)
-    _need(dy.shape[0] == top_k * S, "dy and indices_locations disagree")
-    if out is None:
-        out = torch.empty((S, n_experts), dtype=dy.dtype, device=dy.device)
-    _need(out.dtype == dy.dtype, "the gate gradient takes dy's dtype")
-    st = lib.lancet_moe_encode_dg(_p(dy), _p(indices_locations), S, n_experts, top_k, _gate_code(dy, "dy"), _p(out), _stream())
-    capi.check(st, "lancet_moe_encode_dg")
-    return out
+    return capi.host().moe_encode_dg(dy, indices_locations, n_experts, top_k, out)
 
 
 def moe_encode_dgate(dy, gate, indices_locations, top_k=1, gate_is_logits=False, out=None):
@@ -393,80 +241,24 @@ def moe_encode_dgate(dy, gate, indices_locations, top_k=1, gate_is_logits=False,
     gates_s, gate [S, E] the op's gate input, the result [S, E] the gradient with respect to that input, through the
     top-2 normalisation (docker/resources/sharded_moe.py:304-312) and, with gate_is_logits, the fused softmax.  With
     top_k = 1 on probabilities it is moe_encode_dg (src/op/grad/moe.cc:30-58)."""
-    lib = capi.load()
-    _dev(dy, "dy"), _dev(gate, "gate")
-    _need(dy.dim() == 1 and gate.dim() == 2, "dy must be 1-D and gate 2-D")
-    S = _check_indloc(indices_locations, top_k)
-    _need(dy.shape[0] == top_k * S and gate.shape[0] == S, "dy, gate and indices_locations disagree")
-    _need(dy.dtype == gate.dtype, "dy takes the gate's dtype")
-    if out is None:
-        out = torch.empty_like(gate)
-    _need(out.dtype == gate.dtype and out.shape == gate.shape and out.is_contiguous(), "the gradient has the gate's shape and dtype")
-    st = lib.lancet_moe_encode_dgate(_p(dy), _p(gate), _p(indices_locations), S, gate.shape[1], top_k, _gate_code(gate),
-                                     capi.GATE_IS_LOGITS if gate_is_logits else 0, _p(out), _stream())
-    capi.check(st, "lancet_moe_encode_dgate")
-    return out
+    return capi.host().moe_encode_dgate(dy, gate, indices_locations, top_k, gate_is_logits, out)
 
 
 def moe_decode_dx(dy, gate, indices_locations, n_experts, capacity, top_k=1, workspace=None, out=None):
     """raf.op.moe_decode_dx(dy [S,M], gate [k*S], indices_locations, n_experts, capacity) -> [E, C, M]."""
-    lib = capi.load()
-    _dev(dy, "dy"), _dev(gate, "gate")
-    _need(dy.dim() == 2, "Input dy should be 2-D.")
-    _need(gate.dim() == 1, "gate must be 1-D")
-    S = _check_indloc(indices_locations, top_k)
-    _need(dy.shape[0] == S and gate.shape[0] == top_k * S, "dy, gate and indices_locations disagree")
-    M = dy.shape[1]
-    if out is None:
-        out = torch.empty((n_experts, capacity, M), dtype=dy.dtype, device=dy.device)
-    ws_bytes = int(lib.lancet_moe_decode_dx_workspace_bytes(n_experts, capacity))
-    ws = _workspace(ws_bytes, dy.device, workspace)
-    st = lib.lancet_moe_decode_dx(_p(dy), _p(gate), _p(indices_locations), S, M, n_experts, capacity, top_k,
-                                  _dtype_code(dy), _gate_code(gate), _p(out), _p(ws), ws.numel(), _stream())
-    capi.check(st, "lancet_moe_decode_dx")
-    return out
+    return capi.host().moe_decode_dx(dy, gate, indices_locations, n_experts, capacity, top_k, workspace, out)
 
 
 def moe_decode_dg(dy, data, indices_locations, top_k=1, gate_dtype=torch.float32, out=None):
     """raf.op.moe_decode_dg(dy [S,M], data [E,C,M], indices_locations) -> [k*S] of gate_dtype (the dtype of the
     gates_s the gradient belongs to; the reference gives it dy's dtype, src/op/declare/moe.cc:239)."""
-    lib = capi.load()
-    _dev(dy, "dy"), _dev(data, "data")
-    _need(dy.dim() == 2 and data.dim() == 3 and dy.dtype == data.dtype and dy.shape[1] == data.shape[2],
-          "dy must be [S,M] and data [E,C,M] of one dtype")
-    S = _check_indloc(indices_locations, top_k)
-    _need(dy.shape[0] == S, "dy and indices_locations disagree")
-    E, Cap, M = data.shape
-    if out is None:
-        out = torch.empty(top_k * S, dtype=gate_dtype, device=dy.device)
-    st = lib.lancet_moe_decode_dg(_p(dy), _p(data), _p(indices_locations), S, M, E, Cap, top_k, _dtype_code(dy),
-                                  _gate_code(out, "the gate gradient"), _p(out), _stream())
-    capi.check(st, "lancet_moe_decode_dg")
-    return out
+    return capi.host().moe_decode_dg(dy, data, indices_locations, top_k, gate_dtype, out)
 
 
 def moe_decode_grad(dy, data, gate, indices_locations, top_k=1, workspace=None, out=None):
     """Both gradients of moe_decode(data [E,C,M], gate [k*S], indices_locations) given dy [S,M], in one pass over the rows:
     what moe_decode_dx and moe_decode_dg return (MoeDecodeGrad, src/op/grad/moe.cc:60-90)."""
-    lib = capi.load()
-    _dev(dy, "dy"), _dev(data, "data"), _dev(gate, "gate")
-    _need(dy.dim() == 2 and data.dim() == 3 and dy.dtype == data.dtype and dy.shape[1] == data.shape[2],
-          "dy must be [S,M] and data [E,C,M] of one dtype")
-    S = _check_indloc(indices_locations, top_k)
-    _need(dy.shape[0] == S and gate.dim() == 1 and gate.shape[0] == top_k * S, "dy, gate and indices_locations disagree")
-    E, Cap, M = data.shape
-    if out is None:
-        d_data, d_gate = torch.empty_like(data), torch.empty_like(gate)
-    else:
-        d_data, d_gate = out
-        _dev(d_data, "the expert rows' gradient"), _dev(d_gate, "the gate gradient")
-        _need(d_data.shape == data.shape and d_data.dtype == data.dtype, "the expert rows' gradient has the rows' shape and dtype")
-        _need(d_gate.shape == gate.shape and d_gate.dtype == gate.dtype, "the gate gradient has the gate's shape and dtype")
-    ws = _workspace(int(lib.lancet_moe_decode_dx_workspace_bytes(E, Cap)), dy.device, workspace)
-    st = lib.lancet_moe_decode_grad(_p(dy), _p(data), _p(gate), _p(indices_locations), S, M, E, Cap, top_k, _dtype_code(dy),
-                                    _gate_code(gate), _p(d_data), _p(d_gate), _p(ws), ws.numel(), _stream())
-    capi.check(st, "lancet_moe_decode_grad")
-    return d_data, d_gate
+    return capi.host().moe_decode_grad(dy, data, gate, indices_locations, top_k, workspace, out)
 
 
 def moe_top2_normalize_gates(raw_gates, merged_indices_locations):
@@ -483,54 +275,12 @@ def moe_top2_normalize_gates(raw_gates, merged_indices_locations):
 
 def moe_merge_masks(indices_locations, n_experts, workspace=None, out=None):
     """raf.op.moe_merge_masks(indices_locations: tuple of [2,S], n_experts) -> [2, P*S]."""
-    lib = capi.load()
-    P = len(indices_locations)
-    _need(P >= 1, "need at least one partition")
-    for il in indices_locations:
-        _dev(il, "indices_locations")
-        _need(il.dim() == 2 and il.shape == indices_locations[0].shape and il.dtype == torch.int32,
-              "Expected input indices_locations to be 2D int32 of equal shape.")
-    S = indices_locations[0].shape[1]
-    dev = indices_locations[0].device
-    if out is None:
-        out = torch.empty((2, P * S), dtype=torch.int32, device=dev)
-    ws_bytes = int(lib.lancet_moe_merge_masks_workspace_bytes(P, n_experts))
-    ws = _workspace(ws_bytes, dev, workspace)
-    ptrs = capi.ptr_array([il.data_ptr() for il in indices_locations])
-    st = lib.lancet_moe_merge_masks(ptrs, P, S, n_experts, _p(out), _p(ws), ws.numel(), _stream())
-    capi.check(st, "lancet_moe_merge_masks")
-    return out
+    return capi.host().moe_merge_masks(indices_locations, n_experts, workspace, out)
 
 
 def moe_redispatch(data, indices_locations, workspace=None, out=None):
     """raf.op.moe_redispatch(data: tuple of [E,C,M], indices_locations: tuple of [2,S]) -> [E,C,M]."""
-    lib = capi.load()
-    P = len(indices_locations)
-    _need(P >= 1 and len(data) == P, "data and indices_locations must have one entry per partition")
-    for d in data:
-        _dev(d, "data")
-        _need(d.dim() in (3, 4) and d.shape == data[0].shape and d.dtype == data[0].dtype,
-              "Expected input data to be 3 or 4D of equal shape.")
-    for il in indices_locations:
-        _dev(il, "indices_locations")
-        _need(il.dim() == 2 and il.dtype == torch.int32, "Expected input indices_locations to be 2D.")
-    shape = tuple(data[0].shape)
-    if len(shape) == 4:   # [G, LE, C, M]
-        E, Cap, M = shape[0] * shape[1], shape[2], shape[3]
-    else:
-        E, Cap, M = shape
-    S = indices_locations[0].shape[1]
-    dt = _dtype_code(data[0])
-    dev = data[0].device
-    if out is None:
-        out = torch.empty(shape, dtype=data[0].dtype, device=dev)
-    ws_bytes = int(lib.lancet_moe_redispatch_workspace_bytes(P, E))
-    ws = _workspace(ws_bytes, dev, workspace)
-    dptrs = capi.ptr_array([d.data_ptr() for d in data])
-    iptrs = capi.ptr_array([il.data_ptr() for il in indices_locations])
-    st = lib.lancet_moe_redispatch(dptrs, iptrs, P, S, M, Cap, E, dt, _p(out), _p(ws), ws.numel(), _stream())
-    capi.check(st, "lancet_moe_redispatch")
-    return out
+    return capi.host().moe_redispatch(data, indices_locations, workspace, out)
 
 
 def moe_redispatch_expert_input(data, recv_cnts, local_expert_id, n_local_experts, recv_cnts_scale=1, out=None):
@@ -611,49 +361,21 @@ def memcpy_sparse_ranges_to_cont_3d(src, dst, nelements_per_dim, starts_per_dim,
                                     axis=0):
     """memcpy_sparse_to_cont_3d on row ranges: block b contributes its elements [start_b, start_b + n_b) (both
     arrays indexed b*stride + offset).  Packs what one token partition owns inside a shared buffer."""
-    lib = capi.load()
-    (d0, d1, d2), n_dst, n_cnt = _sparse_copy_args(src, dst, nelements_per_dim, nelements_stride, nelements_offset, axis)
-    _dev(starts_per_dim, "starts_per_dim")
-    _need(starts_per_dim.dtype == nelements_per_dim.dtype and starts_per_dim.numel() == n_cnt and
-          starts_per_dim.is_contiguous(), "starts_per_dim must match nelements_per_dim")
-    st = lib.lancet_memcpy_sparse_ranges_to_cont_3d(_p(src), _p(dst), _p(nelements_per_dim), _p(starts_per_dim), n_cnt,
-                                                    int(nelements_stride), int(nelements_offset), int(axis), d0, d1, d2,
-                                                    n_dst, _dtype_code(src), _stream())
-    capi.check(st, "lancet_memcpy_sparse_ranges_to_cont_3d")
-    return dst
+    return capi.host().memcpy_sparse_ranges_to_cont_3d(src, dst, nelements_per_dim, starts_per_dim, int(nelements_stride),
+                                                       int(nelements_offset), int(axis), None)
 
 
 def memcpy_cont_to_sparse_ranges_3d(src, dst, nelements_per_dim, starts_per_dim, nelements_stride=1, nelements_offset=0,
                                     axis=0):
     """The inverse of memcpy_sparse_ranges_to_cont_3d: only the ranges are written."""
-    lib = capi.load()
-    (d0, d1, d2), n_src, n_cnt = _sparse_copy_args(dst, src, nelements_per_dim, nelements_stride, nelements_offset, axis)
-    _dev(starts_per_dim, "starts_per_dim")
-    _need(starts_per_dim.dtype == nelements_per_dim.dtype and starts_per_dim.numel() == n_cnt and
-          starts_per_dim.is_contiguous(), "starts_per_dim must match nelements_per_dim")
-    st = lib.lancet_memcpy_cont_to_sparse_ranges_3d(_p(src), _p(dst), _p(nelements_per_dim), _p(starts_per_dim), n_cnt,
-                                                    int(nelements_stride), int(nelements_offset), int(axis), d0, d1, d2,
-                                                    n_src, _dtype_code(dst), _stream())
-    capi.check(st, "lancet_memcpy_cont_to_sparse_ranges_3d")
-    return dst
+    return capi.host().memcpy_cont_to_sparse_ranges_3d(src, dst, nelements_per_dim, starts_per_dim, int(nelements_stride),
+                                                       int(nelements_offset), int(axis), None)
 
 
 def moe_partition_ranges(indices_locations, n_partitions, n_experts, M, top_k=1, workspace=None, out=None):
     """Row ranges of n_partitions equal token partitions inside a whole-batch routing: returns (starts, counts), each
     int64 [top_k * n_partitions, E] in elements (rows x M), rows ordered slot-major then partition."""
-    lib = capi.load()
-    S_total = _check_indloc(indices_locations, top_k)
-    _need(n_partitions >= 1 and S_total % n_partitions == 0, "the token count must divide into n_partitions")
-    Q = top_k * int(n_partitions)
-    dev = indices_locations.device
-    if out is None:
-        out = (torch.empty((Q, n_experts), dtype=torch.int64, device=dev), torch.empty((Q, n_experts), dtype=torch.int64, device=dev))
-    starts, counts = out
-    ws = _workspace(lib.lancet_moe_partition_ranges_workspace_bytes(top_k, int(n_partitions), int(n_experts)), dev, workspace)
-    st = lib.lancet_moe_partition_ranges(_p(indices_locations), S_total, top_k, int(n_partitions), int(n_experts), int(M),
-                                         _p(starts), _p(counts), _p(ws), ws.numel(), _stream())
-    capi.check(st, "lancet_moe_partition_ranges")
-    return starts, counts
+    return capi.host().moe_partition_ranges(indices_locations, int(n_partitions), int(n_experts), int(M), top_k, workspace, out, None)
 
 
 # ------------------------------------------------------------------------------------ LANS
@@ -664,9 +386,10 @@ class LansPlan:
     def __init__(self, numels, schedule=None):
         lib = capi.load()
         self.numels = [int(n) for n in numels]
-        arr = (C.c_int64 * len(self.numels))(*self.numels)
+        self._numels = (C.c_int64 * len(self.numels))(*self.numels)
+        self._sizes = C.addressof(self._numels)   # what a step checks its tensors against
         handle = C.c_void_p()
-        capi.check(lib.lancet_lans_plan_create(arr, len(self.numels), C.byref(handle)), "lancet_lans_plan_create")
+        capi.check(lib.lancet_lans_plan_create(self._numels, len(self.numels), C.byref(handle)), "lancet_lans_plan_create")
         self._h = handle
         self._lib = lib
         if schedule is not None:
@@ -727,32 +450,8 @@ class LansPlan:
         the same pass as p.  grad_norms: optional float32 GPU tensor [T] of ||g_i|| in list order (skips the
         step's own pass over g).  Raises LancetError(ERR_STALLED) when an earlier step of the resident
         schedule gave up a wait, until error() has been read."""
-        T = len(self.numels)
-        if grad_norms is not None:
-            _need(grad_norms.is_cuda and grad_norms.dtype == torch.float32 and grad_norms.numel() == T and
-                  grad_norms.is_contiguous(), "grad_norms must be a contiguous float32 GPU tensor of T values")
-        _need(len(g) == len(p) == len(m) == len(v) == T, "tensor lists must have one entry per planned tensor")
-        _need(p_lowp is None or len(p_lowp) == T, "p_lowp must have one entry per planned tensor")
-        g_dtype = g[0].dtype if T else torch.float32
-        _need(g_dtype in _DTYPES, "gradients must be float32, bfloat16 or float16")
-        lowp_dtype = p_lowp[0].dtype if p_lowp else torch.bfloat16
-        _need(lowp_dtype in (torch.bfloat16, torch.float16), "p_lowp must be bfloat16 or float16")
-        for lst, dt in ((g, g_dtype), (p, torch.float32), (m, torch.float32), (v, torch.float32)) + (((p_lowp, lowp_dtype),) if p_lowp else ()):
-            for t, n in zip(lst, self.numels):
-                _need(t.is_cuda and t.is_contiguous() and t.dtype == dt and t.numel() == n,
-                      "LANS tensors must be contiguous GPU tensors of the planned sizes: p, m, v float32, every gradient of "
-                      "one type, every 16-bit parameter copy of one type")
-        arrs = [capi.ptr_array([t.data_ptr() for t in lst]) for lst in (g, p, m, v)]
-        if g_dtype == torch.float32 and not p_lowp:
-            st = self._lib.lancet_lans_step(self._h, arrs[0], arrs[1], arrs[2], arrs[3], int(step),
-                                            _p(step_dev), C.byref(hyper), _p(grad_norms), _stream())
-            capi.check(st, "lancet_lans_step")
-            return
-        low = capi.ptr_array([t.data_ptr() for t in p_lowp]) if p_lowp else None
-        st = self._lib.lancet_lans_step_mixed(self._h, arrs[0], _DTYPES[g_dtype], arrs[1], arrs[2], arrs[3], low,
-                                              _DTYPES[lowp_dtype], int(step), _p(step_dev), C.byref(hyper), _p(grad_norms),
-                                              _stream())
-        capi.check(st, "lancet_lans_step_mixed")
+        capi.host().lans_step(self._h.value, self._sizes, len(self.numels), g, p, m, v, p_lowp, int(step), step_dev,
+                              C.addressof(hyper), grad_norms)
 
     def norms(self):
         """[4, T] float32: (||g||, ||p||, ||u_m||, ||u_g||) of the last step."""
@@ -778,7 +477,7 @@ def lans(tensor_list, step, learning_rate, beta1, beta2, eps, bias_correction, w
     _need(n % 4 == 0 and n > 0, "tensor_list must hold 4 lists of equal length")
     T = n // 4
     g, p, m, v = (list(tensor_list[i * T:(i + 1) * T]) for i in range(4))
-    key = (tuple(t.numel() for t in g), g[0].device.index)
+    key = capi.host().lans_key(g)
     plan = _PLANS.get(key)
     if plan is None:
         plan = _PLANS[key] = LansPlan(key[0])

@@ -21,7 +21,7 @@ launches kernels and records events, so it can be called in a loop.
 """
 import torch
 
-from . import ops
+from . import capi, ops
 
 
 class PartitionedMoeLayer:
@@ -168,11 +168,13 @@ class RoutedOnceMoeLayer:
         self.ranges = (torch.empty((K * P, E), dtype=torch.int64, device=dev),
                        torch.empty((K * P, E), dtype=torch.int64, device=dev))
         self.ranges_ws = torch.empty(max(4, K * P * E * 4), dtype=torch.uint8, device=dev)
+        self.range_rows = tuple(list(t) for t in self.ranges)   # one array per slot and partition
         self.send = torch.empty((E, self.C, M), dtype=dtype, device=dev)
         self.recv = torch.empty((E, self.C, M), dtype=dtype, device=dev)
         # packed streams: one per partition and slot (a partition sends at most Sp rows per slot)
         self.wire = [[torch.empty(Sp * M, dtype=dtype, device=dev) for _ in range(K)] for _ in range(P)]
         self.out = torch.empty((S, M), dtype=dtype, device=dev)
+        self.device = self.out.device
         self.no_rows = torch.empty((0, M), dtype=dtype, device=dev)
         self.routing, self.compute, self.exchange = streams or tuple(torch.cuda.Stream(device=dev) for _ in range(3))
         self.routed = torch.cuda.Event()
@@ -187,36 +189,37 @@ class RoutedOnceMoeLayer:
         for s in (self.routing, self.compute, self.exchange):
             s.wait_event(start)
         g, il, used, _ = self.whole
-        starts, counts = self.ranges
-        with torch.cuda.stream(self.routing):
-            ops.moe_route(gate, None, self.M, self.cf, top_k=K, gate_is_logits=self.gate_is_logits,
-                          workspace=self.whole_ws, out=self.whole)
-            ops.moe_partition_ranges(il, P, E, self.M, top_k=K, workspace=self.ranges_ws, out=self.ranges)
-            # rows of the receive buffer no partition owns: cleared once (a scatter of no tokens is only the tail fill)
-            ops.moe_scatter_tokens(self.no_rows, il, None, used, 0, E, C, top_k=K, zero_tail=True, out=self.recv)
-            self.routed.record(self.routing)
-        self.compute.wait_event(self.routed)
-        self.exchange.wait_event(self.routed)
+        starts, counts = self.range_rows
+        # every buffer is the layer's own, so nothing is allocated and the calls name their stream: entering a stream's
+        # context costs the host as much as a launch, and a pass has 3 + P * (2 + 2 K) of those
+        host, tail = capi.host(), ops._flags(False, True)
+        body = ops._flags(False, False)
+        routing, compute, exchange = (s.cuda_stream for s in (self.routing, self.compute, self.exchange))
 
         def decode(i):
-            ops.moe_decode_tokens(self.recv, g, il, i * Sp, Sp, top_k=K, out=self.out[i * Sp:(i + 1) * Sp])
+            host.moe_decode_tokens(self.recv, g, il, i * Sp, Sp, K, self.out[i * Sp:(i + 1) * Sp], compute)
 
-        for i in range(P):
-            with torch.cuda.stream(self.compute):
-                ops.moe_scatter_tokens(data[i * Sp:(i + 1) * Sp], il, None, used, i * Sp, E, C, top_k=K, zero_tail=False,
-                                       out=self.send)
+        with torch.cuda.device(self.device):
+            host.moe_route(gate, None, None, self.M, self.cf, None, K, ops._flags(self.gate_is_logits, True), self.whole_ws, self.whole,
+                           routing)
+            host.moe_partition_ranges(il, P, E, self.M, K, self.ranges_ws, self.ranges, routing)
+            # rows of the receive buffer no partition owns: cleared once (a scatter of no tokens is only the tail fill)
+            host.moe_scatter_tokens(self.no_rows, il, None, used, 0, E, C, K, tail, self.recv, routing)
+            self.routed.record(self.routing)
+            self.compute.wait_event(self.routed)
+            self.exchange.wait_event(self.routed)
+            for i in range(P):
+                host.moe_scatter_tokens(data[i * Sp:(i + 1) * Sp], il, None, used, i * Sp, E, C, K, body, self.send, compute)
                 self.scattered[i].record(self.compute)
                 if i > 0:
                     self.compute.wait_event(self.received[i - 1])
                     decode(i - 1)
-            with torch.cuda.stream(self.exchange):
                 self.exchange.wait_event(self.scattered[i])
                 for j in range(K):
                     q = j * P + i
-                    ops.memcpy_sparse_ranges_to_cont_3d(self.send, self.wire[i][j], counts[q], starts[q], axis=0)
-                    ops.memcpy_cont_to_sparse_ranges_3d(self.wire[i][j], self.recv, counts[q], starts[q], axis=0)
+                    host.memcpy_sparse_ranges_to_cont_3d(self.send, self.wire[i][j], counts[q], starts[q], 1, 0, 0, exchange)
+                    host.memcpy_cont_to_sparse_ranges_3d(self.wire[i][j], self.recv, counts[q], starts[q], 1, 0, 0, exchange)
                 self.received[i].record(self.exchange)
-        with torch.cuda.stream(self.compute):
             self.compute.wait_event(self.received[P - 1])
             decode(P - 1)
             done = torch.cuda.Event()
