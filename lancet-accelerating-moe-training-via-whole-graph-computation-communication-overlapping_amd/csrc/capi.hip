@@ -251,10 +251,10 @@ extern "C" size_t lancet_moe_encode_workspace_bytes(int64_t S, int64_t E, int to
   return scan_workspace_bytes(S, E, top_k);
 }
 
-extern "C" int lancet_moe_route(const void* gate, const void* gate2_noise, const int32_t* used_in, int64_t S,
-                                int64_t M, int64_t E, int64_t C, int top_k, int gate_dtype, unsigned flags, void* gates_s,
-                                int32_t* indices_locations, int32_t* used_out, uint64_t* elements_per_expert,
-                                void* workspace, size_t workspace_bytes, lancet_stream_t stream) {
+namespace {
+int check_route(const void* gate, const void* gate2_noise, const int32_t* used_in, int64_t S, int64_t M, int64_t E, int64_t C, int top_k,
+                int gate_dtype, const void* gates_s, const int32_t* indices_locations, const int32_t* used_out,
+                const uint64_t* elements_per_expert, const void* workspace, size_t workspace_bytes) {
   if (((!gate || !gates_s || !indices_locations) && S > 0) || !used_out || !elements_per_expert)
     return LANCET_ERR_NULL;
   const int gb = elem_bytes(gate_dtype);
@@ -267,6 +267,17 @@ extern "C" int lancet_moe_route(const void* gate, const void* gate2_noise, const
   if (misaligned(gate, gb) || misaligned(gate2_noise, gb) || misaligned(gates_s, gb) || misaligned(indices_locations, 4) || misaligned(used_in, 4) ||
       misaligned(used_out, 4) || misaligned(elements_per_expert, 8) || misaligned(workspace, 8))
     return LANCET_ERR_ALIGN;
+  return LANCET_OK;
+}
+}  // namespace
+
+extern "C" int lancet_moe_route(const void* gate, const void* gate2_noise, const int32_t* used_in, int64_t S,
+                                int64_t M, int64_t E, int64_t C, int top_k, int gate_dtype, unsigned flags, void* gates_s,
+                                int32_t* indices_locations, int32_t* used_out, uint64_t* elements_per_expert,
+                                void* workspace, size_t workspace_bytes, lancet_stream_t stream) {
+  if (int r = check_route(gate, gate2_noise, used_in, S, M, E, C, top_k, gate_dtype, gates_s, indices_locations, used_out, elements_per_expert,
+                          workspace, workspace_bytes))
+    return r;
   const int s = static_cast<int>(S);
   return rc(run_route_scan(gate, gate2_noise, nullptr, used_in, s, static_cast<int>(E), static_cast<int>(C),
                            static_cast<int>(M), top_k, (flags & LANCET_GATE_IS_LOGITS) != 0, gate_dtype, gates_s,
@@ -307,6 +318,16 @@ extern "C" int lancet_moe_encode(const void* data, const void* gate, const void*
   const int eb = elem_bytes(dtype);
   if (!eb) return LANCET_ERR_DTYPE;
   if (misaligned(data, eb) || misaligned(dispatched, eb)) return LANCET_ERR_ALIGN;
+  if (int r = check_route(gate, gate2_noise, used_in, S, M, E, C, top_k, gate_dtype, gates_s, indices_locations, used_out, elements_per_expert,
+                          workspace, workspace_bytes))
+    return r;
+  const size_t row_bytes = static_cast<size_t>(M) * eb;
+  if (encode_is_short(used_in, used_out, S, E, top_k, row_bytes, (flags & LANCET_SCAN_LOOKBACK) != 0)) {
+    return rc(run_encode_short(data, gate, gate2_noise, used_in, static_cast<int>(S), static_cast<int>(E), static_cast<int>(C), static_cast<int>(M),
+                               top_k, (flags & LANCET_GATE_IS_LOGITS) != 0, eb, gate_dtype, !(flags & LANCET_NO_TAIL_ZERO),
+                               (flags & LANCET_ROWS_AT_USED) != 0, gates_s, indices_locations,
+                               indices_locations + static_cast<size_t>(top_k) * S, used_out, elements_per_expert, dispatched, workspace, S_(stream)));
+  }
   if (int r = lancet_moe_route(gate, gate2_noise, used_in, S, M, E, C, top_k, gate_dtype, flags, gates_s, indices_locations, used_out,
                                elements_per_expert, workspace, workspace_bytes, stream))
     return r;

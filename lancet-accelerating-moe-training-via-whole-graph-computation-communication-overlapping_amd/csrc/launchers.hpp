@@ -31,6 +31,13 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
                           int E, int C, int M, int K, bool is_logits, int gate_dtype, void* gates_s,
                           int32_t* idx_out, int32_t* loc_out, int32_t* used_out,
                           uint64_t* elems_out, void* ws, hipStream_t st, bool force_lookback = false);
+// The whole of an encode (routing and row movement) in one or two launches, where encode_is_short says so; the arguments are
+// those of run_route_scan and run_scatter_rows.  needs_setup: the workspace has to be set up (as the look-back form wants it).
+bool encode_is_short(const int32_t* used_in, const int32_t* used_out, int64_t S, int64_t E, int K, size_t row_bytes, bool force_lookback);
+hipError_t run_encode_short(const void* data, const void* gate, const void* noise, const int32_t* used_in, int S, int E, int C, int M,
+                            int K, bool is_logits, int elem_bytes, int gate_dtype, bool tail, bool rows_at_used, void* gates_s,
+                            int32_t* idx_out, int32_t* loc_out, int32_t* used_out, uint64_t* elems_out, void* out, void* ws,
+                            hipStream_t st);
 // between count and place on long batches: sums of the table's rows in segments of R tiles (scan.hpp)
 hipError_t run_scan_segsum(void* ws, int ntiles, int NC, int R, hipStream_t st);
 hipError_t run_bpr_route(const void* gate, int S0, int E, int C, int M, int n_partitions,

@@ -1,28 +1,10 @@
 // Routing kernels: gate softmax + top-1/top-2 selection (select.hpp) fused with the capacity-bounded
 // position scan (scan.hpp) in its three forms, and the top-2 finalisation.
 #include "launchers.hpp"
-#include "select.hpp"
+#include "route.hpp"
 #include <algorithm>
 
 namespace lancet {
-
-struct RouteArgs {
-  const void* gate;       // [S,E] of gate_dtype (NULL when idx_in is given)
-  const void* noise;      // [S,E] of gate_dtype or NULL: added for the second choice (K = 2)
-  const int32_t* idx_in;  // launcher-level entry: expert per token already chosen (may alias idx_out)
-  const int32_t* used_in; // [E] or NULL (= zeros)
-  void* gates_s;          // [K*S] of gate_dtype (NULL when idx_in is given)
-  int32_t* idx_out;       // [K*S]
-  int32_t* loc_out;       // [K*S]
-  int32_t* used_out;      // [E]
-  uint64_t* elems_out;    // [E]
-  ScanWs ws;
-  int S, E, C, M;
-  int ntiles;
-  int is_logits;
-  int gate_dtype;         // LANCET_F32 / _BF16 / _F16: storage type of gate, noise and gates_s
-  int seg_rows;           // place kernel: tiles per segment of the segment sums, 0 = there are none
-};
 
 // K = 1: everything is final when the tile knows its prefix.
 // K = 2: ranks of both slots are produced in one pass (2E counters); slot-2 locations need the
@@ -208,13 +190,12 @@ __global__ __launch_bounds__(kTile) void route_place_kernel(RouteArgs a) {
       const int r2 = (in2 ? static_cast<int>(s_before[a.E + e2]) : 0) + a.loc_out[a.S + s];
       const int u1 = (a.used_in && in1) ? a.used_in[e1] : 0;
       const int u2 = (a.used_in && in2) ? a.used_in[e2] : 0;
-      const bool keep1 = in1 && r1 < a.C - u1;
-      const int64_t after1 = min(static_cast<int64_t>(u2) + (in2 ? s_total[e2] : 0u), static_cast<int64_t>(a.C));
-      const bool keep2 = in2 && r2 < a.C - after1;
-      a.idx_out[s] = keep1 ? e1 : -1;
-      a.loc_out[s] = keep1 ? r1 : -1;
-      a.idx_out[a.S + s] = keep2 ? e2 : -1;
-      a.loc_out[a.S + s] = keep2 ? r2 + static_cast<int>(after1 - u2) : -1;
+      const Top2Place t = place_top2(e1, r1, e2, r2, u1, u2, in2 ? s_total[e2] : 0u, a.E, a.C);
+      const bool keep1 = t.e1 >= 0, keep2 = t.e2 >= 0;
+      a.idx_out[s] = t.e1;
+      a.loc_out[s] = t.l1;
+      a.idx_out[a.S + s] = t.e2;
+      a.loc_out[a.S + s] = t.l2;
       // the raw values as the first kernel stored them (rounded to the gate type), normalised in fp32, rounded once
       const float g1 = keep1 ? ld_gate(a.gates_s, s, a.gate_dtype) : 0.f;
       const float g2 = keep2 ? ld_gate(a.gates_s, static_cast<size_t>(a.S) + s, a.gate_dtype) : 0.f;
@@ -267,14 +248,12 @@ __global__ __launch_bounds__(kTile) void finalize_top2_kernel(RouteArgs a) {
       const bool in1 = e1 >= 0 && e1 < a.E, in2 = e2 >= 0 && e2 < a.E;  // always, unless the scan left marks behind
       const int u1 = (a.used_in && in1) ? a.used_in[e1] : 0;
       const int u2 = (a.used_in && in2) ? a.used_in[e2] : 0;
-      const bool keep1 = in1 && r1 < a.C - u1;
-      const int64_t after1 = min(static_cast<int64_t>(u2) + (in2 ? static_cast<uint32_t>(ld_desc(tot + e2)) & kDescCountMask : 0u),
-                                 static_cast<int64_t>(a.C));
-      const bool keep2 = in2 && r2 < a.C - after1;
-      a.idx_out[s] = keep1 ? e1 : -1;
-      a.loc_out[s] = keep1 ? r1 : -1;
-      a.idx_out[a.S + s] = keep2 ? e2 : -1;
-      a.loc_out[a.S + s] = keep2 ? r2 + static_cast<int>(after1 - u2) : -1;
+      const Top2Place t = place_top2(e1, r1, e2, r2, u1, u2, in2 ? static_cast<uint32_t>(ld_desc(tot + e2)) & kDescCountMask : 0u, a.E, a.C);
+      const bool keep1 = t.e1 >= 0, keep2 = t.e2 >= 0;
+      a.idx_out[s] = t.e1;
+      a.loc_out[s] = t.l1;
+      a.idx_out[a.S + s] = t.e2;
+      a.loc_out[a.S + s] = t.l2;
       // the raw values as the scan stored them (rounded to the gate type), normalised in fp32, rounded once
       const float g1 = keep1 ? ld_gate(a.gates_s, s, a.gate_dtype) : 0.f;
       const float g2 = keep2 ? ld_gate(a.gates_s, static_cast<size_t>(a.S) + s, a.gate_dtype) : 0.f;
@@ -403,6 +382,17 @@ hipError_t run_gate_topk(const void* gate, const void* noise, int S, int E, int 
   return hipGetLastError();
 }
 
+hipError_t run_route_count(const RouteArgs& a, int K, hipStream_t st) {
+  const SelectLaunch sel = a.idx_in ? SelectLaunch{false, 0} : select_launch(a.gate_dtype, a.gate, a.noise, a.S, a.E, a.is_logits);
+  const size_t lds = std::max(scan_lds_bytes(K * a.E), sel.lds);
+  if (K == 1) {
+    LANCET_SELECT_SWITCH(a.gate_dtype, sel.held, (route_count_kernel<1, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
+  } else {
+    LANCET_SELECT_SWITCH(a.gate_dtype, sel.held, (route_count_kernel<2, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
+  }
+  return hipGetLastError();
+}
+
 hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* idx_in, const int32_t* used_in, int S,
                           int E, int C, int M, int K, bool is_logits, int gate_dtype, void* gates_s,
                           int32_t* idx_out, int32_t* loc_out, int32_t* used_out,
@@ -427,19 +417,14 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
   a.ws = scan_ws_view(ws);
   a.seg_rows = 0;
   hipError_t err = hipSuccess;
+  const ScanForm form = scan_form(a.ntiles, static_cast<int64_t>(K) * E, K, force_lookback);
   const SelectLaunch sel = idx_in ? SelectLaunch{false, 0} : select_launch(gate_dtype, gate, a.noise, S, E, is_logits);
   const size_t lds = std::max(scan_lds_bytes(K * E), sel.lds);
-  const ScanForm form = scan_form(a.ntiles, static_cast<int64_t>(K) * E, K, force_lookback);
   if (form != kScanLookback) {
     // two or three kernels that wait for nothing instead of a look-back between tiles that all run at once
     const int NC = K * E;
     const size_t lds2 = 2 * static_cast<size_t>(NC) * sizeof(uint32_t);
-    if (K == 1) {
-      LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_count_kernel<1, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
-    } else {
-      LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_count_kernel<2, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
-    }
-    err = hipGetLastError();
+    err = run_route_count(a, K, st);
     if (err != hipSuccess) return err;
     if (form == kScanCountSegPlace) {
       a.seg_rows = seg_rows(a.ntiles);

@@ -1,0 +1,88 @@
+"""moe_encode of few tokens (routing and row movement in one kernel up to 256 tokens, in two up to 8192) against the separate
+kernels, which scan_lookback=True asks for, bit for bit, and against the oracle, at the edges of its tiles, workgroups and rules."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as mo
+from tests.gpu_util import TORCH_DT, dev, make_inputs, rows_as_oracle, rows_to_torch, to_np
+
+pytestmark = pytest.mark.gpu
+
+# (S, M, E): one token, ends of a wave and of a tile, one token more; rows of less than a granule, of one and a bit, of whole
+# granules, of more than two per lane; as many tiles as there may be; the most experts a tile of tokens may have
+SHAPES = [(1, 8, 2), (63, 3, 5), (64, 1024, 8), (255, 1003, 60), (256, 4200, 128), (32, 64, 512), (256, 8, 129), (257, 5, 3), (300, 4096, 7),
+          (513, 24, 64), (6000, 77, 33), (8192, 512, 8), (8192, 16, 64), (8000, 2, 128)]
+
+
+@pytest.mark.parametrize("S,M,E", SHAPES)
+@pytest.mark.parametrize("k", [1, 2])
+def test_short_encodes_are_what_the_separate_kernels_give(pkg, S, M, E, k):
+    ops = pkg.ops
+    for i, dt in enumerate(("f32", "bf16", "f16")):
+        data, logits = make_inputs(S + M + k + i, S, M, E, zipf_bias=True, ties=i == 1)
+        rows, logits_in = rows_as_oracle(data, dt), logits.astype(np.float32)
+        d_data = rows_to_torch(data, dt)
+        used0 = (np.arange(E) % 3).astype(np.int32)
+        noise = torch.randn(S, E, device="cuda").to(TORCH_DT[dt]) if k == 2 and i == 0 else None
+        for used, logit, tail, at_used, gdt in ((None, True, True, False, "f32"), (used0, False, True, False, dt), (used0, True, True, True, "f32"),
+                                                (used0, True, False, False, "f32"), (None, True, False, False, dt)):
+            gate = (dev(logits_in) if logit else torch.softmax(dev(logits_in), 1)).to(TORCH_DT[gdt])
+            n = noise.to(gate.dtype) if noise is not None else None
+            args = dict(capacity_factor=0.75, top_k=k, gate_is_logits=logit, zero_tail=tail, gate2_noise=n, rows_at_used=at_used)
+            d_used = None if used is None else dev(used)
+            first = ops.moe_encode(d_data, gate, d_used, **args)
+            outs = [[torch.full_like(t, 7) if t.dtype != torch.uint64 else torch.full((E,), 7, dtype=torch.int64, device="cuda") for t in first]
+                    for _ in range(2)]
+            got = ops.moe_encode(d_data, gate, d_used, out=outs[0], **args)
+            want = ops.moe_encode(d_data, gate, d_used, out=outs[1], scan_lookback=True, **args)
+            for a, b in zip(got, want):
+                assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (dt, used is not None, logit, tail, at_used, gdt)
+        if k == 1:
+            ref = mo.moe_encode(rows, logits_in, used0, 0.75, gate_is_logits=True, fast_scatter=True)
+        else:
+            ref = mo.moe_encode_top2(rows, logits_in, used0, 0.75, gate_is_logits=True, fast_scatter=True)
+        got = ops.moe_encode(d_data, dev(logits_in), dev(used0), 0.75, top_k=k, gate_is_logits=True)
+        for j in (1, 2, 3, 4):
+            np.testing.assert_array_equal(to_np(got[j]), ref[j])
+        np.testing.assert_allclose(to_np(got[0]), ref[0], rtol=1e-5)
+
+
+def test_used_capacity_updated_in_place(pkg):
+    """used_capacity as input and output of one call (rows that feed moe_redispatch): the separate kernels take it, as before."""
+    ops = pkg.ops
+    S, M, E = 200, 32, 6
+    data, logits = make_inputs(9, S, M, E)
+    used = dev(np.full(E, 2, np.int32))
+    want = ops.moe_encode(dev(data), dev(logits), used.clone(), 1.0, gate_is_logits=True, zero_tail=False)
+    outs = [torch.zeros_like(want[0]), torch.zeros_like(want[1]), used, torch.zeros(E, dtype=torch.int64, device="cuda"), torch.zeros_like(want[4])]
+    got = ops.moe_encode(dev(data), dev(logits), used, 1.0, gate_is_logits=True, zero_tail=False, out=outs)
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("S", [100, 3000])
+def test_short_top1_on_memory_that_was_never_set_up(pkg, S):
+    """As the look-back form does: every output marked, the buffer cleared, the error word set; whole again after the set-up."""
+    lib, capi, ops = pkg.capi.load(), pkg.capi, pkg.ops
+    M, E = 8, 8
+    data, logits = make_inputs(3, S, M, E)
+    d_data, d_gate = dev(data), dev(logits)
+    Cap, nws = ops.moe_capacity(S, E, 1.0), int(lib.lancet_moe_encode_workspace_bytes(S, E, 1))
+    ws = torch.full((nws,), 0xff, dtype=torch.uint8, device="cuda")
+    outs = (torch.ones(S, device="cuda"), torch.zeros((2, S), dtype=torch.int32, device="cuda"), torch.zeros(E, dtype=torch.int32, device="cuda"),
+            torch.ones(E, dtype=torch.int64, device="cuda"), torch.ones((E, Cap, M), device="cuda"))
+    p = lambda t: t.data_ptr()
+    call = lambda: lib.lancet_moe_encode(p(d_data), p(d_gate), None, None, S, M, E, Cap, 1, capi.F32, capi.F32, capi.GATE_IS_LOGITS,
+                                         *[p(t) for t in outs], p(ws), nws, None)
+    assert call() == 0
+    torch.cuda.synchronize()
+    err = C.c_int(0)
+    assert (to_np(outs[1]) == -1).all() and (to_np(outs[2]) == -1).all() and not to_np(outs[0]).any()
+    assert not to_np(outs[3]).any() and not to_np(outs[4]).any()
+    assert lib.lancet_scan_workspace_error(p(ws), None, C.byref(err)) == 0 and err.value == 1
+    assert lib.lancet_scan_workspace_init(p(ws), nws, None) == 0 and call() == 0
+    want = mo.moe_encode(data, logits, np.zeros(E, np.int32), 1.0, gate_is_logits=True, fast_scatter=True)
+    np.testing.assert_array_equal(to_np(outs[1]), want[1])
+    np.testing.assert_array_equal(to_np(outs[4]), want[4])
