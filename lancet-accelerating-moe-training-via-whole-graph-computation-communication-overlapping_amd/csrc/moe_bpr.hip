@@ -61,15 +61,16 @@ __device__ __forceinline__ uint32_t par_value(const uint64_t* p) { return static
 // first choice and its gate value (or softmax probability) of every token of the batch
 // (the priority is the gate value as gates_s will hold it: rounded to the gate type); the tile's keys grouped
 // by expert
-template <int GD, bool HELD>
-__global__ __launch_bounds__(kTile) void bpr_prepare_kernel(const void* gate, int is_logits, BprArgs a) {
+template <int GD, int FORM>
+__global__ __launch_bounds__(kSelectThreadsOf<FORM>) void bpr_prepare_kernel(const void* gate, int is_logits, BprArgs a) {
   extern __shared__ uint32_t s_cnt[];
   const int tid = threadIdx.x;
   const uint32_t tile = blockIdx.x;
   const int s = static_cast<int>(tile) * kTile + tid;
   int cls[1] = {-1};
   uint32_t key = 0;
-  const Routed r = route_tile_token<1, GD, HELD>(gate, nullptr, s, a.S0, a.E, is_logits != 0, s_cnt);
+  const Routed r = route_tile_token<1, GD, FORM>(gate, nullptr, s, a.S0, a.E, is_logits != 0, s_cnt);
+  if (threadIdx.x >= kTile) return;
   if (s < a.S0) {
     const float prio = round_gate(r.p0, GD);
     a.tok[s] = foreign_word(static_cast<uint32_t>(r.e0 + 1), __float_as_uint(prio));
@@ -548,7 +549,7 @@ hipError_t run_bpr_route(const void* gate, int S0, int E, int C, int M, int n_pa
   hipError_t err = hipSuccess;
   // (an empty batch still runs one tile, which leaves empty groups for the select kernel)
   const SelectLaunch sel = select_launch(gate_dtype, gate, nullptr, S0, E, is_logits);
-  LANCET_SELECT_SWITCH(gate_dtype, sel.held, (bpr_prepare_kernel<GD, HELD><<<a.ntiles0, kTile, std::max(scan_lds_bytes(E), sel.lds), st>>>(gate, is_logits, a)))
+  LANCET_SELECT_SWITCH(gate_dtype, sel.form, (bpr_prepare_kernel<GD, FORM><<<a.ntiles0, sel.threads, std::max(scan_lds_bytes(E), sel.lds), st>>>(gate, is_logits, a)))
   err = hipGetLastError();
   if (err != hipSuccess) return err;
   bpr_select_kernel<<<E, kSelectThreads, 0, st>>>(a);

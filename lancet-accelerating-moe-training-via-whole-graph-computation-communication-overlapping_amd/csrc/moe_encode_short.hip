@@ -141,8 +141,8 @@ __device__ __forceinline__ bool not_set_up(const EncodeArgs& a) {
 // A tile of tokens (256 and less): every workgroup routes all of them, a token per thread, and moves its own rows; the first
 // also writes the routing.  Routing 64 tokens x 8 experts again in each of 48 workgroups costs nothing that is not waited for
 // anyway: 64 x 1024 bf16 top-2, 8 experts, 9.1 us as three kernels (count, place, scatter), 4.6 as this one.
-template <int K, int GD, bool HELD>
-__global__ __launch_bounds__(kTile) void encode_tile_kernel(EncodeArgs a) {
+template <int K, int GD, int FORM>
+__global__ __launch_bounds__(kSelectThreadsOf<FORM>) void encode_tile_kernel(EncodeArgs a) {
   extern __shared__ uint32_t s_cnt[];
   __shared__ int s_dest[K * kTile];
   const RouteArgs& r = a.r;
@@ -150,14 +150,16 @@ __global__ __launch_bounds__(kTile) void encode_tile_kernel(EncodeArgs a) {
   const bool mover = static_cast<int>(blockIdx.x) < a.token_blocks;
   const int first = static_cast<int>(blockIdx.x) * a.tokens, n = mover ? min(a.tokens, r.S - first) : 0;
   const RowCopy copy(a.row_bytes);
-  RowWork work(a, copy, mover ? first : 0, n);
+  // (the rows wait where sixteen waves select: a thread has half the registers then)
+  RowWork work(a, copy, mover ? first : 0, FORM == kHoldWide ? 0 : n);
   const bool marked = not_set_up(a);
   int e[K];
   float p[K];
   bool mem[K];
   uint32_t rank[K];
   {
-    const Routed t = route_tile_token<K, GD, HELD>(r.gate, r.noise, tid, r.S, r.E, r.is_logits != 0, s_cnt);
+    const Routed t = route_tile_token<K, GD, FORM>(r.gate, r.noise, tid, r.S, r.E, r.is_logits != 0, s_cnt);
+    if (threadIdx.x >= kTile) return;
     e[0] = t.e0, p[0] = t.p0;
     if (K == 2) e[K - 1] = t.e1, p[K - 1] = t.p1;
   }
@@ -209,6 +211,7 @@ __global__ __launch_bounds__(kTile) void encode_tile_kernel(EncodeArgs a) {
     }
   }
   if (blockIdx.x == 0) store_totals<K>(r, totals, marked);
+  if (FORM == kHoldWide) work.load(a, copy, first, n);
   __syncthreads();
   work.store<K>(a, copy, first, n, s_dest);
 }
@@ -344,9 +347,9 @@ hipError_t run_encode_short(const void* data, const void* gate, const void* nois
   if (r.ntiles == 1) {
     const SelectLaunch sel = select_launch(gate_dtype, gate, r.noise, S, E, is_logits);
     const size_t lds = std::max(scan_lds_bytes(NC), sel.lds);
-    LANCET_SELECT_SWITCH(gate_dtype, sel.held,
-      if (K == 1) encode_tile_kernel<1, GD, HELD><<<blocks, kTile, lds, st>>>(a);
-      else encode_tile_kernel<2, GD, HELD><<<blocks, kTile, lds, st>>>(a))
+    LANCET_SELECT_SWITCH(gate_dtype, sel.form,
+      if (K == 1) encode_tile_kernel<1, GD, FORM><<<blocks, sel.threads, lds, st>>>(a);
+      else encode_tile_kernel<2, GD, FORM><<<blocks, sel.threads, lds, st>>>(a))
     return hipGetLastError();
   }
   const hipError_t err = run_route_count(r, K, st);

@@ -10,14 +10,14 @@ namespace lancet {
 // K = 2: ranks of both slots are produced in one pass (2E counters); slot-2 locations need the
 //        slot-1 totals of all tiles, so raw (expert, rank, value) are left in the output arrays
 //        and finalize_top2_kernel completes them.
-template <int K, int GD, bool HELD>
-__global__ __launch_bounds__(kTile) void route_scan_kernel(RouteArgs a) {
+template <int K, int GD, int FORM>
+__global__ __launch_bounds__(kSelectThreadsOf<FORM>) void route_scan_kernel(RouteArgs a) {
   extern __shared__ uint32_t s_cnt[];
   const int tid = threadIdx.x;
   const TileStart me = tile_begin(a.ws, a.ntiles);
   const uint32_t tile = me.tile;
   const int s = static_cast<int>(tile) * kTile + tid;
-  const bool valid = s < a.S;
+  const bool valid = tid < kTile && s < a.S;
   if (!me.ok) {
     // no workspace to scan with: every token of this workgroup's range is marked, and so are the totals
     if (valid) {
@@ -50,7 +50,8 @@ __global__ __launch_bounds__(kTile) void route_scan_kernel(RouteArgs a) {
       e[0] = (x >= 0 && x < a.E) ? x : -1;
     }
   } else {
-    const Routed r = route_tile_token<K, GD, HELD>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
+    const Routed r = route_tile_token<K, GD, FORM>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
+    if (threadIdx.x >= kTile) return;
     if (valid) {
       e[0] = r.e0;
       p[0] = r.p0;
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(kTile) void route_scan_kernel(RouteArgs a) {
 // ---- the same routing as two or three kernels that wait for nothing (scan_form) ------------------------------
 // route_count_kernel: selection, ranks inside the tile, the tile's counts -> table.  Leaves expert, rank inside the
 // tile and raw gate value in idx_out / loc_out / gates_s (idx_out is not written when the experts are given).
-template <int K, int GD, bool HELD>
-__global__ __launch_bounds__(kTile) void route_count_kernel(RouteArgs a) {
+template <int K, int GD, int FORM>
+__global__ __launch_bounds__(kSelectThreadsOf<FORM>) void route_count_kernel(RouteArgs a) {
   extern __shared__ uint32_t s_cnt[];
   const int tid = threadIdx.x;
   const uint32_t tile = blockIdx.x;
@@ -131,7 +132,8 @@ __global__ __launch_bounds__(kTile) void route_count_kernel(RouteArgs a) {
       e[0] = (x >= 0 && x < a.E) ? x : -1;
     }
   } else {
-    const Routed r = route_tile_token<K, GD, HELD>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
+    const Routed r = route_tile_token<K, GD, FORM>(a.gate, a.noise, s, a.S, a.E, a.is_logits != 0, s_cnt);
+    if (threadIdx.x >= kTile) return;
     if (valid) {
       e[0] = r.e0;
       p[0] = r.p0;
@@ -275,13 +277,13 @@ __global__ __launch_bounds__(kTile) void finalize_top2_kernel(RouteArgs a) {
 }
 
 // Selection only (no scan).
-template <int K, int GD, bool HELD>
-__global__ __launch_bounds__(kTile) void gate_topk_kernel(const void* gate, const void* noise, int S, int E,
+template <int K, int GD, int FORM>
+__global__ __launch_bounds__(kSelectThreadsOf<FORM>) void gate_topk_kernel(const void* gate, const void* noise, int S, int E,
                                                           int is_logits, int32_t* idx, void* val) {
   extern __shared__ uint32_t s_stage[];
   const int s = blockIdx.x * kTile + threadIdx.x;
-  const Routed r = route_tile_token<K, GD, HELD>(gate, noise, s, S, E, is_logits != 0, s_stage);
-  if (s >= S) return;
+  const Routed r = route_tile_token<K, GD, FORM>(gate, noise, s, S, E, is_logits != 0, s_stage);
+  if (s >= S || threadIdx.x >= kTile) return;
   idx[s] = r.e0;
   st_gate(val, s, r.p0, GD);
   if (K == 2) {
@@ -376,19 +378,19 @@ hipError_t run_gate_topk(const void* gate, const void* noise, int S, int E, int 
   if (S == 0) return hipSuccess;
   const int blocks = (S + kTile - 1) / kTile;
   const SelectLaunch sel = select_launch(gate_dtype, gate, K == 2 ? noise : nullptr, S, E, is_logits);
-  LANCET_SELECT_SWITCH(gate_dtype, sel.held,
-    if (K == 1) gate_topk_kernel<1, GD, HELD><<<blocks, kTile, sel.lds, st>>>(gate, nullptr, S, E, is_logits, idx, val);
-    else gate_topk_kernel<2, GD, HELD><<<blocks, kTile, sel.lds, st>>>(gate, noise, S, E, is_logits, idx, val))
+  LANCET_SELECT_SWITCH(gate_dtype, sel.form,
+    if (K == 1) gate_topk_kernel<1, GD, FORM><<<blocks, sel.threads, sel.lds, st>>>(gate, nullptr, S, E, is_logits, idx, val);
+    else gate_topk_kernel<2, GD, FORM><<<blocks, sel.threads, sel.lds, st>>>(gate, noise, S, E, is_logits, idx, val))
   return hipGetLastError();
 }
 
 hipError_t run_route_count(const RouteArgs& a, int K, hipStream_t st) {
-  const SelectLaunch sel = a.idx_in ? SelectLaunch{false, 0} : select_launch(a.gate_dtype, a.gate, a.noise, a.S, a.E, a.is_logits);
+  const SelectLaunch sel = a.idx_in ? SelectLaunch{kWalkRows, kTile, 0} : select_launch(a.gate_dtype, a.gate, a.noise, a.S, a.E, a.is_logits);
   const size_t lds = std::max(scan_lds_bytes(K * a.E), sel.lds);
   if (K == 1) {
-    LANCET_SELECT_SWITCH(a.gate_dtype, sel.held, (route_count_kernel<1, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
+    LANCET_SELECT_SWITCH(a.gate_dtype, sel.form, (route_count_kernel<1, GD, FORM><<<a.ntiles, sel.threads, lds, st>>>(a)))
   } else {
-    LANCET_SELECT_SWITCH(a.gate_dtype, sel.held, (route_count_kernel<2, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
+    LANCET_SELECT_SWITCH(a.gate_dtype, sel.form, (route_count_kernel<2, GD, FORM><<<a.ntiles, sel.threads, lds, st>>>(a)))
   }
   return hipGetLastError();
 }
@@ -418,7 +420,7 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
   a.seg_rows = 0;
   hipError_t err = hipSuccess;
   const ScanForm form = scan_form(a.ntiles, static_cast<int64_t>(K) * E, K, force_lookback);
-  const SelectLaunch sel = idx_in ? SelectLaunch{false, 0} : select_launch(gate_dtype, gate, a.noise, S, E, is_logits);
+  const SelectLaunch sel = idx_in ? SelectLaunch{kWalkRows, kTile, 0} : select_launch(gate_dtype, gate, a.noise, S, E, is_logits);
   const size_t lds = std::max(scan_lds_bytes(K * E), sel.lds);
   if (form != kScanLookback) {
     // two or three kernels that wait for nothing instead of a look-back between tiles that all run at once
@@ -436,9 +438,9 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
     return hipGetLastError();
   }
   if (K == 1) {
-    LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_scan_kernel<1, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
+    LANCET_SELECT_SWITCH(gate_dtype, sel.form, (route_scan_kernel<1, GD, FORM><<<a.ntiles, sel.threads, lds, st>>>(a)))
   } else {
-    LANCET_SELECT_SWITCH(gate_dtype, sel.held, (route_scan_kernel<2, GD, HELD><<<a.ntiles, kTile, lds, st>>>(a)))
+    LANCET_SELECT_SWITCH(gate_dtype, sel.form, (route_scan_kernel<2, GD, FORM><<<a.ntiles, sel.threads, lds, st>>>(a)))
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     finalize_top2_kernel<<<a.ntiles, kTile, 0, st>>>(a);

@@ -246,15 +246,17 @@ __device__ __forceinline__ void merge_steps(int q, F f) {
 
 // what route_token returns, for the lane's token of the wave's nrows <= 64 consecutive ones from `rows` on (lanes past
 // them: anything).  All lanes of the wave, uniform control flow.
-template <int K, int GD>
+// WIDE: a lane takes one, two or four granules, so many lanes to a row that the wave's 16 rows fill it.
+template <int K, int GD, bool WIDE = false>
 __device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, int E, bool is_logits) {
   constexpr int gb = GD == LANCET_F32 ? 4 : 2;
   constexpr int V = 16 / gb;
   const int lane = lane_id();
   const uint32_t row_bytes = static_cast<uint32_t>(E) * gb;
   const int n = static_cast<int>((row_bytes + 15u) / 16u);
+  const int mine_n = !WIDE || n > 8 ? kHeldPerLane : n > 4 ? 2 : 1;  // granules per lane
   int q = 0;
-  while (kHeldPerLane << q < n) ++q;
+  while (mine_n << q < n) ++q;
   const int width = 1 << q, per_round = kWave >> q;  // lanes per row, rows per round
   const int sub = lane & (width - 1);
   // where the lane's granules lie in a row; the last of a row that is not whole granules is drawn back to end with it, and
@@ -267,20 +269,22 @@ __device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, i
     at[k] = min(16u * static_cast<uint32_t>(g), row_bytes - 16u);
     dup[k] = g < n ? static_cast<int>(16u * static_cast<uint32_t>(g) - at[k]) / gb : V;
   }
-  const bool ragged = n * 16 != static_cast<int>(row_bytes) || n != kHeldPerLane * width;
+  const bool ragged = n * 16 != static_cast<int>(row_bytes) || n != mine_n * width;
   const auto load = [&](int r, u32x4 (&x)[kHeldPerLane]) {
     const int row = r * per_round + (lane >> q);
     const char* p = rows + static_cast<size_t>(min(row, nrows - 1)) * row_bytes;
 #pragma unroll
-    for (int k = 0; k < kHeldPerLane; ++k) x[k] = *reinterpret_cast<const u32x4_gate*>(p + at[k]);
+    for (int k = 0; k < kHeldPerLane; ++k)
+      if (!WIDE || k < mine_n) x[k] = *reinterpret_cast<const u32x4_gate*>(p + at[k]);
   };
   const int rounds = (nrows + per_round - 1) / per_round;
   float v1 = 0.f, v2 = 0.f, sum = 0.f;  // the lane's own token
   int i1 = 0, i2 = 0;
   u32x4 x[kHeldPerLane], nx[kHeldPerLane];
-  load(0, x);
+  if (!WIDE) load(0, x);
   for (int r = 0; r < rounds; ++r) {
-    if (r + 1 < rounds) load(r + 1, nx);
+    if (WIDE) load(r, x);  // sixteen waves: another one's loads are on their way
+    else if (r + 1 < rounds) load(r + 1, nx);
     float f[kHeldPerLane][V];
 #pragma unroll
     for (int k = 0; k < kHeldPerLane; ++k) each_value<GD>(x[k], [&](float val, int i) { f[k][i] = val; });
@@ -294,6 +298,7 @@ __device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, i
     int j1 = kNoExpert, j2 = kNoExpert;
 #pragma unroll
     for (int k = 0; k < kHeldPerLane; ++k) {
+      if (WIDE && k >= mine_n) break;
       const int j0 = static_cast<int>(at[k] / gb);
 #pragma unroll
       for (int i = 0; i < V; ++i) {
@@ -327,9 +332,11 @@ __device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, i
     });
     float part = 0.f;
 #pragma unroll
-    for (int k = 0; k < kHeldPerLane; ++k)
+    for (int k = 0; k < kHeldPerLane; ++k) {
+      if (WIDE && k >= mine_n) break;
 #pragma unroll
       for (int i = 0; i < V; ++i) part += is_logits ? __expf(f[k][i] - a1) : f[k][i];
+    }
     merge_steps(q, [&](auto step) { part += merge_partner<step.value>(part); });
     // the round's tokens to their lanes
     const int from = (lane & (per_round - 1)) << q;
@@ -346,7 +353,7 @@ __device__ __forceinline__ Routed route_rows_held(const char* rows, int nrows, i
       i2 = mine ? u2 : i2;
     }
 #pragma unroll
-    for (int k = 0; k < kHeldPerLane; ++k) x[k] = nx[k];
+    for (int k = 0; k < kHeldPerLane && !WIDE; ++k) x[k] = nx[k];
   }
   Routed res;
   const bool plain = sum == sum && i1 != kNoExpert && (K == 1 || i2 != kNoExpert);
@@ -453,16 +460,38 @@ __device__ __forceinline__ F walk_rows_staged(const char* rows, int nrows, int E
   return f;
 }
 
-// Selection for token s of a workgroup whose thread t holds token s = first + t (kTile consecutive tokens): what
-// route_token gives, from registers (HELD: rows_are_held), by the direct walk or through LDS.  All kTile threads, uniform
-// control flow; lds = at least kStageBytes when rows_are_staged (it may be reused after the call).  Threads with s >= S get
-// {-1, -1, 0, 0}.
-template <int K, int GD, bool HELD>
+// ---- how a kernel selects ------------------------------------------------------------------------------------------
+enum SelectForm { kWalkRows = 0, kHoldRows = 1, kHoldWide = 2 };
+// Threads of a workgroup that selects for a tile.  Wide: sixteen waves select sixteen tokens each and hand what they chose to the
+// four that go on.  A short launch is over when its waves are, and a wave's 64 rows of a few granules were four rounds of
+// loads, compares and exponentials one after the other.
+template <int FORM>
+constexpr int kSelectThreadsOf = FORM == kHoldWide ? 4 * kTile : kTile;
+constexpr int kWideRows = kTile / 16;
+
+// Selection for token s of a workgroup whose thread t < kTile holds token s = first + t (kTile consecutive tokens): what
+// route_token gives, from registers (kHoldRows, kHoldWide: select_launch), by the direct walk or through LDS.  All threads,
+// uniform control flow; lds = at least kStageBytes when rows_are_staged (it may be reused after the
+// call).  Threads with s >= S get {-1, -1, 0, 0}.  kHoldWide: threads from kTile on have nothing left to do.
+template <int K, int GD, int FORM>
 __device__ __forceinline__ Routed route_tile_token(const void* gate, const void* noise, int s, int S, int E, bool is_logits,
                                                    void* lds) {
   constexpr size_t gb = GD == LANCET_F32 ? 4 : 2;
   Routed r = {-1, -1, 0.f, 0.f};
-  if (HELD) {
+  if constexpr (FORM == kHoldWide) {
+    __shared__ Routed chosen[kTile];
+    const int w = static_cast<int>(threadIdx.x) / kWave, lane = lane_id();
+    const int first = s - static_cast<int>(threadIdx.x) + w * kWideRows;
+    const int nrows = min(S - first, kWideRows);
+    if (nrows > 0) {
+      const Routed held = route_rows_held<K, GD, true>(static_cast<const char*>(gate) + static_cast<size_t>(first) * E * gb, nrows, E, is_logits);
+      if (lane < nrows) chosen[w * kWideRows + lane] = held;
+    }
+    __syncthreads();
+    if (threadIdx.x < kTile && s < S) r = chosen[threadIdx.x];
+    return r;
+  }
+  if constexpr (FORM == kHoldRows) {
     const int first = s - lane_id();  // the wave's first token
     if (first < S) {
       const Routed held = route_rows_held<K, GD>(static_cast<const char*>(gate) + static_cast<size_t>(first) * E * gb,
@@ -512,20 +541,37 @@ __device__ __forceinline__ Routed route_tile_token(const void* gate, const void*
     default: { constexpr int GD = LANCET_F32; __VA_ARGS__; } break;           \
   }
 
-// GD and HELD as compile-time constants inside `...`
-#define LANCET_SELECT_SWITCH(gd, held, ...)                         \
-  LANCET_GATE_SWITCH(gd, if (held) { constexpr bool HELD = true; __VA_ARGS__; } else { constexpr bool HELD = false; __VA_ARGS__; })
+// GD and FORM as compile-time constants inside `...`
+#define LANCET_SELECT_SWITCH(gd, form, ...)                                                              \
+  LANCET_GATE_SWITCH(gd, if (form == kHoldWide) { constexpr int FORM = kHoldWide; __VA_ARGS__; }           \
+                         else if (form == kHoldRows) { constexpr int FORM = kHoldRows; __VA_ARGS__; }      \
+                         else { constexpr int FORM = kWalkRows; __VA_ARGS__; })
 
-// how a kernel that selects is launched: its variant, and the LDS it needs for the rows it stages
+// how a kernel that selects is launched: its form, its threads and the LDS its selection needs
 struct SelectLaunch {
-  bool held;
+  SelectForm form;
+  int threads;
   size_t lds;
 };
+// Wide: short launches (a tile has a CU to itself) of rows long enough for the second barrier and the waves that are started to
+// pay.  moe_encode of 256 / 4096 / 65536 tokens, otherwise / wide, us: 64 fp32 logits top-1 7.3 / 5.6, 10.5 / 8.9, 16.7 / 14.9, top-2
+// 8.8 / 7.7, 12.5 / 11.4, 23.9 / 22.5; 128 top-1 11.2 / 7.3, 14.6 / 10.6, 24.1 / 20.8; 256 21.8 / 13.1, 22.7 / 14.0, 34.5 / 30.3; but 32 top-2 6.5 / 6.9,
+// 9.9 / 10.2 and 16 6.1 / 7.2.  128 bf16 logits top-2 11.3 / 10.6, 15.2 / 14.1, 64 8.1 / 8.6.  64 tokens: 60 bf16 6.1 / 4.8, 32 fp32 6.0 / 5.6.
+// Probabilities: full lanes alone (64 fp32 top-1 6.3 / 5.6, 9.7 / 8.9, 128 8.1 / 7.2; 200 12.2 / 14.2, 60 and 96 the same).
+// 131072 tokens: 64 fp32 23.8 / 24.8.
+constexpr int kWideTiles = 256;
+inline bool rows_are_wide(const void* noise, int S, int E, int gb, bool is_logits) {
+  const int bytes = E * gb;
+  if (noise != nullptr || bytes <= 32 || bytes > 16 * kHeldGranules || (S + kTile - 1) / kTile > kWideTiles) return false;
+  if (!is_logits) return gb == 4 && (E == 64 || E == 128);
+  return E >= (S <= kWave ? 32 : gb == 4 ? 56 : 96);
+}
 inline SelectLaunch select_launch(int gate_dtype, const void* gate, const void* noise, int S, int E, bool is_logits) {
-  SelectLaunch l = {rows_are_held(gate, noise, S, E, gate_dtype == LANCET_F32 ? 4 : 2, is_logits), 0};
-  if (!l.held) {
-    LANCET_GATE_SWITCH(gate_dtype, l.lds = rows_are_staged<GD>(gate, noise, S, E) ? kStageBytes : 0)
-  }
+  const int gb = gate_dtype == LANCET_F32 ? 4 : 2;
+  if (rows_are_wide(noise, S, E, gb, is_logits)) return {kHoldWide, kSelectThreadsOf<kHoldWide>, 0};
+  if (rows_are_held(gate, noise, S, E, gb, is_logits)) return {kHoldRows, kTile, 0};
+  SelectLaunch l = {kWalkRows, kTile, 0};
+  LANCET_GATE_SWITCH(gate_dtype, l.lds = rows_are_staged<GD>(gate, noise, S, E) ? kStageBytes : 0)
   return l;
 }
 

@@ -86,3 +86,27 @@ def test_short_top1_on_memory_that_was_never_set_up(pkg, S):
     want = mo.moe_encode(data, logits, np.zeros(E, np.int32), 1.0, gate_is_logits=True, fast_scatter=True)
     np.testing.assert_array_equal(to_np(outs[1]), want[1])
     np.testing.assert_array_equal(to_np(outs[4]), want[4])
+
+
+@pytest.mark.parametrize("S", [1, 15, 17, 64, 65, 255, 257, 700])
+@pytest.mark.parametrize("E,gdt", [(32, "f32"), (56, "f32"), (63, "f32"), (64, "f32"), (100, "f32"), (256, "f32"), (96, "bf16"), (101, "f16"), (512, "bf16")])
+def test_selection_by_sixteen_waves(pkg, S, E, gdt):
+    """Rows whose selection sixteen waves share: choices against the oracle's on the rounded gate (massive ties of 16-bit values
+    included), rows with a NaN and rows of -inf against the same rows in a batch that sixteen waves do not take (noise of zero
+    sends a top-2 call to the row-by-row walk)."""
+    ops = pkg.ops
+    data, logits = make_inputs(S + E, S, 4, E, ties=S % 2 == 1)
+    gate = dev(logits).to(TORCH_DT[gdt])
+    rounded = gate.float().cpu().numpy()
+    for k in (1, 2):
+        for is_logits in (True, False):
+            sel = mo.select_topk(rounded, k, gate_is_logits=is_logits)[0]
+            got = ops.moe_encode(dev(data), gate, None, float(E), top_k=k, gate_is_logits=is_logits)
+            np.testing.assert_array_equal(to_np(got[1])[0], np.concatenate([sel[j] for j in range(k)]))
+    odd = gate.clone()
+    odd[::3, E // 2] = float("nan")
+    odd[1::3] = float("-inf")
+    for is_logits in (True, False):
+        a = ops.moe_encode(dev(data), odd, None, float(E), top_k=2, gate_is_logits=is_logits)
+        b = ops.moe_encode(dev(data), odd, None, float(E), top_k=2, gate_is_logits=is_logits, gate2_noise=torch.zeros_like(odd))
+        np.testing.assert_array_equal(to_np(a[1]), to_np(b[1]))
