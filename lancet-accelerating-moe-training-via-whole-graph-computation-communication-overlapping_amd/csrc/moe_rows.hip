@@ -652,7 +652,7 @@ __global__ __launch_bounds__(kTile) void encode_dg_kernel(const void* dy, const 
   }
 }
 
-// src[e*C + l] = slot-token id (j*S + s) of the token that owns row (e, l); src is -1 elsewhere.
+// src[e*C + l] = slot-token id (j*S + s) of the token that owns row (e, l); rows nobody owns keep what lies there.
 __global__ __launch_bounds__(kTile) void inverse_map_kernel(const int32_t* idx, const int32_t* loc, int n, int E,
                                                             int C, int32_t* src) {
   const int i = blockIdx.x * kTile + threadIdx.x;
@@ -661,19 +661,28 @@ __global__ __launch_bounds__(kTile) void inverse_map_kernel(const int32_t* idx, 
   if (e >= 0 && e < E && l >= 0 && l < C) src[static_cast<size_t>(e) * C + l] = i;
 }
 
+// The slot-token that owns a row, or -1.  The map is not cleared beforehand (2 to 5 us and a launch in front of every backward
+// pass): an entry counts if the slot it names is routed to that row, which whatever else lies there is not.
+__device__ __forceinline__ int row_owner(const int32_t* src, size_t row, const int32_t* idx, const int32_t* loc, int n, int E, int C) {
+  const int i = src[row];
+  if (i < 0 || i >= n) return -1;
+  const int e = idx[i], l = loc[i];
+  return e >= 0 && e < E && l >= 0 && l < C && static_cast<size_t>(e) * C + l == row ? i : -1;
+}
+
 // grad_expert_out[e, l, :] = gates[i] * dy[s, :] for the slot-token i = src[e*C+l] (s = i mod S), zero
 // for rows nobody owns: decode_backward_data_kernel (tutel_moe_dispatch.cu:118-124, 523-533) without
 // the memset + atomicAdd; every output byte is written once.
 template <int DT, int MODE, int K>
 __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, const void* gates, int gd,
-                                                               const int32_t* src, void* out, int S, int M,
-                                                               long rows, int q) {
+                                                               const int32_t* src, const int32_t* idx, const int32_t* loc,
+                                                               void* out, int S, int M, int E, int C, long rows, int q) {
   typedef Codec<DT> Cd;
   const RowShare h = row_share(q);
   const long r = h.r;
   const int step = h.step;
   if (r >= rows) return;
-  const int i = src[r];
+  const int i = row_owner(src, static_cast<size_t>(r), idx, loc, K * S, E, C);
   // the weight first, then the row: with both asked for at once the reads crowd out the writes here (262144 x 512 bf16
   // top-1: 83 against 90 us)
   const float g1[1] = {i >= 0 ? ld_gate(gates, i, gd) : 0.f};
@@ -825,7 +834,7 @@ struct DecodeGradArgs {
   const void* gates;       // [K*S] of gate_dtype
   const int32_t* idx;      // [K*S]
   const int32_t* loc;      // [K*S]
-  const int32_t* owner;    // [E*C] slot-token that owns a row, -1 = none; null: walk the slots
+  const int32_t* owner;    // [E*C] slot-token that owns a row (row_owner); null: walk the slots
   char* d_expert_out;      // [E, C, M]
   void* d_gates;           // [K*S] of gate_dtype
   int S, E, C, gate_dtype;
@@ -862,7 +871,7 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
     const int q = min(a.q, 6);
     for (int r = first + (static_cast<int>(threadIdx.x) >> q); r < last; r += kTile >> q) {
       const size_t row = static_cast<size_t>(e) * a.C + r;
-      const bool owned = a.owner ? a.owner[row] >= 0 : ((s_owned[(r - first) >> 5] >> ((r - first) & 31)) & 1u) != 0;
+      const bool owned = a.owner ? row_owner(a.owner, row, a.idx, a.loc, K * a.S, a.E, a.C) >= 0 : ((s_owned[(r - first) >> 5] >> ((r - first) & 31)) & 1u) != 0;
       if (owned) continue;
       LANCET_GLOBAL char* dst = as_global(a.d_expert_out + row * a.row_bytes);
       for (int v = threadIdx.x & ((1 << q) - 1); v < a.row_vecs; v += 1 << q) G::st(dst + G::at(v, a.row_bytes), G::zero());
@@ -1172,22 +1181,22 @@ hipError_t run_encode_dg(const void* dy, const int32_t* idx, int S, int E, int K
 }
 
 template <int DT>
-static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, void* out, int S, int M,
-                                   long rows, int K, RowMode mode, hipStream_t st) {
+static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, const int32_t* idx,
+                                   const int32_t* loc, void* out, int S, int M, int E, int C, int K, RowMode mode, hipStream_t st) {
+  const long rows = static_cast<long>(E) * C;
   constexpr int eb = sizeof(typename Codec<DT>::S);
   const int units = row_granules(mode, static_cast<size_t>(M) * eb, eb);
   const int q = row_lanes(units, rows, few_granules(units, rows) && units <= kWave ? 1 : 2);  // two granules per lane: 442 -> 408 us
   const unsigned blocks = static_cast<unsigned>(row_blocks(rows, q));
   LANCET_CODED_ROW_SWITCH(DT, mode,
-    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, q);
-    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, out, S, M, rows, q))
+    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, idx, loc, out, S, M, E, C, rows, q);
+    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, idx, loc, out, S, M, E, C, rows, q))
   return hipGetLastError();
 }
 
-// fills the inverse map src[E*C] (-1: nobody owns the row)
+// the inverse map (row_owner)
 static hipError_t run_inverse_map(const int32_t* idx, const int32_t* loc, int n, int E, int C, int32_t* src, hipStream_t st) {
-  hipError_t err = run_fill_u32(reinterpret_cast<uint32_t*>(src), static_cast<size_t>(E) * C, 0xffffffffu, st);
-  if (err != hipSuccess || n == 0) return err;
+  if (n == 0) return hipSuccess;
   inverse_map_kernel<<<(n + kTile - 1) / kTile, kTile, 0, st>>>(idx, loc, n, E, C, src);
   return hipGetLastError();
 }
@@ -1201,9 +1210,9 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
   const int eb = dtype == LANCET_F32 ? 4 : 2;
   const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(dy) && aligned16(out));
   switch (dtype) {
-    case LANCET_F32: return decode_dx_launch<LANCET_F32>(dy, gates, gate_dtype, src_map, out, S, M, rows, K, mode, st);
-    case LANCET_BF16: return decode_dx_launch<LANCET_BF16>(dy, gates, gate_dtype, src_map, out, S, M, rows, K, mode, st);
-    default: return decode_dx_launch<LANCET_F16>(dy, gates, gate_dtype, src_map, out, S, M, rows, K, mode, st);
+    case LANCET_F32: return decode_dx_launch<LANCET_F32>(dy, gates, gate_dtype, src_map, idx, loc, out, S, M, E, C, K, mode, st);
+    case LANCET_BF16: return decode_dx_launch<LANCET_BF16>(dy, gates, gate_dtype, src_map, idx, loc, out, S, M, E, C, K, mode, st);
+    default: return decode_dx_launch<LANCET_F16>(dy, gates, gate_dtype, src_map, idx, loc, out, S, M, E, C, K, mode, st);
   }
 }
 
