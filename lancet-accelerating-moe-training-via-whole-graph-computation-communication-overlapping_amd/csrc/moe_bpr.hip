@@ -31,7 +31,7 @@ __device__ __forceinline__ uint32_t order_key(float x) {
 // token's expert + 1 in the tag's low bits; par[0..2][e] = threshold, tie quota, ties before the partition,
 // par[3][e] = tokens of the expert before the partition inside the tile of 256 tokens that holds its start.
 // For the select kernel the prepare kernel also leaves every tile's keys grouped by expert, in token order
-// (keys[tile][256]) and where each expert's group lies (groups[e][tile] = start | count << 16): an expert's
+// (keys[tile][256], the token's place in its tile in the tag) and where each expert's group lies (groups[e][tile] = start | count << 16): an expert's
 // workgroup then reads its own keys and one word per tile instead of the whole batch.
 struct BprArgs {
   uint64_t* tok;         // [S0] expert and priority (gate value of the chosen expert) per token
@@ -43,6 +43,7 @@ struct BprArgs {
   int part_lo;           // first token of the partition
   int ntiles;
   int seg_rows;          // place kernel: tiles per segment of the segment sums, 0 = there are none
+  int placed_by_expert;  // the select kernel also places the tokens: no scan follows
   int gate_dtype;        // storage type of gates_s (and of the gate the priorities came from)
   void* gates_s;         // [S]
   int32_t* idx_out;      // [S]
@@ -111,7 +112,8 @@ __global__ __launch_bounds__(kSelectThreadsOf<FORM>) void bpr_prepare_kernel(con
   }
   if (holds_start && cls[0] >= 0 && s < a.part_lo) atomicAdd(&s_early[cls[0]], 1u);
   __syncthreads();
-  if (cls[0] >= 0) a.keys[static_cast<size_t>(tile) * kTile + s_start[cls[0]] + rank[0]] = foreign_word(0u, key);
+  if (cls[0] >= 0) a.keys[static_cast<size_t>(tile) * kTile + s_start[cls[0]] + rank[0]] = foreign_word(static_cast<uint32_t>(tid), key);
+  if (a.placed_by_expert && s >= a.part_lo && s < a.part_lo + a.S) st_gate(a.gates_s, s - a.part_lo, cls[0] >= 0 ? round_gate(r.p0, GD) : 0.f, GD);
   for (int c = tid; c < a.E; c += kTile) {
     a.groups[static_cast<size_t>(c) * a.ntiles0 + tile] = foreign_word(0u, s_start[c] | (s_agg[c] << 16));
     if (holds_start) a.par[3 * a.E + c] = foreign_word(0u, s_early[c]);
@@ -122,6 +124,12 @@ __global__ __launch_bounds__(kSelectThreadsOf<FORM>) void bpr_prepare_kernel(con
 // expert that half of a batch of 65536 tokens chose still fits.
 constexpr int kSelectKeys = 32768;
 constexpr int kSelectTiles = 4096;  // tiles whose group positions fit in LDS (16 KB): batches up to 1M tokens
+// Tokens of a batch up to which an expert's workgroup also places its tokens, which saves the two launches of the scan; in longer
+// batches the expert that most tokens chose is placed by one CU, store by store.  moe_encode_batch_prioritized of rows of 32
+// bytes, scan / placed, us: 64 tokens on 8 experts 14.9 / 12.6, 512 on 16 17.3 / 15.0, 1024 on 64 19.8 / 15.1, 2048 on 4, nearly all on
+// one, 18.0 / 17.7; 4096 on 64 22.9 / 18.6, but nearly all on one of two 18.5 / 20.6, and 32768 on 64, some hot, 35.0 / 42.6.
+constexpr int kPlaceTokens = 2048;
+static_assert(kPlaceTokens <= kSelectKeys, "the keys lie in LDS");
 constexpr int kSelectBits = 10;     // digit of the radix select: one histogram bin per thread
 static_assert((1 << kSelectBits) == kSelectThreads, "a thread owns one bin");
 
@@ -148,7 +156,7 @@ __device__ __forceinline__ uint32_t select_block_scan(uint32_t v, uint32_t* s_wa
   return before + inc - v;
 }
 
-// f(key, position) for every key of the expert, position = its place in token order, from the prepare kernel's groups.
+// f(key's word, tile, position) for every key of the expert, position = its place in token order, from the prepare kernel's groups.
 // A group is read by 2^q neighbouring lanes, q by the expert's mean keys per tile, four loads of a lane in flight:
 // s_pos holds the position of a tile's first key in the low 22 bits and the start of its group inside the tile above
 // them, so nothing is searched for.  (A lane that found the tile of its key by bisection over the positions spent most of
@@ -168,7 +176,7 @@ __device__ __forceinline__ void walk_groups(const BprArgs& a, const uint32_t* s_
       for (int j = 0; j < 4; ++j) k[j] = i + j * width < n ? group[i + j * width] : 0ull;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (i + j * width < n) f(static_cast<uint32_t>(k[j]), pos + i + j * width);
+        if (i + j * width < n) f(k[j], t, pos + i + j * width);
     }
   }
 }
@@ -181,12 +189,18 @@ __device__ __forceinline__ void walk_groups(const BprArgs& a, const uint32_t* s_
 // tokens on 64 experts of which a few are hot (top-1, most keys on one expert): four 8-bit digits from bit 31 on 78 us, three
 // of 10 bits 18.5.  moe_encode_batch_prioritized as a whole, the same two and with the keys compared after the first digit:
 // 256 tokens on 16 experts 17.1 / 18.2 / 15.6 us, 1024 on 64 20.5 / 21.4 / 18.7.
+//
+// PLACE (short batches, whose keys all fit in LDS): the workgroup goes on to place its expert's tokens: two scans over the keys
+// in token order, ties and kept ones, give every kept token its location, and a second walk over the groups, which name the
+// tokens, writes them.
+template <bool PLACE>
 __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
   __shared__ uint32_t s_keys[kSelectKeys];
   __shared__ uint32_t s_pos[kSelectTiles];
   __shared__ uint32_t hist[1 << kSelectBits];
   __shared__ uint32_t s_wave[kSelectThreads / kWave];
   __shared__ uint32_t s_prefix, s_need, s_count, s_min, s_max, s_bin, s_few;
+  __shared__ uint32_t s_thr, s_quota, s_front, s_kept;  // PLACE: what was selected
   const int e = blockIdx.x;
   const int tid = threadIdx.x;
   // The expert's keys, in token order.  Up to kSelectTiles tiles, the prepare kernel's groups say where they are:
@@ -199,6 +213,8 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
     s_few = 0;
     s_min = 0xffffffffu;
     s_max = 0u;
+    s_kept = 0;
+    s_front = 0;
   }
   if (grouped) {
     uint32_t carry = 0;
@@ -223,20 +239,13 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
     __syncthreads();
     count = s_count;
   }
-  if (a.C <= 0) {
-    // nothing fits: no key is above the largest threshold and the tie quota is zero
+  const bool none = a.C <= 0, all = !none && count <= static_cast<uint32_t>(a.C);
+  if (!PLACE && (none || all)) {
+    // nothing fits: no key is above the largest threshold and the tie quota is zero; everything fits: every key is above
+    // threshold 0 or ties with it under an unlimited quota
     if (tid == 0) {
-      a.par[e] = foreign_word(0u, 0xffffffffu);
-      a.par[a.E + e] = foreign_word(0u, 0u);
-      a.par[2 * a.E + e] = foreign_word(0u, 0u);
-    }
-    return;
-  }
-  if (count <= static_cast<uint32_t>(a.C)) {
-    // everything fits: every key is above threshold 0 or ties with it under an unlimited quota
-    if (tid == 0) {
-      a.par[e] = foreign_word(0u, 0u);
-      a.par[a.E + e] = foreign_word(0u, 0x7fffffffu);
+      a.par[e] = foreign_word(0u, none ? 0xffffffffu : 0u);
+      a.par[a.E + e] = foreign_word(0u, none ? 0u : 0x7fffffffu);
       a.par[2 * a.E + e] = foreign_word(0u, 0u);
     }
     return;
@@ -249,7 +258,7 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
     if (in_lds) {
       for (uint32_t i = tid; i < count; i += kSelectThreads) f(s_keys[i], i < nfront);
     } else if (grouped) {
-      walk_groups(a, s_pos, count, q, [&](uint32_t k, uint32_t pos) { f(k, pos < nfront); });
+      walk_groups(a, s_pos, count, q, [&](uint64_t w, int, uint32_t pos) { f(static_cast<uint32_t>(w), pos < nfront); });
     } else {
       for (int s = tid; s < a.S0; s += kSelectThreads) {
         const uint64_t t = a.tok[s];
@@ -257,100 +266,165 @@ __global__ __launch_bounds__(kSelectThreads) void bpr_select_kernel(BprArgs a) {
       }
     }
   };
-  uint32_t lo = 0xffffffffu, hi = 0u;
-  if (in_lds) {
-    walk_groups(a, s_pos, count, q, [&](uint32_t k, uint32_t pos) {
-      s_keys[pos] = k;
-      lo = min(lo, k), hi = max(hi, k);
-    });
-  } else {
-    every_key([&](uint32_t k, bool) { lo = min(lo, k), hi = max(hi, k); });
-  }
+  const auto select = [&] {
+    uint32_t lo = 0xffffffffu, hi = 0u;
+    if (in_lds) {
+      walk_groups(a, s_pos, count, q, [&](uint64_t w, int, uint32_t pos) {
+        const uint32_t k = static_cast<uint32_t>(w);
+        s_keys[pos] = k;
+        lo = min(lo, k), hi = max(hi, k);
+      });
+    } else {
+      every_key([&](uint32_t k, bool) { lo = min(lo, k), hi = max(hi, k); });
+    }
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    lo = min(lo, static_cast<uint32_t>(__shfl_xor(lo, off, kWave)));
-    hi = max(hi, static_cast<uint32_t>(__shfl_xor(hi, off, kWave)));
-  }
-  if (lane_id() == 0) {
-    atomicMin(&s_min, lo);
-    atomicMax(&s_max, hi);
-  }
-  if (tid == 0) s_need = static_cast<uint32_t>(a.C);
-  __syncthreads();
-  // digits from the highest bit in which two keys differ; `left` bits are still to be found
-  int left = s_min == s_max ? 0 : 32 - __clz(s_min ^ s_max);
-  uint32_t prefix = left == 32 ? 0u : s_min >> left;
-  uint32_t open = count;  // keys that share what is found of the threshold
-  while (left > 0 && open > kWave) {
-    const int bits = min(left, kSelectBits);
-    const int shift = left - bits;
-    const uint32_t digits = (1u << bits) - 1u;
-    hist[tid] = 0;
-    __syncthreads();
-    const uint32_t need = s_need;
-    every_key([&](uint32_t k, bool) {
-      if (left == 32 || (k >> left) == prefix) atomicAdd(&hist[(k >> shift) & digits], 1u);
-    });
-    __syncthreads();
-    // the digit that holds the need-th largest of the keys counted, and what is needed inside it: bins in descending
-    // order, one per thread
-    const uint32_t bin = static_cast<uint32_t>(kSelectThreads - 1 - tid);
-    const uint32_t h = hist[bin];
-    uint32_t total;
-    const uint32_t above = select_block_scan(h, s_wave, &total);
-    // (fewer keys than needed does not happen with consistent counts: digit 0 takes what is left)
-    if ((above < need && need <= above + h) || (bin == 0u && total < need)) {
-      s_need = need - above;
-      s_prefix = (left == 32 ? 0u : prefix << bits) | bin;
-      s_bin = h;
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      lo = min(lo, static_cast<uint32_t>(__shfl_xor(lo, off, kWave)));
+      hi = max(hi, static_cast<uint32_t>(__shfl_xor(hi, off, kWave)));
     }
+    if (lane_id() == 0) {
+      atomicMin(&s_min, lo);
+      atomicMax(&s_max, hi);
+    }
+    if (tid == 0) s_need = static_cast<uint32_t>(a.C);
     __syncthreads();
-    prefix = s_prefix;
-    open = s_bin;
-    left = shift;
-  }
-  if (left > 0) {
-    // no more keys than a wave has lanes: it compares them with one another, and counts the threshold's equals that
-    // precede the partition on the way
-    every_key([&](uint32_t k, bool early) {
-      if (left == 32 || (k >> left) == prefix) {
-        const uint32_t at = atomicAdd(&s_few, 1u);
-        hist[at] = k;
-        hist[kWave + at] = early;
-      }
-    });
-    __syncthreads();
-    if (tid < static_cast<int>(open)) {
-      const uint32_t mine = hist[tid];
-      uint32_t above = 0, same = 0, front = 0;
-      for (uint32_t i = 0; i < open; ++i) {
-        above += hist[i] > mine;
-        same += hist[i] == mine;
-        front += (hist[i] == mine) & hist[kWave + i];
-      }
+    // digits from the highest bit in which two keys differ; `left` bits are still to be found
+    int left = s_min == s_max ? 0 : 32 - __clz(s_min ^ s_max);
+    uint32_t prefix = left == 32 ? 0u : s_min >> left;
+    uint32_t open = count;  // keys that share what is found of the threshold
+    while (left > 0 && open > kWave) {
+      const int bits = min(left, kSelectBits);
+      const int shift = left - bits;
+      const uint32_t digits = (1u << bits) - 1u;
+      hist[tid] = 0;
+      __syncthreads();
       const uint32_t need = s_need;
-      if (above < need && need <= above + same) {  // equal keys write the same words
-        a.par[e] = foreign_word(0u, mine);
-        a.par[a.E + e] = foreign_word(0u, need - above);
-        a.par[2 * a.E + e] = foreign_word(0u, front);
+      every_key([&](uint32_t k, bool) {
+        if (left == 32 || (k >> left) == prefix) atomicAdd(&hist[(k >> shift) & digits], 1u);
+      });
+      __syncthreads();
+      // the digit that holds the need-th largest of the keys counted, and what is needed inside it: bins in descending
+      // order, one per thread
+      const uint32_t bin = static_cast<uint32_t>(kSelectThreads - 1 - tid);
+      const uint32_t h = hist[bin];
+      uint32_t total;
+      const uint32_t above = select_block_scan(h, s_wave, &total);
+      // (fewer keys than needed does not happen with consistent counts: digit 0 takes what is left)
+      if ((above < need && need <= above + h) || (bin == 0u && total < need)) {
+        s_need = need - above;
+        s_prefix = (left == 32 ? 0u : prefix << bits) | bin;
+        s_bin = h;
       }
+      __syncthreads();
+      prefix = s_prefix;
+      open = s_bin;
+      left = shift;
     }
-    return;
-  }
-  const uint32_t thr = prefix;
-  // ties that precede the partition
-  if (a.part_lo > 0) {
-    uint32_t local = 0;
-    every_key([&](uint32_t k, bool early) { local += early && k == thr; });
-    if (!grouped && tid == 0) s_count = 0;  // held the expert's count
+    if (left > 0) {
+      // no more keys than a wave has lanes: it compares them with one another, and counts the threshold's equals that
+      // precede the partition on the way
+      every_key([&](uint32_t k, bool early) {
+        if (left == 32 || (k >> left) == prefix) {
+          const uint32_t at = atomicAdd(&s_few, 1u);
+          hist[at] = k;
+          hist[kWave + at] = early;
+        }
+      });
+      __syncthreads();
+      if (tid < static_cast<int>(open)) {
+        const uint32_t mine = hist[tid];
+        uint32_t above = 0, same = 0, front = 0;
+        for (uint32_t i = 0; i < open; ++i) {
+          above += hist[i] > mine;
+          same += hist[i] == mine;
+          front += (hist[i] == mine) & hist[kWave + i];
+        }
+        const uint32_t need = s_need;
+        if (above < need && need <= above + same) {  // equal keys write the same words
+          if (PLACE) {
+            s_thr = mine;
+            s_quota = need - above;
+          } else {
+            a.par[e] = foreign_word(0u, mine);
+            a.par[a.E + e] = foreign_word(0u, need - above);
+            a.par[2 * a.E + e] = foreign_word(0u, front);
+          }
+        }
+      }
+      return;
+    }
+    if (PLACE) {
+      if (tid == 0) {
+        s_thr = prefix;
+        s_quota = s_need;
+      }
+      return;
+    }
+    const uint32_t thr = prefix;
+    // ties that precede the partition
+    if (a.part_lo > 0) {
+      uint32_t local = 0;
+      every_key([&](uint32_t k, bool early) { local += early && k == thr; });
+      if (!grouped && tid == 0) s_count = 0;  // held the expert's count
+      __syncthreads();
+      if (local) atomicAdd(&s_count, local);
+      __syncthreads();
+    }
+    if (tid == 0) {
+      a.par[e] = foreign_word(0u, thr);
+      a.par[a.E + e] = foreign_word(0u, s_need);
+      a.par[2 * a.E + e] = foreign_word(0u, a.part_lo > 0 ? s_count : 0u);
+    }
+  };
+  if (!none && !all) select();
+  if (!PLACE) return;
+
+  // ---- the tokens' places -----------------------------------------------------------------------------------------
+  __syncthreads();
+  if (!none && !all) {
+    // a thread owns consecutive keys, an odd number of them (LDS banks): how many tie with the threshold before them, which of
+    // them stay, how many stay before
+    const uint32_t thr = s_thr, quota = s_quota;
+    const uint32_t per = (count + kSelectThreads - 1) / kSelectThreads | 1u, lo = min(count, tid * per), hi = min(count, lo + per);
+    uint32_t ties = 0, total;
+    for (uint32_t p = lo; p < hi; ++p) ties += s_keys[p] == thr;
+    ties = select_block_scan(ties, s_wave, &total);
+    const uint32_t first_tie = ties;
+    uint32_t kept = 0;
+    for (uint32_t p = lo; p < hi; ++p) {
+      const uint32_t k = s_keys[p];
+      kept += k > thr || (k == thr && ties < quota);
+      ties += k == thr;
+    }
+    uint32_t before = select_block_scan(kept, s_wave, &total);
+    ties = first_tie;
+    for (uint32_t p = lo; p < hi; ++p) {
+      const uint32_t k = s_keys[p];
+      const bool stays = k > thr || (k == thr && ties < quota);
+      ties += k == thr;
+      if (p == nfront) s_front = before;
+      s_keys[p] = stays ? before : 0xffffffffu;
+      before += stays;
+    }
+    if (tid == 0 && nfront >= count) s_front = total;
     __syncthreads();
-    if (local) atomicAdd(&s_count, local);
-    __syncthreads();
   }
+  const uint32_t front = all ? nfront : s_front;
+  uint32_t kept = 0;
+  walk_groups(a, s_pos, count, q, [&](uint64_t w, int t, uint32_t pos) {
+    const int sl = t * kTile + static_cast<int>((w >> 32) & 0xffu) - a.part_lo;
+    if (sl < 0 || sl >= a.S) return;
+    const uint32_t place = none ? 0xffffffffu : all ? pos : s_keys[pos];
+    const bool stays = place != 0xffffffffu;
+    a.idx_out[sl] = stays ? e : -1;
+    a.loc_out[sl] = stays ? static_cast<int>(place - front) : -1;
+    kept += stays;
+  });
+  if (kept) atomicAdd(&s_kept, kept);
+  __syncthreads();
   if (tid == 0) {
-    a.par[e] = foreign_word(0u, thr);
-    a.par[a.E + e] = foreign_word(0u, s_need);
-    a.par[2 * a.E + e] = foreign_word(0u, a.part_lo > 0 ? s_count : 0u);
+    a.used_out[e] = static_cast<int32_t>(s_kept);
+    a.elems_out[e] = static_cast<uint64_t>(s_kept) * static_cast<uint64_t>(a.M);
   }
 }
 
@@ -547,12 +621,17 @@ hipError_t run_bpr_route(const void* gate, int S0, int E, int C, int M, int n_pa
   a.used_out = used_out;
   a.elems_out = elems_out;
   hipError_t err = hipSuccess;
+  a.placed_by_expert = !force_lookback && S0 <= kPlaceTokens;
   // (an empty batch still runs one tile, which leaves empty groups for the select kernel)
   const SelectLaunch sel = select_launch(gate_dtype, gate, nullptr, S0, E, is_logits);
   LANCET_SELECT_SWITCH(gate_dtype, sel.form, (bpr_prepare_kernel<GD, FORM><<<a.ntiles0, sel.threads, std::max(scan_lds_bytes(E), sel.lds), st>>>(gate, is_logits, a)))
   err = hipGetLastError();
   if (err != hipSuccess) return err;
-  bpr_select_kernel<<<E, kSelectThreads, 0, st>>>(a);
+  if (a.placed_by_expert) {
+    bpr_select_kernel<true><<<E, kSelectThreads, 0, st>>>(a);
+    return hipGetLastError();
+  }
+  bpr_select_kernel<false><<<E, kSelectThreads, 0, st>>>(a);
   err = hipGetLastError();
   if (err != hipSuccess) return err;
   a.seg_rows = 0;
