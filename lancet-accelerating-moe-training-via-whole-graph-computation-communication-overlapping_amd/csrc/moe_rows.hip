@@ -27,14 +27,15 @@ __device__ __forceinline__ T ld_now(const T* p) {
 struct RowShare {
   int r, v, step;
 };
-__device__ __forceinline__ RowShare row_share(int q) {
-  const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kTile + threadIdx.x;
+__device__ __forceinline__ RowShare row_share(int q, uint32_t block) {
+  const uint64_t t = static_cast<uint64_t>(block) * kTile + threadIdx.x;
   RowShare h;
   h.r = static_cast<int>(t >> q);
   h.step = 1 << q;
   h.v = static_cast<int>(static_cast<uint32_t>(t) & static_cast<uint32_t>(h.step - 1));
   return h;
 }
+__device__ __forceinline__ RowShare row_share(int q) { return row_share(q, blockIdx.x); }
 // sum over the row's lanes inside a wave
 __device__ __forceinline__ float share_sum(float x, int q) {
   if (q >= 6) return wave_sum(x);
@@ -116,14 +117,25 @@ struct ScatterArgs {
   int q;                      // 2^q lanes share one token row
   int token_blocks;
   int tail_chunks;            // tail workgroups per expert
+  int tail_groups;            // eights of tail workgroups that stand among the tokens', 0 = all stand behind them
+  int tail_every;             // ... one in this many eights
 };
+
+constexpr int kXcds = 8;  // workgroups go round them: what comes in turns comes in eights, or a few XCDs do all of it
 
 template <int MODE, int K, bool DEST = false>
 __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
   typedef Granule<MODE> G;
   typedef typename G::V V;
-  if (static_cast<int>(blockIdx.x) < a.token_blocks) {
-    const RowShare h = row_share(a.q);
+  int token = static_cast<int>(blockIdx.x), tail = token - a.token_blocks;  // tail: negative in a workgroup of tokens
+  if (a.tail_groups) {
+    const int eight = token / kXcds, turn = eight / a.tail_every;
+    const bool clears = turn < a.tail_groups && eight - turn * a.tail_every == a.tail_every - 1;
+    tail = clears ? turn * kXcds + token % kXcds : -1;
+    token -= kXcds * min(turn, a.tail_groups);
+  }
+  if (tail < 0) {
+    const RowShare h = row_share(a.q, static_cast<uint32_t>(token));
     const int s = h.r, step = h.step;
     int v = h.v;
     if (s >= a.S) return;
@@ -184,20 +196,22 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
         if (j < nd) G::st(dst[j] + o, x);
     }
   } else {
-    // tail: zero rows [used, C) of expert e, kTailRows rows per workgroup
-    const int tb = blockIdx.x - a.token_blocks;
-    const int e = tb / a.tail_chunks;
-    const int ch = tb - e * a.tail_chunks;
+    // tail: zero rows [used, C) of expert e, kTailRows rows per workgroup and turn
+    const int e = tail / a.tail_chunks;
+    const int ch = tail - e * a.tail_chunks;
+    if (e >= a.E) return;  // the last eight may be more than there are
     const int used = a.rows_hi[e] - (a.rows_lo ? a.rows_lo[e] : 0);
-    const int first = max(used, 0) + ch * kTailRows;
-    const int last = min(first + kTailRows, a.C);
     // the rows lie one behind the other: one run of granules, or one per row where the run's length takes more than 32 bits
-    const int rows = a.row_bytes <= 0xffffffffu / kTailRows ? kTailRows : 1;
-    for (int r = first; r < last; r += rows) {
-      LANCET_GLOBAL char* run = as_global(a.out + (static_cast<size_t>(e) * a.C + r) * a.row_bytes);
-      const uint32_t bytes = static_cast<uint32_t>(min(rows, last - r)) * a.row_bytes;
-      const uint32_t n = static_cast<uint32_t>((bytes + sizeof(V) - 1) / sizeof(V));
-      for (uint32_t v = threadIdx.x; v < n; v += kTile) G::st(run + G::at(v, bytes), G::zero());
+    const uint32_t rows = a.row_bytes <= 0xffffffffu / kTailRows ? kTailRows : 1;
+    const uint32_t C = static_cast<uint32_t>(a.C), stride = static_cast<uint32_t>(a.tail_chunks) * kTailRows;
+    for (uint32_t first = static_cast<uint32_t>(max(used, 0)) + static_cast<uint32_t>(ch) * kTailRows; first < C; first += stride) {
+      const uint32_t last = min(first + kTailRows, C);
+      for (uint32_t r = first; r < last; r += rows) {
+        LANCET_GLOBAL char* run = as_global(a.out + (static_cast<size_t>(e) * a.C + r) * a.row_bytes);
+        const uint32_t bytes = min(rows, last - r) * a.row_bytes;
+        const uint32_t n = static_cast<uint32_t>((bytes + sizeof(V) - 1) / sizeof(V));
+        for (uint32_t v = threadIdx.x; v < n; v += kTile) G::st(run + G::at(v, bytes), G::zero());
+      }
     }
   }
 }
@@ -1053,7 +1067,14 @@ hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, con
   a.q = row_lanes(a.row_vecs, S, 1);
   a.token_blocks = static_cast<int>(row_blocks(S, a.q));
   a.tail_chunks = rows_hi ? (C + kTailRows - 1) / kTailRows : 0;
-  const long blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_chunks) * E;
+  a.tail_groups = a.tail_every = 0;
+  long blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_chunks) * E;
+  if (a.tail_chunks && a.token_blocks && E <= kMixedTails && mode == kWhole16 && (K == 2 || row_bytes <= kMixedTop1Bytes)) {
+    a.tail_chunks = std::min(a.tail_chunks, kMixedTails / E);
+    a.tail_groups = (a.tail_chunks * E + kXcds - 1) / kXcds;
+    blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_groups) * kXcds;
+    a.tail_every = static_cast<int>(blocks / kXcds / a.tail_groups);
+  }
   if (blocks == 0) return hipSuccess;
   const size_t lds = a.row_vecs > kWave ? kScatterLds : 0;
   if (dest) {
