@@ -860,7 +860,8 @@ struct DecodeGradArgs {
   int tail_chunks;         // such workgroups per expert
 };
 
-template <int DT, int K, int MODE>
+// EARLY: every lane has granules of its token for two turns and more; the first two are asked for before the routing words.
+template <int DT, int K, int MODE, bool EARLY>
 __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
   typedef Codec<DT> Cd;
   typedef Granule<MODE> G;
@@ -898,6 +899,13 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
 #pragma unroll
   for (int j = 0; j < K; ++j) acc[j] = 0.f;
   if (s < a.S) {
+    const char* dy = a.dy + static_cast<size_t>(s) * a.row_bytes;
+    int v = h.v;
+    u32x4 early[2];
+    if constexpr (EARLY) {
+      early[0] = G::ld(dy + G::at(v, a.row_bytes));
+      early[1] = G::ld(dy + G::at(v + step, a.row_bytes));
+    }
     RowWords<K> words;
     words.load(a.idx, a.loc, a.gates, a.gate_dtype, a.S, s);
     bool ok[K];
@@ -912,8 +920,6 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
       dst[j] = as_global(a.d_expert_out + at);
       any = any || ok[j];
     }
-    const char* dy = a.dy + static_cast<size_t>(s) * a.row_bytes;
-    int v = h.v;
     if constexpr (MODE == kWhole16 || MODE == kAny16) {
       // two granules of the token and of each slot's row in flight
       for (; any && v < a.row_vecs; v += 2 * step) {
@@ -923,7 +929,8 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
           d[b] = G::zero();
-          if (b == 0 || two) d[b] = G::ld(dy + o[b]);
+          if (EARLY && v == h.v) d[b] = early[b];
+          else if (b == 0 || two) d[b] = G::ld(dy + o[b]);
 #pragma unroll
           for (int j = 0; j < K; ++j) {
             x[b][j] = G::zero();
@@ -1037,6 +1044,17 @@ static inline int row_granules(RowMode mode, size_t row_bytes, int elem_bytes) {
 // 2048.  Rows of one wave want every slot: 90 / 92 / 99 / 108 us at 262144 x 512.  The gather kernels do not gain.
 constexpr size_t kCuLds = 160 * 1024;
 constexpr size_t kScatterLds = kCuLds / 6 + 1;  // six do not fit, however LDS is rounded up; five do
+
+// Where the workgroups that clear the experts' tails stand.  Behind the tokens' they are an end of the launch that only
+// writes, or, where nearly all find nothing to clear, a row of empty starts; among them both hide behind the rows' traffic.
+// Behind / among, us for the whole encode: 16384 x 1024 fp32 top-2, 16 experts, some hot, 40.8 / 36.4; 8192 x 4096 bf16 top-2 44.2 /
+// 42.5, 16384 x 8192 173.1 / 169.8; 20000 x 3072 fp16, capacity 2, 125.5 / 122.8; 131072 x 512 88.8 / 85.6; 65536 x 4096
+// 333.6 / 333.4; top-1 32768 x 2048, some hot, 64.0 / 60.0, 12000 x 768 fp32, capacity 2, 26.1 / 22.4, 262144 x 512, some hot, 115.8 /
+// 113.3.  Not for top-1 rows of more than 4 KB, whose reads and writes are in balance without (65536 x 4096 211.2 / 214.0, 20000 x
+// 3072 62.1 / 66.6), nor for rows that end inside a granule (10007 x 1003 bf16 24.8 / 25.6).  At most kMixedTails of them,
+// each then with several turns: one eight in four at 65536 x 1024 93.2, one in five 90.0 (behind: 91.3).
+constexpr size_t kMixedTop1Bytes = 4096;
+constexpr int kMixedTails = 8192;
 
 hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, const int32_t* loc,
                             const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
@@ -1245,6 +1263,8 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
 constexpr int kScanSlots = 8192;
 constexpr int kGradTailRows = 16;  // rows per clearing workgroup with the inverse map
 constexpr int kGradScanRows = 64;  // ... that walks the slots
+constexpr size_t kGradWideLds = kCuLds / 5 + 1;  // five workgroups do not fit, four do
+constexpr size_t kMemoryCache = size_t(256) << 20;  // what the cache in front of the HBM holds
 
 template <int DT>
 static hipError_t decode_grad_launch(DecodeGradArgs a, int K, int M, RowMode mode, hipStream_t st) {
@@ -1259,12 +1279,22 @@ static hipError_t decode_grad_launch(DecodeGradArgs a, int K, int M, RowMode mod
   a.tail_chunks = (a.C + a.tail_rows - 1) / a.tail_rows;
   const unsigned blocks = static_cast<unsigned>(a.token_blocks + static_cast<long>(a.tail_chunks) * a.E);
   if (blocks == 0) return hipSuccess;
-  // top-1 rows of several waves: as in the scatter, 317 against 329 us at 65536 x 4096 bf16 (top-2 577 / 581, 52 / 51 at
-  // 16384 x 1024 fp32; rows of one wave 182 / 151)
-  const size_t lds = K == 1 && a.q > 6 ? kScatterLds : 0;
+  // top-1 rows of several waves: as in the scatter, 317 against 329 us at 65536 x 4096 bf16 (rows of one wave 182 / 151).
+  // top-2 rows with more granules than a workgroup has lanes, of which a lane keeps twice the loads in flight, in passes that
+  // come from the HBM: four workgroups on a CU instead of eight (20000 x 3072 bf16 122 against 126 us; rows of 4 KB 157 / 137, 66 / 49
+  // at 16384 x 1024 fp32), and where all lanes have two granules of it the token's row is asked for before the routing words: both
+  // together 549 / 570 at 65536 x 4096, 156 / 165 at 20000, 96 / 101 at 12000, 51.3 / 52.7 at 6000.  In the cache neither pays (4200 x
+  // 4096 with half as many rows kept 29 / 25), nor the latter for rows of 384 granules (158 / 153) or top-1 (20000 x 4096 92 / 90).
+  const bool wide = K == 2 && mode == kWhole16 && a.row_vecs > kTile &&
+                    (static_cast<size_t>(a.S) + 2 * static_cast<size_t>(a.E) * a.C) * a.row_bytes > kMemoryCache;
+  const size_t lds = wide ? kGradWideLds : K == 1 && a.q > 6 ? kScatterLds : 0;
+  if (wide && a.row_vecs >= 2 * kTile) {
+    decode_grad_kernel<DT, 2, kWhole16, true><<<blocks, kTile, lds, st>>>(a);
+    return hipGetLastError();
+  }
   LANCET_CODED_ROW_SWITCH(DT, mode,
-    if (K == 1) decode_grad_kernel<DT, 1, MODE><<<blocks, kTile, lds, st>>>(a);
-    else decode_grad_kernel<DT, 2, MODE><<<blocks, kTile, 0, st>>>(a))
+    if (K == 1) decode_grad_kernel<DT, 1, MODE, false><<<blocks, kTile, lds, st>>>(a);
+    else decode_grad_kernel<DT, 2, MODE, false><<<blocks, kTile, lds, st>>>(a))
   return hipGetLastError();
 }
 
