@@ -279,10 +279,10 @@ __device__ __forceinline__ void st_lowp1(LANCET_GLOBAL uint16_t* p, float x) {
 }
 
 // ---- the three phases on one chunk, executed by one workgroup ------------------------------
-// phase 1: sum of squares of g (L2NormFunctor, multi_tensor_lans.cu:95-167); valid on thread 0.
+// phase 1: squares of g (L2NormFunctor, multi_tensor_lans.cu:95-167), the share of thread tid of kLansThreads.
 // (The sum of squares of p is not needed before phase 3 and is taken in phase 2, which reads p anyway.)
 template <int GT>
-__device__ __forceinline__ float chunk_norm_g(const LansTables& t, const ChunkView& c, float* s_red) {
+__device__ __forceinline__ float chunk_squares_g(const LansTables& t, const ChunkView& c, int tid) {
   typedef Grad<GT> G;
   const LANCET_GLOBAL typename G::S* g = as_global(static_cast<const typename G::S*>(t.g[c.tensor]) + c.begin);
   float ag = 0.f;
@@ -290,17 +290,17 @@ __device__ __forceinline__ float chunk_norm_g(const LansTables& t, const ChunkVi
   if (((uintptr_t)g & G::kAlign4) == 0) {
     const int nv = c.n / 4;
 #pragma unroll 8
-    for (int i = threadIdx.x; i < nv; i += kLansThreads) {
+    for (int i = tid; i < nv; i += kLansThreads) {
       const f32x4 x = G::ld4(g + 4 * i);
       ag += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
     }
     scalar_from = nv * 4;
   }
-  for (int i = scalar_from + threadIdx.x; i < c.n; i += kLansThreads) {
+  for (int i = scalar_from + tid; i < c.n; i += kLansThreads) {
     const float x = G::ld1(g + i);
     ag += x * x;
   }
-  return block_sum(ag, s_red);
+  return ag;
 }
 
 // phase 2: moments + sums of squares of p and of the two updates (LANSStage1Functor :207-322 and the
@@ -438,8 +438,8 @@ __device__ __forceinline__ ChunkView slice_view(const LansTables& t, int chunk_b
 }
 
 // The sweep over g covers chunks [chunk_base, chunk_base + gridDim.x), the other two
-// [chunk_base, chunk_base + gridDim.x / kSweepSplit): all of them, or the ones the resident
-// kernel takes (first sweep only), or the ones it leaves (tensors too large for it).
+// [chunk_base, chunk_base + gridDim.x / kSweepSplit): all of them, or the ones the resident kernel leaves (tensors too
+// large for it).  Up to kEarlyNorms chunks are summed by the first kernel instead.
 template <int GT>
 __global__ __launch_bounds__(kLansThreads) void lans_norm_g_kernel(LansTables t, int chunk_base) {
   __shared__ float s_red[kLansThreads / kWave];
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(kLansThreads) void lans_norm_g_kernel(LansTables t,
   const int chunk = chunk_base + blockIdx.x;  // a whole chunk per workgroup: this sweep only reads, and splitting it costs more in reductions than it gains
   const ChunkView c = chunk_view(t, chunk);
   if (c.tensor < 0) return;  // padding slot (uniform over the workgroup)
-  const float sg = chunk_norm_g<GT>(t, c, s_red);
+  const float sg = block_sum(chunk_squares_g<GT>(t, c, threadIdx.x), s_red);
   if (threadIdx.x == 0) t.partial[chunk] = sg;
 }
 
@@ -1218,10 +1218,17 @@ __device__ __forceinline__ void small_step(const LansTables& t, const LansScalar
 // registers are all spoken for) and brings the caller's gradient norms into the plan's order.  The epoch lives on the
 // device so that a step recorded in a graph tags every replay differently; when it wraps (2^31 steps) every word of
 // earlier steps is forgotten.  The error word is left alone.
-// The other workgroups update one small tensor each; they look at the error word itself, which no workgroup of this
-// launch writes.
+// The workgroups behind it update one small tensor each, those behind them sum the squares of g over kNormChunks chunks each of
+// the tensors that go through the sweeps; both look at the error word itself, which no workgroup of this launch writes.
+// (In a launch of their own behind the resident kernel the sums took 11 us of a step of 60M parameters of which a table of 20M
+// is swept, 398 us, now 391; here they fill a chip that the small tensors' dependent round trips leave idle.  40M fp32 parameters
+// by sweeps 329 / 322.  Of many chunks the sweep is as fast as the memory only with more waves than this kernel's registers
+// allow: 60M in one tensor 508 in a launch of their own against 515, 400M in 16 tensors 3237 / 3254.)
+constexpr int kEarlyNorms = 6144;
+constexpr int kNormChunks = kSmallThreads / kLansThreads;
 template <int GT, int PL>
-__global__ __launch_bounds__(kSmallThreads) void lans_begin_kernel(LansTables t, LansScalars sc, size_t nwords, int small_base) {
+__global__ __launch_bounds__(kSmallThreads) void lans_begin_kernel(LansTables t, LansScalars sc, size_t nwords, int small_base,
+                                                                   int norm_slot, int norm_slot_end) {
   __shared__ double s_red[3 * kSmallThreads / kWave];
   __shared__ float s_bc[2];
   const bool skip = ld_agent(t.ctl + kCtlError) != 0u;
@@ -1243,6 +1250,24 @@ __global__ __launch_bounds__(kSmallThreads) void lans_begin_kernel(LansTables t,
   }
   if (skip) return;
   const int tensor = small_base + static_cast<int>(blockIdx.x) - 1;
+  if (tensor >= t.T) {
+    __shared__ float s_sum[kSmallThreads / kWave];
+    const int part = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kLansThreads), tid = threadIdx.x % kLansThreads;
+    const int chunk = norm_slot + (tensor - t.T) * kNormChunks + part;
+    ChunkView c;
+    c.tensor = -1;  // a padding slot too
+    if (chunk < norm_slot_end) c = chunk_view(t, chunk);
+    const float squares = wave_sum(c.tensor >= 0 ? chunk_squares_g<GT>(t, c, tid) : 0.f);
+    if (lane_id() == 0) s_sum[threadIdx.x / kWave] = squares;
+    __syncthreads();
+    if (tid == 0 && c.tensor >= 0) {
+      float sum = 0.f;
+#pragma unroll
+      for (int k = 0; k < kWavesPerTile; ++k) sum += s_sum[part * kWavesPerTile + k];
+      t.partial[chunk] = sum;
+    }
+    return;
+  }
   if (threadIdx.x == 0) bias_corrections(sc, s_bc[0], s_bc[1]);
   __syncthreads();
   const float bc1 = s_bc[0], bc2 = s_bc[1];
@@ -1683,18 +1708,18 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   pl->last_resident_slots = t.nres;
   const int sweep_tensor = resident ? pl->big_first : 0, sweep_slot = resident ? pl->big_slot : 0;
   const int sweep_tensor_end = ragged ? pl->ragged_first : pl->small_first, sweep_slot_end = ragged ? pl->ragged_slot : pl->small_slot;
-  LANS_TYPE_SWITCH(g_dtype, plt, (lans_begin_kernel<GT, PL><<<1 + (T - pl->small_first), kSmallThreads, 0, st>>>(
-                                     t, sc, pl->words_bytes / sizeof(uint64_t), pl->small_first)))
+  const int nsweep = sweep_slot_end - sweep_slot, rest = sweep_tensor_end - sweep_tensor;
+  const int norm_blocks = grad_norms || nsweep <= 0 || nsweep > kEarlyNorms ? 0 : (nsweep + kNormChunks - 1) / kNormChunks;
+  LANS_TYPE_SWITCH(g_dtype, plt, (lans_begin_kernel<GT, PL><<<1 + (T - pl->small_first) + norm_blocks, kSmallThreads, 0, st>>>(
+                                     t, sc, pl->words_bytes / sizeof(uint64_t), pl->small_first, sweep_slot, sweep_slot_end)))
   if (t.nres > 0) {
     const int grid = std::min(pl->resident_grid, t.nres);
     LANS_TYPE_SWITCH(g_dtype, plt, (lans_resident_kernel<GT, PL><<<grid, kLansThreads, 0, st>>>(t, sc)))
   }
-  const int nsweep = sweep_slot_end - sweep_slot, rest = sweep_tensor_end - sweep_tensor;
   if (nsweep > 0) {
-    if (!grad_norms) {
+    if (!grad_norms && nsweep > kEarlyNorms)
       LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_norm_g_kernel<GT><<<nsweep, kLansThreads, 0, st>>>(t, sweep_slot)))
-      lans_reduce_kernel<<<dim3(rest, 1), kReduceThreads, 0, st>>>(t, 0, sweep_tensor, 1);
-    }
+    if (!grad_norms) lans_reduce_kernel<<<dim3(rest, 1), kReduceThreads, 0, st>>>(t, 0, sweep_tensor, 1);
     LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_moments_kernel<GT><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, sweep_slot)))
     lans_reduce_kernel<<<dim3(rest, 3), kReduceThreads, 0, st>>>(t, 1, sweep_tensor, kSweepSplit);
     LANS_TYPE_SWITCH(g_dtype, plt, (lans_update_kernel<GT, PL><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, sweep_slot)))
