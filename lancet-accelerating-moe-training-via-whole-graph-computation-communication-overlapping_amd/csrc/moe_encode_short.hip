@@ -7,7 +7,6 @@
 
 namespace lancet {
 
-constexpr int kShortTailRows = 16;  // rows cleared by one tail workgroup
 
 struct EncodeArgs {
   RouteArgs r;
@@ -17,7 +16,9 @@ struct EncodeArgs {
   int q;              // 2^q lanes of a workgroup share one token row
   int tokens;         // tokens per workgroup: a power of two, kTile at most
   int token_blocks;
-  int tail_chunks;    // workgroups per expert that clear the rows behind the used ones (0: nobody does)
+  int tail_rows;      // rows that a tail workgroup clears in a turn
+  int tail_chunks;    // turns that clear an expert's rows if none is used (0: nobody clears them)
+  int tail_blocks;    // workgroups that clear: one tile: of all experts; a few tiles: of each expert
   int rows_at_used;   // rows start behind those that earlier calls used
   int needs_setup;    // the outputs are marked where the workspace was never set up
 };
@@ -100,14 +101,17 @@ __device__ __forceinline__ int buffer_row(const EncodeArgs& a, int e, int l) {
   return l < a.r.C ? e * a.r.C + l : -1;
 }
 
-// rows [used, C) of one expert, kShortTailRows of them per workgroup; total = tokens of the batch that chose it, used_before =
-// rows of earlier calls (0 where this call's rows start behind them: they are in the buffer already)
-__device__ __forceinline__ void clear_tail(const EncodeArgs& a, int e, int chunk, int64_t total, bool marked) {
+// the first of an expert's rows that is to be cleared; total = tokens of the batch that chose it (rows of earlier calls are in
+// the buffer already where this call's start behind them)
+__device__ __forceinline__ int64_t tail_start(const EncodeArgs& a, int e, int64_t total, bool marked) {
   const int64_t used_in = a.r.used_in ? a.r.used_in[e] : 0;
   const int64_t used_out = min(used_in + total, static_cast<int64_t>(a.r.C));
-  const int64_t used = marked ? 0 : used_out - (a.rows_at_used ? 0 : used_in);
-  const int first = static_cast<int>(max(used, static_cast<int64_t>(0))) + chunk * kShortTailRows;
-  const int last = min(first + kShortTailRows, a.r.C);
+  return marked ? 0 : max(used_out - (a.rows_at_used ? 0 : used_in), static_cast<int64_t>(0));
+}
+// a turn: tail_rows rows of the expert's tail, which starts at row `from`
+__device__ __forceinline__ void clear_tail(const EncodeArgs& a, int e, int64_t from, int chunk) {
+  const int64_t first = from + static_cast<int64_t>(chunk) * a.tail_rows;
+  const int64_t last = min(first + a.tail_rows, static_cast<int64_t>(a.r.C));
   if (first >= last) return;
   LANCET_GLOBAL char* run = as_global(a.out + (static_cast<size_t>(e) * a.r.C + first) * a.row_bytes);
   const size_t bytes = static_cast<size_t>(last - first) * a.row_bytes;
@@ -173,8 +177,13 @@ __global__ __launch_bounds__(kSelectThreadsOf<FORM>) void encode_tile_kernel(Enc
   tile_scan<K, false>(e, mem, r.E, me, r.ws, s_cnt, rank);
   const uint32_t* totals = s_cnt + kWavesPerTile * K * r.E;
   if (!mover) {
-    const int tb = static_cast<int>(blockIdx.x) - a.token_blocks, x = tb / a.tail_chunks;
-    clear_tail(a, x, tb - x * a.tail_chunks, static_cast<int64_t>(totals[x]) + (K == 2 ? totals[r.E + x] : 0u), marked);
+    // (turns are no more than rows of the buffer, which 31 bits count)
+    const uint32_t chunks = static_cast<uint32_t>(a.tail_chunks), turns = chunks * static_cast<uint32_t>(r.E);
+    for (uint32_t turn = blockIdx.x - static_cast<uint32_t>(a.token_blocks); turn < turns; turn += static_cast<uint32_t>(a.tail_blocks)) {
+      const int x = static_cast<int>(turn / chunks);
+      const int64_t total = static_cast<int64_t>(totals[x]) + (K == 2 ? totals[r.E + x] : 0u);
+      clear_tail(a, x, tail_start(a, x, total, marked), static_cast<int>(turn - static_cast<uint32_t>(x) * chunks));
+    }
     return;
   }
   if (tid < r.S) {
@@ -229,7 +238,7 @@ __global__ __launch_bounds__(kTile) void encode_place_rows_kernel(EncodeArgs a) 
   const bool marked = not_set_up(a);
   if (static_cast<int>(blockIdx.x) >= a.token_blocks) {
     // the totals of one expert
-    const int tb = static_cast<int>(blockIdx.x) - a.token_blocks, x = tb / a.tail_chunks;
+    const int tb = static_cast<int>(blockIdx.x) - a.token_blocks, x = tb / a.tail_blocks;
     const int PP = count_pairs(NC);
     uint32_t t = 0;
     for (int i = tid; i < K * r.ntiles; i += kTile) {
@@ -241,7 +250,8 @@ __global__ __launch_bounds__(kTile) void encode_place_rows_kernel(EncodeArgs a) 
     __syncthreads();
     if (t) atomicAdd(&s_sum[0], t);
     __syncthreads();
-    clear_tail(a, x, tb - x * a.tail_chunks, s_sum[0], marked);
+    const int64_t from = tail_start(a, x, s_sum[0], marked);
+    for (int chunk = tb - x * a.tail_blocks; chunk < a.tail_chunks; chunk += a.tail_blocks) clear_tail(a, x, from, chunk);
     return;
   }
   const int first = static_cast<int>(blockIdx.x) * a.tokens, n = min(a.tokens, r.S - first);
@@ -312,6 +322,19 @@ constexpr size_t kShortRows1 = 64u << 20, kShortRows2 = 12u << 20;  // bytes of 
 // 13.8 / 13.8 / 11.7 / 11.7 us, 6000 x 1024 12.6 / 10.9 / 10.9 / 9.7 (separate kernels 12.8), 4096 x 4096 20.5 / 20.4 / 20.1 / 20.1; top-2
 // 8192 x 512 12.4 / 12.4 / 13.6 / 13.6, 6000 x 1024 16.6 / 13.7 / 13.7 / 15.1.
 constexpr int kShortBlocks1 = 1536, kShortBlocks2 = 768;
+// Tails.  A turn clears 32 KB, 16 rows at least.  Of one tile, every workgroup that clears has to route the tile first, so there
+// are only as many as the movers leave CUs idle, each with several turns; a second one on a CU costs the routing again (256 x
+// 1024 top-2, 128 experts, capacity 20: 10.9 us with 192 of them beside 64 movers, 15.9 with 256), and one per 16 rows, as many as
+// the buffer has, made the capacity the bound: separate kernels / one workgroup per turn of 16 rows / now, us: 256 x 64 top-1, 128
+// experts, capacity 256 14.2 / 39.4 / 7.8, 4096 33.6 / 530 / 18.2; 256 x 1024 top-2, 128 experts, capacity 256 28.7 / 58.9 / 20.2, 4096
+// 209 / 744 / 204; 64 x 64 top-2, 128 experts, capacity 128 15.2 / 18.4 / 7.5; 1 x 1024 top-2, 512 experts 36.1 / 47.2 / 34.6.  (fp32 logits of
+// more than 256 experts for 17 to 32 tokens run faster with two on a CU, 32 x 1024 top-1 23.2 / 26.9, and for 16 tokens slower,
+// 35.0 / 26.6: not understood.)  Of a few tiles, a workgroup adds up its expert's counts: 8192 x 64 top-1, 64 experts, capacity 8192
+// 31.7 / 52.5 / 19.4, 8192 x 1024, capacity 160 16.8 / 14.0 / 13.8.
+constexpr int kShortTailRows = 16;
+constexpr uint32_t kShortTailBytes = 32768;
+constexpr int kCus = 256, kTileTails = 128;  // (movers on every CU: half as many again)
+constexpr int kShortTails = 4096;            // of a few tiles, all experts together
 constexpr int kShortPerLane = 2;  // granules per lane (one: 6000 x 1024 top-1 12.3 us against 10.9, top-2 16.8 against 13.7)
 
 bool encode_is_short(const int32_t* used_in, const int32_t* used_out, int64_t S, int64_t E, int K, size_t row_bytes, bool force_lookback) {
@@ -339,10 +362,13 @@ hipError_t run_encode_short(const void* data, const void* gate, const void* nois
   a.tokens = kTile >> a.q;
   while (a.tokens < kTile && (S + a.tokens - 1) / a.tokens > (K == 1 ? kShortBlocks1 : kShortBlocks2)) a.tokens *= 2;
   a.token_blocks = (S + a.tokens - 1) / a.tokens;
-  a.tail_chunks = tail ? (C + kShortTailRows - 1) / kShortTailRows : 0;
+  a.tail_rows = std::max(kShortTailRows, static_cast<int>(kShortTailBytes / a.row_bytes));
+  a.tail_chunks = tail ? (C + a.tail_rows - 1) / a.tail_rows : 0;
+  const int64_t turns = static_cast<int64_t>(a.tail_chunks) * E;
+  a.tail_blocks = static_cast<int>(r.ntiles == 1 ? std::min<int64_t>(turns, std::max(kCus - a.token_blocks, kTileTails)) : std::min(a.tail_chunks, std::max(kShortTails / E, 1)));
   a.rows_at_used = rows_at_used && used_in != nullptr;
   a.needs_setup = scan_form(r.ntiles, static_cast<int64_t>(K) * E, K) == kScanLookback;
-  const unsigned blocks = static_cast<unsigned>(a.token_blocks + static_cast<long>(a.tail_chunks) * E);
+  const unsigned blocks = static_cast<unsigned>(a.token_blocks + (r.ntiles == 1 ? a.tail_blocks : a.tail_blocks * E));
   const int NC = K * E;
   if (r.ntiles == 1) {
     const SelectLaunch sel = select_launch(gate_dtype, gate, r.noise, S, E, is_logits);

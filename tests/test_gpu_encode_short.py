@@ -110,3 +110,23 @@ def test_selection_by_sixteen_waves(pkg, S, E, gdt):
         a = ops.moe_encode(dev(data), odd, None, float(E), top_k=2, gate_is_logits=is_logits)
         b = ops.moe_encode(dev(data), odd, None, float(E), top_k=2, gate_is_logits=is_logits, gate2_noise=torch.zeros_like(odd))
         np.testing.assert_array_equal(to_np(a[1]), to_np(b[1]))
+
+
+# buffers far larger than the load: turns of one expert (E = 2), of all (more experts than workgroups clear), an end of a turn off
+# the expert's last row, rows of less than a granule; a few tiles; more rows than one workgroup per turn could be launched for
+@pytest.mark.parametrize("S,M,E,C", [(1, 8, 2, 5000), (64, 24, 128, 700), (256, 1024, 128, 33), (256, 4104, 3, 300), (20, 3, 512, 129),
+                                     (256, 1, 128, (1 << 19) + 5), (300, 8, 60, 4096), (2000, 1024, 5, 2500), (8192, 2, 64, 9000)])
+@pytest.mark.parametrize("k", [1, 2])
+def test_tails_of_buffers_larger_than_the_load(pkg, S, M, E, C, k):
+    """Every row of the buffer as the separate kernels leave it, in memory that held something else."""
+    ops = pkg.ops
+    data, logits = make_inputs(S + C, S, M, E, zipf_bias=True)
+    d_data, gate = rows_to_torch(data, "bf16"), dev(logits)
+    used0 = torch.arange(E, dtype=torch.int32, device="cuda") % 3
+    for used, at_used in ((None, False), (used0, False), (used0, True)):
+        got, want = (ops.moe_encode(d_data, gate, used, top_k=k, gate_is_logits=True, capacity=C, rows_at_used=at_used, scan_lookback=separate,
+                                    out=[torch.empty(k * S, device="cuda"), torch.empty((2, k * S), dtype=torch.int32, device="cuda"),
+                                         torch.empty(E, dtype=torch.int32, device="cuda"), torch.empty(E, dtype=torch.int64, device="cuda"),
+                                         torch.full((E, C, M), 7.0, dtype=torch.bfloat16, device="cuda")]) for separate in (False, True))
+        for a, b in zip(got, want):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
