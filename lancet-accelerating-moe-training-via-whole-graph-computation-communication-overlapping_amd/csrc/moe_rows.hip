@@ -675,12 +675,19 @@ __global__ __launch_bounds__(kTile) void inverse_map_kernel(const int32_t* idx, 
   if (e >= 0 && e < E && l >= 0 && l < C) src[static_cast<size_t>(e) * C + l] = i;
 }
 
-// The slot-token that owns a row, or -1.  The map is not cleared beforehand (2 to 5 us and a launch in front of every backward
-// pass): an entry counts if the slot it names is routed to that row, which whatever else lies there is not.
-__device__ __forceinline__ int row_owner(const int32_t* src, size_t row, const int32_t* idx, const int32_t* loc, int n, int E, int C) {
+// The slot-token that owns a row, or -1.  A map that was not cleared beforehand is checked (kClearedRows): an entry counts if the
+// slot it names is routed to that row, which whatever else lies there is not.  f(i) asks for what else is needed of the slot named
+// together with its routing words: behind them it would be one more round trip in front of the row.
+template <typename F>
+__device__ __forceinline__ int row_owner(const int32_t* src, size_t row, const int32_t* idx, const int32_t* loc, int n, int E, int C, bool checked, F f) {
   const int i = src[row];
   if (i < 0 || i >= n) return -1;
+  if (!checked) {
+    f(i);
+    return i;
+  }
   const int e = idx[i], l = loc[i];
+  f(i);
   return e >= 0 && e < E && l >= 0 && l < C && static_cast<size_t>(e) * C + l == row ? i : -1;
 }
 
@@ -690,16 +697,16 @@ __device__ __forceinline__ int row_owner(const int32_t* src, size_t row, const i
 template <int DT, int MODE, int K>
 __global__ __launch_bounds__(kTile) void decode_dx_rows_kernel(const void* dy, const void* gates, int gd,
                                                                const int32_t* src, const int32_t* idx, const int32_t* loc,
-                                                               void* out, int S, int M, int E, int C, long rows, int q) {
+                                                               void* out, int S, int M, int E, int C, long rows, int q, bool checked) {
   typedef Codec<DT> Cd;
   const RowShare h = row_share(q);
   const long r = h.r;
   const int step = h.step;
   if (r >= rows) return;
-  const int i = row_owner(src, static_cast<size_t>(r), idx, loc, K * S, E, C);
   // the weight first, then the row: with both asked for at once the reads crowd out the writes here (262144 x 512 bf16
   // top-1: 83 against 90 us)
-  const float g1[1] = {i >= 0 ? ld_gate(gates, i, gd) : 0.f};
+  float g1[1] = {0.f};
+  const int i = row_owner(src, static_cast<size_t>(r), idx, loc, K * S, E, C, checked, [&](int slot) { g1[0] = ld_gate(gates, slot, gd); });
   const size_t s = i >= 0 ? static_cast<size_t>(i % S) : 0;
   if constexpr (MODE == kWhole16 || MODE == kAny16) {
     typedef Granule<MODE> G;
@@ -839,7 +846,7 @@ __global__ __launch_bounds__(kTile) void decode_dg_kernel(const void* dy, const 
 // Same products and roundings as decode_dx; the dot products of rows of more than 64 granules are summed in another order
 // than decode_dg's.
 // Workgroups behind the tokens' clear the rows no slot owns.  Which those are, they look up in the inverse map
-// (decode_dx) or, in short batches, find out themselves by walking all slots, which saves the two launches that make
+// (decode_dx) or, in short batches, find out themselves by walking all slots, which saves the launch that makes
 // the map (kScanSlots below).
 // ---------------------------------------------------------------------------------------
 struct DecodeGradArgs {
@@ -851,12 +858,13 @@ struct DecodeGradArgs {
   const int32_t* owner;    // [E*C] slot-token that owns a row (row_owner); null: walk the slots
   char* d_expert_out;      // [E, C, M]
   void* d_gates;           // [K*S] of gate_dtype
+  int checked;             // the map was not cleared
   int S, E, C, gate_dtype;
   uint32_t row_bytes;
   int row_vecs;            // granules per row
   int q;                   // 2^q lanes of one workgroup share a token
   int token_blocks;
-  int tail_rows;           // rows looked at by one workgroup behind the tokens' (at most 32 * kTile)
+  int tail_rows;           // rows looked at by one workgroup behind the tokens' (at most 32 * kTile; kWave with a map)
   int tail_chunks;         // such workgroups per expert
 };
 
@@ -884,10 +892,19 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
       __syncthreads();
     }
     const int q = min(a.q, 6);
+    const auto mapped = [&](int r) {
+      return row_owner(a.owner, static_cast<size_t>(e) * a.C + r, a.idx, a.loc, K * a.S, a.E, a.C, a.checked, [](int) {}) >= 0;
+    };
+    // where a wave has several rows one after the other, it looks all up at once: one chain of round trips instead of one per row
+    // (65536 x 512 bf16 top-2 73.8 -> 71.1 us, 262144 x 512 top-1 173 -> 168)
+    const bool at_once = a.owner && (kTile >> q) < a.tail_rows;
+    uint64_t owned_rows = 0;
+    if (at_once) owned_rows = __ballot(first + lane < last && mapped(first + lane));
     for (int r = first + (static_cast<int>(threadIdx.x) >> q); r < last; r += kTile >> q) {
-      const size_t row = static_cast<size_t>(e) * a.C + r;
-      const bool owned = a.owner ? row_owner(a.owner, row, a.idx, a.loc, K * a.S, a.E, a.C) >= 0 : ((s_owned[(r - first) >> 5] >> ((r - first) & 31)) & 1u) != 0;
+      const int at = r - first;
+      const bool owned = at_once ? (owned_rows >> at) & 1u : a.owner ? mapped(r) : (s_owned[at >> 5] >> (at & 31)) & 1u;
       if (owned) continue;
+      const size_t row = static_cast<size_t>(e) * a.C + r;
       LANCET_GLOBAL char* dst = as_global(a.d_expert_out + row * a.row_bytes);
       for (int v = threadIdx.x & ((1 << q) - 1); v < a.row_vecs; v += 1 << q) G::st(dst + G::at(v, a.row_bytes), G::zero());
     }
@@ -1219,6 +1236,12 @@ hipError_t run_encode_dg(const void* dy, const int32_t* idx, int S, int E, int K
   return hipGetLastError();
 }
 
+// Rows of the buffer up to which the map is checked instead of cleared.  Clearing is a launch of 2 to 3 us, checking two words more to
+// gather per row.  Cleared / checked, us: moe_decode_dx 16384 x 64 bf16 top-1 (20480 rows) 7.8 / 6.1, 32768 x 2048 (40960) 59.0 / 58.0,
+// 65536 x 64 (81920) 10.7 / 9.0; 131072 x 16 (163840) 10.9 / 10.3, x 64 16.0 / 16.5; 262144 x 64 (327680) 25.9 / 27.3, x 512 111.1 /
+// 109.6, 1000000 x 64 80.3 / 95.4; moe_decode_grad 65536 x 1024 82.0 / 80.2, 262144 x 64 35.4 / 35.8.
+constexpr long kClearedRows = 131072;
+
 template <int DT>
 static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, const int32_t* idx,
                                    const int32_t* loc, void* out, int S, int M, int E, int C, int K, RowMode mode, hipStream_t st) {
@@ -1228,13 +1251,17 @@ static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, co
   const int q = row_lanes(units, rows, few_granules(units, rows) && units <= kWave ? 1 : 2);  // two granules per lane: 442 -> 408 us
   const unsigned blocks = static_cast<unsigned>(row_blocks(rows, q));
   LANCET_CODED_ROW_SWITCH(DT, mode,
-    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, idx, loc, out, S, M, E, C, rows, q);
-    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, idx, loc, out, S, M, E, C, rows, q))
+    if (K == 1) decode_dx_rows_kernel<DT, MODE, 1><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, idx, loc, out, S, M, E, C, rows, q, rows <= kClearedRows);
+    else decode_dx_rows_kernel<DT, MODE, 2><<<blocks, kTile, 0, st>>>(dy, gates, gd, src, idx, loc, out, S, M, E, C, rows, q, rows <= kClearedRows))
   return hipGetLastError();
 }
 
 // the inverse map (row_owner)
 static hipError_t run_inverse_map(const int32_t* idx, const int32_t* loc, int n, int E, int C, int32_t* src, hipStream_t st) {
+  if (static_cast<long>(E) * C > kClearedRows) {
+    const hipError_t err = run_fill_u32(reinterpret_cast<uint32_t*>(src), static_cast<size_t>(E) * C, 0xffffffffu, st);
+    if (err != hipSuccess) return err;
+  }
   if (n == 0) return hipSuccess;
   inverse_map_kernel<<<(n + kTile - 1) / kTile, kTile, 0, st>>>(idx, loc, n, E, C, src);
   return hipGetLastError();
@@ -1256,11 +1283,10 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
 }
 
 // Slots up to which the clearing workgroups of decode_grad_kernel walk all of them themselves instead of looking rows up in
-// a map that two launches before it make.  Map / walk by workgroups of 64 rows, us: 1024 slots, 4 to 512 experts, rows of 64
-// bf16 6.3 / 3.0; 4096 slots 6.6 / 4.5, rows of 2048 14.6 / 14.5 with 4 experts and 14.6 / 12.1 with 512; 8192 slots 7.0 / 7.1,
-// rows of 2048 23.3 / 24.7 and 24.0 / 23.3; 12000 slots 7.2 / 9.6.  (128 rows per workgroup: those that have rows to clear
-// become the launch's end, 18.1 us for the 14.5 above.)
-constexpr int kScanSlots = 8192;
+// a map that the launch before it makes.  Map / walk by workgroups of 64 rows, us: 1024 slots, rows of 64 bf16, 4 experts 4.6 /
+// 2.9 and 512 experts 4.9 / 3.0, rows of 2048 6.7 / 8.2 and 6.5 / 4.5; 4096 slots 5.0 / 4.3, 5.3 / 4.9, 13.0 / 15.1 and 12.7 / 11.2; 6000 slots
+// 5.2 / 5.5, 5.6 / 6.3, 16.0 / 19.1 and 16.1 / 15.5; 8192 slots 5.3 / 7.0, 5.6 / 7.5, 19.2 / 22.8 and 20.2 / 20.4.
+constexpr int kScanSlots = 4096;
 constexpr int kGradTailRows = 16;  // rows per clearing workgroup with the inverse map
 constexpr int kGradScanRows = 64;  // ... that walks the slots
 constexpr size_t kGradWideLds = kCuLds / 5 + 1;  // five workgroups do not fit, four do
@@ -1314,10 +1340,12 @@ hipError_t run_decode_grad(const void* dy, const void* expert_out, const void* g
   a.E = E;
   a.C = C;
   a.owner = nullptr;
+  a.checked = 0;
   if (K * static_cast<long>(S) > kScanSlots && M > 0 && C > 0) {
     const hipError_t err = run_inverse_map(idx, loc, K * S, E, C, src_map, st);
     if (err != hipSuccess) return err;
     a.owner = src_map;
+    a.checked = static_cast<long>(E) * C <= kClearedRows;
   }
   const int eb = dtype == LANCET_F32 ? 4 : 2;
   const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(dy) && aligned16(expert_out) && aligned16(d_expert_out));

@@ -61,3 +61,26 @@ def test_row_map_in_memory_that_holds_anything(pkg, k, fill):
     np.testing.assert_array_equal(to_np(got), want)
     d_rows, d_g = ops.moe_decode_grad(dev(tok), dev(disp), dev(g), dev(il), top_k=k, workspace=ws.clone())
     np.testing.assert_array_equal(to_np(d_rows), want)
+
+
+# a wave with one row to look up and with several, ends inside them; up to 131072 rows the map is checked, beyond it is cleared
+@pytest.mark.parametrize("S,M,E,cf", [(9000, 512, 5, 0.9), (9000, 520, 33, 1.3), (5000, 2050, 7, 1.1), (60000, 8, 3, 3.0), (70000, 264, 64, 2.0)])
+@pytest.mark.parametrize("k", [1, 2])
+def test_row_map_of_rows_looked_up_together(pkg, S, M, E, cf, k):
+    """Gradients of the expert rows, bit for bit: a copy of dy where the weight is a power of two, zero where nobody owns the row."""
+    ops, lib = pkg.ops, pkg.capi.load()
+    logits = torch.randn((S, E), device="cuda", generator=torch.Generator(device="cuda").manual_seed(S)) + torch.arange(E, device="cuda") % 3
+    C = ops.moe_capacity(S, E, cf)
+    dy = torch.randn((S, M), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M)).bfloat16()
+    _, il, _, _ = ops.moe_route(logits, None, M, top_k=k, gate_is_logits=True, capacity=C)
+    g = torch.exp2(-(torch.arange(k * S, device="cuda") % 4).float())
+    want = torch.zeros((E, C, M), dtype=torch.bfloat16, device="cuda")
+    keep = il[0] >= 0
+    want[il[0][keep].long(), il[1][keep].long()] = (dy.repeat(k, 1) * g[:, None].bfloat16())[keep]
+    assert (~keep).any() or cf > 1.0
+    ws = (torch.arange(int(lib.lancet_moe_decode_dx_workspace_bytes(E, C)) // 4, dtype=torch.int32, device="cuda") % (k * S)).view(torch.uint8)
+    got = ops.moe_decode_dx(dy, g, il, E, C, top_k=k, workspace=ws.clone())
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    rows = torch.randn((E, C, M), device="cuda").bfloat16()
+    d_rows, _ = ops.moe_decode_grad(dy, rows, g, il, top_k=k, workspace=ws.clone())
+    assert torch.equal(d_rows.view(torch.int16), want.view(torch.int16))
