@@ -91,7 +91,8 @@ _scan_pool = {}
 
 def _scan_workspace(nbytes, device, given):
     """The workspace a scan call uses: the caller's ScanWorkspace, or one kept per (device, stream) and grown on
-    demand (calls on one stream run one after the other, so they can share)."""
+    demand (calls on one stream run one after the other, so they can share; threads that call on one stream take
+    turns, torch_host/torch_host.cc launches_on)."""
     if given is not None:
         if not isinstance(given, ScanWorkspace):
             raise TypeError("workspace of a scan call must be an ops.ScanWorkspace (it is set up once and carries "

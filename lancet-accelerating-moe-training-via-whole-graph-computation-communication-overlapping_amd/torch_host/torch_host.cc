@@ -29,7 +29,7 @@
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
 
-#include <cmath>
+#include <mutex>
 #include <optional>
 #include <string>
 #include <vector>
@@ -183,6 +183,15 @@ Tensor scan_workspace(size_t nbytes, const Tensor& data, PyObject* given) {
   if (!buf) throw python_error();
   return tensor_arg(buf.get(), "workspace");
 }
+// A call is several launches that pass tables through its workspace, and the interpreter's lock is released around them: threads
+// that share a stream share the workspace kept for it, so one enqueues all its launches before the next may (they then run
+// one after the other on the stream).  Taken without the interpreter's lock, held over launches alone; a workspace given by
+// the caller serves one call at a time by its contract.
+std::unique_lock<std::mutex> launches_on(const Tensor& workspace, bool kept) {
+  static std::mutex locks[64];  // by address, so that threads on streams of their own do not wait for one another
+  if (!kept) return {};
+  return std::unique_lock<std::mutex>(locks[(reinterpret_cast<uintptr_t>(workspace.data_ptr()) >> 12) % 64]);
+}
 // a plain scratch buffer: the caller's, or a new one
 Tensor scratch(size_t nbytes, const Tensor& like, const Tensor& given) {
   if (given.defined()) {
@@ -205,6 +214,7 @@ struct EncodeArgs {
   bool prioritized = false;  // batch-prioritised: the batch is cut into n_partitions, the call covers one
   int64_t n_partitions = 0, partition_id = 0;
   Tensor workspace;
+  bool kept_workspace = false;  // scan_workspace's own, which other threads may find too
 };
 
 size_t encode_workspace_bytes(const Tensor& gate, const EncodeArgs& a) {
@@ -242,6 +252,7 @@ void encode(const Tensor& data, const Tensor& gate, const Tensor& noise, const T
   const auto elems = static_cast<uint64_t*>(ptr(o.elems));
   const auto il = static_cast<int32_t*>(ptr(o.indloc));
   const auto used_out = static_cast<int32_t*>(ptr(o.used));
+  const auto lock = launches_on(a.workspace, a.kept_workspace);
   if (a.prioritized) {
     check(lancet_moe_encode_bpr(ptr(data), ptr(gate), data.size(0), data.size(1), gate.size(1), cap, static_cast<int>(a.n_partitions),
                                 static_cast<int>(a.partition_id), dt, gd, a.flags, ptr(o.gates_s), il, used_out, elems,
@@ -494,7 +505,7 @@ PyObject* py_encode(PyObject*, Args p, Py_ssize_t n) {
                used = optional_arg(p[3], "used_capacity");
   EncodeArgs a = encode_args(p[4], p[5], p[6], p[7]);
   const int64_t cap = check_encode(data, gate, noise, used, a);
-  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), data, p[8]);
+  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), data, p[8]), a.kept_workspace = p[8] == Py_None;
   return encode_into(data, gate, noise, used, cap, a, p[9]);
   LANCET_CATCH
 }
@@ -507,7 +518,7 @@ PyObject* py_encode_bpr(PyObject*, Args p, Py_ssize_t n) {
   a.capacity_factor = float_arg(p[4]), a.flags = static_cast<unsigned>(int_arg(p[5]));
   a.prioritized = true, a.n_partitions = int_arg(p[2]), a.partition_id = int_arg(p[3]);
   const int64_t cap = check_encode(data, gate, Tensor(), Tensor(), a);
-  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), data, p[6]);
+  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), data, p[6]), a.kept_workspace = p[6] == Py_None;
   return encode_into(data, gate, Tensor(), Tensor(), cap, a, p[7]);
   LANCET_CATCH
 }
@@ -520,7 +531,7 @@ PyObject* py_encode_diff(PyObject*, Args p, Py_ssize_t n) {
   EncodeArgs a = encode_args(p[4], p[5], p[6], p[7]);
   if (p[8] != Py_None) a.prioritized = true, a.n_partitions = int_arg(p[8]), a.partition_id = int_arg(p[9]);
   const int64_t cap = check_encode(data, gate, noise, used, a);
-  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), data, Py_None);
+  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), data, Py_None), a.kept_workspace = true;
   const auto some = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
   variable_list all;
   {
@@ -751,11 +762,12 @@ PyObject* py_route(PyObject*, Args p, Py_ssize_t n) {
     NEED(seq.n >= 4, "out must be a sequence of four tensors");
     o = {seq.at(0, "gates_s"), seq.at(1, "indices_locations"), seq.at(2, "used_capacity"), seq.at(3, "elements_per_expert"), Tensor()};
   }
-  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), gate, p[8]);
+  a.workspace = scan_workspace(encode_workspace_bytes(gate, a), gate, p[8]), a.kept_workspace = p[8] == Py_None;
   NEED(o.gates_s.scalar_type() == gate.scalar_type(), "gates_s takes the gate's dtype");
   void* const stream = stream_arg(p[10]);
   {
     pybind11::gil_scoped_release unlocked;
+    const auto lock = launches_on(a.workspace, a.kept_workspace);
     check(lancet_moe_route(ptr(gate), ptr(noise), static_cast<const int32_t*>(ptr(used)), S, M, E, cap, static_cast<int>(a.top_k), gd,
                            a.flags, ptr(o.gates_s), static_cast<int32_t*>(ptr(o.indloc)), static_cast<int32_t*>(ptr(o.used)),
                            static_cast<uint64_t*>(ptr(o.elems)), ptr(a.workspace), a.workspace.numel(), stream),
