@@ -451,6 +451,10 @@ class LansPlan:
         the same pass as p.  grad_norms: optional float32 GPU tensor [T] of ||g_i|| in list order (skips the
         step's own pass over g).  Raises LancetError(ERR_STALLED) when an earlier step of the resident
         schedule gave up a wait, until error() has been read."""
+        if not isinstance(hyper, capi.LansHyper):   # the native call takes its address
+            raise TypeError("hyper must be a capi.LansHyper, got %s" % type(hyper).__name__)
+        if self._h is None:
+            raise capi.LancetError(capi.ERR_PLAN, "lancet_lans_step on a closed plan")
         capi.host().lans_step(self._h.value, self._sizes, len(self.numels), g, p, m, v, p_lowp, int(step), step_dev,
                               C.addressof(hyper), grad_norms)
 
