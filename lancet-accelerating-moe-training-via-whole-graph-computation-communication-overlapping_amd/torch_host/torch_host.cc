@@ -733,9 +733,11 @@ PyObject* py_redispatch(PyObject*, Args p, Py_ssize_t n) {
 }
 
 // ---- the halves and token ranges of the operators (a caller with streams of its own names the stream) ---------------
-// None: the current device's current stream; else the handle of one
-void* stream_arg(PyObject* o) {
+// None: the current device's current stream; else the handle of one, for calls whose arrays are all given: what is allocated
+// here, and the workspace kept, belong to the current stream, and could be handed on while the named one still uses them
+void* stream_arg(PyObject* o, bool all_given) {
   if (o == Py_None) return current_stream();
+  NEED(all_given, "a call on a named stream takes its outputs and its workspace from the caller");
   return reinterpret_cast<void*>(static_cast<intptr_t>(int_arg(o)));
 }
 
@@ -753,6 +755,7 @@ PyObject* py_route(PyObject*, Args p, Py_ssize_t n) {
   NEED(a.top_k == 1 || a.top_k == 2, "top_k must be 1 or 2");
   check_noise(noise, gate, a.top_k);
   const int64_t cap = a.capacity ? *a.capacity : capacity_of(S, E, a.capacity_factor * (a.top_k == 2 ? 2.0 : 1.0));
+  void* const stream = stream_arg(p[10], p[8] != Py_None && p[9] != Py_None);
   Encoded o;
   if (p[9] == Py_None) {
     o = {new_tensor({a.top_k * S}, gate.scalar_type(), gate), new_tensor({2, a.top_k * S}, at::kInt, gate), new_tensor({E}, at::kInt, gate),
@@ -764,7 +767,6 @@ PyObject* py_route(PyObject*, Args p, Py_ssize_t n) {
   }
   a.workspace = scan_workspace(encode_workspace_bytes(gate, a), gate, p[8]), a.kept_workspace = p[8] == Py_None;
   NEED(o.gates_s.scalar_type() == gate.scalar_type(), "gates_s takes the gate's dtype");
-  void* const stream = stream_arg(p[10]);
   {
     pybind11::gil_scoped_release unlocked;
     const auto lock = launches_on(a.workspace, a.kept_workspace);
@@ -789,7 +791,7 @@ PyObject* py_scatter_tokens(PyObject*, Args p, Py_ssize_t n) {
   NEED(data.dim() == 2, "Expected input data to be 2D.");
   const int64_t total = mask_tokens(il, k), count = data.size(0), M = data.size(1);
   NEED(0 <= first && first + count <= total, "token range outside the routed batch");
-  void* const stream = stream_arg(p[10]);
+  void* const stream = stream_arg(p[10], out.defined());
   {
     pybind11::gil_scoped_release unlocked;
     if (!out.defined()) out = new_tensor({E, C, M}, data.scalar_type(), data);
@@ -815,7 +817,7 @@ PyObject* py_decode_tokens(PyObject*, Args p, Py_ssize_t n) {
   NEED(gate.size(0) == k * total, "gate and indices_locations disagree on the token count");
   NEED(0 <= first && 0 <= count && first + count <= total, "token range outside the routed batch");
   const int64_t E = data.size(0), C = data.size(1), M = data.size(2);
-  void* const stream = stream_arg(p[7]);
+  void* const stream = stream_arg(p[7], out.defined());
   {
     pybind11::gil_scoped_release unlocked;
     if (!out.defined()) out = new_tensor({count, M}, data.scalar_type(), data);
@@ -840,7 +842,7 @@ PyObject* py_partition_ranges(PyObject*, Args p, Py_ssize_t n) {
     NEED(seq.n == 2, "out must be two tensors");
     starts = seq.at(0, "starts"), counts = seq.at(1, "counts");
   }
-  void* const stream = stream_arg(p[7]);
+  void* const stream = stream_arg(p[7], starts.defined() && given.defined());
   {
     pybind11::gil_scoped_release unlocked;
     if (!starts.defined()) starts = new_tensor({k * P, E}, at::kLong, il), counts = new_tensor({k * P, E}, at::kLong, il);
@@ -869,7 +871,7 @@ PyObject* py_sparse_ranges(PyObject*, Args p, Py_ssize_t n) {
   NEED(wide == at::kLong || wide == at::kUInt64, "nelements_per_dim must be contiguous 64-bit counts");
   on_device(start, "starts_per_dim");
   NEED(start.scalar_type() == wide && start.numel() == count.numel(), "starts_per_dim must match nelements_per_dim");
-  void* const stream = stream_arg(p[7]);
+  void* const stream = stream_arg(p[7], true);
   {
     pybind11::gil_scoped_release unlocked;
     const auto copy = PACK ? lancet_memcpy_sparse_ranges_to_cont_3d : lancet_memcpy_cont_to_sparse_ranges_3d;

@@ -119,3 +119,25 @@ def test_bpr_gradient_covers_the_partition_alone(pkg):
     dx, dg = torch.autograd.grad((out[0].sum() + out[4].sum()), (data, gate))
     assert dx.shape == data.shape and dg.shape == gate.shape
     assert not dx[:S // 2].any() and not dg[:S // 2].any() and dx[S // 2:].any() and dg[S // 2:].any()
+
+
+@pytest.mark.parametrize("case", ["route", "route_workspace", "scatter", "decode", "ranges", "ranges_workspace"])
+def test_named_streams_take_given_arrays_alone(pkg, case):
+    """What a native call would allocate belongs to the current stream, not to the one that is named."""
+    ops, host = pkg.ops, pkg.capi.host()
+    data, gate = _inputs()
+    il, g = torch.zeros((2, S), dtype=torch.int32, device="cuda"), torch.ones(S, device="cuda")
+    used, buf = torch.zeros(E, dtype=torch.int32, device="cuda"), torch.zeros((E, 8, M), device="cuda")
+    outs = (g, il, used, torch.zeros(E, dtype=torch.int64, device="cuda"))
+    pair = (torch.zeros((2, E), dtype=torch.int64, device="cuda"),) * 2
+    side = torch.cuda.Stream().cuda_stream
+    calls = {
+        "route": lambda: host.moe_route(gate, None, None, M, 1.0, 8, 1, 0, ops.ScanWorkspace(1 << 16), None, side),
+        "route_workspace": lambda: host.moe_route(gate, None, None, M, 1.0, 8, 1, 0, None, outs, side),
+        "scatter": lambda: host.moe_scatter_tokens(data, il, None, used, 0, E, 8, 1, 0, None, side),
+        "decode": lambda: host.moe_decode_tokens(buf, g, il, 0, S, 1, None, side),
+        "ranges": lambda: host.moe_partition_ranges(il, 2, E, M, 1, torch.zeros(4096, dtype=torch.uint8, device="cuda"), None, side),
+        "ranges_workspace": lambda: host.moe_partition_ranges(il, 2, E, M, 1, None, pair, side),
+    }
+    with pytest.raises(ValueError, match="named stream"):
+        calls[case]()
