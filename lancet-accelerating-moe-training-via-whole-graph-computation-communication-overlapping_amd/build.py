@@ -66,11 +66,20 @@ def build_ops():
 
 
 def build_torch_host():
-    """The native host path of the operators: a Python extension over the C ABI and torch's own libraries."""
+    """The native host path of the operators: a Python extension over the C ABI and torch's own libraries.  None where torch or
+    its headers are not installed: the C ABI and the op layer stand without it (and ops.py cannot be imported there)."""
     import sysconfig
-    from torch.utils import cpp_extension
+    try:
+        from torch.utils import cpp_extension
+        torch_include = cpp_extension.include_paths()
+    except ImportError as e:
+        print("lancet_torch_host.so is not built, torch is not there: %s" % e, flush=True)
+        return None
+    if not any(os.path.exists(os.path.join(d, "torch", "csrc", "autograd", "python_variable.h")) for d in torch_include):
+        print("lancet_torch_host.so is not built, torch's headers are not there", flush=True)
+        return None
     out = os.path.join(LIBDIR, "lancet_torch_host.so")
-    include = [sysconfig.get_paths()["include"]] + cpp_extension.include_paths() + ["/opt/rocm/include"]
+    include = [sysconfig.get_paths()["include"]] + torch_include + ["/opt/rocm/include"]
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"] +
          [x for d in include for x in ("-isystem", d)] +
          ["-o", out, os.path.join(HERE, "torch_host", "torch_host.cc")] +
