@@ -554,21 +554,39 @@ struct SelectLaunch {
   size_t lds;
 };
 // Wide: short launches (a tile has a CU to itself) of rows long enough for the second barrier and the waves that are started to
-// pay.  moe_encode of 256 / 4096 / 65536 tokens, otherwise / wide, us: 64 fp32 logits top-1 7.3 / 5.6, 10.5 / 8.9, 16.7 / 14.9, top-2
-// 8.8 / 7.7, 12.5 / 11.4, 23.9 / 22.5; 128 top-1 11.2 / 7.3, 14.6 / 10.6, 24.1 / 20.8; 256 21.8 / 13.1, 22.7 / 14.0, 34.5 / 30.3; but 32 top-2 6.5 / 6.9,
-// 9.9 / 10.2 and 16 6.1 / 7.2.  128 bf16 logits top-2 11.3 / 10.6, 15.2 / 14.1, 64 8.1 / 8.6.  64 tokens: 60 bf16 6.1 / 4.8, 32 fp32 6.0 / 5.6.
-// Probabilities: full lanes alone (64 fp32 top-1 6.3 / 5.6, 9.7 / 8.9, 128 8.1 / 7.2; 200 12.2 / 14.2, 60 and 96 the same).
-// 131072 tokens: 64 fp32 23.8 / 24.8.
+// pay, where few lanes take granules that the row has not (as in rows_are_held).  moe_encode of 256 / 4096 / 65536 tokens,
+// otherwise / wide, us: 64 fp32 logits top-1 7.3 / 5.6, 10.5 / 8.9, 16.7 / 14.9, top-2 8.8 / 7.7, 12.5 / 11.4, 23.9 / 22.5; 128 top-1
+// 11.2 / 7.3, 14.6 / 10.6, 24.1 / 20.8; 256 21.8 / 13.1, 22.7 / 14.0, 34.5 / 30.3; but 32 top-2 6.5 / 6.9, 9.9 / 10.2 and 16 6.1 / 7.2.  128
+// bf16 logits top-2 11.3 / 10.6, 15.2 / 14.1, 64 8.1 / 8.6.  131072 tokens: 64 fp32 23.8 / 24.8.  The rest is moe_route alone:
+//   * logits of more than half a tile: five lanes in eight, whatever the type.  256 tokens top-2: 68 fp32 (17 granules, lanes for
+//     32) 10.0 / 11.1, 76 10.9 / 11.2, 80 11.2 / 11.2, 96 13.8 / 11.4; 132 (33 of 64) 13.2 / 16.4, 152 15.4 / 16.4, 160 18.8 / 16.4; 136 bf16
+//     14.3 / 16.0, 160 15.8 / 15.9, 272 22.1 / 25.1, 320 26.5 / 25.3; 4096 tokens top-1: 132 fp32 12.3 / 14.2, 144 14.5 / 15.2, 160 18.4 / 15.3,
+//     272 bf16 19.5 / 22.0, 320 23.5 / 22.0.  Rows that are not whole aligned granules are held otherwise, by the same lanes, and
+//     always gain (65 fp32 14.3 / 11.1, 129 23.6 / 16.4, 257 bf16 31.9 / 24.9), and so do few tokens (64: 132 fp32 12.8 / 11.3; moe_encode of
+//     128: 72 fp32 8.6 / 7.9, 136 bf16 16.4 / 14.3);
+//   * probabilities, which are a few compares per value: all lanes, four granules each.  256 tokens top-1: 64 fp32 6.8 / 6.3, 128
+//     8.6 / 7.8, 256 12.1 / 10.8, 128 bf16 8.4 / 7.9, 256 11.5 / 10.2, 512 17.9 / 15.8; 65536 top-2: 64 fp32 15.2 / 14.2, 128 bf16 19.9 / 18.2, 512
+//     46.0 / 40.4; but lanes with two granules and fewer 32 fp32 5.6 / 5.9, 64 bf16 6.1 / 6.8, and lanes without, 120 fp32 7.2 / 7.6, 200
+//     9.0 / 11.1.  What fills the lanes and is not whole granules gains too (1000 tokens: 61 fp32 9.2 / 8.3, 253 20.2 / 13.3, 505 bf16
+//     27.6 / 20.3), but for the tokens of one of the sixteen waves (16: 253 fp32 7.2 / 7.4).  64 granules of fp32: the walk is faster
+//     again from 193 tiles on (49152 tokens 21.6 / 20.8, 65536 22.9 / 25.9).
 constexpr int kWideTiles = 256;
-inline bool rows_are_wide(const void* noise, int S, int E, int gb, bool is_logits) {
-  const int bytes = E * gb;
-  if (noise != nullptr || bytes <= 32 || bytes > 16 * kHeldGranules || (S + kTile - 1) / kTile > kWideTiles) return false;
-  if (!is_logits) return gb == 4 && (E == 64 || E == 128);
-  return E >= (S <= kWave ? 32 : gb == 4 ? 56 : 96);
+constexpr int kWideLongTiles = 192;
+inline bool rows_are_wide(const void* gate, const void* noise, int S, int E, int gb, bool is_logits) {
+  const int bytes = E * gb, n = (bytes + 15) / 16, tiles = (S + kTile - 1) / kTile;
+  if (noise != nullptr || bytes <= 32 || bytes > 16 * kHeldGranules || tiles > kWideTiles) return false;
+  int taken = kHeldPerLane;
+  while (taken < n) taken *= 2;
+  const bool walked = bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(gate) & 15u) == 0;  // otherwise held
+  if (!is_logits) {
+    if (n != taken || n <= 8 || (!walked && S <= kWideRows)) return false;
+    return !walked || gb == 2 || n < kHeldGranules || tiles <= kWideLongTiles;
+  }
+  return E >= (S <= kWave ? 32 : gb == 4 ? 56 : 96) && (!walked || S <= kTile / 2 || 8 * n >= 5 * taken);
 }
 inline SelectLaunch select_launch(int gate_dtype, const void* gate, const void* noise, int S, int E, bool is_logits) {
   const int gb = gate_dtype == LANCET_F32 ? 4 : 2;
-  if (rows_are_wide(noise, S, E, gb, is_logits)) return {kHoldWide, kSelectThreadsOf<kHoldWide>, 0};
+  if (rows_are_wide(gate, noise, S, E, gb, is_logits)) return {kHoldWide, kSelectThreadsOf<kHoldWide>, 0};
   if (rows_are_held(gate, noise, S, E, gb, is_logits)) return {kHoldRows, kTile, 0};
   SelectLaunch l = {kWalkRows, kTile, 0};
   LANCET_GATE_SWITCH(gate_dtype, l.lds = rows_are_staged<GD>(gate, noise, S, E) ? kStageBytes : 0)

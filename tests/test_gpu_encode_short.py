@@ -88,10 +88,12 @@ def test_short_top1_on_memory_that_was_never_set_up(pkg, S):
     np.testing.assert_array_equal(to_np(outs[4]), want[4])
 
 
-@pytest.mark.parametrize("S", [1, 15, 17, 64, 65, 255, 257, 700])
-@pytest.mark.parametrize("E,gdt", [(32, "f32"), (56, "f32"), (63, "f32"), (64, "f32"), (100, "f32"), (256, "f32"), (96, "bf16"), (101, "f16"), (512, "bf16")])
+# lanes that are full, five in eight, fewer (logits of more than half a tile are walked then), rows that end inside a granule
+@pytest.mark.parametrize("S", [1, 15, 17, 64, 65, 128, 129, 257, 700])
+@pytest.mark.parametrize("E,gdt", [(32, "f32"), (56, "f32"), (61, "f32"), (64, "f32"), (76, "f32"), (80, "f32"), (100, "f32"), (125, "f32"), (129, "f32"), (132, "f32"),
+                                   (256, "f32"), (96, "bf16"), (128, "bf16"), (249, "bf16"), (101, "f16"), (272, "f16"), (512, "bf16")])
 def test_selection_by_sixteen_waves(pkg, S, E, gdt):
-    """Rows whose selection sixteen waves share: choices against the oracle's on the rounded gate (massive ties of 16-bit values
+    """Rows whose selection sixteen waves share, and those beside them: choices against the oracle's on the rounded gate (massive ties of 16-bit values
     included), rows with a NaN and rows of -inf against the same rows in a batch that sixteen waves do not take (noise of zero
     sends a top-2 call to the row-by-row walk)."""
     ops = pkg.ops
