@@ -27,11 +27,11 @@ def _capture(fn):
     return g
 
 
-# (4096, 256, 16): the scan as one look-back kernel (top-1) or as count + place (top-2); (140000, 8, 64): count +
-# segment sums + place, gate rows staged through LDS
-@pytest.mark.parametrize("S,M,E", [(4096, 256, 16), (140000, 8, 64)])
+# (200, 40, 8): the encode as one kernel; (4096, 256, 16): count, then placement and rows in one, and on request the scan as one
+# look-back kernel; (140000, 8, 64): count + segment sums + place
+@pytest.mark.parametrize("S,M,E,lookback", [(200, 40, 8, False), (4096, 256, 16, False), (4096, 256, 16, True), (140000, 8, 64, False)])
 @pytest.mark.parametrize("k,dt", [(1, torch.float32), (2, torch.bfloat16)])
-def test_encode_decode_graph_replays(pkg, k, dt, S, M, E):
+def test_encode_decode_graph_replays(pkg, k, dt, S, M, E, lookback):
     ops = pkg.ops
     cf = 0.8
     data = torch.empty((S, M), dtype=dt, device="cuda")
@@ -45,7 +45,7 @@ def test_encode_decode_graph_replays(pkg, k, dt, S, M, E):
     zero = torch.zeros(E, dtype=torch.int32, device="cuda")
 
     def step():
-        ops.moe_encode(data, logits, zero, cf, top_k=k, gate_is_logits=True, workspace=ws, out=outs)
+        ops.moe_encode(data, logits, zero, cf, top_k=k, gate_is_logits=True, workspace=ws, out=outs, scan_lookback=lookback)
         ops.moe_decode(outs[4], outs[0], outs[1], top_k=k, out=dec)
 
     def fresh(seed):

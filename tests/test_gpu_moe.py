@@ -455,8 +455,8 @@ def test_scan_epoch_wraps(pkg):
 
 def test_scan_on_a_workspace_that_is_not_set_up(pkg):
     """A call handed memory that lancet_scan_workspace_init never saw must not hang or run wild: the look-back form of
-    the scan (top-1 on few tiles here) marks its outputs (-1) and sets the error word, and after the set-up the same
-    memory works; the form without waits (top-2 here) keeps no state and simply gives the right result."""
+    the scan marks its outputs (-1) and sets the error word, as every top-1 encode on few tiles does, and after the set-up the
+    same memory works; the forms without waits keep no state and top-2 simply gives the right result."""
     import ctypes as C
     lib = pkg.capi.load()
     capi = pkg.capi
@@ -464,20 +464,21 @@ def test_scan_on_a_workspace_that_is_not_set_up(pkg):
     data, logits = make_inputs(2, S, M, E)
     d_data, d_gate = dev(data), dev(logits)
     p = lambda t: C.c_void_p(t.data_ptr())
-    for k in (1, 2):
+    for k, lookback in ((1, 0), (1, capi.SCAN_LOOKBACK), (2, 0), (2, capi.SCAN_LOOKBACK)):
         nws = int(lib.lancet_moe_encode_workspace_bytes(S, E, k))
+        flags = capi.GATE_IS_LOGITS | lookback
         for fill in (0, 0xff):
             ws = torch.full((nws,), fill, dtype=torch.uint8, device="cuda")
             Cap = ops_cap = pkg.ops.moe_capacity(S, E, float(k))
             outs = (torch.zeros(k * S, device="cuda"), torch.zeros((2, k * S), dtype=torch.int32, device="cuda"),
                     torch.zeros(E, dtype=torch.int32, device="cuda"), torch.zeros(E, dtype=torch.int64, device="cuda"),
                     torch.zeros((E, Cap, M), device="cuda"))
-            st = lib.lancet_moe_encode(p(d_data), p(d_gate), None, None, S, M, E, Cap, k, capi.F32, capi.F32, capi.GATE_IS_LOGITS,
+            st = lib.lancet_moe_encode(p(d_data), p(d_gate), None, None, S, M, E, Cap, k, capi.F32, capi.F32, flags,
                                        *[p(t) for t in outs], p(ws), nws, None)
             assert st == 0
             torch.cuda.synchronize()
             err = C.c_int(0)
-            if k == 1:
+            if k == 1 or lookback:
                 assert (to_np(outs[1]) == -1).all() and (to_np(outs[2]) == -1).all()
                 assert (to_np(outs[4]) == 0).all(), "no token has a place: the buffer is all tail"
                 assert lib.lancet_scan_workspace_error(p(ws), None, C.byref(err)) == 0 and err.value == 1
@@ -486,7 +487,7 @@ def test_scan_on_a_workspace_that_is_not_set_up(pkg):
                 np.testing.assert_array_equal(to_np(outs[1]), want[1])
                 np.testing.assert_array_equal(to_np(outs[4]), want[4])
             assert lib.lancet_scan_workspace_init(p(ws), nws, None) == 0
-            st = lib.lancet_moe_encode(p(d_data), p(d_gate), None, None, S, M, E, Cap, k, capi.F32, capi.F32, capi.GATE_IS_LOGITS,
+            st = lib.lancet_moe_encode(p(d_data), p(d_gate), None, None, S, M, E, Cap, k, capi.F32, capi.F32, flags,
                                        *[p(t) for t in outs], p(ws), nws, None)
             assert st == 0
             enc = mo.moe_encode_top2 if k == 2 else mo.moe_encode
@@ -996,11 +997,13 @@ def test_capacity_override_gshard_formula(pkg):
     np.testing.assert_array_equal(to_np(r[1]), want[1])
 
 
-def test_default_workspaces_are_kept_per_stream(pkg):
+@pytest.mark.parametrize("lookback", [False, True])
+def test_default_workspaces_are_kept_per_stream(pkg, lookback):
     """Calls without a workspace argument share one kept per (device, stream): calls on two streams that run at the
-    same time must not share theirs (the look-back form keeps state in it), and scan_errors() reads them all."""
+    same time must not share theirs (the look-back form keeps state in it, the others pass tables through it), and scan_errors()
+    reads them all."""
     ops = pkg.ops
-    S, M, E = 6000, 32, 16           # top-1 on 24 tiles: the look-back form
+    S, M, E = 6000, 32, 16
     data, logits = make_inputs(77, S, M, E)
     want = mo.moe_encode(data, logits, np.zeros(E, np.int32), 1.0, gate_is_logits=True, fast_scatter=True)
     d_data, d_gate = dev(data), dev(logits)
@@ -1009,9 +1012,9 @@ def test_default_workspaces_are_kept_per_stream(pkg):
     before = len(ops._scan_pool)
     outs = []
     for _ in range(20):
-        outs.append(ops.moe_encode(d_data, d_gate, None, 1.0, gate_is_logits=True))
+        outs.append(ops.moe_encode(d_data, d_gate, None, 1.0, gate_is_logits=True, scan_lookback=lookback))
         with torch.cuda.stream(side):
-            outs.append(ops.moe_encode(d_data, d_gate, None, 1.0, gate_is_logits=True))
+            outs.append(ops.moe_encode(d_data, d_gate, None, 1.0, gate_is_logits=True, scan_lookback=lookback))
     torch.cuda.synchronize()
     assert len(ops._scan_pool) >= max(before, 2)
     keys = {k for k in ops._scan_pool if k[1] in (side.cuda_stream, torch.cuda.current_stream().cuda_stream)}

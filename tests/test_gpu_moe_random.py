@@ -95,14 +95,17 @@ def test_routing_over_many_tiles(pkg, S, E, k, cf, skew, scan_lookback=False):
         used0 = rng.integers(0, max(mo.capacity(S, E, cf), 1) + 1, E).astype(np.int32)
     want = (mo.moe_encode_top2 if k == 2 else mo.moe_encode)(data, logits, used0, cf, gate_is_logits=True, fast_scatter=True)
     got = pkg.ops.moe_encode(dev(data), dev(logits), dev(used0), cf, top_k=k, gate_is_logits=True, scan_lookback=scan_lookback)
-    np.testing.assert_array_equal(to_np(got[1]), want[1])
-    np.testing.assert_array_equal(to_np(got[2]), want[2])
-    np.testing.assert_array_equal(to_np(got[3]), want[3])
-    np.testing.assert_allclose(to_np(got[0]), want[0], rtol=1e-5, atol=0)
+    # the routing alone as well: an encode of few tiles has kernels of its own
+    alone = pkg.ops.moe_route(dev(logits), dev(used0), M, cf, top_k=k, gate_is_logits=True, scan_lookback=scan_lookback)
+    for r in (got, alone):
+        np.testing.assert_array_equal(to_np(r[1]), want[1])
+        np.testing.assert_array_equal(to_np(r[2]), want[2])
+        np.testing.assert_array_equal(to_np(r[3]).astype(np.uint64), want[3])
+        np.testing.assert_allclose(to_np(r[0]), want[0], rtol=1e-5, atol=0)
     np.testing.assert_array_equal(to_np(got[4]), want[4])
 
 
-# one counter set on at most 32 tiles: one look-back kernel; tiles x counters up to 32768: two kernels without waits;
+# the routing alone, one counter set on at most 32 tiles: one look-back kernel; tiles x counters up to 32768: two kernels without waits;
 # beyond: three (segment sums between count and place).  Every case also as one look-back kernel.
 @pytest.mark.parametrize("S,E,k,cf,skew", [
     (32768, 512, 2, 1.0, 2.0),    # 128 tiles x 1024 counters: two pairs of counters per thread and row, segments of 32
