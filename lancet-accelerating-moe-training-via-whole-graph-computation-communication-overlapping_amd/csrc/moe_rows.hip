@@ -118,7 +118,8 @@ struct ScatterArgs {
   int token_blocks;
   int tail_chunks;            // tail workgroups per expert
   int tail_groups;            // eights of tail workgroups that stand among the tokens', 0 = all stand behind them
-  int tail_every;             // ... one in this many eights
+  int tail_every;             // ... one in this many eights, two at least
+  uint32_t tail_inverse;      // 2^32 / tail_every, rounded up
 };
 
 constexpr int kXcds = 8;  // workgroups go round them: what comes in turns comes in eights, or a few XCDs do all of it
@@ -129,7 +130,9 @@ __global__ __launch_bounds__(kTile) void scatter_rows_kernel(ScatterArgs a) {
   typedef typename G::V V;
   int token = static_cast<int>(blockIdx.x), tail = token - a.token_blocks;  // tail: negative in a workgroup of tokens
   if (a.tail_groups) {
-    const int eight = token / kXcds, turn = eight / a.tail_every;
+    // (a division would stand in front of every workgroup's first load: top-1 scatters with tails that are mostly empty 1.03 against 1.06
+    // of the time they take with the tails behind)
+    const int eight = token / kXcds, turn = static_cast<int>(__umulhi(static_cast<uint32_t>(eight), a.tail_inverse));
     const bool clears = turn < a.tail_groups && eight - turn * a.tail_every == a.tail_every - 1;
     tail = clears ? turn * kXcds + token % kXcds : -1;
     token -= kXcds * min(turn, a.tail_groups);
@@ -1063,15 +1066,27 @@ constexpr size_t kCuLds = 160 * 1024;
 constexpr size_t kScatterLds = kCuLds / 6 + 1;  // six do not fit, however LDS is rounded up; five do
 
 // Where the workgroups that clear the experts' tails stand.  Behind the tokens' they are an end of the launch that only
-// writes, or, where nearly all find nothing to clear, a row of empty starts; among them both hide behind the rows' traffic.
-// Behind / among, us for the whole encode: 16384 x 1024 fp32 top-2, 16 experts, some hot, 40.8 / 36.4; 8192 x 4096 bf16 top-2 44.2 /
-// 42.5, 16384 x 8192 173.1 / 169.8; 20000 x 3072 fp16, capacity 2, 125.5 / 122.8; 131072 x 512 88.8 / 85.6; 65536 x 4096
-// 333.6 / 333.4; top-1 32768 x 2048, some hot, 64.0 / 60.0, 12000 x 768 fp32, capacity 2, 26.1 / 22.4, 262144 x 512, some hot, 115.8 /
-// 113.3.  Not for top-1 rows of more than 4 KB, whose reads and writes are in balance without (65536 x 4096 211.2 / 214.0, 20000 x
-// 3072 62.1 / 66.6), nor for rows that end inside a granule (10007 x 1003 bf16 24.8 / 25.6).  At most kMixedTails of them,
-// each then with several turns: one eight in four at 65536 x 1024 93.2, one in five 90.0 (behind: 91.3).
+// writes, or, where nearly all find nothing to clear, a row of empty starts; among them they hide behind the rows' traffic, but an
+// empty start there costs more than one at the end.  Among them pays for long rows, which need few workgroups of tails per byte, in
+// passes that are long themselves.  Behind / among, us, tokens x bytes of a row, arrays that change from call to call:
+//   top-1, 40 to 60 % of the buffer filled: 34818 x 2912 64.9 / 60.2, 57288 x 2864 77.5 / 73.8, 135909 x 896 64.1 / 60.9 (the same arrays again
+//   and again 62 / 44, 68 / 58, 61 / 52); more filled than that: 141135 x 2352 171 / 170, 34914 x 3456 51.6 / 51.1, 218661 x 1552 120 / 125;
+//   top-2, half filled: 19356 x 2112 28.3 / 25.3, 28776 x 2160 38.2 / 35.2, 160407 x 912 98.9 / 94.7; filled: 119178 x 2240 210 / 207, 42771 x 2528 65.4 /
+//   68.5, 13773 x 6256 48.9 / 48.3; 16384 x 4096 half filled 40.8 / 36.4 for the whole encode.
+// Not for shorter rows and passes: 86769 x 48 top-2 6.5 / 10.8, 83468 x 64 top-1 5.4 / 7.3, 38382 x 448 10.2 / 12.2, 37842 x 1152 34.4 / 39.6, 69009 x 1216
+// top-1 37.1 / 39.3, 12474 x 1536 11.5 / 11.9; nor for top-1 rows of more than 4 KB, whose reads and writes are in balance without (65536 x 8192
+// 211.2 / 214.0, 45919 x 4752 107 / 119); nor for rows that end inside a granule (10007 x 2006 24.8 / 25.6).  At most
+// kMixedTails of them, each then with several turns: one eight in four at 65536 x 2048 93.2, one in five 90.0 (behind: 91.3).
+constexpr size_t kMixedRowBytes = 1536, kMixedBytes = size_t(64) << 20;
+constexpr size_t kMixedLongRowBytes = 768, kMixedLongBytes = size_t(256) << 20;
 constexpr size_t kMixedTop1Bytes = 4096;
 constexpr int kMixedTails = 8192;
+constexpr long kMixedBlocks = 1L << 19;  // up to here the multiplication by tail_inverse divides exactly
+static bool tails_among_tokens(size_t row_bytes, int S, int E, int C, int K) {
+  const size_t pass = (static_cast<size_t>(S) + static_cast<size_t>(E) * C) * row_bytes;
+  if (E > kMixedTails || (K == 1 && row_bytes > kMixedTop1Bytes)) return false;
+  return (row_bytes >= kMixedRowBytes && pass >= kMixedBytes) || (row_bytes >= kMixedLongRowBytes && pass >= kMixedLongBytes);
+}
 
 hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, const int32_t* loc,
                             const int32_t* avail_used, const int32_t* row_base, const int32_t* rows_lo,
@@ -1102,13 +1117,17 @@ hipError_t run_scatter_rows(const void* data, void* out, const int32_t* idx, con
   a.q = row_lanes(a.row_vecs, S, 1);
   a.token_blocks = static_cast<int>(row_blocks(S, a.q));
   a.tail_chunks = rows_hi ? (C + kTailRows - 1) / kTailRows : 0;
-  a.tail_groups = a.tail_every = 0;
+  a.tail_groups = a.tail_every = 0, a.tail_inverse = 0u;
   long blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_chunks) * E;
-  if (a.tail_chunks && a.token_blocks && E <= kMixedTails && mode == kWhole16 && (K == 2 || row_bytes <= kMixedTop1Bytes)) {
-    a.tail_chunks = std::min(a.tail_chunks, kMixedTails / E);
-    a.tail_groups = (a.tail_chunks * E + kXcds - 1) / kXcds;
-    blocks = static_cast<long>(a.token_blocks) + static_cast<long>(a.tail_groups) * kXcds;
-    a.tail_every = static_cast<int>(blocks / kXcds / a.tail_groups);
+  if (a.tail_chunks && a.token_blocks && mode == kWhole16 && tails_among_tokens(row_bytes, S, E, C, K)) {
+    const int chunks = std::min(a.tail_chunks, kMixedTails / E), groups = (chunks * E + kXcds - 1) / kXcds;
+    const long mixed = static_cast<long>(a.token_blocks) + static_cast<long>(groups) * kXcds;
+    const int every = static_cast<int>(mixed / kXcds / groups);
+    if (every >= 2 && mixed <= kMixedBlocks) {  // (more tails than tokens would stand in front of them)
+      a.tail_chunks = chunks, a.tail_groups = groups, a.tail_every = every;
+      a.tail_inverse = static_cast<uint32_t>((0x100000000ull + static_cast<uint64_t>(every) - 1) / static_cast<uint64_t>(every));
+      blocks = mixed;
+    }
   }
   if (blocks == 0) return hipSuccess;
   const size_t lds = a.row_vecs > kWave ? kScatterLds : 0;

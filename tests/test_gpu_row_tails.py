@@ -10,10 +10,12 @@ from tests.gpu_util import TORCH_DT, dev, make_inputs, rows_as_oracle, rows_to_t
 pytestmark = pytest.mark.gpu
 
 
-# one granule per row: fewer workgroups of tokens than of tails; tails that are no multiple of eight; more tails than there may be
-# workgroups (64 x 256, 512 x 19, one per expert); rows up to which top-1 has its tails among the tokens, and one granule more
-@pytest.mark.parametrize("S,M,E,C", [(8200, 8, 5, 2000), (8193, 8, 2, 9000), (8200, 8, 64, 4096), (8200, 8, 512, 300), (70001, 16, 3, 100),
-                                     (8200, 2048, 7, 1500), (8200, 2056, 7, 1300)])
+# tails among the tokens: one eight in two to in many, tails that are no multiple of eight, the most tails there may be workgroups (64 x
+# 256, 512 x 19: one per expert has several turns), long passes of shorter rows; behind them: more workgroups of tails than of tokens, rows and passes just
+# short of that, top-1 rows just longer, short rows
+@pytest.mark.parametrize("S,M,E,C", [(8200, 768, 5, 8000), (8193, 776, 2, 15001), (20000, 768, 64, 4096), (40000, 768, 512, 300), (8200, 2048, 7, 1500), (30000, 1600, 3, 100),
+                                     (150000, 384, 11, 20000), (8200, 768, 5, 30000), (8200, 760, 7, 4900), (8200, 768, 7, 4700), (8200, 2056, 7, 1300),
+                                     (8200, 8, 64, 4096), (70001, 16, 3, 100)])
 @pytest.mark.parametrize("k", [1, 2])
 def test_every_row_of_the_buffer_is_written_once(pkg, S, M, E, C, k):
     """Rows of tokens are copies, all others zero; with rows_at_used the rows below used_capacity stay as they were."""
