@@ -1325,12 +1325,13 @@ static hipError_t decode_grad_launch(DecodeGradArgs a, int K, int M, RowMode mod
   const unsigned blocks = static_cast<unsigned>(a.token_blocks + static_cast<long>(a.tail_chunks) * a.E);
   if (blocks == 0) return hipSuccess;
   // top-1 rows of several waves: as in the scatter, 317 against 329 us at 65536 x 4096 bf16 (rows of one wave 182 / 151).
-  // top-2 rows with more granules than a workgroup has lanes, of which a lane keeps twice the loads in flight, in passes that
-  // come from the HBM: four workgroups on a CU instead of eight (20000 x 3072 bf16 122 against 126 us; rows of 4 KB 157 / 137, 66 / 49
-  // at 16384 x 1024 fp32), and where all lanes have two granules of it the token's row is asked for before the routing words: both
+  // top-2 rows with half as many granules again as a workgroup has lanes, of which those keep twice the loads in flight, in passes that
+  // come from the HBM: four workgroups on a CU instead of eight (20000 x 3072 bf16 122 against 126 us, 13357 x 11376 bytes 150 / 160, 6797 x
+  // 6304 the same; of fewer granules, which most lanes have one of, eight are faster: 17248 x 5040 bytes 85 / 70, 28302 x 4480 129 / 101,
+  // 16384 x 4096 66 / 49), and where all lanes have two granules of it the token's row is asked for before the routing words: both
   // together 549 / 570 at 65536 x 4096, 156 / 165 at 20000, 96 / 101 at 12000, 51.3 / 52.7 at 6000.  In the cache neither pays (4200 x
   // 4096 with half as many rows kept 29 / 25), nor the latter for rows of 384 granules (158 / 153) or top-1 (20000 x 4096 92 / 90).
-  const bool wide = K == 2 && mode == kWhole16 && a.row_vecs > kTile &&
+  const bool wide = K == 2 && mode == kWhole16 && 2 * a.row_vecs >= 3 * kTile &&
                     (static_cast<size_t>(a.S) + 2 * static_cast<size_t>(a.E) * a.C) * a.row_bytes > kMemoryCache;
   const size_t lds = wide ? kGradWideLds : K == 1 && a.q > 6 ? kScatterLds : 0;
   if (wide && a.row_vecs >= 2 * kTile) {
