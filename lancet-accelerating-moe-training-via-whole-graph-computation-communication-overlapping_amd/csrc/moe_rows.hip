@@ -867,7 +867,7 @@ struct DecodeGradArgs {
   int row_vecs;            // granules per row
   int q;                   // 2^q lanes of one workgroup share a token
   int token_blocks;
-  int tail_rows;           // rows looked at by one workgroup behind the tokens' (at most 32 * kTile; kWave with a map)
+  int tail_rows;           // rows looked at by one workgroup behind the tokens' (kWave at most)
   int tail_chunks;         // such workgroups per expert
 };
 
@@ -877,7 +877,7 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
   typedef Codec<DT> Cd;
   typedef Granule<MODE> G;
   __shared__ float s_dot[kRowsPerBlock][K];
-  __shared__ uint32_t s_owned[kTile];
+  __shared__ uint32_t s_owned[2];
   const int w = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   if (static_cast<int>(blockIdx.x) >= a.token_blocks) {
@@ -885,28 +885,26 @@ __global__ __launch_bounds__(kTile) void decode_grad_kernel(DecodeGradArgs a) {
     const int e = tb / a.tail_chunks;
     const int first = (tb - e * a.tail_chunks) * a.tail_rows;
     const int last = min(first + a.tail_rows, a.C);
-    if (!a.owner) {
-      s_owned[threadIdx.x] = 0u;
+    // which of the rows are owned, a bit each: a wave that has rows looks all up at once, one chain of round trips instead of one per
+    // row (65536 x 512 bf16 top-2 73.8 -> 71.1 us, 262144 x 512 top-1 173 -> 168)
+    const int q = min(a.q, 6);
+    uint64_t owned = 0;
+    if (a.owner) {
+      if (first + (w * kWave >> q) >= last) return;
+      owned = __ballot(first + lane < last &&
+                       row_owner(a.owner, static_cast<size_t>(e) * a.C + first + lane, a.idx, a.loc, K * a.S, a.E, a.C, a.checked, [](int) {}) >= 0);
+    } else {
+      if (threadIdx.x < 2) s_owned[threadIdx.x] = 0u;
       __syncthreads();
       for (int i = threadIdx.x; i < K * a.S; i += kTile) {
         const int l = a.loc[i];
         if (a.idx[i] == e && l >= first && l < last) atomicOr(&s_owned[(l - first) >> 5], 1u << ((l - first) & 31));
       }
       __syncthreads();
+      owned = s_owned[0] | static_cast<uint64_t>(s_owned[1]) << 32;
     }
-    const int q = min(a.q, 6);
-    const auto mapped = [&](int r) {
-      return row_owner(a.owner, static_cast<size_t>(e) * a.C + r, a.idx, a.loc, K * a.S, a.E, a.C, a.checked, [](int) {}) >= 0;
-    };
-    // where a wave has several rows one after the other, it looks all up at once: one chain of round trips instead of one per row
-    // (65536 x 512 bf16 top-2 73.8 -> 71.1 us, 262144 x 512 top-1 173 -> 168)
-    const bool at_once = a.owner && (kTile >> q) < a.tail_rows;
-    uint64_t owned_rows = 0;
-    if (at_once) owned_rows = __ballot(first + lane < last && mapped(first + lane));
     for (int r = first + (static_cast<int>(threadIdx.x) >> q); r < last; r += kTile >> q) {
-      const int at = r - first;
-      const bool owned = at_once ? (owned_rows >> at) & 1u : a.owner ? mapped(r) : (s_owned[at >> 5] >> (at & 31)) & 1u;
-      if (owned) continue;
+      if ((owned >> (r - first)) & 1u) continue;
       const size_t row = static_cast<size_t>(e) * a.C + r;
       LANCET_GLOBAL char* dst = as_global(a.d_expert_out + row * a.row_bytes);
       for (int v = threadIdx.x & ((1 << q) - 1); v < a.row_vecs; v += 1 << q) G::st(dst + G::at(v, a.row_bytes), G::zero());
@@ -1257,9 +1255,10 @@ hipError_t run_encode_dg(const void* dy, const int32_t* idx, int S, int E, int K
 
 // Rows of the buffer up to which the map is checked instead of cleared.  Clearing is a launch of 2 to 3 us, checking two words more to
 // gather per row.  Cleared / checked, us: moe_decode_dx 16384 x 64 bf16 top-1 (20480 rows) 7.8 / 6.1, 32768 x 2048 (40960) 59.0 / 58.0,
-// 65536 x 64 (81920) 10.7 / 9.0; 131072 x 16 (163840) 10.9 / 10.3, x 64 16.0 / 16.5; 262144 x 64 (327680) 25.9 / 27.3, x 512 111.1 /
-// 109.6, 1000000 x 64 80.3 / 95.4; moe_decode_grad 65536 x 1024 82.0 / 80.2, 262144 x 64 35.4 / 35.8.
-constexpr long kClearedRows = 131072;
+// 65536 x 64 (81920) 10.7 / 9.0; 131072 x 16 (163840) 10.9 / 10.3, 107376 x 8 (214752) 8.3 / 6.5, 57693 x 928 top-2 (230820) 94.3 / 91.4, 119642 x 24 top-2 (239400)
+// 20.4 / 18.9; 131072 x 64 (163840) 16.0 / 16.5, 262144 x 64 (327680) 25.9 / 27.3, 87380 x 576 top-2 (349520) 112.9 / 113.9, 1000000 x 64 80.3 / 95.4;
+// moe_decode_grad 65536 x 1024 82.0 / 80.2, 26295 x 8 top-2 (105184) 9.4 / 7.4, 90630 x 552 top-2 (226610) 142.4 / 138.9, 262144 x 64 35.4 / 35.8.
+constexpr long kClearedRows = 262144;
 
 template <int DT>
 static hipError_t decode_dx_launch(const void* dy, const void* gates, int gd, const int32_t* src, const int32_t* idx,
@@ -1304,8 +1303,11 @@ hipError_t run_decode_dx(const void* dy, const void* gates, int gate_dtype, cons
 // Slots up to which the clearing workgroups of decode_grad_kernel walk all of them themselves instead of looking rows up in
 // a map that the launch before it makes.  Map / walk by workgroups of 64 rows, us: 1024 slots, rows of 64 bf16, 4 experts 4.6 /
 // 2.9 and 512 experts 4.9 / 3.0, rows of 2048 6.7 / 8.2 and 6.5 / 4.5; 4096 slots 5.0 / 4.3, 5.3 / 4.9, 13.0 / 15.1 and 12.7 / 11.2; 6000 slots
-// 5.2 / 5.5, 5.6 / 6.3, 16.0 / 19.1 and 16.1 / 15.5; 8192 slots 5.3 / 7.0, 5.6 / 7.5, 19.2 / 22.8 and 20.2 / 20.4.
-constexpr int kScanSlots = 4096;
+// rows of 2048 16.0 / 19.1 and 16.1 / 15.5.  Rows of less than 768 bytes, bytes and slots: top-1 144 x 4734 5.8 / 5.6, 48 x 5087 5.6 / 5.3, 16 x
+// 5225 5.5 / 5.9, 304 x 6343 6.1 / 7.0; top-2, whose map takes twice the writes, 320 x 4832 7.0 / 6.0, 160 x 5664 6.9 / 5.9, 238 x 6418 7.3 / 6.2, 100 x
+// 6982 6.8 / 6.4, 304 x 7426 7.6 / 8.5; longer rows 2102 x 4358 top-1 11.6 / 14.2, 1596 x 5214 top-2 10.7 / 11.7.
+constexpr int kScanSlots = 4096, kScanShortSlots1 = 5000, kScanShortSlots2 = 6900;
+constexpr size_t kScanShortRow = 768;
 constexpr int kGradTailRows = 16;  // rows per clearing workgroup with the inverse map
 constexpr int kGradScanRows = 64;  // ... that walks the slots
 constexpr size_t kGradWideLds = kCuLds / 5 + 1;  // five workgroups do not fit, four do
@@ -1361,13 +1363,14 @@ hipError_t run_decode_grad(const void* dy, const void* expert_out, const void* g
   a.C = C;
   a.owner = nullptr;
   a.checked = 0;
-  if (K * static_cast<long>(S) > kScanSlots && M > 0 && C > 0) {
+  const int eb = dtype == LANCET_F32 ? 4 : 2;
+  const int walked = static_cast<size_t>(M) * eb >= kScanShortRow ? kScanSlots : K == 1 ? kScanShortSlots1 : kScanShortSlots2;
+  if (K * static_cast<long>(S) > walked && M > 0 && C > 0) {
     const hipError_t err = run_inverse_map(idx, loc, K * S, E, C, src_map, st);
     if (err != hipSuccess) return err;
     a.owner = src_map;
     a.checked = static_cast<long>(E) * C <= kClearedRows;
   }
-  const int eb = dtype == LANCET_F32 ? 4 : 2;
   const RowMode mode = row_mode(static_cast<size_t>(M) * eb, eb, aligned16(dy) && aligned16(expert_out) && aligned16(d_expert_out));
   switch (dtype) {
     case LANCET_F32: return decode_grad_launch<LANCET_F32>(a, K, M, mode, st);

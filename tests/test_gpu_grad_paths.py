@@ -63,7 +63,7 @@ def test_row_map_in_memory_that_holds_anything(pkg, k, fill):
     np.testing.assert_array_equal(to_np(d_rows), want)
 
 
-# a wave with one row to look up and with several, ends inside them; up to 131072 rows the map is checked, beyond it is cleared
+# a wave with one row to look up and with several, ends inside them; up to 262144 rows the map is checked, beyond it is cleared
 @pytest.mark.parametrize("S,M,E,cf", [(9000, 512, 5, 0.9), (9000, 520, 33, 1.3), (5000, 2050, 7, 1.1), (60000, 8, 3, 3.0), (70000, 264, 64, 2.0)])
 @pytest.mark.parametrize("k", [1, 2])
 def test_row_map_of_rows_looked_up_together(pkg, S, M, E, cf, k):

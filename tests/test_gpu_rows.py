@@ -69,11 +69,12 @@ def test_rows_of_any_length_and_alignment(pkg, dt, M, offset, k):
 
 
 @pytest.mark.parametrize("S,k,M,dt,gdt", [(7, 1, 64, "f32", "f32"), (4096, 2, 24, "bf16", "bf16"), (4097, 2, 24, "bf16", "f32"), (8192, 1, 8, "f16", "f16"),
-                                          (4096, 1, 24, "bf16", "bf16"), (4097, 1, 24, "f32", "f16"), (2048, 2, 520, "bf16", "f32"),
+                                          (5000, 1, 24, "bf16", "bf16"), (5001, 1, 24, "f32", "f16"), (3450, 2, 24, "f32", "f32"), (3451, 2, 360, "bf16", "bf16"),
+                                          (4096, 1, 384, "bf16", "bf16"), (4097, 1, 192, "f32", "f16"), (2048, 2, 520, "bf16", "f32"),
                                           (8193, 1, 8, "f32", "bf16"), (700, 2, 512, "bf16", "f32"), (700, 2, 1024, "f32", "f32"), (300, 2, 4100, "bf16", "f16")])
 def test_decode_gradients_in_one_pass(pkg, S, k, M, dt, gdt):
     """moe_decode_grad against the two ops it stands for: rows bit for bit (the same products and roundings), weights within
-    1e-5 of sum|a_i * b_i| plus one rounding to the gate's type.  Sizes on both sides of the 4096 slots up to which the
+    1e-5 of sum|a_i * b_i| plus one rounding to the gate's type.  Sizes on both sides of the slots up to which the
     workgroups that clear unowned rows walk the slots themselves; rows of one wave, of several, and longer than a pass."""
     ops = pkg.ops
     E = 5
