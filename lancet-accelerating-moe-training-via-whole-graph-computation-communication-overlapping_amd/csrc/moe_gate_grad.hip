@@ -16,6 +16,7 @@
 #include "launchers.hpp"
 #include "select.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace lancet {
 
@@ -25,15 +26,20 @@ struct GateGradArgs {
   const int32_t* idx;    // [K*S] expert per slot after the drop (row 0 of indices_locations)
   void* out;             // [S,E]
   int S, E;
-  int is_logits;
-  int whole;             // rows of 16 bytes and more: walked in granules
-  int vec;               // both arrays are aligned to granules
 };
 
-// What bounds it is its length: two dependent round trips to memory and the exponentials of a row's lanes.  Rows that are not
-// whole granules used to be walked and written value by value, and every value decided by itself whether it is the largest so
-// far: 10007 x 60 bf16 top-2 logits 11.5 us, now 6.7; 30000 x 61 fp32 10.9 and 7.6, 65536 x 32 8.4 and 7.8, 65536 x 256 top-1 36.1
-// and 32.7, 4096 x 128 fp16 11.0 and 9.3.
+// How a workgroup writes its block of the result.
+enum GateGradBlock {
+  kValues = 0,      // value by value
+  kGranules = 1,    // in granules, which rows are whole ones of
+  kCutGranules = 2  // in granules that rows end inside of
+};
+
+// What bounds it is its length: two dependent round trips to memory, the exponentials of a row's lanes, and, in a kernel of 3 us,
+// the code itself: one kernel for logits and probabilities, and for every way to write a block, fetched more of it than it ran.
+// Rows that are not whole granules value by value / all rows in granules, one such kernel for both / now, us: 8192 x 60 bf16 top-2 logits 11.8 / 7.0 / 5.2, 8192 x 128 fp32 12.9 / 10.3 / 7.8,
+// 65536 x 128 bf16 probabilities top-1 7.2 / 7.7 / 6.7, 65536 x 256 fp32 top-1 logits 37.8 / 33.9 / 32.8, 8192 x 4 bf16 top-2 3.5 / 4.6 / 3.2,
+// 131072 x 10 bf16 top-2 8.4 / 12.3 / 8.0.  856 shapes of 500 to 131072 tokens and 2 to 512 experts: 0.82 of the first, 0.83 of the second.
 
 // A token's row is walked by kSub lanes, each taking every kSub-th 16-byte granule (or element), two at a time, with the
 // maximum and the sum of exponentials kept together and rescaled when a larger value comes; the lanes' pairs are then
@@ -41,6 +47,9 @@ struct GateGradArgs {
 // only gets up to the memory system's speed when many waves are in flight.
 constexpr int kSub = 4;                      // lanes per token
 constexpr int kGradTokens = kTile / kSub;    // tokens per workgroup
+// Rows of fewer granules than lanes are read value by value, so that all lanes have some, and as many at a time as the row has, each
+// of which costs an exponential: 131072 x 10 bf16 top-1 6.9 us, in granules 9.8; 131072 x 2 top-2 5.5, always four values 6.3.
+constexpr int kShortValues = 4;
 
 // Maximum and sum of exponentials of a row WITHOUT the entries that carry a slot gradient: with those the sum would
 // hide how far a selected probability is from 1 (1 - p = rest / sum loses every digit to rounding once the row is
@@ -48,13 +57,13 @@ constexpr int kGradTokens = kTile / kSub;    // tokens per workgroup
 // granules at a time, those left out as -inf, whose term is zero.
 struct MaxSum {
   float top = -INFINITY, sum = 0.f;
-  template <int N>
+  template <int N, bool FIRST = false>  // FIRST: nothing has been added before
   __device__ __forceinline__ void add(const float (&f)[N]) {
     float m = top;
 #pragma unroll
     for (int i = 0; i < N; ++i) m = fmaxf(m, f[i]);
     const float ref = m == -INFINITY ? 0.f : m;  // nothing but -inf so far: every term is zero
-    float s = sum * expf(top - ref);
+    float s = FIRST ? 0.f : sum * expf(top - ref);
 #pragma unroll
     for (int i = 0; i < N; ++i) s += expf(f[i] - ref);
     sum = s;
@@ -71,7 +80,7 @@ struct GateGradTile {
   float top[kGradTokens], inv[kGradTokens];  // logits: row maximum and 1 / sum_e exp(x - max)
 };
 
-template <int K, int GD>
+template <int K, int GD, bool LOGITS, int BLOCK>
 __global__ __launch_bounds__(kTile) void encode_dgate_kernel(GateGradArgs a) {
   __shared__ GateGradTile sh;
   constexpr size_t gb = GD == LANCET_F32 ? 4 : 2;
@@ -91,38 +100,53 @@ __global__ __launch_bounds__(kTile) void encode_dgate_kernel(GateGradArgs a) {
       if (x >= 0 && x < a.E) {
         e[j] = x;
         dy[j] = ld_gate(a.dy, static_cast<size_t>(j) * a.S + s, GD);
-        if (K == 2 || a.is_logits) raw[j] = gate_at<GD>(row, x);  // top-1 on probabilities needs no gate
+        if (K == 2 || LOGITS) raw[j] = gate_at<GD>(row, x);  // top-1 on probabilities needs no gate
       }
     }
     float top = 0.f, inv = 1.f, rest = 0.f;  // rest: sum of exponentials of the entries without a slot gradient
     float g[2] = {raw[0], raw[1]};           // the two kept probabilities (0 for a dropped slot)
-    if (a.is_logits) {
+    if (LOGITS) {
       MaxSum ms;
-      if (a.whole) {
-        // two granules in flight per lane, at any alignment; the last one of a row that ends inside it is drawn back, and the
-        // values it shares with the one before are left out
-        const int n = (a.E + V - 1) / V;
-        for (int g0 = sub; g0 < n; g0 += 2 * kSub) {
-          float f[2 * V];
-          u32x4 x[2];
-          int j0[2];
+      const int n = (a.E + V - 1) / V;  // granules of the row
+      if (n < kSub && a.E <= kSub * kShortValues) {
+        const auto values = [&](auto per_lane) {
+          float f[per_lane.value];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            j0[h] = min((g0 + h * kSub) * V, a.E - V);
-            x[h] = *reinterpret_cast<const u32x4_gate*>(row + j0[h] * static_cast<int>(gb));
+          for (int i = 0; i < per_lane.value; ++i) {
+            const int j = sub + i * kSub;
+            const float x = gate_at<GD>(row, min(j, a.E - 1));
+            f[i] = ((j < a.E) & (j != e[0]) & (j != e[1])) ? x : -INFINITY;
           }
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            each_value<GD>(x[h], [&](float val, int i) {
-              const int j = j0[h] + i;
-              f[h * V + i] = ((j >= (g0 + h * kSub) * V) & (j != e[0]) & (j != e[1])) ? val : -INFINITY;
-            });
-          ms.add(f);
-        }
+          ms.template add<per_lane.value, true>(f);
+        };
+        if (a.E <= kSub) values(std::integral_constant<int, 1>());
+        else if (a.E <= 2 * kSub) values(std::integral_constant<int, 2>());
+        else values(std::integral_constant<int, kShortValues>());
       } else {
-        for (int j = sub; j < a.E; j += kSub) {
-          const float f[1] = {((j != e[0]) & (j != e[1])) ? gate_at<GD>(row, j) : -INFINITY};
-          ms.add(f);
+        // granules at any alignment; the last one of a row that ends inside it is drawn back, and the values it shares with the one
+        // before are left out
+        const auto ask = [&](int g0, u32x4& x) { x = *reinterpret_cast<const u32x4_gate*>(row + min(g0 * V, a.E - V) * static_cast<int>(gb)); };
+        const auto take = [&](int g0, u32x4 x, float* f) {
+          const int j0 = min(g0 * V, a.E - V);
+          each_value<GD>(x, [&](float val, int i) {
+            const int j = j0 + i;
+            f[i] = ((j >= g0 * V) & (j != e[0]) & (j != e[1])) ? val : -INFINITY;
+          });
+        };
+        if (n <= kSub) {
+          float f[V];
+          u32x4 x;
+          ask(sub, x);
+          take(sub, x, f);
+          ms.template add<V, true>(f);
+        } else {
+          for (int g0 = sub; g0 < n; g0 += 2 * kSub) {  // two in flight per lane
+            float f[2 * V];
+            u32x4 x0, x1;
+            ask(g0, x0), ask(g0 + kSub, x1);
+            take(g0, x0, f), take(g0 + kSub, x1, f + V);
+            ms.add(f);
+          }
         }
       }
       // merge the kSub lanes' (max, sum) pairs: they are neighbours in the wave
@@ -166,7 +190,7 @@ __global__ __launch_bounds__(kTile) void encode_dgate_kernel(GateGradArgs a) {
       sh.i2[t] = e[1];
       sh.top[t] = top;
       sh.inv[t] = inv;
-      if (a.is_logits) {  // 1 - p_1 = rest + p_2 and 1 - p_2 = rest + p_1: sums of positive terms
+      if (LOGITS) {  // 1 - p_1 = rest + p_2 and 1 - p_2 = rest + p_1: sums of positive terms
         sh.c1[t] = d[0] * (rest + g[1]) - g[1] * d[1];
         sh.c2[t] = d[1] * (rest + g[0]) - g[0] * d[0];
         sh.rest[t] = -(g[0] * d[0] + g[1] * d[1]);
@@ -185,24 +209,23 @@ __global__ __launch_bounds__(kTile) void encode_dgate_kernel(GateGradArgs a) {
     float c = sh.rest[tk];
     if (ex == sh.i1[tk]) c = sh.c1[tk];
     if (K == 2 && ex == sh.i2[tk]) c = sh.c2[tk];
-    if (!a.is_logits) return c;
+    if (!LOGITS) return c;
     return expf(x - sh.top[tk]) * sh.inv[tk] * c;
   };
   const int n = ntok * a.E;
   const char* src = static_cast<const char*>(a.gate) + base * gb;
   char* dst = static_cast<char*>(a.out) + base * gb;
   int done = 0;
-  if (a.vec) {
+  if constexpr (BLOCK != kValues) {
     // (64 rows of any length are whole granules, so every workgroup's block starts on one)
     done = n / V * V;
-    const bool cut = a.E % V != 0;  // rows end inside granules
     for (int q = tid * V; q < done; q += kTile * V) {
       const int tk = q / a.E, ex = q - tk * a.E;
       u32x4 x = {0u, 0u, 0u, 0u}, r;
-      if (a.is_logits) x = *reinterpret_cast<const u32x4*>(src + q * gb);
+      if (LOGITS) x = *reinterpret_cast<const u32x4*>(src + q * gb);
       float v[V];
       each_value<GD>(x, [&](float val, int i) { v[i] = val; });
-      if (!cut) {
+      if constexpr (BLOCK == kGranules) {
 #pragma unroll
         for (int i = 0; i < V; ++i) v[i] = value(tk, ex + i, v[i]);
       } else {
@@ -232,10 +255,23 @@ __global__ __launch_bounds__(kTile) void encode_dgate_kernel(GateGradArgs a) {
   for (int q = done + tid; q < n; q += kTile) {
     const int tk = q / a.E;
     const int ex = q - tk * a.E;
-    const float x = a.is_logits ? ld_gate(a.gate, base + q, GD) : 0.f;
+    const float x = LOGITS ? ld_gate(a.gate, base + q, GD) : 0.f;
     st_gate(a.out, base + q, value(tk, ex, x), GD);
   }
 }
+
+template <int K, int GD, bool LOGITS>
+static void dgate_launch(const GateGradArgs& a, int block, hipStream_t st) {
+  const int blocks = (a.S + kGradTokens - 1) / kGradTokens;
+  if (block == kGranules) encode_dgate_kernel<K, GD, LOGITS, kGranules><<<blocks, kTile, 0, st>>>(a);
+  else if (block == kCutGranules) encode_dgate_kernel<K, GD, LOGITS, kCutGranules><<<blocks, kTile, 0, st>>>(a);
+  else encode_dgate_kernel<K, GD, LOGITS, kValues><<<blocks, kTile, 0, st>>>(a);
+}
+
+// Rows that end inside granules are written in granules from this length on (bytes): below, few threads have one, each with a chain
+// of lookups.  Values / granules, us, 131072 top-2 on logits: 10 bf16 8.2 / 8.7, 12 bf16 8.4 / 8.8, 5 fp32 6.7 / 6.9; 14 fp32 9.7 / 9.4, and of 500
+// tokens 3.6 / 3.3, 28 bf16 5.4 / 4.3.
+constexpr int kCutRowBytes = 48;
 
 hipError_t run_encode_dgate(const void* dy, const void* gate, const int32_t* idx, int S, int E, int K, bool is_logits,
                             int gate_dtype, void* out, hipStream_t st) {
@@ -247,14 +283,18 @@ hipError_t run_encode_dgate(const void* dy, const void* gate, const int32_t* idx
   a.out = out;
   a.S = S;
   a.E = E;
-  a.is_logits = is_logits;
   const int gb = gate_dtype == LANCET_F32 ? 4 : 2;
-  a.whole = E * gb >= 16;
-  a.vec = ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-  const int blocks = (S + kGradTokens - 1) / kGradTokens;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+  const bool whole_rows = static_cast<size_t>(E) * gb % 16 == 0;
+  const int block = !aligned ? kValues : whole_rows ? kGranules : E * gb >= kCutRowBytes ? kCutGranules : kValues;
   LANCET_GATE_SWITCH(gate_dtype,
-    if (K == 1) encode_dgate_kernel<1, GD><<<blocks, kTile, 0, st>>>(a);
-    else encode_dgate_kernel<2, GD><<<blocks, kTile, 0, st>>>(a))
+    if (K == 1) {
+      if (is_logits) dgate_launch<1, GD, true>(a, block, st);
+      else dgate_launch<1, GD, false>(a, block, st);
+    } else {
+      if (is_logits) dgate_launch<2, GD, true>(a, block, st);
+      else dgate_launch<2, GD, false>(a, block, st);
+    })
   return hipGetLastError();
 }
 

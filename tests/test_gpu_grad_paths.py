@@ -40,6 +40,36 @@ def test_gate_gradient_of_rows_of_any_length(pkg, S, E, k, gdt, offset):
     assert (np.abs(got - want) <= eps * np.abs(want) + 1e-6 * scale + tiny).all()
 
 
+# one, two and four values per lane; one granule per lane, and the first rows with two; blocks written by value and in granules
+@pytest.mark.parametrize("S,E", [(64, 3), (65, 4), (129, 5), (64, 8), (70, 12), (63, 14), (64, 16), (66, 17), (257, 24), (65, 32), (64, 33)])
+@pytest.mark.parametrize("k", [1, 2])
+@pytest.mark.parametrize("gdt,offset", [("f32", 0), ("bf16", 0), ("f16", 3)])
+def test_gate_gradient_of_short_rows(pkg, S, E, k, gdt, offset):
+    test_gate_gradient_of_rows_of_any_length(pkg, S, E, k, gdt, offset)
+    # on probabilities, and on logits of which some are masked out: those get no gradient, the others what the oracle says
+    tdt = TORCH_DT[gdt]
+    logits = make_inputs(E, S, 4, E)[1]
+    masked = logits.copy()
+    masked[::3, ::2] = -np.inf
+    for gate, is_logits in ((np.exp(logits) / np.exp(logits).sum(axis=1, keepdims=True), False), (masked, True)):
+        gate = dev(gate.astype(np.float32)).to(tdt)
+        rounded = gate.float().cpu().numpy()
+        il = np.zeros((2, k * S), np.int32)
+        il[0] = np.argsort(-rounded, axis=1, kind="stable")[:, :k].T.reshape(-1)
+        il[0][::7] = -1
+        if is_logits:                              # a masked expert is nobody's choice
+            chosen = rounded[np.tile(np.arange(S), k), il[0]]
+            il[0][np.isinf(chosen)] = -1
+        dy = dev(np.random.default_rng(S).standard_normal(k * S).astype(np.float32)).to(tdt)
+        want = mo.moe_encode_dgate(dy.float().cpu().numpy(), rounded, il, k, is_logits)
+        out = _off(torch.full((S, E), 7.0, dtype=tdt, device="cuda"), offset)
+        got = to_np(pkg.ops.moe_encode_dgate(dy, _off(gate, offset), dev(il), top_k=k, gate_is_logits=is_logits, out=out)).astype(np.float64)
+        scale = np.abs(want).max(axis=1, keepdims=True)
+        eps = {"f32": 1e-5, "bf16": 2.0 ** -7, "f16": 2.0 ** -10}[gdt]
+        tiny = {"f32": 1e-30, "bf16": 1e-30, "f16": 2.0 ** -24}[gdt]
+        assert np.isfinite(got).all() and (np.abs(got - want) <= eps * np.abs(want) + 1e-6 * scale + tiny).all()
+
+
 @pytest.mark.parametrize("k", [1, 2])
 @pytest.mark.parametrize("fill", ["zeros", "ones", "last", "others", "large"])
 def test_row_map_in_memory_that_holds_anything(pkg, k, fill):
