@@ -1223,8 +1223,10 @@ __device__ __forceinline__ void small_step(const LansTables& t, const LansScalar
 // (In a launch of their own behind the resident kernel the sums took 11 us of a step of 60M parameters of which a table of 20M
 // is swept, 398 us, now 391; here they fill a chip that the small tensors' dependent round trips leave idle.  40M fp32 parameters
 // by sweeps 329 / 322.  Of many chunks the sweep is as fast as the memory only with more waves than this kernel's registers
-// allow: 60M in one tensor 508 in a launch of their own against 515, 400M in 16 tensors 3237 / 3254.)
-constexpr int kEarlyNorms = 6144;
+// allow: 60M in one tensor 508 in a launch of their own against 515, 400M in 16 tensors 3237 / 3254; and where there are no small
+// tensors to hide behind, from fewer on: 44M alone 373 / 375, 48M 411 / 416, 48M beside 8M resident 475 / 478, but 40M 342 / 342 and
+// 33M 283 / 281; with 40 small tensors 44M 382 / 376, 48M 422 / 421.)
+constexpr int kEarlyNorms = 6144, kEarlyNormsAlone = 5120;
 constexpr int kNormChunks = kSmallThreads / kLansThreads;
 template <int GT, int PL>
 __global__ __launch_bounds__(kSmallThreads) void lans_begin_kernel(LansTables t, LansScalars sc, size_t nwords, int small_base,
@@ -1709,7 +1711,8 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
   const int sweep_tensor = resident ? pl->big_first : 0, sweep_slot = resident ? pl->big_slot : 0;
   const int sweep_tensor_end = ragged ? pl->ragged_first : pl->small_first, sweep_slot_end = ragged ? pl->ragged_slot : pl->small_slot;
   const int nsweep = sweep_slot_end - sweep_slot, rest = sweep_tensor_end - sweep_tensor;
-  const int norm_blocks = grad_norms || nsweep <= 0 || nsweep > kEarlyNorms ? 0 : (nsweep + kNormChunks - 1) / kNormChunks;
+  const bool early = nsweep <= (pl->small_first < T ? kEarlyNorms : kEarlyNormsAlone);
+  const int norm_blocks = grad_norms || nsweep <= 0 || !early ? 0 : (nsweep + kNormChunks - 1) / kNormChunks;
   LANS_TYPE_SWITCH(g_dtype, plt, (lans_begin_kernel<GT, PL><<<1 + (T - pl->small_first) + norm_blocks, kSmallThreads, 0, st>>>(
                                      t, sc, pl->words_bytes / sizeof(uint64_t), pl->small_first, sweep_slot, sweep_slot_end)))
   if (t.nres > 0) {
@@ -1717,7 +1720,7 @@ int lans_step_impl(lancet_lans_plan_t pl, const void* const* g, int g_dtype, flo
     LANS_TYPE_SWITCH(g_dtype, plt, (lans_resident_kernel<GT, PL><<<grid, kLansThreads, 0, st>>>(t, sc)))
   }
   if (nsweep > 0) {
-    if (!grad_norms && nsweep > kEarlyNorms)
+    if (!grad_norms && !early)
       LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_norm_g_kernel<GT><<<nsweep, kLansThreads, 0, st>>>(t, sweep_slot)))
     if (!grad_norms) lans_reduce_kernel<<<dim3(rest, 1), kReduceThreads, 0, st>>>(t, 0, sweep_tensor, 1);
     LANS_TYPE_SWITCH(g_dtype, kNoLowp, (lans_moments_kernel<GT><<<nsweep * kSweepSplit, kLansThreads, 0, st>>>(t, sc, sweep_slot)))
