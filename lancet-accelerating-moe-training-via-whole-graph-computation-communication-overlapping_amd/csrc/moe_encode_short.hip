@@ -312,16 +312,21 @@ __global__ __launch_bounds__(kTile) void encode_place_rows_kernel(EncodeArgs a) 
 //   16.8 / 12.9; but 128 tokens, 256 experts 22.6 / 24.8 and 256 tokens, 512 experts 43 / 90.
 //   A few tiles: a workgroup adds up the counts of all tiles, so there must be few; and what the saved launch gives is lost again
 //   where long rows go to two places, which many short workgroups do better.  Buffers that no cache holds, 8 experts: top-1
-//   2000 x 1024 9.4 / 7.5, 8192 x 1024 14.6 / 11.7, 8192 x 2048 22.4 / 19.9, 8192 x 4096 34.6 / 34.2; top-2 4096 x 512 10.6 / 10.0,
-//   6000 x 1024 14.9 / 13.7, 4096 x 2048 17.5 / 19.4, 8192 x 4096 48.4 / 52.0.  64 tiles, top-1: x 256 10.1 / 9.5, x 512 13.3 / 13.6,
-//   x 2048 34.0 / 33.7; 128 tiles x 256 14.0 / 14.5.
+//   2000 x 1024 9.4 / 7.5, 8192 x 1024 14.6 / 11.7, 8192 x 2048 22.4 / 19.9; top-2 4096 x 512 10.6 / 10.0, 4096 x 2048 17.5 / 19.4, 8192 x
+//   4096 48.4 / 52.0.  64 tiles, top-1: x 256 10.1 / 9.5, x 512 13.3 / 13.6, x 2048 34.0 / 33.7; 128 tiles x 256 14.0 / 14.5.
+//   Long top-1 rows: 40 MB of 8192 bytes 23.6 / 24.6, 50 MB 26.6 / 27.9, 62 MB 30.6 / 34; with 64 experts, whose separate routing takes
+//   longer, 28.2 / 26.5, 34.7 / 34.2 and 35.2 / 36.0.
 constexpr int64_t kTileGate = 16384, kTileExperts = 128;
 constexpr int64_t kShortTiles = 32, kShortCounts = 4096;
-constexpr size_t kShortRows1 = 64u << 20, kShortRows2 = 12u << 20;  // bytes of token rows, top-1 and top-2
-// Workgroups that move rows: each takes twice the tokens while there are more than this.  Top-1, 512 / 768 / 1024 / 1536: 8192 x 1024
-// 13.8 / 13.8 / 11.7 / 11.7 us, 6000 x 1024 12.6 / 10.9 / 10.9 / 9.7 (separate kernels 12.8), 4096 x 4096 20.5 / 20.4 / 20.1 / 20.1; top-2
-// 8192 x 512 12.4 / 12.4 / 13.6 / 13.6, 6000 x 1024 16.6 / 13.7 / 13.7 / 15.1.
-constexpr int kShortBlocks1 = 1536, kShortBlocks2 = 768;
+constexpr size_t kShortRows2 = 12u << 20;  // bytes of token rows, top-2
+static size_t short_rows1(int64_t E) { return static_cast<size_t>(E >= 32 ? 52 : 36) << 20; }  // ... top-1
+// Workgroups that move rows: each takes twice the tokens while there are more than this.  Best are 1000 to 1700, and half of what just
+// exceeds the limit is the worst case.  Arrays that no cache holds, tokens x bytes, us by workgroups (separate kernels): top-2 6510 x
+// 1536 407 17.4, 814 14.9, 1628 14.5 (15.0); 3255 x 3072 407 18.1, 814 15.6, 1628 13.7 (15.1); 7812 x 1536 488 18.5, 977 15.8, 1953 17.4 (16.0);
+// 2000 x 6000 500 18.8, 1000 16.9, 2000 17.5 (16.6); 1220 x 8192 610 15.0, 1220 13.0 (14.9); 5859 x 2048 732 15.4, 1465 15.5 (15.7); top-1 6666 x
+// 6000 834 28.5, 1667 25.0 (24.4); 3333 x 6000 834 17.2, 1667 14.5, 3333 15.6 (17.1); 6510 x 3072 814 16.2, 1628 14.8, 3255 16.1 (16.6); 3662 x 8192
+// 916 20.4, 1831 19.4, 3662 20.0 (19.4); 4882 x 4096 1221 14.0, 2441 15.3 (15.8).
+constexpr int kShortBlocks1 = 2000, kShortBlocks2 = 1700;
 // Tails.  A turn clears 32 KB, 16 rows at least.  Of one tile, every workgroup that clears has to route the tile first, so there
 // are only as many as the movers leave CUs idle, each with several turns; a second one on a CU costs the routing again (256 x
 // 1024 top-2, 128 experts, capacity 20: 10.9 us with 192 of them beside 64 movers, 15.9 with 256), and one per 16 rows, as many as
@@ -342,7 +347,7 @@ bool encode_is_short(const int32_t* used_in, const int32_t* used_out, int64_t S,
   if (force_lookback || S < 1 || row_bytes == 0 || (used_in != nullptr && used_in == used_out)) return false;
   if (S <= kTile) return S * E <= kTileGate || E <= kTileExperts;
   const int64_t tiles = scan_num_tiles(S);
-  return tiles <= kShortTiles && tiles * K * E <= kShortCounts && static_cast<size_t>(S) * row_bytes <= (K == 1 ? kShortRows1 : kShortRows2);
+  return tiles <= kShortTiles && tiles * K * E <= kShortCounts && static_cast<size_t>(S) * row_bytes <= (K == 1 ? short_rows1(E) : kShortRows2);
 }
 
 hipError_t run_encode_short(const void* data, const void* gate, const void* noise, const int32_t* used_in, int S, int E, int C, int M,

@@ -50,6 +50,14 @@ def test_short_encodes_are_what_the_separate_kernels_give(pkg, S, M, E, k):
         np.testing.assert_allclose(to_np(got[0]), ref[0], rtol=1e-5)
 
 
+# one and two tokens more than workgroups there may be, of one and of two tokens; rows of either side of the limits of 36 MB (below 32
+# experts) and 12 MB
+@pytest.mark.parametrize("S,M,E", [(1701, 1500, 6), (3402, 772, 5), (2001, 1540, 3), (2305, 4096, 31), (2305, 4096, 32)])
+@pytest.mark.parametrize("k", [1, 2])
+def test_short_encodes_at_the_limits_of_their_rule(pkg, S, M, E, k):
+    test_short_encodes_are_what_the_separate_kernels_give(pkg, S, M, E, k)
+
+
 def test_used_capacity_updated_in_place(pkg):
     """used_capacity as input and output of one call (rows that feed moe_redispatch): the separate kernels take it, as before."""
     ops = pkg.ops
