@@ -83,9 +83,11 @@ extern "C" {
  * indices_locations are unchanged (locations stay relative to the call, as moe_merge_masks expects). */
 #define LANCET_ROWS_AT_USED 8u
 /* lancet_moe_encode / lancet_moe_route / lancet_moe_encode_bpr: run the position scan as ONE kernel with a
- * decoupled look-back between its tiles, whatever the size.  By default only top-1 calls of at most 8192 tokens
- * do; everything else is faster as two or three kernels in which no workgroup waits for another.  For callers
- * that want the fewest launches, and for tests of the look-back's bounded waits. */
+ * decoupled look-back between its tiles, whatever the size.  By default only lancet_moe_route of top-1 on at most
+ * 8192 tokens does (and lancet_moe_encode where its short form, which routes and moves the rows in one or two
+ * kernels without a look-back, does not serve such a call); everything else is faster as two or three kernels in which
+ * no workgroup waits for another.  For callers that want the fewest routing launches, and for tests of the look-back's
+ * bounded waits. */
 #define LANCET_SCAN_LOOKBACK 16u
 
 typedef void* lancet_stream_t;
@@ -465,7 +467,10 @@ int lancet_lans_plan_norms(lancet_lans_plan_t plan, float* norms4xT, lancet_stre
  * (8192 tokens), and calls with LANCET_SCAN_LOOKBACK, run as one kernel with a look-back between tiles, to which
  * everything said here about state and waits applies.  All others run as two kernels (three on long batches: tiles
  * x counters above 32768) in which no workgroup waits for another: they use the workspace as plain scratch (no
- * state, no wait that could give up, and memory that was never set up works as well).
+ * state, no wait that could give up, and memory that was never set up works as well).  lancet_moe_encode of up to 8192
+ * tokens mostly runs as one or two kernels of its own without a look-back; top-1, which by the rule above is a look-back,
+ * they still ask for a workspace that is set up and mark their outputs where it is not, so that the answer does not
+ * depend on which of the two forms served the call.
  * Every wait inside the scan is bounded.  A wait that gives up sets the workspace's sticky error word, and
  * every token whose position was built on it gets indices = locations = -1 (gates_s 0 for top_k = 2), as if
  * dropped, so that no consumer moves a row on a wrong position; when the totals themselves were built on it,
@@ -476,8 +481,8 @@ int lancet_lans_plan_norms(lancet_lans_plan_t plan, float* norms4xT, lancet_stre
 int lancet_scan_workspace_init(void* workspace, size_t workspace_bytes, lancet_stream_t stream);
 int lancet_scan_workspace_error(void* workspace, lancet_stream_t stream, int* error_out);
 /* 1 when a call of these sizes and flags (batch_prioritized != 0: lancet_moe_encode_bpr, S = S0 / n_partitions; else
- * lancet_moe_encode / lancet_moe_route) runs the scan in its look-back form, the only form that reads state from
- * the workspace: such a call needs the first lancet_moe_encode_workspace_bytes(S, E, top_k or 2) bytes of its
+ * lancet_moe_encode / lancet_moe_route) is one of the look-back form, the only form that reads state from
+ * the workspace (or a short top-1 encode in its place, which checks that it is set up): such a call needs the first lancet_moe_encode_workspace_bytes(S, E, top_k or 2) bytes of its
  * workspace set up and can give up a wait; 0: it uses the whole workspace as plain scratch, which needs neither
  * set-up nor a look at the error word.  For executors that hand an operator fresh workspace memory before every
  * call (src/impl/vm/vm.cc:1260-1266) and would otherwise pay a set-up launch each time. */

@@ -32,7 +32,8 @@ hipError_t run_route_scan(const void* gate, const void* noise, const int32_t* id
                           int32_t* idx_out, int32_t* loc_out, int32_t* used_out,
                           uint64_t* elems_out, void* ws, hipStream_t st, bool force_lookback = false);
 // The whole of an encode (routing and row movement) in one or two launches, where encode_is_short says so; the arguments are
-// those of run_route_scan and run_scatter_rows.  needs_setup: the workspace has to be set up (as the look-back form wants it).
+// those of run_route_scan and run_scatter_rows.  Where the look-back form would serve the routing alone, the workspace has to be set
+// up for these kernels too, which mark their outputs otherwise.
 bool encode_is_short(const int32_t* used_in, const int32_t* used_out, int64_t S, int64_t E, int K, size_t row_bytes, bool force_lookback);
 hipError_t run_encode_short(const void* data, const void* gate, const void* noise, const int32_t* used_in, int S, int E, int C, int M,
                             int K, bool is_logits, int elem_bytes, int gate_dtype, bool tail, bool rows_at_used, void* gates_s,

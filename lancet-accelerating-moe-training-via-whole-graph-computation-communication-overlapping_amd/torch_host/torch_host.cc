@@ -19,7 +19,6 @@
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
-#include <ATen/ops/empty_like.h>
 #include <ATen/ops/zeros.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/DynamicTypes.h>
